@@ -15,6 +15,8 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libgpukern.so")
 
 SOURCES = ["gk_basic.hip", "gk_fft.hip", "gk_fft_any.hip", "conv.hip", "rk.hip", "sim.hip", "batch.hip", "io.cpp"]
+# kernels with many length instantiations, compiled in parts (-DGK_PART=i): they set the build's time
+PARTS = {"conv_z.hip": 5, "batch_z.hip": 5, "batch_any.hip": 4}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -27,9 +29,12 @@ FLAGS = [
 ]
 
 
-def _compile(src):
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+def _compile(job):
+    src, part = job
+    name = os.path.splitext(src)[0] + ("" if part is None else "_%d" % part)
+    obj = os.path.join(BUILD, name + ".o")
+    defs = [] if part is None else ["-DGK_PART=%d" % part]
+    cmd = [HIPCC, *FLAGS, *defs, "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     msgs = [l for l in (r.stdout + r.stderr).splitlines() if "packed-fp32" not in l and "warning: feature" not in l]
     if r.returncode != 0:
@@ -39,8 +44,9 @@ def _compile(src):
 
 def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 4)) as ex:
-        objs = list(ex.map(_compile, SOURCES))
+    jobs = [(src, i) for src, n in PARTS.items() for i in range(n)] + [(src, None) for src in SOURCES]
+    with ThreadPoolExecutor(max_workers=min(len(jobs), os.cpu_count() or 4)) as ex:
+        objs = list(ex.map(_compile, jobs))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)

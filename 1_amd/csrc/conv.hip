@@ -36,6 +36,7 @@
 #include "engine.h"
 #include "fft_device.h"
 #include "gk_fft.h"
+#include "conv_z.h"
 #include "passes.h"
 
 namespace gk {
@@ -732,45 +733,6 @@ double conv_build_kernel(ConvPlan& cp, const KernelSpec& ks, float* full_host, f
 // =============================================================== launchers
 
 
-// rows per Z block: enough consecutive y for 64-128 B transposed segments, at most 1024 threads
-template <int M> constexpr int z_rows() {
-    constexpr int G = RegFFT<M>::G;
-    int tr = 1024 / G;
-    if (tr > 16) tr = 16;
-    while (tr > 1 && tr * (M + 1) * 8 > 72 * 1024) tr /= 2;
-    return tr;
-}
-
-// rows per Z forward block of shape variant v: 0 the default, 1 half of it, 2
-// double (while the block stays within 1024 threads and 80 KB of LDS).  Short
-// rows (M < 32) have one shape; a variant that does not exist gives the default.
-template <int M> constexpr int z_rows_v(int v) {
-    constexpr int d = z_rows<M>();
-    if (M < 32) return d;
-    if (v == 1) return d > 1 ? d / 2 : d;
-    if (v == 2) {
-        const int t = 2 * d;
-        const int fft = t * RegFFT<M>::LDS, tile = (M + 1) * (t + 1);
-        return (t * RegFFT<M>::G <= 1024 && (fft > tile ? fft : tile) * 8 <= 80 * 1024) ? t : d;
-    }
-    return d;
-}
-
-template <int M, int TR>
-static void zfwd_launch(const ConvPlan& cp, const StageIn& si, int NKp, const float2* twM, const float2* twP,
-                        hipStream_t s) {
-    const int Nx = cp.N[0], Ny = cp.N[1], Nz = cp.N[2];
-    const dim3 g(div_up(Ny, TR), Nx, 3);
-    constexpr int nt = TR * RegFFT<M>::G;
-    switch (NKp) {
-    case 0: k_zfwd<M, TR, 0><<<g, nt, 0, s>>>(si, cp.B1, twM, twP, Nx, Ny, Nz); break;
-    case 1: k_zfwd<M, TR, 1><<<g, nt, 0, s>>>(si, cp.B1, twM, twP, Nx, Ny, Nz); break;
-    case 2: k_zfwd<M, TR, 2><<<g, nt, 0, s>>>(si, cp.B1, twM, twP, Nx, Ny, Nz); break;
-    case 3: k_zfwd<M, TR, 3><<<g, nt, 0, s>>>(si, cp.B1, twM, twP, Nx, Ny, Nz); break;
-    default: k_zfwd<M, TR, 5><<<g, nt, 0, s>>>(si, cp.B1, twM, twP, Nx, Ny, Nz); break;
-    }
-}
-
 static void launch_zfwd(const ConvPlan& cp, const StageIn& in, hipStream_t s) {
     const int M = cp.M;
     const float2* twM = twiddle_f32(M);
@@ -787,9 +749,7 @@ static void launch_zfwd(const ConvPlan& cp, const StageIn& in, hipStream_t s) {
     switch (M) {
 #define GK_CASE(n)                                                                               \
     case n:                                                                                      \
-        if (cp.tp.zr == 1) zfwd_launch<n, z_rows_v<n>(1)>(cp, si, NKp, twM, twP, s);             \
-        else if (cp.tp.zr == 2) zfwd_launch<n, z_rows_v<n>(2)>(cp, si, NKp, twM, twP, s);        \
-        else zfwd_launch<n, z_rows_v<n>(0)>(cp, si, NKp, twM, twP, s);                           \
+        zfwd_run<n>(cp, si, NKp, twM, twP, s);                                                   \
         break;
         GK_LEN_M(GK_CASE)
 #undef GK_CASE
@@ -811,41 +771,17 @@ bool conv_zr_valid(int M, int v) {
 }
 
 static void launch_zinv(const ConvPlan& cp, float* h, const EngineState* st, hipStream_t s) {
-    const int M = cp.M, Nx = cp.N[0], Ny = cp.N[1], Nz = cp.N[2];
+    const int M = cp.M;
     const float2* twM = twiddle_f32(M);
     const float2* twP = twiddle_f32(cp.P[2]);
     switch (M) {
 #define GK_CASE(n)                                                                              \
-    case n: {                                                                                   \
-        constexpr int TR = z_rows<n>();                                                         \
-        dim3 g(div_up(Ny, TR), Nx, 3);                                                          \
-        k_zinv<n, TR><<<g, TR * RegFFT<n>::G, 0, s>>>(cp.B1, h, twM, twP, st, Nx, Ny, Nz);      \
-        break;                                                                                  \
-    }
+    case n: zinv_run<n>(cp, h, st, twM, twP, s); break;
         GK_LEN_M(GK_CASE)
 #undef GK_CASE
     default: abort();
     }
     GK_LAUNCH_CHECK();
-}
-
-// rows per block of the fused Z inverse: 3 x TR lane groups <= 1024 threads, its
-// LDS (transposed tiles, FFT exchange buffers) within 80 KB (two blocks per CU)
-template <int M> constexpr int epi_rows() {
-    constexpr int G = RegFFT<M>::G;
-    int tr = 1024 / (3 * G);
-    if (tr > 16) tr = 16;
-    int p = 1;
-    while (p * 2 <= tr) p *= 2;
-    tr = p;
-    while (tr > 1 && zinv_epi_lds_elems(M, tr) * 8 > 80 * 1024) tr /= 2;
-    return tr;
-}
-
-// rows per fused Z inverse block of shape variant v: 0 the default, 1 half of it
-template <int M> constexpr int epi_rows_v(int v) {
-    constexpr int d = epi_rows<M>();
-    return (v == 1 && M >= 32 && d > 1) ? d / 2 : d;
 }
 
 int conv_epi_rows(int M, int v) {
@@ -861,25 +797,6 @@ int conv_epi_rows(int M, int v) {
 bool conv_er_valid(int M, int v) { return v == 0 || (v == 1 && conv_epi_rows(M, 1) != conv_epi_rows(M, 0)); }
 
 int conv_epi_blocks(const ConvPlan& cp) { return div_up(cp.N[1], conv_epi_rows(cp.M, cp.tp.er)) * cp.N[0]; }
-
-template <int M, int TR>
-static void zinv_epi_launch(const ConvPlan& cp, const EpiArgs& e, const EngineState* st, const float2* twM,
-                            const float2* twP, hipStream_t s) {
-    const int Nx = cp.N[0], Ny = cp.N[1], Nz = cp.N[2], nu = e.nu;
-    const dim3 g(div_up(Ny, TR), Nx), b(3 * TR * RegFFT<M>::G);
-    if (e.fin == 1) {
-        if (nu <= 1) k_zinv_epi<M, TR, 1, 1><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
-        else k_zinv_epi<M, TR, 3, 1><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
-    } else if (e.fin == 2) {
-        if (nu <= 3) k_zinv_epi<M, TR, 3, 2><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
-        else k_zinv_epi<M, TR, 6, 2><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
-    } else {
-        if (nu == 0) k_zinv_epi<M, TR, 0, 0><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
-        else if (nu == 1) k_zinv_epi<M, TR, 1, 0><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
-        else if (nu <= 3) k_zinv_epi<M, TR, 3, 0><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
-        else k_zinv_epi<M, TR, 6, 0><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
-    }
-}
 
 static void launch_zinv_epi(const ConvPlan& cp, const EpiArgs& ea, const EngineState* st, hipStream_t s) {
     const int M = cp.M;
@@ -900,8 +817,7 @@ static void launch_zinv_epi(const ConvPlan& cp, const EpiArgs& ea, const EngineS
     switch (M) {
 #define GK_CASE(n)                                                                               \
     case n:                                                                                      \
-        if (cp.tp.er == 1) zinv_epi_launch<n, epi_rows_v<n>(1)>(cp, e, st, twM, twP, s);         \
-        else zinv_epi_launch<n, epi_rows_v<n>(0)>(cp, e, st, twM, twP, s);                       \
+        zinv_epi_run<n>(cp, e, st, twM, twP, s);                                                 \
         break;
         GK_LEN_M(GK_CASE)
 #undef GK_CASE

@@ -13,6 +13,13 @@
 #define GK_LEN_M(X)                                                                                              \
     X(1) X(2) X(3) X(4) X(6) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512) \
         X(768) X(1024) X(1536) X(2048)
+// the same list in parts: the Z kernels are compiled one part per translation
+// unit (conv_z.hip, batch_z.hip; build.py), since they are most of the build time
+#define GK_LEN_M_PART0(X) X(1) X(2) X(3) X(4) X(6) X(8) X(12) X(16) X(24) X(32)
+#define GK_LEN_M_PART1(X) X(48) X(64) X(96) X(128)
+#define GK_LEN_M_PART2(X) X(192) X(256) X(384) X(512)
+#define GK_LEN_M_PART3(X) X(768) X(1024)
+#define GK_LEN_M_PART4(X) X(1536) X(2048)
 #define GK_LEN_Y(X)                                                                                              \
     X(2) X(4) X(6) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768)    \
         X(1024) X(1536) X(2048) X(3072) X(4096)
