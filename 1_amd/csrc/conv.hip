@@ -42,7 +42,7 @@
 namespace gk {
 
 // =============================================================== kernel setup
-__constant__ int c_kern_idx[3][3] = {{0, 5, 4}, {5, 1, 3}, {4, 3, 2}};  // xx yy zz yz xz xy
+// kernel components in the order xx yy zz yz xz xy
 
 // faceIntegral (demag.go:142-183) in FP64
 __device__ void face_integral_f64(double B[3], const double R[3], const double cell[3], int s, int n) {
@@ -62,8 +62,8 @@ __device__ void face_integral_f64(double B[3], const double R[3], const double c
                 pos[w] = pw;
                 const double d0 = R[0] - pos[0], d1 = R[1] - pos[1], d2 = R[2] - pos[2];
                 const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-                const double r = sqrt(r2);
-                const double q = (pole == 0 ? charge : -charge) * inv4pi / (r2 * r);
+                const double ir = rsqrt(r2);
+                const double q = (pole == 0 ? charge : -charge) * inv4pi * (ir * ir * ir);
                 B[0] += d0 * q;
                 B[1] += d1 * q;
                 B[2] += d2 * q;
@@ -136,30 +136,68 @@ struct KernelImages {
     int period[3], images[3];
 };
 
-__global__ void k_facekernel6(double* __restrict__ K, int P0, int P1, int P2, double c0, double c1, double c2,
-                              int acc, KernelImages im) {
-    const long NP = (long)P0 * P1 * P2;
+// Value v of component k at index idx of a real-space kernel array: a double,
+// or (CPLX) the complex number (v, 0) that the spectrum's transform starts from.
+template <bool CPLX> __device__ __forceinline__ void kern_put(double* __restrict__ K, long i, double v) {
+    if constexpr (CPLX) reinterpret_cast<double2*>(K)[i] = make_double2(v, 0.0);
+    else K[i] = v;
+}
+
+// The kernel is even or odd along each axis whose displacement range is
+// symmetric (even padded length, and an even period where the axis is
+// periodic), so only the indices 0..P/2 of such an axis are evaluated (H of them;
+// H = P where an axis has no such symmetry) and each value is written to all
+// its mirror images with the component's sign: xx, yy, zz even; yz odd in y and
+// z, xz in x and z, xy in x and y.  An evaluation costs 6 acc^2 inverse cubes of
+// distances in FP64 against 48 B of stores per index, so the kernel is bound by
+// FP64 arithmetic, and the octant takes an eighth of it.  Source faces along
+// axis s = blockIdx.y give the components (s, d >= s), so each axis has threads
+// of its own: small kernels fill the chip and each has a shorter serial chain.
+// Padded 16 x 256 x 256, acc 8: every index 626 us, the octant 156 us, one axis
+// per thread and the inverse cube from rsqrt 52 us.
+template <bool CPLX>
+__global__ void k_facekernel6(double* __restrict__ K, int P0, int P1, int P2, int H0, int H1, int H2, double c0,
+                              double c1, double c2, int acc, KernelImages im) {
+    const long NP = (long)P0 * P1 * P2, NH = (long)H0 * H1 * H2;
     const double cell[3] = {c0, c1, c2};
-    for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < NP; idx += (long)gridDim.x * blockDim.x) {
-        const int zw = (int)(idx % P2);
-        const long r = idx / P2;
-        const int yw = (int)(r % P1), xw = (int)(r / P1);
+    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < NH; t += (long)gridDim.x * blockDim.x) {
+        const int zw = (int)(t % H2);
+        const long r = t / H2;
+        const int yw = (int)(r % H1), xw = (int)(r / H1);
         const AxisImages ax = axis_images(xw, P0, im.period[0], im.images[0], true);
         const AxisImages ay = axis_images(yw, P1, im.period[1], im.images[1], false);
         const AxisImages az = axis_images(zw, P2, im.period[2], im.images[2], false);
-        double kk[6] = {0, 0, 0, 0, 0, 0};
+        const int f = blockIdx.y;
+        double kk[3] = {0, 0, 0};  // B[d] of the faces along f
         for (int i = 0; i < ax.count; i++)
             for (int j = 0; j < ay.count; j++)
                 for (int l = 0; l < az.count; l++) {
                     const double R[3] = {(ax.first + i * ax.step) * c0, (ay.first + j * ay.step) * c1,
                                          (az.first + l * az.step) * c2};
-                    for (int s = 0; s < 3; s++) {
-                        double B[3];
-                        face_integral_f64(B, R, cell, s, acc);
-                        for (int d = s; d < 3; d++) kk[c_kern_idx[s][d]] += B[d];
-                    }
+                    double B[3];
+                    if (f == 0) face_integral_f64(B, R, cell, 0, acc);
+                    else if (f == 1) face_integral_f64(B, R, cell, 1, acc);
+                    else face_integral_f64(B, R, cell, 2, acc);
+                    for (int d = 0; d < 3; d++) kk[d] += B[d];
                 }
-        for (int k = 0; k < 6; k++) K[k * NP + idx] = kk[k];
+        // mirror images; an axis that is not mirrored, index 0 and index P/2 have none
+        const bool mx = H0 < P0 && xw > 0 && 2 * xw != P0, my = H1 < P1 && yw > 0 && 2 * yw != P1;
+        const bool mz = H2 < P2 && zw > 0 && 2 * zw != P2;
+        for (int q = 0; q < 8; q++) {
+            const bool fx = q & 4, fy = q & 2, fz = q & 1;
+            if ((fx && !mx) || (fy && !my) || (fz && !mz)) continue;
+            const long o = ((long)(fx ? P0 - xw : xw) * P1 + (fy ? P1 - yw : yw)) * P2 + (fz ? P2 - zw : zw);
+            if (f == 0) {
+                kern_put<CPLX>(K, o, kk[0]);
+                kern_put<CPLX>(K, 5 * NP + o, fx != fy ? -kk[1] : kk[1]);
+                kern_put<CPLX>(K, 4 * NP + o, fx != fz ? -kk[2] : kk[2]);
+            } else if (f == 1) {
+                kern_put<CPLX>(K, NP + o, kk[1]);
+                kern_put<CPLX>(K, 3 * NP + o, fy != fz ? -kk[2] : kk[2]);
+            } else {
+                kern_put<CPLX>(K, 2 * NP + o, kk[2]);
+            }
+        }
     }
 }
 
@@ -282,6 +320,7 @@ __global__ void k_newell_octant(double* __restrict__ O, int H0, int H1, int H2, 
 
 // the wrapped grid from the octant: diagonal even, yz odd in y and z, xz odd
 // in x and z, xy odd in x and y; FaceKernel6's displacement range (unwrap)
+template <bool CPLX>
 __global__ void k_newell_expand(const double* __restrict__ O, int H0, int H1, int H2, double* __restrict__ K,
                                 int P0, int P1, int P2) {
     const long NP = (long)P0 * P1 * P2, NH = (long)H0 * H1 * H2;
@@ -301,7 +340,7 @@ __global__ void k_newell_expand(const double* __restrict__ O, int H0, int H1, in
             kk[4] = sx * sz * O[4 * NH + o];
             kk[5] = sx * sy * O[5 * NH + o];
         }
-        for (int k = 0; k < 6; k++) K[k * NP + idx] = kk[k];
+        for (int k = 0; k < 6; k++) kern_put<CPLX>(K, k * NP + idx, kk[k]);
     }
 }
 
@@ -315,6 +354,7 @@ struct ExchPoints {
     int n;
     int R[3], period[3];
 };
+template <bool CPLX>
 __global__ void k_add_exch_points(double* __restrict__ K, int P0, int P1, int P2, ExchPoints p) {
     const long NP = (long)P0 * P1 * P2;
     for (long w = blockIdx.x * (long)blockDim.x + threadIdx.x; w < NP; w += (long)gridDim.x * blockDim.x) {
@@ -336,7 +376,7 @@ __global__ void k_add_exch_points(double* __restrict__ K, int P0, int P1, int P2
         const long id = ((long)rho[0] * p.R[1] + rho[1]) * p.R[2] + rho[2];
         for (int i = 0; i < p.n; i++)
             if (p.idx[i] == id)
-                for (int comp = 0; comp < 3; comp++) K[comp * NP + w] += p.val[i];  // xx, yy, zz
+                for (int comp = 0; comp < 3; comp++) K[(comp * NP + w) * (CPLX ? 2 : 1)] += p.val[i];  // xx, yy, zz
     }
 }
 
@@ -353,30 +393,96 @@ __device__ __forceinline__ void atomic_max_nonneg(unsigned long long* a, double 
 // Compressed layouts: 2-D [comp][kz][ky]; 3-D [kz][ky][kx][comp] (the 6 values
 // of one frequency together, for the X . K . X pass); thin 3-D plane-pass
 // plans [kz][comp][kx][ky] (consecutive ky together, one thread per ky).
-__global__ void k_extract_kernel(const double2* __restrict__ W, int P0, int P1, int P2, int Q, double norm,
-                                 float* __restrict__ Kc, int comp, int nK, int plane_layout,
-                                 float* __restrict__ full_comp, unsigned long long* maxre,
-                                 unsigned long long* maxim) {
-    const long total = (long)P0 * P1 * Q;
-    const int hx = P0 / 2 + 1, hy = P1 / 2 + 1;
-    double lre = 0, lim = 0;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total; t += (long)gridDim.x * blockDim.x) {
-        const int kz = (int)(t % Q);
-        const long r = t / Q;
-        const int ky = (int)(r % P1), kx = (int)(r / P1);
-        const double2 w = W[((long)kx * P1 + ky) * P2 + kz];
-        const double re = w.x * norm, im = w.y * norm;
-        lre = fmax(lre, fabs(re));
-        lim = fmax(lim, fabs(im));
-        if (full_comp) full_comp[t] = (float)re;
-        if (kx < hx && ky < hy) {
-            if (P0 == 1) Kc[((long)comp * Q + kz) * hy + ky] = (float)re;
-            else if (plane_layout) Kc[(((long)kz * nK + comp) * hx + kx) * hy + ky] = (float)re;
-            else Kc[(((long)kz * hy + ky) * hx + kx) * nK + comp] = (float)re;
-        }
+// Components comp0..comp0+ncomp of W ([component][P0][P1][P2]): the stored
+// quarter kx <= P0/2, ky <= P1/2, whose maxima are those of the whole spectrum
+// by its parity.  A tile is 16 kz of EXT_P stored elements (component, kx, ky)
+// that are neighbours in Kc: it is read along kz (256 B runs of W) and written
+// along the elements (256 B runs of Kc) through LDS, and the maxima are reduced
+// per block before its two atomics.  Bound by memory: padded 16 x 256 x 256, 6
+// components, 1186 us with one atomic per element, 86 us with these maxima but
+// 4-byte stores a plane apart, 29 us through the tile.
+constexpr int EXT_Z = 16, EXT_P = 64;
+// stored element p of a kz plane (of the ncomp components) -> component, kx, ky
+__device__ __forceinline__ void kc_element(int p, int hx, int hy, int ncomp, int plane_layout, int& ci, int& kx,
+                                           int& ky) {
+    if (hx == 1 || plane_layout) {  // [comp][kx][ky]
+        ky = p % hy;
+        p /= hy;
+        kx = p % hx;
+        ci = p / hx;
+    } else {  // [ky][kx][comp]
+        ci = p % ncomp;
+        p /= ncomp;
+        kx = p % hx;
+        ky = p / hx;
     }
-    atomic_max_nonneg(maxre, lre);
-    atomic_max_nonneg(maxim, lim);
+}
+__global__ __launch_bounds__(256) void k_extract_kernel(const double2* __restrict__ W, int P0, int P1, int P2, int Q,
+                                                        double norm, float* __restrict__ Kc, int comp0, int ncomp,
+                                                        int nK, int plane_layout, unsigned long long* maxre,
+                                                        unsigned long long* maxim) {
+    __shared__ float tile[EXT_Z][EXT_P + 1];
+    __shared__ double red[2][4];
+    const int hx = P0 / 2 + 1, hy = P1 / 2 + 1;
+    const int np = ncomp * hx * hy, ptiles = (np + EXT_P - 1) / EXT_P, ztiles = (Q + EXT_Z - 1) / EXT_Z;
+    const long tiles = (long)ptiles * ztiles;
+    double lre = 0, lim = 0;
+    for (long t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const int p0 = (int)(t % ptiles) * EXT_P, z0 = (int)(t / ptiles) * EXT_Z;
+        for (int i = threadIdx.x; i < EXT_Z * EXT_P; i += 256) {
+            const int z = i % EXT_Z, p = i / EXT_Z;
+            if (z0 + z < Q && p0 + p < np) {
+                int ci, kx, ky;
+                kc_element(p0 + p, hx, hy, ncomp, plane_layout, ci, kx, ky);
+                const double2 w = W[(((long)ci * P0 + kx) * P1 + ky) * P2 + z0 + z];
+                const double re = w.x * norm, im = w.y * norm;
+                lre = fmax(lre, fabs(re));
+                lim = fmax(lim, fabs(im));
+                tile[z][p] = (float)re;
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < EXT_Z * EXT_P; i += 256) {
+            const int p = i % EXT_P, z = i / EXT_P, kz = z0 + z;
+            if (kz < Q && p0 + p < np) {
+                int ci, kx, ky;
+                kc_element(p0 + p, hx, hy, ncomp, plane_layout, ci, kx, ky);
+                const int comp = comp0 + ci;
+                long o;
+                if (P0 == 1) o = ((long)comp * Q + kz) * hy + ky;
+                else if (plane_layout) o = (((long)kz * nK + comp) * hx + kx) * hy + ky;
+                else o = (((long)kz * hy + ky) * hx + kx) * nK + comp;
+                Kc[o] = tile[z][p];
+            }
+        }
+        __syncthreads();
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        lre = fmax(lre, __shfl_xor(lre, off, 64));
+        lim = fmax(lim, __shfl_xor(lim, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = lre;
+        red[1][threadIdx.x >> 6] = lim;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; w++) {
+            lre = fmax(lre, red[0][w]);
+            lim = fmax(lim, red[1][w]);
+        }
+        atomic_max_nonneg(maxre, lre);
+        atomic_max_nonneg(maxim, lim);
+    }
+}
+// the reference's full layout, [component][P0][P1][Q] floats
+__global__ void k_extract_full(const double2* __restrict__ W, int P0, int P1, int P2, int Q, double norm, int comp0,
+                               int ncomp, float* __restrict__ full) {
+    const long rows = (long)ncomp * P0 * P1, total = rows * Q;
+    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total; t += (long)gridDim.x * blockDim.x) {
+        const long r = t / Q;
+        full[(long)comp0 * P0 * P1 * Q + t] = (float)(W[r * P2 + t % Q].x * norm);
+    }
 }
 
 // =============================================================== plan
@@ -593,13 +699,13 @@ static int wrapi(int number, int max) {
 }
 
 // real-space demag kernel (FaceKernel6 or Newell) + Exch6 over the padded grid
-// P, 6 x P doubles on the device
-static double* realspace_kernel_f64(const int P[3], const KernelSpec& ks, hipStream_t s) {
+// P, 6 x P doubles on the device (CPLX: double2 with zero imaginary parts)
+template <bool CPLX> static double* realspace_kernel_f64(const int P[3], const KernelSpec& ks, hipStream_t s) {
     const int P0 = P[0], P1 = P[1], P2 = P[2];
     const double* cell = ks.cell;
     const long NP = (long)P0 * P1 * P2;
     double* K = nullptr;
-    K = (double*)cached_malloc(6 * NP * sizeof(double));
+    K = (double*)cached_malloc((CPLX ? 12 : 6) * NP * sizeof(double));
     for (int a = 0; a < 3; a++)
         GK_ASSERT(ks.period[a] == 0 || (ks.images[a] > 0 && (ks.period[a] == P[a] || P[a] >= 2 * ks.period[a])),
                   "periodic axis %d: period %d, %d images, padded length %d", a, ks.period[a], ks.images[a], P[a]);
@@ -613,7 +719,7 @@ static double* realspace_kernel_f64(const int P[3], const KernelSpec& ks, hipStr
         O = (double*)cached_malloc(6 * NH * sizeof(double));
         k_newell_octant<<<grid1d(NH, 64), 64, 0, s>>>(O, H0, H1, H2, cell[0], cell[1], cell[2]);
         GK_LAUNCH_CHECK();
-        k_newell_expand<<<grid1d(NP), kBlock, 0, s>>>(O, H0, H1, H2, K, P0, P1, P2);
+        k_newell_expand<CPLX><<<grid1d(NP), kBlock, 0, s>>>(O, H0, H1, H2, K, P0, P1, P2);
         GK_LAUNCH_CHECK();
         GK_CHECK(hipStreamSynchronize(s));
         cached_free(O);
@@ -624,7 +730,11 @@ static double* realspace_kernel_f64(const int P[3], const KernelSpec& ks, hipStr
             im.period[a] = ks.period[a];
             im.images[a] = ks.images[a];
         }
-        k_facekernel6<<<grid1d(NP), kBlock, 0, s>>>(K, P0, P1, P2, cell[0], cell[1], cell[2], ks.accuracy, im);
+        int H[3];
+        for (int a = 0; a < 3; a++) H[a] = P[a] % 2 == 0 && ks.period[a] % 2 == 0 ? P[a] / 2 + 1 : P[a];
+        // one wave per block: the evaluations are long, and small kernels then spread over more CUs
+        const dim3 g(grid1d((long)H[0] * H[1] * H[2], 64).x, 3);
+        k_facekernel6<CPLX><<<g, 64, 0, s>>>(K, P0, P1, P2, H[0], H[1], H[2], cell[0], cell[1], cell[2], ks.accuracy, im);
         GK_LAUNCH_CHECK();
     }
     if (ks.exch) {
@@ -661,7 +771,7 @@ static double* realspace_kernel_f64(const int P[3], const KernelSpec& ks, hipStr
             ep.R[a] = R[a];
             ep.period[a] = ks.period[a];
         }
-        k_add_exch_points<<<grid1d(NP), kBlock, 0, s>>>(K, P0, P1, P2, ep);
+        k_add_exch_points<CPLX><<<grid1d(NP), kBlock, 0, s>>>(K, P0, P1, P2, ep);
         GK_LAUNCH_CHECK();
     }
     return K;
@@ -675,7 +785,7 @@ __global__ void k_to_float(const double* __restrict__ in, float* __restrict__ ou
 void conv_realspace_kernel_f64(const int P[3], const KernelSpec& ks, double* out_host) {
     hipStream_t s = stream();
     const long NP = (long)P[0] * P[1] * P[2];
-    double* K = realspace_kernel_f64(P, ks, s);
+    double* K = realspace_kernel_f64<false>(P, ks, s);
     GK_CHECK(hipMemcpyAsync(out_host, K, 6 * NP * sizeof(double), hipMemcpyDeviceToHost, s));
     sync();
     cached_free(K);
@@ -684,7 +794,7 @@ void conv_realspace_kernel_f64(const int P[3], const KernelSpec& ks, double* out
 void conv_realspace_kernel(const int P[3], const KernelSpec& ks, float* out_host) {
     hipStream_t s = stream();
     const long NP = (long)P[0] * P[1] * P[2];
-    double* K = realspace_kernel_f64(P, ks, s);
+    double* K = realspace_kernel_f64<false>(P, ks, s);
     float* f = nullptr;
     f = (float*)cached_malloc(6 * NP * sizeof(float));
     k_to_float<<<grid1d(6 * NP), kBlock, 0, s>>>(K, f, 6 * NP);
@@ -695,26 +805,52 @@ void conv_realspace_kernel(const int P[3], const KernelSpec& ks, float* out_host
     cached_free(f);
 }
 
+// Up to this size all components of a kernel's set-up are transformed together
+// (launches of 6x the lines: a padded 16 x 256 x 256 leaves CUs idle per component).
+constexpr long kKernelSetupBytes = 2L << 30;
+
 double conv_build_kernel(ConvPlan& cp, const KernelSpec& ks, float* full_host, float* full_dev) {
     hipStream_t s = stream();
     const int P0 = cp.P[0], P1 = cp.P[1], P2 = cp.P[2];
     const long NP = (long)P0 * P1 * P2;
-    double* K = realspace_kernel_f64(cp.P, ks, s);
-    double2* W = nullptr;
-    unsigned long long* mx = nullptr;
-    W = (double2*)cached_malloc(NP * sizeof(double2));
-    mx = (unsigned long long*)cached_malloc(2 * sizeof(unsigned long long));
+    unsigned long long* mx = (unsigned long long*)cached_malloc(2 * sizeof(unsigned long long));
     GK_CHECK(hipMemsetAsync(mx, 0, 2 * sizeof(unsigned long long), s));
     const int hx = P0 / 2 + 1, hy = P1 / 2 + 1;
     const long fulls = (long)P0 * P1 * cp.Q;
     const double norm = 1.0 / (double)NP;
-    // components stored: 3-D xx yy zz yz xz xy; 2-D xx yy zz yz
-    for (int k = 0; k < cp.nK; k++) {
-        k_real_to_complex<<<grid1d(NP), kBlock, 0, s>>>(K + k * NP, W, NP);
-        fft3_c2c_f64(W, cp.P, -1, s);
-        k_extract_kernel<<<grid1d(fulls), kBlock, 0, s>>>(W, P0, P1, P2, cp.Q, norm, cp.Kc, k, cp.nK, cp.yxy,
-                                                            full_dev ? full_dev + k * fulls : nullptr, mx, mx + 1);
+    auto extract = [&](const double2* W, int comp0, int ncomp) {
+        const long tiles = (long)div_up((long)ncomp * hx * hy, EXT_P) * div_up(cp.Q, EXT_Z);
+        k_extract_kernel<<<(unsigned)std::min<long>(tiles, 4096), 256, 0, s>>>(W, P0, P1, P2, cp.Q, norm, cp.Kc, comp0,
+                                                                             ncomp, cp.nK, cp.yxy, mx, mx + 1);
         GK_LAUNCH_CHECK();
+        if (full_dev) {
+            k_extract_full<<<grid1d(ncomp * fulls), kBlock, 0, s>>>(W, P0, P1, P2, cp.Q, norm, comp0, ncomp, full_dev);
+            GK_LAUNCH_CHECK();
+        }
+    };
+    // components stored: 3-D xx yy zz yz xz xy; 2-D xx yy zz yz
+    double* K = nullptr;
+    double2* W = nullptr;
+    if (6 * NP * (long)sizeof(double2) <= kKernelSetupBytes) {
+        // all components as complex numbers, one launch per axis; after the Z
+        // transform only kz < Q is needed, and for the compressed spectrum only
+        // ky <= P1/2 of the X transform
+        W = reinterpret_cast<double2*>(realspace_kernel_f64<true>(cp.P, ks, s));
+        const long n12 = (long)P1 * P2;
+        const int ny = full_dev ? P1 : hy;
+        fft_lines_any<double, -1>(W, P2, (long)cp.nK * P0 * P1, (long)cp.nK * P0 * P1, P2, 0, 1, P2, P2, s);
+        if (P1 > 1) fft_lines_any<double, -1>(W, P1, (long)cp.nK * P0 * cp.Q, cp.Q, 1, n12, P2, P1, P1, s);
+        if (P0 > 1) fft_lines_any<double, -1>(W, P0, (long)cp.nK * ny * P2, (long)ny * P2, 1, P0 * n12, n12, P0, P0, s);
+        extract(W, 0, cp.nK);
+    } else {
+        // large grids: one component at a time, 64 instead of 96 bytes per padded cell
+        K = realspace_kernel_f64<false>(cp.P, ks, s);
+        W = (double2*)cached_malloc(NP * sizeof(double2));
+        for (int k = 0; k < cp.nK; k++) {
+            k_real_to_complex<<<grid1d(NP), kBlock, 0, s>>>(K + k * NP, W, NP);
+            fft3_c2c_f64(W, cp.P, -1, s);
+            extract(W, k, 1);
+        }
     }
     unsigned long long h[2];
     GK_CHECK(hipMemcpyAsync(h, mx, sizeof(h), hipMemcpyDeviceToHost, s));
