@@ -310,11 +310,20 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// an exchange buffer whose elements are 2^sh apart (2^sh lines interleaved, so that
+// neighbouring lanes on neighbouring lines use neighbouring banks)
+struct StridedBuf {
+    float2* p;
+    int sh;
+    __device__ __forceinline__ float2& operator[](int i) const { return p[i << sh]; }
+};
+
 // EE: elements per lane (default RegFFT<L>::E; a smaller power-of-two EE spreads
 // a line over more lanes, L / EE, with the same exchange buffer); WS: wave-level
 // instead of block-level barriers around the exchanges (see wave_sync)
-template <typename T, int L, int DIR, int NS = 1, int EE = reg_fft_E(L), bool WS = true>
-__device__ __forceinline__ void reg_fft(C2<T>* v, int g, C2<T>* lds, const C2<T>* tw) {
+// Buf: the exchange buffer, a pointer or anything indexed like one (StridedBuf)
+template <typename T, int L, int DIR, int NS = 1, int EE = reg_fft_E(L), bool WS = true, class Buf = C2<T>*>
+__device__ __forceinline__ void reg_fft(C2<T>* v, int g, Buf lds, const C2<T>* tw) {
     if constexpr (NS < L) {
         constexpr int E = EE, G = L / EE;
         static_assert(L % EE == 0, "elements per lane must divide the length");

@@ -13,8 +13,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <map>
-#include <mutex>
 
 #include "../../include/gpukern.h"
 #include "fft_device.h"
@@ -73,84 +71,128 @@ __global__ __launch_bounds__(NT) void k_fft_lines(C2<T>* __restrict__ data, cons
     }
 }
 
-// rows of n_real floats -> M+1 complex (real transform of length P = 2M, zero padded)
-template <int M, int NL, int NT>
-__global__ __launch_bounds__(NT) void k_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
-                                                 const float2* __restrict__ twM, const float2* __restrict__ twP,
-                                                 long nrows, long n_inner, long in_inner, long in_outer,
-                                                 long out_inner, long out_outer, int n_real) {
-    constexpr int LS = M + 1;
-    __shared__ float2 lds[NL * LS];
-    const long r0 = (long)blockIdx.x * NL;
-    const int npair = (n_real + 1) / 2;
-    batched_copy<float2, NT>(
-        NL * npair,
-        [&](int t) {
-            const int i = t / npair, e = t % npair;
-            const long r = r0 + i;
-            float2 v = make_float2(0.f, 0.f);
-            if (r < nrows) {
-                const float* src = in + (r / n_inner) * in_outer + (r % n_inner) * in_inner;
-                v.x = src[2 * e];
-                v.y = (2 * e + 1 < n_real) ? src[2 * e + 1] : 0.f;
-            }
-            return v;
-        },
-        [&](int t, float2 v) { lds[(t / npair) * LS + t % npair] = v; });
+// ----------------------------------------------------------------------------
+// Register transforms (FP32, 2^a and 3 * 2^a).  A line is held by G lanes with
+// up to 8 (2^a) or 12 (3 * 2^a) elements each, so a lane keeps 16-24 data
+// registers whatever the length, and the radix passes exchange through LDS.
+//
+// Strided lines (Y and X of the drop-in layout): 2^sh neighbouring lines per
+// block, line index fastest over the lanes, so a load touches runs of 2^sh x 8 B;
+// the exchange buffers are interleaved the same way.  Contiguous rows: lane
+// index fastest.  All of a lane's loads and the block's copy of the twiddle
+// table are issued together, one memory latency for the whole kernel (the LDS
+// Stockham kernels these replace read the table from global memory in every
+// pass).  Blocks hold as many lines as leave about two blocks per CU: small
+// transforms are latency-bound and need the CUs, not the occupancy.
+// Measured per launch (before / now): 2064 lines of 256 12.9 / 9.0 us, 33024 of 32
+// 8.0 / 5.7 us, 2048 rows of 256 reals 8.9 / 4.2 us; 64 rows of 512 12.4 / 4.0 us.
+constexpr int line_E(int L) { return L % 3 == 0 ? (L < 12 ? L : 12) : (L < 8 ? L : 8); }
+constexpr int line_G(int L) { return L / line_E(L); }
+constexpr int line_buf(int L) { return L + L / 8 + 1; }
+
+template <int L, int DIR>
+__global__ __launch_bounds__(1024) void k_lines_reg(float2* __restrict__ data, const float2* __restrict__ tw,
+                                                    LineArgs a, int sh) {
+    constexpr int E = line_E(L), G = line_G(L);
+    extern __shared__ float2 dyn_lines[];
+    float2* twl = dyn_lines;
+    float2* buf = dyn_lines + L;
+    const int i = threadIdx.x & ((1 << sh) - 1), g = threadIdx.x >> sh;
+    const unsigned l = (blockIdx.x << sh) + i;
+    const bool ok = l < a.nlines;
+    float2* p = data + a.start(ok ? l : 0);
+    float2 v[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int n = g + G * e;
+        v[e] = (ok && n < a.nvalid) ? p[n * a.estride] : make_float2(0.f, 0.f);
+    }
+    for (int t = threadIdx.x; t < L; t += G << sh) twl[t] = tw[t];
     __syncthreads();
-    fft_lds<float, M, -1, NL, NT>(lds, LS, twM, npair);
-    for (int t = threadIdx.x; t < NL * (M + 1); t += NT) {
-        const int i = t / (M + 1), k = t % (M + 1);
-        const long r = r0 + i;
-        if (r < nrows) {
-            float2 zk = lds[i * LS + (k % M)], zmk = lds[i * LS + ((M - k) % M)];
-            out[(r / n_inner) * out_outer + (r % n_inner) * out_inner + k] = r2c_split<float>(zk, zmk, twP[k]);
-        }
+    reg_fft<float, L, DIR, 1, E, false>(v, g, StridedBuf{buf + i, sh}, twl);
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int n = g + G * e;
+        if (ok && n < a.nkeep) p[n * a.estride] = v[e];
     }
 }
 
-// M+1 complex per row -> first n_real floats of the length-2M real inverse transform
-template <int M, int NL, int NT>
-__global__ __launch_bounds__(NT) void k_rows_c2r(const float2* __restrict__ in, float* __restrict__ out,
-                                                 const float2* __restrict__ twM, const float2* __restrict__ twP,
-                                                 long nrows, long n_inner, long in_inner, long in_outer,
-                                                 long out_inner, long out_outer, int n_real) {
-    constexpr int LS = M + 1;
-    constexpr int NY = (NL * M + NT - 1) / NT;
-    __shared__ float2 lds[NL * LS];
-    const long r0 = (long)blockIdx.x * NL;
-    batched_copy<float2, NT>(
-        NL * (M + 1),
-        [&](int t) {
-            const int i = t / (M + 1), k = t % (M + 1);
-            const long r = r0 + i;
-            return r < nrows ? in[(r / n_inner) * in_outer + (r % n_inner) * in_inner + k] : make_float2(0.f, 0.f);
-        },
-        [&](int t, float2 v) { lds[(t / (M + 1)) * LS + t % (M + 1)] = v; });
-    __syncthreads();
-    float2 y[NY];
+// rows of n_real floats -> M+1 complex (real transform of length P = 2M, zero padded)
+template <int M>
+__global__ __launch_bounds__(1024) void k_rows_r2c_reg(const float* __restrict__ in, float2* __restrict__ out,
+                                                       const float2* __restrict__ twM, const float2* __restrict__ twP,
+                                                       RowArgs a, int nr) {
+    constexpr int E = line_E(M), G = line_G(M);
+    extern __shared__ float2 dyn_lines[];
+    float2* twl = dyn_lines;
+    const int g = threadIdx.x % G, row = threadIdx.x / G;
+    float2* buf = dyn_lines + M + row * line_buf(M);
+    const unsigned r = blockIdx.x * nr + row;
+    const bool ok = r < a.nrows;
+    const float* src = in + a.real_at(ok ? r : 0);
+    float2 v[E], wp[E];
 #pragma unroll
-    for (int q = 0; q < NY; q++) {
-        const int t = threadIdx.x + q * NT;
-        if (t < NL * M) {
-            const int i = t / M, k = t % M;
-            y[q] = c2r_merge<float>(lds[i * LS + k], lds[i * LS + (M - k)], twP[k]);
+    for (int e = 0; e < E; e++) {
+        const int n = g + G * e;
+        float2 x = make_float2(0.f, 0.f);
+        if (a.vec) {
+            if (ok && 2 * n < a.n_real) x = *reinterpret_cast<const float2*>(src + 2 * n);
+        } else {
+            if (ok && 2 * n < a.n_real) x.x = src[2 * n];
+            if (ok && 2 * n + 1 < a.n_real) x.y = src[2 * n + 1];
         }
+        v[e] = x;
+        wp[e] = twP[n];
     }
+    for (int t = threadIdx.x; t < M; t += G * nr) twl[t] = twM[t];
+    __syncthreads();
+    reg_fft<float, M, -1, 1, E, false>(v, g, buf, twl);
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NY; q++) {
-        const int t = threadIdx.x + q * NT;
-        if (t < NL * M) lds[(t / M) * LS + (t % M)] = y[q];
-    }
+    for (int e = 0; e < E; e++) buf[g + G * e] = v[e];
     __syncthreads();
-    fft_lds<float, M, +1, NL, NT>(lds, LS, twM, M);
-    for (int t = threadIdx.x; t < NL * n_real; t += NT) {
-        const int i = t / n_real, e = t % n_real;
-        const long r = r0 + i;
-        if (r < nrows) {
-            float2 z = lds[i * LS + (e >> 1)];
-            out[(r / n_inner) * out_outer + (r % n_inner) * out_inner + e] = (e & 1) ? z.y : z.x;
+    if (!ok) return;
+    float2* dst = out + a.cplx_at(r);
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int k = g + G * e;
+        dst[k] = r2c_split<float>(v[e], buf[k ? M - k : 0], wp[e]);
+    }
+    if (g == 0) dst[M] = make_float2(v[0].x - v[0].y, 0.f);
+}
+
+// M+1 complex per row -> first n_real floats of the length-2M real inverse transform
+template <int M>
+__global__ __launch_bounds__(1024) void k_rows_c2r_reg(const float2* __restrict__ in, float* __restrict__ out,
+                                                       const float2* __restrict__ twM, const float2* __restrict__ twP,
+                                                       RowArgs a, int nr) {
+    constexpr int E = line_E(M), G = line_G(M);
+    extern __shared__ float2 dyn_lines[];
+    float2* twl = dyn_lines;
+    const int g = threadIdx.x % G, row = threadIdx.x / G;
+    float2* buf = dyn_lines + M + row * line_buf(M);
+    const unsigned r = blockIdx.x * nr + row;
+    const bool ok = r < a.nrows;
+    const float2* src = in + a.cplx_at(ok ? r : 0);
+    float2 v[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int k = g + G * e;
+        v[e] = c2r_merge<float>(src[k], src[M - k], twP[k]);
+    }
+    for (int t = threadIdx.x; t < M; t += G * nr) twl[t] = twM[t];
+    __syncthreads();
+    reg_fft<float, M, +1, 1, E, false>(v, g, buf, twl);
+    if (!ok) return;
+    float* dst = out + a.real_at(r);
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int n = g + G * e;
+        if (a.vec) {
+            if (2 * n < a.n_real) *reinterpret_cast<float2*>(dst + 2 * n) = v[e];
+        } else {
+            if (2 * n < a.n_real) dst[2 * n] = v[e].x;
+            if (2 * n + 1 < a.n_real) dst[2 * n + 1] = v[e].y;
         }
     }
 }
@@ -203,49 +245,92 @@ void fft_lines(C2<T>* data, int L, long nlines, long n_inner, long inner, long o
     GK_LAUNCH_CHECK();
 }
 
-template void fft_lines<float, -1>(float2*, int, long, long, long, long, long, int, int, hipStream_t);
-template void fft_lines<float, +1>(float2*, int, long, long, long, long, long, int, int, hipStream_t);
 template void fft_lines<double, -1>(double2*, int, long, long, long, long, long, int, int, hipStream_t);
 template void fft_lines<double, +1>(double2*, int, long, long, long, long, long, int, int, hipStream_t);
 
-void fft_rows_r2c(const float* in, float2* out, int P, long nrows, long n_inner, long in_inner, long in_outer,
-                  long out_inner, long out_outer, int n_real, hipStream_t s) {
-    if (nrows <= 0) return;
-    GK_ASSERT(P % 2 == 0 && n_real <= P, "real FFT length %d (data %d)", P, n_real);
+// 2^a up to 4096 and 3 * 2^a up to 3072
+#define GK_FOR_EACH_REG(X) GK_FOR_EACH_POW2(X) X(3) X(6) X(12) X(24) X(48) X(96) X(192) X(384) X(768) X(1536) X(3072)
+
+bool fft_reg_length(int L) {
+    switch (L) {
+#define GK_CASE(n) case n:
+        GK_FOR_EACH_REG(GK_CASE)
+#undef GK_CASE
+        return true;
+    default: return false;
+    }
+}
+
+// log2 of the lines per block: up to 256 threads (64 B or longer runs: at least
+// 8 lines) and 60 KB of LDS, then fewer while the launch has under two blocks per
+// CU (512) and a block a whole wave and 4 lines (32 B runs)
+static int lines_shift(int L, int G, unsigned nlines) {
+    int sh = 3;
+    while ((G << (sh + 1)) <= 256) sh++;
+    while (sh > 0 && ((G << sh) > 1024 || (((line_buf(L) << sh) + L) * 8) > 60 * 1024)) sh--;
+    while (sh > 2 && (G << (sh - 1)) >= 64 && (nlines >> sh) < 512) sh--;
+    return sh;
+}
+// rows per block: 256 threads, fewer while the launch has under 512 blocks and a block a whole wave
+static int rows_per_launch_block(int M, int G, unsigned nrows) {
+    int nr = 1;
+    while (2 * nr * G <= 256 && (2 * nr * line_buf(M) + M) * 8 <= 60 * 1024) nr *= 2;
+    while (nr > 1 && nr / 2 * G >= 64 && nrows / nr < 512) nr /= 2;
+    return nr;
+}
+
+template <int DIR> void fft_lines_reg(float2* data, int L, const LineArgs& a, hipStream_t s) {
+    if (a.nlines == 0) return;
+    const float2* tw = twiddle_f32(L);
+    switch (L) {
+#define GK_CASE(n)                                                                                              \
+    case n: {                                                                                                   \
+        const int sh = lines_shift(n, line_G(n), a.nlines);                                                     \
+        k_lines_reg<n, DIR><<<div_up(a.nlines, 1L << sh), line_G(n) << sh, ((line_buf(n) << sh) + n) * 8, s>>>( \
+            data, tw, a, sh);                                                                                   \
+        break;                                                                                                  \
+    }
+        GK_FOR_EACH_REG(GK_CASE)
+#undef GK_CASE
+    default: fprintf(stderr, "libgpukern: FFT length %d is not supported\n", L); abort();
+    }
+    GK_LAUNCH_CHECK();
+}
+template void fft_lines_reg<-1>(float2*, int, const LineArgs&, hipStream_t);
+template void fft_lines_reg<+1>(float2*, int, const LineArgs&, hipStream_t);
+
+void fft_rows_r2c_reg(const float* in, float2* out, int P, const RowArgs& a, hipStream_t s) {
     const int M = P / 2;
     const float2* twM = twiddle_f32(M);
     const float2* twP = twiddle_f32(P);
     switch (M) {
-#define GK_CASE(n)                                                                                              \
-    case n: {                                                                                                   \
-        constexpr int NL = lines_per_block<float>(n);                                                           \
-        k_rows_r2c<n, NL, kFFTThreads><<<div_up(nrows, NL), kFFTThreads, 0, s>>>(                               \
-            in, out, twM, twP, nrows, n_inner, in_inner, in_outer, out_inner, out_outer, n_real);               \
-        break;                                                                                                  \
+#define GK_CASE(n)                                                                                       \
+    case n: {                                                                                            \
+        const int nr = rows_per_launch_block(n, line_G(n), a.nrows);                                     \
+        k_rows_r2c_reg<n><<<div_up(a.nrows, nr), line_G(n) * nr, (line_buf(n) * nr + n) * 8, s>>>(       \
+            in, out, twM, twP, a, nr);                                                                   \
+        break;                                                                                           \
     }
-        GK_FOR_EACH_POW2(GK_CASE)
+        GK_FOR_EACH_REG(GK_CASE)
 #undef GK_CASE
     default: fprintf(stderr, "libgpukern: real FFT length %d is not supported\n", P); abort();
     }
     GK_LAUNCH_CHECK();
 }
 
-void fft_rows_c2r(const float2* in, float* out, int P, long nrows, long n_inner, long in_inner, long in_outer,
-                  long out_inner, long out_outer, int n_real, hipStream_t s) {
-    if (nrows <= 0) return;
-    GK_ASSERT(P % 2 == 0 && n_real <= P, "real FFT length %d (data %d)", P, n_real);
+void fft_rows_c2r_reg(const float2* in, float* out, int P, const RowArgs& a, hipStream_t s) {
     const int M = P / 2;
     const float2* twM = twiddle_f32(M);
     const float2* twP = twiddle_f32(P);
     switch (M) {
-#define GK_CASE(n)                                                                                              \
-    case n: {                                                                                                   \
-        constexpr int NL = lines_per_block<float>(n);                                                           \
-        k_rows_c2r<n, NL, kFFTThreads><<<div_up(nrows, NL), kFFTThreads, 0, s>>>(                               \
-            in, out, twM, twP, nrows, n_inner, in_inner, in_outer, out_inner, out_outer, n_real);               \
-        break;                                                                                                  \
+#define GK_CASE(n)                                                                                       \
+    case n: {                                                                                            \
+        const int nr = rows_per_launch_block(n, line_G(n), a.nrows);                                     \
+        k_rows_c2r_reg<n><<<div_up(a.nrows, nr), line_G(n) * nr, (line_buf(n) * nr + n) * 8, s>>>(       \
+            in, out, twM, twP, a, nr);                                                                   \
+        break;                                                                                           \
     }
-        GK_FOR_EACH_POW2(GK_CASE)
+        GK_FOR_EACH_REG(GK_CASE)
 #undef GK_CASE
     default: fprintf(stderr, "libgpukern: real FFT length %d is not supported\n", P); abort();
     }
@@ -272,28 +357,9 @@ void fft3_c2c_f64(double2* d, const int n[3], int dir, hipStream_t s) {
 // drop-in plan
 using namespace gk;
 
-// Scratch of gpuFFT3dPlan_forward_noalloc: the packed rows and Bluestein buffers
-// of the any-length transforms, 4 Mi float2 (32 MiB) per device, held by every
-// device the library runs on until the process ends.  Host code never passes
-// `scratch` itself to a kernel: it takes the device address that
-// hipGetSymbolAddress gives on each device (scratch_device_ptr).
+// gpuFFT3dPlan_forward_noalloc refuses plans above this many elements of what
+// its contract counts (forward_scratch_elems).
 constexpr size_t kFFTScratchElems = size_t(4) << 20;
-static __device__ __align__(256) float2 scratch[kFFTScratchElems];
-
-static float2* scratch_device_ptr() {
-    static std::mutex mu;
-    static std::map<int, float2*> ptr;  // device -> address of its copy of `scratch`
-    int dev = 0;
-    GK_CHECK(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = ptr.find(dev);
-    if (it != ptr.end()) return it->second;
-    void* a = nullptr;
-    GK_CHECK(hipGetSymbolAddress(&a, HIP_SYMBOL(scratch)));
-    GK_ASSERT(a != nullptr, "no device address for the FFT scratch array");
-    ptr[dev] = static_cast<float2*>(a);
-    return ptr[dev];
-}
 
 struct gpuFFT3dPlan {
     int size[3];
@@ -333,29 +399,36 @@ void delete_gpuFFT3dPlan(gpuFFT3dPlan* plan) { delete plan; }
 
 int gpuFFT3dPlan_normalization(gpuFFT3dPlan* p) { return p->padded[0] * p->padded[1] * p->padded[2]; }
 
-void gpuFFT3dPlan_forward(gpuFFT3dPlan* p, float* input, float* output) {
+// The no-allocation transform's size limit counts, for the largest pass, the
+// packed rows and padded lines of lengths that are no power of two (the transforms
+// themselves use registers and LDS only, for every plan).
+static size_t forward_scratch_elems(const gpuFFT3dPlan* p) {
+    const long N0 = p->size[0], N1 = p->size[1];
+    const int P0 = p->padded[0], P1 = p->padded[1], P2 = p->padded[2], Q = p->pzc;
+    const int H = P2 % 2 == 0 ? P2 / 2 : P2;
+    size_t need = 0;
+    if (P2 % 2 || !fft_length_supported(H)) need = (size_t)(N0 * N1) * (H + fft_blue_length(H));
+    if (P1 > 1) need = std::max(need, (size_t)(N0 * Q) * fft_blue_length(P1));
+    if (P0 > 1) need = std::max(need, (size_t)P1 * Q * fft_blue_length(P0));
+    return need;
+}
+
+// the forward transform on stream s: rows, then columns; twiddle and chirp tables
+// come from the plan's construction
+static void plan_forward(gpuFFT3dPlan* p, const float* input, float2* out, hipStream_t s) {
     const int N0 = p->size[0], N1 = p->size[1], N2 = p->size[2];
     const int P0 = p->padded[0], P1 = p->padded[1], P2 = p->padded[2], Q = p->pzc;
-    float2* out = (float2*)output;
-    hipStream_t s = stream();
     // Z: real rows (x<N0, y<N1) -> out[x][y][0..Q)
     fft_rows_r2c_any(input, out, P2, (long)N0 * N1, N1, N2, (long)N1 * N2, Q, (long)P1 * Q, N2, s);
     // Y: columns (x<N0, kz) over y; rows y>=N1 are zero padding and not read
     if (P1 > 1) fft_lines_any<float, -1>(out, P1, (long)N0 * Q, Q, 1, (long)P1 * Q, Q, N1, P1, s);
     // X: every (ky,kz) column; planes x>=N0 are zero padding and not read
     if (P0 > 1) fft_lines_any<float, -1>(out, P0, (long)P1 * Q, (long)P1 * Q, 1, 0, (long)P1 * Q, N0, P0, s);
-    sync();
 }
 
-// float2 elements of scratch the forward transform of plan p needs: its three
-// passes run one after the other on one stream, so they share it
-static size_t forward_scratch_elems(const gpuFFT3dPlan* p) {
-    const long N0 = p->size[0], N1 = p->size[1];
-    const int P0 = p->padded[0], P1 = p->padded[1], P2 = p->padded[2], Q = p->pzc;
-    size_t need = fft_rows_r2c_any_scratch(P2, N0 * N1);
-    if (P1 > 1) need = std::max(need, fft_lines_any_scratch(P1, N0 * Q));
-    if (P0 > 1) need = std::max(need, fft_lines_any_scratch(P0, (long)P1 * Q));
-    return need;
+void gpuFFT3dPlan_forward(gpuFFT3dPlan* p, float* input, float* output) {
+    plan_forward(p, input, (float2*)output, stream());
+    sync();
 }
 
 void gpuFFT3dPlan_forward_noalloc(gpuFFT3dPlan* p, float* input, float* output) {
@@ -364,15 +437,8 @@ void gpuFFT3dPlan_forward_noalloc(gpuFFT3dPlan* p, float* input, float* output) 
               "gpuFFT3dPlan_forward_noalloc: padded size %d x %d x %d needs %zu scratch elements (8 bytes each); "
               "the maximum is %zu (use gpuFFT3dPlan_forward)",
               p->padded[0], p->padded[1], p->padded[2], need, kFFTScratchElems);
-    const int N0 = p->size[0], N1 = p->size[1], N2 = p->size[2];
-    const int P0 = p->padded[0], P1 = p->padded[1], P2 = p->padded[2], Q = p->pzc;
-    const FFTScratch sc{need ? scratch_device_ptr() : nullptr, kFFTScratchElems};
-    float2* out = (float2*)output;
-    hipStream_t s = stream();
     tables_frozen(true);
-    fft_rows_r2c_any(input, out, P2, (long)N0 * N1, N1, N2, (long)N1 * N2, Q, (long)P1 * Q, N2, s, &sc);
-    if (P1 > 1) fft_lines_any<float, -1>(out, P1, (long)N0 * Q, Q, 1, (long)P1 * Q, Q, N1, P1, s, &sc);
-    if (P0 > 1) fft_lines_any<float, -1>(out, P0, (long)P1 * Q, (long)P1 * Q, 1, 0, (long)P1 * Q, N0, P0, s, &sc);
+    plan_forward(p, input, (float2*)output, stream());
     tables_frozen(false);
     sync();
 }

@@ -44,52 +44,42 @@ static bool factor_radices(int L, RadixList& rl) {
     return true;
 }
 
-// one Stockham pass of radix RR over a line of L held in LDS (src -> dst)
+// one Stockham pass of radix RR over 2^sh lines of L held interleaved in LDS
+// (element i of line q at (i << sh) + q, src -> dst)
 template <typename T, int DIR, int RR>
-__device__ __forceinline__ void stockham_pass_rt(const C2<T>* src, C2<T>* dst, int L, int NS,
+__device__ __forceinline__ void stockham_pass_rt(const C2<T>* src, C2<T>* dst, unsigned L, unsigned NS, int sh,
                                                  const C2<T>* __restrict__ tw) {
-    const int nb = L / RR;
-    for (int j = threadIdx.x; j < nb; j += blockDim.x) {
-        const int k = j % NS;
+    const unsigned nb = L / RR, mask = (1u << sh) - 1;
+    for (unsigned b = threadIdx.x; b < (nb << sh); b += blockDim.x) {
+        const unsigned q = b & mask, j = b >> sh, jq = j / NS, k = j - jq * NS;
         C2<T> v[RR];
 #pragma unroll
-        for (int r = 0; r < RR; r++) v[r] = src[j + r * nb];
+        for (unsigned r = 0; r < RR; r++) v[r] = src[((j + r * nb) << sh) + q];
         if (NS > 1) {
-            const int step = L / (NS * RR);
+            const unsigned step = L / (NS * RR);
 #pragma unroll
-            for (int r = 1; r < RR; r++) v[r] = cmul<T>(v[r], twid<T, DIR>(tw, r * k * step));
+            for (unsigned r = 1; r < RR; r++) v[r] = cmul<T>(v[r], twid<T, DIR>(tw, r * k * step));
         }
         dft<T, RR, DIR>(v);
-        const int base = (j / NS) * NS * RR + k;
+        const unsigned base = jq * NS * RR + k;
 #pragma unroll
-        for (int r = 0; r < RR; r++) dst[base + r * NS] = v[r];
+        for (unsigned r = 0; r < RR; r++) dst[((base + r * NS) << sh) + q] = v[r];
     }
 }
-
-// lines as in k_fft_lines: line l starts at (l / n_inner) outer + (l % n_inner) inner,
-// elements at stride estride; the first nvalid inputs are read, the first nkeep stored
+// all passes; returns the buffer holding the result (every thread of the block calls it)
 template <typename T, int DIR>
-__global__ __launch_bounds__(256) void k_fft_lines_rt(C2<T>* __restrict__ data, const C2<T>* __restrict__ tw, int L,
-                                                      RadixList rl, long nlines, long n_inner, long inner, long outer,
-                                                      long estride, int nvalid, int nkeep) {
-    extern __shared__ __align__(16) unsigned char smem_rt[];
-    C2<T>* a = reinterpret_cast<C2<T>*>(smem_rt);
-    C2<T>* b = a + L;
-    const long l = blockIdx.x;
-    if (l >= nlines) return;
-    C2<T>* line = data + (l / n_inner) * outer + (l % n_inner) * inner;
-    for (int i = threadIdx.x; i < L; i += blockDim.x) a[i] = i < nvalid ? line[(long)i * estride] : mk<T>(0, 0);
-    __syncthreads();
+__device__ __forceinline__ C2<T>* stockham_rt(C2<T>* a, C2<T>* b, int L, const RadixList& rl, int sh,
+                                              const C2<T>* __restrict__ tw) {
     int NS = 1;
     for (int p = 0; p < rl.n; p++) {
         const int R = rl.r[p];
         switch (R) {
-        case 8: stockham_pass_rt<T, DIR, 8>(a, b, L, NS, tw); break;
-        case 4: stockham_pass_rt<T, DIR, 4>(a, b, L, NS, tw); break;
-        case 2: stockham_pass_rt<T, DIR, 2>(a, b, L, NS, tw); break;
-        case 3: stockham_pass_rt<T, DIR, 3>(a, b, L, NS, tw); break;
-        case 5: stockham_pass_rt<T, DIR, 5>(a, b, L, NS, tw); break;
-        default: stockham_pass_rt<T, DIR, 7>(a, b, L, NS, tw); break;
+        case 8: stockham_pass_rt<T, DIR, 8>(a, b, L, NS, sh, tw); break;
+        case 4: stockham_pass_rt<T, DIR, 4>(a, b, L, NS, sh, tw); break;
+        case 2: stockham_pass_rt<T, DIR, 2>(a, b, L, NS, sh, tw); break;
+        case 3: stockham_pass_rt<T, DIR, 3>(a, b, L, NS, sh, tw); break;
+        case 5: stockham_pass_rt<T, DIR, 5>(a, b, L, NS, sh, tw); break;
+        default: stockham_pass_rt<T, DIR, 7>(a, b, L, NS, sh, tw); break;
         }
         __syncthreads();
         C2<T>* t = a;
@@ -97,7 +87,108 @@ __global__ __launch_bounds__(256) void k_fft_lines_rt(C2<T>* __restrict__ data, 
         b = t;
         NS *= R;
     }
-    for (int i = threadIdx.x; i < nkeep; i += blockDim.x) line[(long)i * estride] = a[i];
+    return a;
+}
+
+// Lines (LineArgs), 2^sh neighbours per block: strided lines load and store runs
+// of 2^sh elements, contiguous ones (estride 1) along the line.  One line per
+// block, the form this replaces, moved 8 B (16 B in FP64) per 64 B of memory: 1070
+// lines of 150 11.2 us, now 7.7 us.
+template <typename T, int DIR>
+__global__ __launch_bounds__(256) void k_fft_lines_rt(C2<T>* __restrict__ data, const C2<T>* __restrict__ tw, int L,
+                                                      RadixList rl, LineArgs la, int sh) {
+    extern __shared__ __align__(16) unsigned char smem_rt[];
+    C2<T>* a = reinterpret_cast<C2<T>*>(smem_rt);
+    C2<T>* b = a + ((long)L << sh);
+    const unsigned l0 = blockIdx.x << sh, mask = (1u << sh) - 1, nl = min(la.nlines - l0, 1u << sh);
+    const bool col = la.estride != 1;
+    for (unsigned t = threadIdx.x; t < ((unsigned)L << sh); t += blockDim.x) {
+        const unsigned q = col ? t & mask : t / L, n = col ? t >> sh : t - q * L;
+        const bool in = q < nl && (int)n < la.nvalid;
+        a[(n << sh) + q] = in ? data[la.start(l0 + q) + (long)n * la.estride] : mk<T>(0, 0);
+    }
+    __syncthreads();
+    a = stockham_rt<T, DIR>(a, b, L, rl, sh, tw);
+    for (unsigned t = threadIdx.x; t < ((unsigned)la.nkeep << sh); t += blockDim.x) {
+        const unsigned q = col ? t & mask : t / la.nkeep, n = col ? t >> sh : t - q * la.nkeep;
+        if (q < nl) data[la.start(l0 + q) + (long)n * la.estride] = a[(n << sh) + q];
+    }
+}
+
+// Real rows of length P: even P through the packed transform of H = P/2 and
+// the split, odd P as H = P complex numbers
+__global__ __launch_bounds__(256) void k_rows_r2c_rt(const float* __restrict__ in, float2* __restrict__ out,
+                                                     const float2* __restrict__ tw, const float2* __restrict__ twP,
+                                                     int H, int even, RadixList rl, RowArgs ra, int sh) {
+    extern __shared__ __align__(16) unsigned char smem_rt[];
+    float2* a = reinterpret_cast<float2*>(smem_rt);
+    float2* b = a + ((long)H << sh);
+    const unsigned r0 = blockIdx.x << sh, nr = min(ra.nrows - r0, 1u << sh);
+    for (unsigned t = threadIdx.x; t < ((unsigned)H << sh); t += blockDim.x) {
+        const unsigned q = t / H, n = t - q * H;
+        float2 v = make_float2(0.f, 0.f);
+        if (q < nr) {
+            const float* row = in + ra.real_at(r0 + q);
+            if (even) {
+                if (2 * (int)n < ra.n_real) v.x = row[2 * n];
+                if (2 * (int)n + 1 < ra.n_real) v.y = row[2 * n + 1];
+            } else if ((int)n < ra.n_real) {
+                v.x = row[n];
+            }
+        }
+        a[(n << sh) + q] = v;
+    }
+    __syncthreads();
+    a = stockham_rt<float, -1>(a, b, H, rl, sh, tw);
+    const unsigned Q = even ? H + 1 : H / 2 + 1;
+    for (unsigned t = threadIdx.x; t < (Q << sh); t += blockDim.x) {
+        const unsigned q = t / Q, k = t - q * Q;
+        if (q >= nr) continue;
+        const float2 zk = a[((k == (unsigned)H ? 0 : k) << sh) + q];
+        float2 X = zk;
+        if (even) {
+            if (k == (unsigned)H) X = make_float2(zk.x - zk.y, 0.f);
+            else X = r2c_split<float>(zk, a[((k ? H - k : 0) << sh) + q], twP[k]);
+        }
+        out[ra.cplx_at(r0 + q) + k] = X;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_rows_c2r_rt(const float2* __restrict__ in, float* __restrict__ out,
+                                                     const float2* __restrict__ tw, const float2* __restrict__ twP,
+                                                     int H, int even, RadixList rl, RowArgs ra, int sh) {
+    extern __shared__ __align__(16) unsigned char smem_rt[];
+    float2* a = reinterpret_cast<float2*>(smem_rt);
+    float2* b = a + ((long)H << sh);
+    const unsigned r0 = blockIdx.x << sh, nr = min(ra.nrows - r0, 1u << sh);
+    for (unsigned t = threadIdx.x; t < ((unsigned)H << sh); t += blockDim.x) {
+        const unsigned q = t / H, k = t - q * H;
+        float2 v = make_float2(0.f, 0.f);
+        if (q < nr) {
+            const float2* X = in + ra.cplx_at(r0 + q);
+            if (even) v = c2r_merge<float>(X[k], X[H - k], twP[k]);
+            else v = (int)k <= H / 2 ? X[k] : cconj<float>(X[H - k]);
+        }
+        a[(k << sh) + q] = v;
+    }
+    __syncthreads();
+    a = stockham_rt<float, +1>(a, b, H, rl, sh, tw);
+    const unsigned n_real = ra.n_real;
+    for (unsigned t = threadIdx.x; t < (n_real << sh); t += blockDim.x) {
+        const unsigned q = t / n_real, i = t - q * n_real;
+        if (q >= nr) continue;
+        const float2 y = a[((even ? i >> 1 : i) << sh) + q];
+        out[ra.real_at(r0 + q) + i] = even && (i & 1) ? y.y : y.x;
+    }
+}
+
+// log2 of the lines per block: 8 (64 B runs of float2), fewer where both buffers
+// pass 48 KB or, down to 4, where the launch has under 512 blocks
+template <typename T> static int rt_shift(int L, unsigned nlines) {
+    int sh = 3;
+    while (sh > 0 && (2L * L * (long)sizeof(C2<T>) << sh) > 48 * 1024) sh--;
+    while (sh > 2 && (nlines >> sh) < 512) sh--;
+    return sh;
 }
 
 // ---------------------------------------------------------------- Bluestein
@@ -162,55 +253,206 @@ static const BlueTables& blue_tables(int L, int dir) {
     return cache.emplace(std::make_pair(L, dir), t).first->second;
 }
 
-// scratch[l][n] = x_l[n] w[n] (n < nvalid), zero up to Lp
-__global__ void k_blue_pre(const float2* __restrict__ data, float2* __restrict__ scr, const float2* __restrict__ w,
-                           int L, int Lp, long nlines, long n_inner, long inner, long outer, long estride, int nvalid) {
-    const long tot = nlines * Lp;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long l = t / Lp;
-        const int n = (int)(t - l * Lp);
-        float2 v = make_float2(0.f, 0.f);
-        if (n < nvalid && n < L) {
-            const float2 x = data[(l / n_inner) * outer + (l % n_inner) * inner + (long)n * estride];
-            v = cmul<float>(x, w[n]);
+// One kernel per transform: the chirped inputs go through the length-Lp forward
+// transform, the filter, the inverse transform and the second chirp in registers
+// (fft_device.h; E elements per lane, G lanes per line), and real rows are packed,
+// split or merged at its ends.  L <= Lp / 2, so the upper half of each lane's
+// inputs is zero and of its outputs dead at compile time.  The separate kernels
+// this replaces (pack, chirp, transform, multiply, transform, chirp, split) moved
+// the Lp-padded lines through memory eight times and allocated them per call:
+// 750 rows of 212 reals (H = 106, Lp = 256) took 49 us and seven launches, now 6.3 us.
+enum { BLUE_LINES = 0, BLUE_R2C = 1, BLUE_C2R = 2 };
+constexpr int blue_G(int Lp) { return Lp / 8; }
+constexpr int blue_buf(int Lp) { return Lp + Lp / 8 + 1; }
+
+template <int Lp, int DIR>
+__device__ __forceinline__ void blue_transform(float2* v, int g, StridedBuf buf, const float2* __restrict__ w,
+                                               const float2* __restrict__ B, const float2* tw, int L) {
+    constexpr int G = blue_G(Lp);
+    float2 c[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int n = g + G * e;
+        c[e] = n < L ? w[n] : make_float2(0.f, 0.f);
+        v[e] = cmul<float>(v[e], c[e]);
+        v[e + 4] = make_float2(0.f, 0.f);
+    }
+    reg_fft<float, Lp, -1, 1, 8, false>(v, g, buf, tw);
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = cmul<float>(v[e], B[g + G * e]);
+    reg_fft<float, Lp, +1, 1, 8, false>(v, g, buf, tw);
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = cmul<float>(v[e], c[e]);
+}
+
+// strided lines: 2^sh neighbours per block, line index fastest (as k_lines_reg)
+template <int Lp, int DIR>
+__global__ __launch_bounds__(1024) void k_lines_blue(float2* __restrict__ data, const float2* __restrict__ w,
+                                                     const float2* __restrict__ B, const float2* __restrict__ tw,
+                                                     int L, LineArgs a, int sh) {
+    constexpr int G = blue_G(Lp);
+    extern __shared__ float2 dyn_blue[];
+    float2* twl = dyn_blue;
+    const int i = threadIdx.x & ((1 << sh) - 1), g = threadIdx.x >> sh;
+    const unsigned l = (blockIdx.x << sh) + i;
+    const bool ok = l < a.nlines;
+    float2* p = data + a.start(ok ? l : 0);
+    float2 v[8];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int n = g + G * e;
+        v[e] = (ok && n < a.nvalid && n < L) ? p[n * a.estride] : make_float2(0.f, 0.f);
+    }
+    for (int t = threadIdx.x; t < Lp; t += G << sh) twl[t] = tw[t];
+    __syncthreads();
+    blue_transform<Lp, DIR>(v, g, StridedBuf{dyn_blue + Lp + i, sh}, w, B, twl, L);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int n = g + G * e;
+        if (ok && n < a.nkeep) p[n * a.estride] = v[e];
+    }
+}
+
+// real rows through a transform of H = P/2 (even P) or H = P (odd) complex numbers
+template <int Lp, int MODE>
+__global__ __launch_bounds__(1024) void k_rows_blue(const float* __restrict__ rin, float* __restrict__ rout,
+                                                    const float2* __restrict__ cin, float2* __restrict__ cout,
+                                                    const float2* __restrict__ w, const float2* __restrict__ B,
+                                                    const float2* __restrict__ tw, const float2* __restrict__ twP,
+                                                    int H, int even, RowArgs a, int nr) {
+    constexpr int G = blue_G(Lp);
+    extern __shared__ float2 dyn_blue[];
+    float2* twl = dyn_blue;
+    const int g = threadIdx.x % G, row = threadIdx.x / G;
+    float2* buf = dyn_blue + Lp + row * blue_buf(Lp);
+    const unsigned r = blockIdx.x * nr + row;
+    const bool ok = r < a.nrows;
+    float2 v[8];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int n = g + G * e;
+        float2 x = make_float2(0.f, 0.f);
+        if (ok && n < H) {
+            if constexpr (MODE == BLUE_R2C) {
+                const float* src = rin + a.real_at(r);
+                if (even) {
+                    if (2 * n < a.n_real) x.x = src[2 * n];
+                    if (2 * n + 1 < a.n_real) x.y = src[2 * n + 1];
+                } else if (n < a.n_real) {
+                    x.x = src[n];
+                }
+            } else {
+                const float2* X = cin + a.cplx_at(r);
+                if (even) x = c2r_merge<float>(X[n], X[H - n], twP[n]);
+                else x = n <= H / 2 ? X[n] : cconj<float>(X[H - n]);
+            }
         }
-        scr[t] = v;
+        v[e] = x;
     }
-}
-__global__ void k_blue_mul(float2* __restrict__ scr, const float2* __restrict__ B, int Lp, long nlines) {
-    const long tot = nlines * Lp;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x)
-        scr[t] = cmul<float>(scr[t], B[t % Lp]);
-}
-__global__ void k_blue_post(float2* __restrict__ data, const float2* __restrict__ scr, const float2* __restrict__ w,
-                            int Lp, long nlines, long n_inner, long inner, long outer, long estride, int nkeep) {
-    const long tot = nlines * nkeep;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long l = t / nkeep;
-        const int k = (int)(t - l * nkeep);
-        data[(l / n_inner) * outer + (l % n_inner) * inner + (long)k * estride] = cmul<float>(scr[l * Lp + k], w[k]);
+    for (int t = threadIdx.x; t < Lp; t += G * nr) twl[t] = tw[t];
+    __syncthreads();
+    blue_transform<Lp, MODE == BLUE_R2C ? -1 : +1>(v, g, StridedBuf{buf, 0}, w, B, twl, H);
+    if constexpr (MODE == BLUE_R2C) {
+        if (even) {  // uniform over the launch
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (g + G * e < H) buf[g + G * e] = v[e];
+            __syncthreads();
+        }
+        if (!ok) return;
+        float2* dst = cout + a.cplx_at(r);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int k = g + G * e;
+            if (even) {
+                if (k < H) dst[k] = r2c_split<float>(v[e], buf[k ? H - k : 0], twP[k]);
+                if (k == 0) dst[H] = make_float2(v[e].x - v[e].y, 0.f);
+            } else if (k <= H / 2) {
+                dst[k] = v[e];
+            }
+        }
+    } else {
+        if (!ok) return;
+        float* dst = rout + a.real_at(r);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int n = g + G * e;
+            if (n >= H) continue;
+            if (even) {
+                if (2 * n < a.n_real) dst[2 * n] = v[e].x;
+                if (2 * n + 1 < a.n_real) dst[2 * n + 1] = v[e].y;
+            } else if (n < a.n_real) {
+                dst[n] = v[e].x;
+            }
+        }
     }
 }
 
-static int grid_for(long n) {
-    long g = (n + 255) / 256;
-    if (g > 65536) g = 65536;
-    return (int)(g < 1 ? 1 : g);
-}
+#define GK_FOR_EACH_BLUE(X) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096)
 
-static int blue_length(int L) {
+int fft_blue_length(int L) {
+    RadixList rl;
+    if (fft_length_supported(L) || factor_radices(L, rl)) return 0;
     int Lp = 1;
     while (Lp < 2 * L - 1) Lp *= 2;
     return Lp;
 }
 
-size_t fft_lines_any_scratch(int L, long nlines) {
-    if (nlines <= 0 || fft_length_supported(L)) return 0;
-    RadixList rl;
-    if (factor_radices(L, rl)) return 0;
-    return (size_t)nlines * blue_length(L);
+// lines (log2) and rows per block: the choices of k_lines_reg and k_rows_r2c_reg
+static int blue_shift(int Lp, unsigned nlines) {
+    const int G = Lp / 8;
+    int sh = 3;
+    while ((G << (sh + 1)) <= 256) sh++;
+    while (sh > 0 && ((G << sh) > 1024 || (((blue_buf(Lp) << sh) + Lp) * 8) > 60 * 1024)) sh--;
+    while (sh > 2 && (G << (sh - 1)) >= 64 && (nlines >> sh) < 512) sh--;
+    return sh;
+}
+static int blue_rows(int Lp, unsigned nrows) {
+    const int G = Lp / 8;
+    int nr = 1;
+    while (2 * nr * G <= 256 && (2 * nr * blue_buf(Lp) + Lp) * 8 <= 60 * 1024) nr *= 2;
+    while (nr > 1 && nr / 2 * G >= 64 && nrows / nr < 512) nr /= 2;
+    return nr;
+}
+template <int DIR> static void lines_blue(float2* data, int L, const LineArgs& a, hipStream_t s) {
+    const BlueTables& bt = blue_tables(L, DIR);
+    const float2* tw = twiddle_f32(bt.Lp);
+    const int sh = blue_shift(bt.Lp, a.nlines);
+    switch (bt.Lp) {
+#define GK_CASE(n)                                                                                               \
+    case n:                                                                                                      \
+        k_lines_blue<n, DIR><<<div_up(a.nlines, 1L << sh), blue_G(n) << sh, ((blue_buf(n) << sh) + n) * 8, s>>>( \
+            data, bt.w, bt.B, tw, L, a, sh);                                                                     \
+        break;
+        GK_FOR_EACH_BLUE(GK_CASE)
+#undef GK_CASE
+    default: GK_ASSERT(false, "FFT length %d is not supported", L);
+    }
+    GK_LAUNCH_CHECK();
+}
+template <int MODE>
+static void rows_blue(const float* rin, float* rout, const float2* cin, float2* cout, int P, const RowArgs& a,
+                      hipStream_t s) {
+    const int even = P % 2 == 0, H = even ? P / 2 : P;
+    const BlueTables& bt = blue_tables(H, MODE == BLUE_R2C ? -1 : +1);
+    const float2* tw = twiddle_f32(bt.Lp);
+    const float2* twP = even ? twiddle_f32(P) : nullptr;
+    const int nr = blue_rows(bt.Lp, a.nrows);
+    switch (bt.Lp) {
+#define GK_CASE(n)                                                                                                \
+    case n:                                                                                                       \
+        k_rows_blue<n, MODE><<<div_up(a.nrows, nr), blue_G(n) * nr, (blue_buf(n) * nr + n) * 8, s>>>(             \
+            rin, rout, cin, cout, bt.w, bt.B, tw, twP, H, even, a, nr);                                           \
+        break;
+        GK_FOR_EACH_BLUE(GK_CASE)
+#undef GK_CASE
+    default: GK_ASSERT(false, "FFT length %d is not supported", P);
+    }
+    GK_LAUNCH_CHECK();
 }
 
+// ---------------------------------------------------------------- any length
 void fft_lines_any_tables(int L, int dir) {
     RadixList rl;
     if (fft_length_supported(L) || factor_radices(L, rl)) {
@@ -218,16 +460,26 @@ void fft_lines_any_tables(int L, int dir) {
         return;
     }
     blue_tables(L, dir);
-    twiddle_f32(blue_length(L));
+    twiddle_f32(fft_blue_length(L));
 }
 
 template <typename T, int DIR>
 void fft_lines_any(C2<T>* data, int L, long nlines, long n_inner, long inner, long outer, long estride, int nvalid,
-                   int nkeep, hipStream_t s, const FFTScratch* sc) {
+                   int nkeep, hipStream_t s) {
     if (nlines <= 0) return;
-    if (fft_length_supported(L)) {
-        fft_lines<T, DIR>(data, L, nlines, n_inner, inner, outer, estride, nvalid, nkeep, s);
-        return;
+    if constexpr (sizeof(T) == 8) {
+        if (fft_length_supported(L)) {
+            fft_lines<T, DIR>(data, L, nlines, n_inner, inner, outer, estride, nvalid, nkeep, s);
+            return;
+        }
+    }
+    GK_ASSERT(nlines < (1L << 31) && n_inner < (1L << 31), "FFT of %ld lines", nlines);
+    const LineArgs a{(unsigned)nlines, (unsigned)n_inner, inner, outer, estride, nvalid, nkeep};
+    if constexpr (sizeof(T) == 4) {
+        if (fft_reg_length(L)) {
+            fft_lines_reg<DIR>(data, L, a, s);
+            return;
+        }
     }
     RadixList rl;
     if (factor_radices(L, rl)) {
@@ -235,192 +487,71 @@ void fft_lines_any(C2<T>* data, int L, long nlines, long n_inner, long inner, lo
         const C2<T>* tw;
         if constexpr (sizeof(T) == 4) tw = twiddle_f32(L);
         else tw = twiddle_f64(L);
-        const int nt = L <= 512 ? 64 : 256;
-        k_fft_lines_rt<T, DIR><<<(unsigned)nlines, nt, 2 * L * sizeof(C2<T>), s>>>(data, tw, L, rl, nlines, n_inner,
-                                                                                   inner, outer, estride, nvalid, nkeep);
+        const int sh = rt_shift<T>(L, a.nlines);
+        k_fft_lines_rt<T, DIR><<<div_up(nlines, 1L << sh), 256, (2 * L * sizeof(C2<T>)) << sh, s>>>(data, tw, L, rl, a, sh);
         GK_LAUNCH_CHECK();
         return;
     }
-    if constexpr (sizeof(T) == 4) {
-        const BlueTables& bt = blue_tables(L, DIR);
-        GK_ASSERT(bt.Lp <= 4096 * 2 && fft_length_supported(bt.Lp), "FFT length %d is not supported", L);
-        float2* scr = nullptr;
-        if (sc) {
-            GK_ASSERT((size_t)nlines * bt.Lp <= sc->cap, "FFT scratch of %zu elements, %ld needed", sc->cap,
-                      nlines * (long)bt.Lp);
-            scr = sc->base;
-        } else {
-            GK_CHECK(hipMalloc(&scr, nlines * bt.Lp * sizeof(float2)));
-        }
-        k_blue_pre<<<grid_for(nlines * bt.Lp), 256, 0, s>>>(data, scr, bt.w, L, bt.Lp, nlines, n_inner, inner, outer,
-                                                          estride, nvalid);
-        GK_LAUNCH_CHECK();
-        fft_lines<float, -1>(scr, bt.Lp, nlines, nlines, bt.Lp, 0, 1, bt.Lp, bt.Lp, s);
-        k_blue_mul<<<grid_for(nlines * bt.Lp), 256, 0, s>>>(scr, bt.B, bt.Lp, nlines);
-        GK_LAUNCH_CHECK();
-        fft_lines<float, +1>(scr, bt.Lp, nlines, nlines, bt.Lp, 0, 1, bt.Lp, bt.Lp, s);
-        k_blue_post<<<grid_for(nlines * nkeep), 256, 0, s>>>(data, scr, bt.w, bt.Lp, nlines, n_inner, inner, outer,
-                                                           estride, nkeep);
-        GK_LAUNCH_CHECK();
-        if (!sc) {
-            GK_CHECK(hipStreamSynchronize(s));
-            GK_CHECK(hipFree(scr));
-        }
-    } else {
-        GK_ASSERT(false, "FP64 FFT length %d is not supported", L);
-    }
+    if constexpr (sizeof(T) == 4) lines_blue<DIR>(data, L, a, s);
+    else GK_ASSERT(false, "FP64 FFT length %d is not supported", L);
 }
 
-template void fft_lines_any<float, -1>(float2*, int, long, long, long, long, long, int, int, hipStream_t,
-                                       const FFTScratch*);
-template void fft_lines_any<float, +1>(float2*, int, long, long, long, long, long, int, int, hipStream_t,
-                                       const FFTScratch*);
-template void fft_lines_any<double, -1>(double2*, int, long, long, long, long, long, int, int, hipStream_t,
-                                        const FFTScratch*);
-template void fft_lines_any<double, +1>(double2*, int, long, long, long, long, long, int, int, hipStream_t,
-                                        const FFTScratch*);
-
-// ---------------------------------------------------------------- real rows of any length
-// row r: input at (r / n_inner) in_outer + (r % n_inner) in_inner (n_real floats),
-// output at (r / n_inner) out_outer + (r % n_inner) out_inner (P/2+1 complex)
-__global__ void k_rows_pack(const float* __restrict__ in, float2* __restrict__ z, int H, long nrows, long n_inner,
-                            long in_inner, long in_outer, int n_real, int interleave) {
-    const long tot = nrows * H;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long r = t / H;
-        const int n = (int)(t - r * H);
-        const float* row = in + (r / n_inner) * in_outer + (r % n_inner) * in_inner;
-        float a = 0.f, b = 0.f;
-        if (interleave) {  // z[n] = x[2n] + i x[2n+1]
-            if (2 * n < n_real) a = row[2 * n];
-            if (2 * n + 1 < n_real) b = row[2 * n + 1];
-        } else if (n < n_real) {
-            a = row[n];
-        }
-        z[t] = make_float2(a, b);
-    }
-}
-__global__ void k_rows_split(const float2* __restrict__ Z, float2* __restrict__ out, const float2* __restrict__ twP,
-                             int M, long nrows, long n_inner, long out_inner, long out_outer) {
-    const long tot = nrows * (M + 1);
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long r = t / (M + 1);
-        const int k = (int)(t - r * (M + 1));
-        const float2* z = Z + r * M;
-        float2 X;
-        if (k == M) X = make_float2(z[0].x - z[0].y, 0.f);
-        else X = r2c_split<float>(z[k], z[(M - k) % M], twP[k]);
-        out[(r / n_inner) * out_outer + (r % n_inner) * out_inner + k] = X;
-    }
-}
-__global__ void k_rows_keep(const float2* __restrict__ Z, float2* __restrict__ out, int P, int Q, long nrows,
-                            long n_inner, long out_inner, long out_outer) {
-    const long tot = nrows * Q;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long r = t / Q;
-        const int k = (int)(t - r * Q);
-        out[(r / n_inner) * out_outer + (r % n_inner) * out_inner + k] = Z[r * P + k];
-    }
-}
-// inverse: even P -> merged half-length spectrum; odd P -> full Hermitian spectrum
-__global__ void k_rows_merge(const float2* __restrict__ in, float2* __restrict__ Y, const float2* __restrict__ twP,
-                             int P, long nrows, long n_inner, long in_inner, long in_outer) {
-    const int even = (P & 1) == 0, H = even ? P / 2 : P;
-    const long tot = nrows * H;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long r = t / H;
-        const int k = (int)(t - r * H);
-        const float2* X = in + (r / n_inner) * in_outer + (r % n_inner) * in_inner;
-        if (even) Y[t] = c2r_merge<float>(X[k], X[H - k], twP[k]);
-        else Y[t] = k <= P / 2 ? X[k] : cconj<float>(X[P - k]);
-    }
-}
-__global__ void k_rows_unpack(const float2* __restrict__ Y, float* __restrict__ out, int H, long nrows, long n_inner,
-                              long out_inner, long out_outer, int n_real, int interleave) {
-    const long tot = nrows * (long)n_real;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long r = t / n_real;
-        const int i = (int)(t - r * n_real);
-        const float2 y = interleave ? Y[r * H + i / 2] : Y[r * H + i];
-        out[(r / n_inner) * out_outer + (r % n_inner) * out_inner + i] = interleave ? ((i & 1) ? y.y : y.x) : y.x;
-    }
-}
-
-size_t fft_rows_r2c_any_scratch(int P, long nrows) {
-    if (nrows <= 0 || (P % 2 == 0 && fft_length_supported(P / 2))) return 0;
-    const int H = P % 2 == 0 ? P / 2 : P;
-    return (size_t)nrows * H + fft_lines_any_scratch(H, nrows);
-}
+template void fft_lines_any<float, -1>(float2*, int, long, long, long, long, long, int, int, hipStream_t);
+template void fft_lines_any<float, +1>(float2*, int, long, long, long, long, long, int, int, hipStream_t);
+template void fft_lines_any<double, -1>(double2*, int, long, long, long, long, long, int, int, hipStream_t);
+template void fft_lines_any<double, +1>(double2*, int, long, long, long, long, long, int, int, hipStream_t);
 
 void fft_rows_any_tables(int P, int dir) {
-    if (P % 2 == 0) {
-        twiddle_f32(P);
-        if (fft_length_supported(P / 2)) {
-            twiddle_f32(P / 2);
-            return;
-        }
-        fft_lines_any_tables(P / 2, dir);
-    } else {
-        fft_lines_any_tables(P, dir);
-    }
+    const int H = P % 2 == 0 ? P / 2 : P;
+    if (P % 2 == 0) twiddle_f32(P);
+    fft_lines_any_tables(H, dir);
+}
+
+static RowArgs row_args(const void* real, long nrows, long n_inner, long real_inner, long real_outer, long cplx_inner,
+                        long cplx_outer, int n_real) {
+    GK_ASSERT(nrows < (1L << 31) && n_inner < (1L << 31), "FFT of %ld rows", nrows);
+    const int vec = n_real % 2 == 0 && real_inner % 2 == 0 && real_outer % 2 == 0 && (uintptr_t)real % 8 == 0;
+    return RowArgs{(unsigned)nrows, (unsigned)n_inner, real_inner, real_outer, cplx_inner, cplx_outer, n_real, vec};
 }
 
 void fft_rows_r2c_any(const float* in, float2* out, int P, long nrows, long n_inner, long in_inner, long in_outer,
-                      long out_inner, long out_outer, int n_real, hipStream_t s, const FFTScratch* sc) {
+                      long out_inner, long out_outer, int n_real, hipStream_t s) {
     if (nrows <= 0) return;
-    if (P % 2 == 0 && fft_length_supported(P / 2)) {
-        fft_rows_r2c(in, out, P, nrows, n_inner, in_inner, in_outer, out_inner, out_outer, n_real, s);
-        return;
-    }
-    const bool even = P % 2 == 0;
-    const int H = even ? P / 2 : P;
-    float2* z = nullptr;
-    FFTScratch rest;  // what the packed rows leave for the line transform
-    if (sc) {
-        GK_ASSERT(fft_rows_r2c_any_scratch(P, nrows) <= sc->cap, "FFT scratch of %zu elements, %zu needed", sc->cap,
-                  fft_rows_r2c_any_scratch(P, nrows));
-        z = sc->base;
-        rest.base = sc->base + (size_t)nrows * H;
-        rest.cap = sc->cap - (size_t)nrows * H;
+    GK_ASSERT(n_real <= P, "real FFT length %d (data %d)", P, n_real);
+    const RowArgs a = row_args(in, nrows, n_inner, in_inner, in_outer, out_inner, out_outer, n_real);
+    const int even = P % 2 == 0, H = even ? P / 2 : P;
+    RadixList rl;
+    if (even && fft_reg_length(H)) {
+        fft_rows_r2c_reg(in, out, P, a, s);
+    } else if (factor_radices(H, rl)) {
+        GK_ASSERT(2L * H * 8 <= 65536, "FFT length %d is too long for one block", H);
+        const int sh = rt_shift<float>(H, a.nrows);
+        k_rows_r2c_rt<<<div_up(nrows, 1L << sh), 256, (2 * H * 8) << sh, s>>>(
+            in, out, twiddle_f32(H), even ? twiddle_f32(P) : nullptr, H, even, rl, a, sh);
+        GK_LAUNCH_CHECK();
     } else {
-        GK_CHECK(hipMalloc(&z, nrows * H * sizeof(float2)));
-    }
-    k_rows_pack<<<grid_for(nrows * H), 256, 0, s>>>(in, z, H, nrows, n_inner, in_inner, in_outer, n_real, even);
-    GK_LAUNCH_CHECK();
-    fft_lines_any<float, -1>(z, H, nrows, nrows, H, 0, 1, H, H, s, sc ? &rest : nullptr);
-    if (even) {
-        k_rows_split<<<grid_for(nrows * (H + 1)), 256, 0, s>>>(z, out, twiddle_f32(P), H, nrows, n_inner, out_inner,
-                                                              out_outer);
-    } else {
-        k_rows_keep<<<grid_for(nrows * (P / 2 + 1)), 256, 0, s>>>(z, out, P, P / 2 + 1, nrows, n_inner, out_inner,
-                                                                 out_outer);
-    }
-    GK_LAUNCH_CHECK();
-    if (!sc) {
-        GK_CHECK(hipStreamSynchronize(s));
-        GK_CHECK(hipFree(z));
+        rows_blue<BLUE_R2C>(in, nullptr, nullptr, out, P, a, s);
     }
 }
 
 void fft_rows_c2r_any(const float2* in, float* out, int P, long nrows, long n_inner, long in_inner, long in_outer,
                       long out_inner, long out_outer, int n_real, hipStream_t s) {
     if (nrows <= 0) return;
-    if (P % 2 == 0 && fft_length_supported(P / 2)) {
-        fft_rows_c2r(in, out, P, nrows, n_inner, in_inner, in_outer, out_inner, out_outer, n_real, s);
-        return;
+    GK_ASSERT(n_real <= P, "real FFT length %d (data %d)", P, n_real);
+    const RowArgs a = row_args(out, nrows, n_inner, out_inner, out_outer, in_inner, in_outer, n_real);
+    const int even = P % 2 == 0, H = even ? P / 2 : P;
+    RadixList rl;
+    if (even && fft_reg_length(H)) {
+        fft_rows_c2r_reg(in, out, P, a, s);
+    } else if (factor_radices(H, rl)) {
+        GK_ASSERT(2L * H * 8 <= 65536, "FFT length %d is too long for one block", H);
+        const int sh = rt_shift<float>(H, a.nrows);
+        k_rows_c2r_rt<<<div_up(nrows, 1L << sh), 256, (2 * H * 8) << sh, s>>>(
+            in, out, twiddle_f32(H), even ? twiddle_f32(P) : nullptr, H, even, rl, a, sh);
+        GK_LAUNCH_CHECK();
+    } else {
+        rows_blue<BLUE_C2R>(nullptr, out, in, nullptr, P, a, s);
     }
-    const bool even = P % 2 == 0;
-    const int H = even ? P / 2 : P;
-    float2* y = nullptr;
-    GK_CHECK(hipMalloc(&y, nrows * H * sizeof(float2)));
-    k_rows_merge<<<grid_for(nrows * H), 256, 0, s>>>(in, y, twiddle_f32(P), P, nrows, n_inner, in_inner, in_outer);
-    GK_LAUNCH_CHECK();
-    fft_lines_any<float, +1>(y, H, nrows, nrows, H, 0, 1, H, H, s);
-    k_rows_unpack<<<grid_for(nrows * (long)n_real), 256, 0, s>>>(y, out, H, nrows, n_inner, out_inner, out_outer,
-                                                                n_real, even);
-    GK_LAUNCH_CHECK();
-    GK_CHECK(hipStreamSynchronize(s));
-    GK_CHECK(hipFree(y));
 }
 
 }  // namespace gk
