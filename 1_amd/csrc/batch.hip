@@ -172,6 +172,7 @@ int epi_rows_host(int M) {
     abort();
 }
 int lanes_host(int L) { return reg_fft_G(L); }  // RegFFT<L>::G
+int y2_cols_host(int L) { return std::max(1, 64 / (L / y2_E(L))); }  // Y2<L>::COLS
 
 // per length: threads and dynamic LDS bytes of a block in the dispatch kernels
 struct AnyShape {
@@ -204,7 +205,7 @@ AnyShape any_shape(int pass, int L) {
     }
     case 3:  // 2-D, L = PY
         switch (L) {
-#define GK_CASE(n) case n: return {kNT, y2r_lds<n>() * 8};
+#define GK_CASE(n) case n: return {Y2<n>::NT, Y2<n>::LDS * 8};
             GK_ANY_Y(GK_CASE)
 #undef GK_CASE
         }
@@ -408,7 +409,7 @@ void bl_y2d(mmBatch* b, const LaunchSet& ls, const BStage& sg) {
     const float2* tw = twiddle_f32(ls.L);
     switch (ls.L) {
 #define GK_CASE(n)                                                                                           \
-    case n: kb_y2r<n><<<ls.blocks, kNT, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, sg, tw); \
+    case n: kb_y2r<n><<<ls.blocks, Y2<n>::NT, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, sg, tw); \
         break;
         GK_LEN_Y(GK_CASE)
 #undef GK_CASE
@@ -563,6 +564,8 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
         d.twP = twiddle_f32(s->cp.P[2]);
         d.twY = s->cp.P[1] > 1 ? twiddle_f32(s->cp.P[1]) : nullptr;
         d.twX = s->cp.P[0] > 1 ? twiddle_f32(s->cp.P[0]) : nullptr;
+        d.dx = FastDiv(s->cp.N[0]);
+        d.dq = FastDiv(s->cp.Q);
         d.cp = ctrl_params(s);
         d.cp.n_err = d.nfin;
         d.cp.part_e = nullptr;  // the batched epilogue computes no energy
@@ -589,7 +592,7 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
         const int lpr = std::min(lpb, s->cp.P[1]);
         return s->cp.Q * div_up(s->cp.P[1], lpr);
     });
-    b->y2 = make_sets(b, d2, PY, [](const mmSim* s) { return div_up(s->cp.Q, 256 / lanes_host(s->cp.P[1])); });
+    b->y2 = make_sets(b, d2, PY, [](const mmSim* s) { return div_up(s->cp.Q, y2_cols_host(s->cp.P[1])); });
     b->yx = make_sets(b, dt, [](const mmSim* s) { return s->cp.P[1] * 64 + s->cp.P[0]; },
                       [](const mmSim* s) { return s->cp.Q; });
     b->fin = make_sets(b, all, [](const mmSim*) { return 0; }, [](const mmSim* s) { return fin_blocks(s); });

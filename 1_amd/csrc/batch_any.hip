@@ -121,14 +121,18 @@ __global__ __launch_bounds__(kYxyThreads) void kb_yxy_any(const BSim* sims, cons
     }
 }
 
-__global__ __launch_bounds__(kNT) void kb_y2r_any(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(Y2<1024>::NT) void kb_y2r_any(const BSim* sims, const int* idx, const int* start, int n,
                                                   BStage sg) {
     extern __shared__ float2 dyn[];
     const BBlock bb = bblock(sims, idx, start, n);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     switch (d.PY) {
-#define GK_CASE(py)     case py: b_y2r<py>(d, bb.lb, d.twY, dyn); break;
+#define GK_CASE(py)                                 \
+    case py:                                        \
+        if (threadIdx.x >= Y2<py>::NT) return;      \
+        b_y2r<py>(d, bb.lb, d.twY, dyn);            \
+        break;
         GK_ANY_Y(GK_CASE)
 #undef GK_CASE
     }

@@ -30,6 +30,7 @@ struct BSim {
     const float2* twP;  // Z padded length 2M
     const float2* twY;  // padded Y
     const float2* twX;  // padded X
+    FastDiv dx, dq;     // by Nx and Q (3-D Y passes)
 };
 
 // one RK stage, the same for every simulation of the batch
@@ -119,13 +120,13 @@ __device__ __forceinline__ void b_ypass(const BSim& d, int lb, const float2* __r
     if constexpr (TWL)
         for (int i = threadIdx.x; i < PY; i += kNT) twl[i] = tw[i];
     const int li = threadIdx.x / G, g = threadIdx.x % G;
-    const long nlines = 3L * d.Nx * d.Q;
-    const long line = (long)lb * LPB + li;
+    const unsigned nlines = 3u * d.Nx * d.Q, line = (unsigned)lb * LPB + li;
+    const YLine ln = ypass_line(line < nlines ? line : 0, d.dx, d.dq, d.Ny, PY);
     float2 v[E];
-    ypass_load<PY, FWD>(v, FWD ? d.B1 : d.B2, line, line < nlines, d.Nx, d.Ny, d.Q, g);
+    ypass_load<PY, FWD>(v, FWD ? d.B1 : d.B2, ln, line < nlines, d.Ny, g);
     __syncthreads();  // twiddle table
     reg_fft<float, PY, FWD ? -1 : +1>(v, g, lds + li * F::LDS, TWL ? twl : tw);
-    if (line < nlines) ypass_store<PY, FWD>(v, FWD ? d.B2 : d.B1, line, d.Nx, d.Ny, d.Q, g);
+    if (line < nlines) ypass_store<PY, FWD>(v, FWD ? d.B2 : d.B1, ln, d.Ny, g);
 }
 
 template <int PY, bool FWD>
@@ -150,7 +151,7 @@ __device__ __forceinline__ void b_xmul(const BSim& d, int lb, const float2* __re
     const int lpr = LPB < d.PY ? LPB : d.PY;
     const int rows = (d.PY + lpr - 1) / lpr;
     int kz, ky;
-    xmul_column(lb, (long)d.Q * rows, rows, lpr, li, d.PY, kz, ky);
+    xmul_column(lb, (unsigned)d.Q * rows, rows, lpr, li, d.PY, kz, ky);
     float2 v[3][E];
     xmul_load<PX>(v, d.B2, kz, ky, d.Nx, d.PY, d.Q, g);
     __syncthreads();  // twiddle table
@@ -195,36 +196,16 @@ __global__ __launch_bounds__(kYxyThreads) void kb_yxy(const BSim* sims, const in
     b_yxy<PY, PX>(d, bb.lb, twY, twX, lds);
 }
 
-// 2-D: lds holds the exchange buffers (LPB RegFFT<PY>::LDS) and then the
-// twiddle copy (PY, for PY <= 1024)
-template <int PY> constexpr int y2r_lds() {
-    return (kNT / RegFFT<PY>::G) * RegFFT<PY>::LDS + (PY <= 1024 ? PY : 1);
-}
+// 2-D: the columns of block lb
 template <int PY>
 __device__ __forceinline__ void b_y2r(const BSim& d, int lb, const float2* __restrict__ tw, float2* lds) {
-    using F = RegFFT<PY>;
-    constexpr int E = F::E, G = F::G, LPB = kNT / G;
-    constexpr bool TWL = PY <= 1024;
-    float2* twl = lds + LPB * F::LDS;
-    if constexpr (TWL)
-        for (int i = threadIdx.x; i < PY; i += kNT) twl[i] = tw[i];
-    const int li = threadIdx.x / G, g = threadIdx.x % G;
-    const long kz = (long)lb * LPB + li;
-    __syncthreads();  // twiddle table
-    if constexpr (E > 16) {
-        y2r_column_split<PY>(d.B1, d.Kc, kz, kz < d.Q, d.Ny, d.Q, g, lds + li * F::LDS, TWL ? twl : tw);
-    } else {
-        float2 v[3][E];
-        y2r_load<PY>(v, d.B1, kz, kz < d.Q, d.Ny, d.Q, g);
-        y2r_column<PY>(v, d.Kc, kz, kz < d.Q, d.Q, g, lds + li * F::LDS, TWL ? twl : tw);
-        if (kz < d.Q) y2r_store<PY>(v, d.B1, kz, d.Ny, d.Q, g);
-    }
+    y2_columns<PY>(d.B1, d.Kc, tw, (long)lb * Y2<PY>::COLS, d.Ny, d.Q, lds);
 }
 
 template <int PY>
-__global__ __launch_bounds__(kNT) void kb_y2r(const BSim* sims, const int* idx, const int* start, int n, BStage sg,
-                                              const float2* __restrict__ tw) {
-    __shared__ float2 lds[y2r_lds<PY>()];
+__global__ __launch_bounds__(Y2<PY>::NT) void kb_y2r(const BSim* sims, const int* idx, const int* start, int n,
+                                                     BStage sg, const float2* __restrict__ tw) {
+    __shared__ float2 lds[Y2<PY>::LDS];
     const BBlock bb = bblock(sims, idx, start, n);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
@@ -299,7 +280,7 @@ template <int M> constexpr int epi_rows_c() {
 // from dynamic shared memory sized for the launch's largest class.  A batch of
 // many small simulations of different sizes then issues a few launches per
 // stage instead of one per length class and pass.
-constexpr int kAnyLds = 80 * 1024;
+constexpr int kAnyLds = 96 * 1024;
 #define GK_ANY_M(X) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
 #define GK_ANY_Y(X) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(1024)
 inline bool any_m(int M) {

@@ -985,14 +985,16 @@ static void launch_y3d(const ConvPlan& cp, const EngineState* st, bool fwd, hipS
     const int PY = cp.P[1], Nx = cp.N[0], Ny = cp.N[1], Q = cp.Q;
     const float2* tw = twiddle_f32(PY);
     const long nlines = 3L * Nx * Q;
+    GK_ASSERT(nlines < (1L << 31), "%ld Y lines", nlines);
+    const FastDiv dx(Nx), dq(Q);
     switch (PY) {
 #define GK_CASE(n)                                                                              \
     case n: {                                                                                   \
         constexpr int LPB = kNT / RegFFT<n>::G;                                                 \
         int g = 0;                                                                              \
         const int nit = pipeline_split(div_up(nlines, LPB), (long)cp.tp.yb * cu_count(), &g); \
-        if (fwd) k_ypass<n, true><<<g, kNT, 0, s>>>(cp.B1, cp.B2, tw, st, Nx, Ny, Q, nit);      \
-        else k_ypass<n, false><<<g, kNT, 0, s>>>(cp.B2, cp.B1, tw, st, Nx, Ny, Q, nit);          \
+        if (fwd) k_ypass<n, true><<<g, kNT, 0, s>>>(cp.B1, cp.B2, tw, st, dx, dq, Ny, nit);     \
+        else k_ypass<n, false><<<g, kNT, 0, s>>>(cp.B2, cp.B1, tw, st, dx, dq, Ny, nit);         \
         break;                                                                                  \
     }
         GK_LEN_Y(GK_CASE)
@@ -1055,10 +1057,9 @@ static void launch_y2d(const ConvPlan& cp, const EngineState* st, hipStream_t s)
     switch (PY) {
 #define GK_CASE(n)                                                                              \
     case n: {                                                                                   \
-        constexpr int LPB = kNT / RegFFT<n>::G;                                                 \
         int g = 0;                                                                              \
-        const int nit = pipeline_split(div_up(Q, LPB), (long)cp.tp.y2b * cu_count(), &g);  \
-        k_y2r<n><<<g, kNT, 0, s>>>(cp.B1, cp.Kc, tw, st, Ny, Q, nit);                           \
+        const int nit = pipeline_split(div_up(Q, Y2<n>::COLS), (long)cp.tp.y2b * cu_count(), &g); \
+        k_y2r<n><<<g, Y2<n>::NT, 0, s>>>(cp.B1, cp.Kc, tw, st, Ny, Q, nit);                     \
         break;                                                                                  \
     }
         GK_LEN_Y(GK_CASE)

@@ -60,10 +60,19 @@ template <int W> __device__ __forceinline__ float2 shfl2(float2 v, int src) {
 // m + sum dt a_ij k_j applied while loading), transformed in registers; the
 // r2c split takes Z[M-k] from the partner lane by a shuffle, and the spectrum is
 // transposed through a padded LDS tile into B1[c][x][kz][y] (TR consecutive y).
-template <int M, int TR> constexpr int zfwd_lds() {
+//
+// The pass is bound by instruction issue as much as by memory (a wave takes 4
+// cycles per instruction, and small grids leave one or two waves per SIMD), so
+// index arithmetic is kept out of the loops: a thread's tile elements are a
+// fixed row r and kz = k0 + G u, one addition apart.  All of a lane's loads
+// (m, the earlier k_j, the twiddles of the split) are issued together, and the
+// transform's twiddles come from LDS.
+constexpr bool z_twl(int M) { return M > 1 && M <= 512; }  // longer tables stay in global memory
+template <int M, int TR> constexpr int zfwd_core() {
     constexpr int FFT_LDS = TR * RegFFT<M>::LDS, TILE_LDS = (M + 1) * (TR + 1);
     return FFT_LDS > TILE_LDS ? FFT_LDS : TILE_LDS;
 }
+template <int M, int TR> constexpr int zfwd_lds() { return zfwd_core<M, TR>() + (z_twl(M) ? M : 0); }
 
 // body: component c, plane x, rows y0..y0+TR; lds holds zfwd_lds<M,TR>() complex.
 // NK earlier stages enter the stage build (a compile-time count, so every load
@@ -81,48 +90,69 @@ __device__ __forceinline__ void zfwd_tile(const StageIn& si, float2* __restrict_
     const bool ok = row < nrows;
     const long N = (long)Nx * Ny * Nz;
     const long rbase = c * N + ((long)x * Ny + y0 + row) * Nz;
-    const float dt = si.st ? si.st->dt_used : 0.f;
-    float coef[6];
-#pragma unroll
-    for (int j = 0; j < 6; j++) coef[j] = dt * si.a[j];
-    float2 v[E];
+    float2 v[E], wp[E];
     if ((Nz & 1) == 0) {
         // pairs (2n, 2n+1) as float2: rows start at an even float offset
+        float2 kv[NK > 0 ? NK : 1][E];
 #pragma unroll
         for (int e = 0; e < E; e++) {
             const int n = g + G * e;
-            float2 z = make_float2(0.f, 0.f);
-            if (!pad_half<M>(e) && ok && 2 * n < Nz) {
-                z = *reinterpret_cast<const float2*>(si.m + rbase + 2 * n);
+            const bool in = !pad_half<M>(e) && ok && 2 * n < Nz;
+            v[e] = in ? *reinterpret_cast<const float2*>(si.m + rbase + 2 * n) : make_float2(0.f, 0.f);
 #pragma unroll
-                for (int j = 0; j < NK; j++) {
-                    const float2 kv = *reinterpret_cast<const float2*>(si.k[j] + rbase + 2 * n);
-                    z.x = fmaf(coef[j], kv.x, z.x);
-                    z.y = fmaf(coef[j], kv.y, z.y);
-                }
-                if (si.mout) *reinterpret_cast<float2*>(si.mout + rbase + 2 * n) = z;
+            for (int j = 0; j < NK; j++)
+                kv[j][e] = in ? *reinterpret_cast<const float2*>(si.k[j] + rbase + 2 * n) : make_float2(0.f, 0.f);
+        }
+#pragma unroll
+        for (int e = 0; e < E; e++) wp[e] = twP[g + G * e];
+        const float dt = si.st ? si.st->dt_used : 0.f;
+        const bool store = si.mout != nullptr;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int n = g + G * e;
+#pragma unroll
+            for (int j = 0; j < NK; j++) {
+                v[e].x = fmaf(dt * si.a[j], kv[j][e].x, v[e].x);
+                v[e].y = fmaf(dt * si.a[j], kv[j][e].y, v[e].y);
             }
-            v[e] = z;
+            if (store && !pad_half<M>(e) && ok && 2 * n < Nz) *reinterpret_cast<float2*>(si.mout + rbase + 2 * n) = v[e];
         }
     } else {
+        float ks[NK > 0 ? NK : 1][E][2], ms[E][2];
+#pragma unroll
+        for (int e = 0; e < E; e++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int i = 2 * (g + G * e) + h;
+                const bool in = !pad_half<M>(e) && ok && i < Nz;
+                ms[e][h] = in ? si.m[rbase + i] : 0.f;
+#pragma unroll
+                for (int j = 0; j < NK; j++) ks[j][e][h] = in ? si.k[j][rbase + i] : 0.f;
+            }
+#pragma unroll
+        for (int e = 0; e < E; e++) wp[e] = twP[g + G * e];
+        const float dt = si.st ? si.st->dt_used : 0.f;
+        const bool store = si.mout != nullptr;
 #pragma unroll
         for (int e = 0; e < E; e++) {
-            const int n = g + G * e;
-            float z2[2] = {0.f, 0.f};
-            for (int h = 0; h < 2; h++) {
-                const int i = 2 * n + h;
-                if (!pad_half<M>(e) && ok && i < Nz) {
-                    float a = si.m[rbase + i];
 #pragma unroll
-                    for (int j = 0; j < NK; j++) a = fmaf(coef[j], si.k[j][rbase + i], a);
-                    if (si.mout) si.mout[rbase + i] = a;
-                    z2[h] = a;
-                }
+            for (int h = 0; h < 2; h++) {
+                const int i = 2 * (g + G * e) + h;
+#pragma unroll
+                for (int j = 0; j < NK; j++) ms[e][h] = fmaf(dt * si.a[j], ks[j][e][h], ms[e][h]);
+                if (store && !pad_half<M>(e) && ok && i < Nz) si.mout[rbase + i] = ms[e][h];
             }
-            v[e] = make_float2(z2[0], z2[1]);
+            v[e] = make_float2(ms[e][0], ms[e][1]);
         }
     }
-    reg_fft<float, M, -1>(v, g, lds + row * F::LDS, twM);
+    const float2* tw = twM;
+    if constexpr (z_twl(M)) {
+        float2* twl = lds + zfwd_core<M, TR>();
+        for (int i = threadIdx.x; i < M; i += NT) twl[i] = twM[i];
+        tw = twl;
+    }
+    if constexpr (z_twl(M)) __syncthreads();
+    reg_fft<float, M, -1>(v, g, lds + row * F::LDS, tw);
     // r2c split: lane g holds Z[k], k = g + G e; Z[M-k] is in lane (G-g) % G at e' = E-1-e
     // (or, for g = 0, in this lane at e' = (E-e) % E)
     const int partner = (G - g) % G;
@@ -131,7 +161,7 @@ __device__ __forceinline__ void zfwd_tile(const StageIn& si, float2* __restrict_
     for (int e = 0; e < E; e++) {
         const float2 t = shfl2<G>(v[E - 1 - e], partner);
         const float2 zmk = g == 0 ? v[(E - e) % E] : t;
-        X[e] = r2c_split<float>(v[e], zmk, twP[g + G * e]);
+        X[e] = r2c_split<float>(v[e], zmk, wp[e]);
     }
     const float2 nyq = make_float2(v[0].x - v[0].y, 0.f);  // X[M], valid in lane 0
     __syncthreads();  // the FFT exchange buffer becomes the transpose tile
@@ -139,10 +169,13 @@ __device__ __forceinline__ void zfwd_tile(const StageIn& si, float2* __restrict_
     for (int e = 0; e < E; e++) lds[(g + G * e) * TS + row] = X[e];
     if (g == 0) lds[M * TS + row] = nyq;
     __syncthreads();
-    float2* dst = B1 + ((long)c * Nx + x) * Q * Ny + y0;
-    for (int t = threadIdx.x; t < Q * TR; t += NT) {
-        const int r = t % TR, kz = t / TR;
-        if (r < nrows) dst[(long)kz * Ny + r] = lds[kz * TS + r];
+    const int r = threadIdx.x % TR, k0 = threadIdx.x / TR;  // kz = k0 + G u (and kz = M)
+    float2* dst = B1 + ((long)c * Nx + x) * Q * Ny + y0 + (k0 * Ny + r);
+    const float2* tile = lds + k0 * TS + r;
+    if (r < nrows) {
+#pragma unroll
+        for (int u = 0; u < E; u++) dst[(long)(u * G * Ny)] = tile[u * G * TS];
+        if (k0 == 0) dst[(long)(M * Ny)] = tile[M * TS];
     }
 }
 
@@ -153,6 +186,31 @@ __global__ __launch_bounds__(TR * RegFFT<M>::G) void k_zfwd(StageIn si, float2* 
     __shared__ float2 lds[zfwd_lds<M, TR>()];
     if (si.st && !si.st->trial_active) return;
     zfwd_tile<M, TR, NK>(si, B1, twM, twP, Nx, Ny, Nz, blockIdx.z, blockIdx.y, blockIdx.x * TR, lds);
+}
+
+// A plane's spectra B1[kz][y0..y0+TR) (src, row pitch Ny) into the padded tile
+// [kz][TS]: thread t of the component's TR G threads takes row t % TR and kz =
+// t / TR + G u, loads issued 8 at a time.
+template <int M, int TR>
+__device__ __forceinline__ void zinv_load_tile(const float2* __restrict__ src, int Ny, int nrows, int t, float2* tile) {
+    constexpr int E = RegFFT<M>::E, G = RegFFT<M>::G, TS = TR + 1;
+    const int r = t % TR, k0 = t / TR;
+    const bool in = r < nrows;
+    src += k0 * Ny + (in ? r : 0);
+    tile += k0 * TS + r;
+    float2 last = make_float2(0.f, 0.f);
+    if (in && k0 == 0) last = src[(long)(M * Ny)];
+#pragma unroll
+    for (int u0 = 0; u0 < E; u0 += kUnroll) {
+        float2 w[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; u++)
+            if (u0 + u < E) w[u] = in ? src[(long)((u0 + u) * G * Ny)] : make_float2(0.f, 0.f);
+#pragma unroll
+        for (int u = 0; u < kUnroll; u++)
+            if (u0 + u < E) tile[(u0 + u) * G * TS] = w[u];
+    }
+    if (k0 == 0) tile[M * TS] = last;
 }
 
 // Z inverse: B1[c][x][kz][y0..y0+TR) -> rows of h.  The spectrum is read through
@@ -171,13 +229,13 @@ __global__ __launch_bounds__(TR * RegFFT<M>::G) void k_zinv(const float2* __rest
     const int c = blockIdx.z, x = blockIdx.y, y0 = blockIdx.x * TR;
     const int nrows = min(TR, Ny - y0);
     const float2* src = B1 + ((long)c * Nx + x) * Q * Ny + y0;
-    batched_copy<float2, NT>(
-        Q * TR,
-        [&](int t) {
-            const int r = t % TR, kz = t / TR;
-            return r < nrows ? src[(long)kz * Ny + r] : make_float2(0.f, 0.f);
-        },
-        [&](int t, float2 val) { lds[(t / TR) * TS + t % TR] = val; });
+    zinv_load_tile<M, TR>(src, Ny, nrows, threadIdx.x, lds);
+    const float2* tw = twM;
+    if constexpr (z_twl(M)) {
+        float2* twl = lds + zfwd_core<M, TR>();
+        for (int i = threadIdx.x; i < M; i += NT) twl[i] = twM[i];
+        tw = twl;
+    }
     __syncthreads();
     float2 v[E];
 #pragma unroll
@@ -186,7 +244,7 @@ __global__ __launch_bounds__(TR * RegFFT<M>::G) void k_zinv(const float2* __rest
         v[e] = c2r_merge<float>(lds[k * TS + row], lds[(M - k) * TS + row], twP[k]);
     }
     __syncthreads();  // the tile becomes the FFT exchange buffer
-    reg_fft<float, M, +1>(v, g, lds + row * F::LDS, twM);
+    reg_fft<float, M, +1>(v, g, lds + row * F::LDS, tw);
     if (row < nrows) {
         const long N = (long)Nx * Ny * Nz;
         float* dst = h + c * N + ((long)x * Ny + y0 + row) * Nz;
@@ -225,7 +283,7 @@ __host__ __device__ constexpr int zinv_epi_lds_elems(int M, int TR) {
 }
 template <int M, int TR> constexpr int zinv_epi_lds() {
     static_assert(RegFFT<M>::LDS == M + M / 8, "exchange buffer size");
-    return zinv_epi_lds_elems(M, TR);
+    return zinv_epi_lds_elems(M, TR) + (z_twl(M) ? M : 0);  // + the twiddle table
 }
 
 // body: plane x, rows y0..y0+TR, all 3 components; the per-block max |k| goes to
@@ -236,6 +294,11 @@ template <int M, int TR> constexpr int zinv_epi_lds() {
 // is the high-order solution (a_Sj = b_j): it is stored to ea.mhigh and the
 // error dt sum (b2_j - b_j) k_j, this stage's k included, is reduced per block
 // into ea.part_err (rk.go:381-403), in place of a separate final pass.
+// Where few earlier stages enter (NU <= 1) the cells' m and k_j are loaded with the
+// spectra, before the transform.  As in the forward pass, a thread's tile
+// elements, cells and twiddles need no division or 64-bit product per element
+// (the copy's, 16 per thread, and the cells' had cost more instructions than the
+// transform).
 template <int M, int TR, int NU, int FIN>
 __device__ __forceinline__ void zinv_epi_tile(const float2* __restrict__ B1, const EpiArgs& ea,
                                               const float2* __restrict__ twM, const float2* __restrict__ twP,
@@ -247,40 +310,13 @@ __device__ __forceinline__ void zinv_epi_tile(const float2* __restrict__ B1, con
     const int c = threadIdx.x / NR, rem = threadIdx.x - c * NR, row = rem / G, g = rem % G;
     const int nrows = min(TR, Ny - y0);
     if (threadIdx.x == 0) stage_field(ea.t, st, hext_s);
-    const long cst = (long)Nx * Q * Ny;
-    const float2* src = B1 + (long)x * Q * Ny + y0;
-    batched_copy<float2, NT>(
-        3 * Q * TR,
-        [&](int t) {
-            const int cc = t / (Q * TR), u = t - cc * (Q * TR), kz = u / TR, r = u - kz * TR;
-            return r < nrows ? src[cc * cst + (long)kz * Ny + r] : make_float2(0.f, 0.f);
-        },
-        [&](int t, float2 val) {
-            const int cc = t / (Q * TR), u = t - cc * (Q * TR), kz = u / TR, r = u - kz * TR;
-            lds[(cc * Q + kz) * TS + r] = val;
-        });
-    __syncthreads();
-    float2 v[E];
-    {
-        const float2* tile = lds + c * Q * TS;
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            const int k = g + G * e;
-            v[e] = c2r_merge<float>(tile[k * TS + row], tile[(M - k) * TS + row], twP[k]);
-        }
+    zinv_load_tile<M, TR>(B1 + ((long)c * Nx + x) * Q * Ny + y0, Ny, nrows, rem, lds + c * Q * TS);
+    const float2* tw = twM;
+    if constexpr (z_twl(M)) {
+        float2* twl = lds + zinv_epi_lds_elems(M, TR);
+        for (int i = threadIdx.x; i < M; i += NT) twl[i] = twM[i];
+        tw = twl;
     }
-    __syncthreads();  // the tiles become the FFT exchange buffers
-    reg_fft<float, M, +1>(v, g, lds + (c * TR + row) * F::LDS, twM);
-    __syncthreads();  // ... and then the h rows
-    const int nh = (Nz + 1) >> 1;
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        const int n = g + G * e;
-        if (!pad_half<M>(e) && n < nh) lds[(c * TR + row) * HS + n] = v[e];
-    }
-    __syncthreads();
-
-    const float hext[3] = {hext_s[0], hext_s[1], hext_s[2]};
     const float dt = st->dt_used;
     float ca[NU > 0 ? NU : 1], cb[NU > 0 ? NU : 1];
 #pragma unroll
@@ -294,6 +330,89 @@ __device__ __forceinline__ void zinv_epi_tile(const float2* __restrict__ B1, con
     for (int j = 0; j < NU; j++) ce[j] = FIN == 2 ? ea.ce[j] * (double)dt : 0.0;
     const double ce_self = FIN == 2 ? ea.ce_self * (double)dt : 0.0;
     const long N = (long)Nx * Ny * Nz;
+    const long rowbase = ((long)x * Ny + y0) * Nz;
+    // A thread's cells: pairs (2n, 2n+1) as float2 where rows start at an even
+    // float (VW = 2), else single cells.  The stage input mi (and the final sum hi,
+    // or the error of the earlier stages er) is accumulated from m and the k_j.
+    constexpr int IT2 = (TR * HS + NT - 1) / NT, IT1 = (2 * TR * HS + NT - 1) / NT;
+    struct Cells {
+        float mi[IT1][3], hi[FIN == 1 ? IT1 : 1][3];
+        double er[FIN == 2 ? IT1 : 1][3];
+    };
+    const bool pairs = (Nz & 1) == 0;
+    // cell index of slot it of this thread, -1 if none; row r and column z of the tile
+    auto cell1 = [&](int it, int& r, int& z) -> long {
+        const int p = threadIdx.x + it * NT;
+        r = p / (2 * HS);
+        z = p % (2 * HS);
+        return r < nrows && z < Nz ? rowbase + (r * Nz + z) : -1;
+    };
+    auto cell2 = [&](int it, int& r, int& n) -> long {
+        const int p = threadIdx.x + it * NT;
+        r = p / HS;
+        n = p % HS;
+        return r < nrows && 2 * n < Nz ? rowbase + (r * Nz + 2 * n) : -1;
+    };
+    float2 ai[IT2][3], af[IT2][3];
+    double ex[FIN == 2 ? IT2 : 1][3], ey[FIN == 2 ? IT2 : 1][3];
+    auto build2 = [&]() {
+#pragma unroll
+        for (int it = 0; it < IT2; it++) {
+            int r, n;
+            const long gi = cell2(it, r, n);
+            if (gi >= 0) {
+#pragma unroll
+                for (int q = 0; q < 3; q++) ai[it][q] = af[it][q] = *reinterpret_cast<const float2*>(ea.m + q * N + gi);
+                if constexpr (FIN == 2)
+#pragma unroll
+                    for (int q = 0; q < 3; q++) ex[it][q] = ey[it][q] = 0.0;
+#pragma unroll
+                for (int j = 0; j < NU; j++)
+#pragma unroll
+                    for (int q = 0; q < 3; q++) {
+                        const float2 kv = *reinterpret_cast<const float2*>(ea.k[j] + q * N + gi);
+                        ai[it][q].x = fmaf(ca[j], kv.x, ai[it][q].x);
+                        ai[it][q].y = fmaf(ca[j], kv.y, ai[it][q].y);
+                        if constexpr (FIN == 1) {
+                            af[it][q].x = fmaf(cb[j], kv.x, af[it][q].x);
+                            af[it][q].y = fmaf(cb[j], kv.y, af[it][q].y);
+                        }
+                        if constexpr (FIN == 2) {
+                            ex[it][q] = fma(ce[j], (double)kv.x, ex[it][q]);
+                            ey[it][q] = fma(ce[j], (double)kv.y, ey[it][q]);
+                        }
+                    }
+            }
+        }
+    };
+    constexpr bool PRE = NU <= 1 && FIN != 2 && E <= 12;
+    if constexpr (PRE)
+        if (pairs) build2();
+    float2 wp[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) wp[e] = twP[g + G * e];
+    __syncthreads();
+    float2 v[E];
+    {
+        const float2* tile = lds + c * Q * TS;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int k = g + G * e;
+            v[e] = c2r_merge<float>(tile[k * TS + row], tile[(M - k) * TS + row], wp[e]);
+        }
+    }
+    __syncthreads();  // the tiles become the FFT exchange buffers
+    reg_fft<float, M, +1>(v, g, lds + (c * TR + row) * F::LDS, tw);
+    __syncthreads();  // ... and then the h rows
+    const int nh = (Nz + 1) >> 1;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int n = g + G * e;
+        if (!pad_half<M>(e) && n < nh) lds[(c * TR + row) * HS + n] = v[e];
+    }
+    __syncthreads();
+
+    const float hext[3] = {hext_s[0], hext_s[1], hext_s[2]};
     float lmax = 0.f, emax = 0.f;
     double esum = 0.0;
     const bool want_e = ea.epart != nullptr;
@@ -332,48 +451,13 @@ __device__ __forceinline__ void zinv_epi_tile(const float2* __restrict__ B1, con
             for (int q = 0; q < 3; q++) o[q] = k[q];
         }
     };
-    const long rowbase = ((long)x * Ny + y0) * Nz;
-    if ((Nz & 1) == 0) {
-        // cell pairs (2n, 2n+1) as float2
-        constexpr int IT = (TR * HS + NT - 1) / NT;
-        const int nzh = Nz >> 1, P = nrows * nzh;
-        float2 ai[IT][3], af[IT][3];
-        double ex[FIN == 2 ? IT : 1][3], ey[FIN == 2 ? IT : 1][3];
+    if (pairs) {
+        if constexpr (!PRE) build2();
 #pragma unroll
-        for (int it = 0; it < IT; it++) {
-            const int p = threadIdx.x + it * NT;
-            if (p < P) {
-                const int r = p / nzh, n = p - r * nzh;
-                const long gi = rowbase + (long)r * Nz + 2 * n;
-#pragma unroll
-                for (int q = 0; q < 3; q++) ai[it][q] = af[it][q] = *reinterpret_cast<const float2*>(ea.m + q * N + gi);
-                if constexpr (FIN == 2)
-#pragma unroll
-                    for (int q = 0; q < 3; q++) ex[it][q] = ey[it][q] = 0.0;
-#pragma unroll
-                for (int j = 0; j < NU; j++)
-#pragma unroll
-                    for (int q = 0; q < 3; q++) {
-                        const float2 kv = *reinterpret_cast<const float2*>(ea.k[j] + q * N + gi);
-                        ai[it][q].x = fmaf(ca[j], kv.x, ai[it][q].x);
-                        ai[it][q].y = fmaf(ca[j], kv.y, ai[it][q].y);
-                        if constexpr (FIN == 1) {
-                            af[it][q].x = fmaf(cb[j], kv.x, af[it][q].x);
-                            af[it][q].y = fmaf(cb[j], kv.y, af[it][q].y);
-                        }
-                        if constexpr (FIN == 2) {
-                            ex[it][q] = fma(ce[j], (double)kv.x, ex[it][q]);
-                            ey[it][q] = fma(ce[j], (double)kv.y, ey[it][q]);
-                        }
-                    }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < IT; it++) {
-            const int p = threadIdx.x + it * NT;
-            if (p < P) {
-                const int r = p / nzh, n = p - r * nzh;
-                const long gi = rowbase + (long)r * Nz + 2 * n;
+        for (int it = 0; it < IT2; it++) {
+            int r, n;
+            const long gi = cell2(it, r, n);
+            if (gi >= 0) {
                 float2 hv[3];
 #pragma unroll
                 for (int q = 0; q < 3; q++) hv[q] = lds[(q * TR + r) * HS + n];
@@ -404,30 +488,45 @@ __device__ __forceinline__ void zinv_epi_tile(const float2* __restrict__ B1, con
             }
         }
     } else {
+        // rows of odd length: single cells, all of a thread's loads issued first
         const float* hf = reinterpret_cast<const float*>(lds);
-        const int P = nrows * Nz;
-        for (int p = threadIdx.x; p < P; p += NT) {
-            const int r = p / Nz, z = p - r * Nz;
-            const long gi = rowbase + (long)r * Nz + z;
-            float mi[3], hi[3], h[3], o[3];
-            double er[3] = {0.0, 0.0, 0.0};
+        Cells a;
 #pragma unroll
-            for (int q = 0; q < 3; q++) {
-                mi[q] = hi[q] = ea.m[q * N + gi];
-                h[q] = hf[(q * TR + r) * 2 * HS + z];
+        for (int it = 0; it < IT1; it++) {
+            int r, z;
+            const long gi = cell1(it, r, z);
+            if (gi >= 0) {
 #pragma unroll
-                for (int j = 0; j < NU; j++) {
-                    const float kv = ea.k[j][q * N + gi];
-                    mi[q] = fmaf(ca[j], kv, mi[q]);
-                    hi[q] = fmaf(cb[j], kv, hi[q]);
-                    if constexpr (FIN == 2) er[q] = fma(ce[j], (double)kv, er[q]);
+                for (int q = 0; q < 3; q++) {
+                    float mi = ea.m[q * N + gi], hi = mi;
+                    double er = 0.0;
+#pragma unroll
+                    for (int j = 0; j < NU; j++) {
+                        const float kv = ea.k[j][q * N + gi];
+                        mi = fmaf(ca[j], kv, mi);
+                        if constexpr (FIN == 1) hi = fmaf(cb[j], kv, hi);
+                        if constexpr (FIN == 2) er = fma(ce[j], (double)kv, er);
+                    }
+                    a.mi[it][q] = mi;
+                    if constexpr (FIN == 1) a.hi[it][q] = hi;
+                    if constexpr (FIN == 2) a.er[it][q] = er;
                 }
             }
-            finish(gi, mi, hi, er, h, o);
+        }
 #pragma unroll
-            for (int q = 0; q < 3; q++) {
-                ea.out[q * N + gi] = o[q];
-                if constexpr (FIN == 2) ea.mhigh[q * N + gi] = mi[q];
+        for (int it = 0; it < IT1; it++) {
+            int r, z;
+            const long gi = cell1(it, r, z);
+            if (gi >= 0) {
+                float h[3], o[3];
+#pragma unroll
+                for (int q = 0; q < 3; q++) h[q] = hf[(q * TR + r) * 2 * HS + z];
+                finish(gi, a.mi[it], a.hi[FIN == 1 ? it : 0], a.er[FIN == 2 ? it : 0], h, o);
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    ea.out[q * N + gi] = o[q];
+                    if constexpr (FIN == 2) ea.mhigh[q * N + gi] = a.mi[it][q];
+                }
             }
         }
     }
@@ -489,59 +588,54 @@ __global__ __launch_bounds__(3 * TR * RegFFT<M>::G) void k_zinv_epi(const float2
 // before transforming line i, so the memory of one line overlaps the FFT of
 // the previous one; twiddles come from LDS, so no global load sits between a
 // prefetch and its use.
-// B1 line (c, x, kz) and B2 line (c, kz, x) of a Y-pass line number (x fastest)
-__device__ __forceinline__ long ypass_b1(long ln, int Nx, int Ny, int Q) {
-    const int x = (int)(ln % Nx);
-    const long r = ln / Nx;
-    const int kz = (int)(r % Q), c = (int)(r / Q);
-    return (((long)c * Nx + x) * Q + kz) * Ny;
-}
-__device__ __forceinline__ long ypass_b2(long ln, int Nx, int Q, int PY) {
-    const int x = (int)(ln % Nx);
-    const long r = ln / Nx;
-    const int kz = (int)(r % Q), c = (int)(r / Q);
-    return (((long)c * Q + kz) * Nx + x) * PY;
+// Division of n < 2^31 by a runtime constant d >= 1 as a product: a pass's lines
+// cost two of these instead of four 64-bit divisions (about 100 instructions each,
+// twice the line's transform).
+struct FastDiv {
+    unsigned d, mul, shift;
+    FastDiv() = default;
+    explicit FastDiv(unsigned dv) : d(dv), mul(0), shift(31) {
+        while ((1ull << (shift - 31)) < dv) shift++;               // 2^(shift-31) >= d
+        mul = (unsigned)(((1ull << shift) + dv - 1) / dv);         // ceil(2^shift / d) <= 2^31 + 1
+    }
+    __device__ __forceinline__ unsigned div(unsigned n) const { return (unsigned)(((unsigned long long)n * mul) >> shift); }
+};
+// offsets of B1 line (c, x, kz) and B2 line (c, kz, x) of a Y-pass line number (x fastest)
+struct YLine {
+    long b1, b2;
+};
+__device__ __forceinline__ YLine ypass_line(unsigned ln, FastDiv dx, FastDiv dq, int Ny, int PY) {
+    const unsigned r = dx.div(ln), x = ln - r * dx.d;
+    const unsigned c = dq.div(r), kz = r - c * dq.d;
+    return YLine{(long)((c * dx.d + x) * dq.d + kz) * Ny, (long)((c * dq.d + kz) * dx.d + x) * PY};
 }
 // one line into the lane-strided registers of lane g (zeros when !ok)
 template <int PY, bool FWD>
-__device__ __forceinline__ void ypass_load(float2* v, const float2* __restrict__ src, long ln, bool ok, int Nx,
-                                           int Ny, int Q, int g) {
+__device__ __forceinline__ void ypass_load(float2* v, const float2* __restrict__ src, const YLine& ln, bool ok, int Ny,
+                                           int g) {
     using F = RegFFT<PY>;
-    if constexpr (FWD) {
-        const float2* p = src + ypass_b1(ok ? ln : 0, Nx, Ny, Q);
+    const float2* p = src + (FWD ? ln.b1 : ln.b2) + g;
 #pragma unroll
-        for (int e = 0; e < F::E; e++) {
-            const int i = g + F::G * e;
-            v[e] = (!pad_half<PY>(e) && ok && i < Ny) ? p[i] : make_float2(0.f, 0.f);
-        }
-    } else {
-        const float2* p = src + ypass_b2(ok ? ln : 0, Nx, Q, PY);
-#pragma unroll
-        for (int e = 0; e < F::E; e++) v[e] = ok ? p[g + F::G * e] : make_float2(0.f, 0.f);
+    for (int e = 0; e < F::E; e++) {
+        if constexpr (FWD) v[e] = (!pad_half<PY>(e) && ok && g + F::G * e < Ny) ? p[F::G * e] : make_float2(0.f, 0.f);
+        else v[e] = ok ? p[F::G * e] : make_float2(0.f, 0.f);
     }
 }
 template <int PY, bool FWD>
-__device__ __forceinline__ void ypass_store(const float2* v, float2* __restrict__ dst, long ln, int Nx, int Ny,
-                                            int Q, int g) {
+__device__ __forceinline__ void ypass_store(const float2* v, float2* __restrict__ dst, const YLine& ln, int Ny, int g) {
     using F = RegFFT<PY>;
-    if constexpr (FWD) {
-        float2* p = dst + ypass_b2(ln, Nx, Q, PY);
+    float2* p = dst + (FWD ? ln.b2 : ln.b1) + g;
 #pragma unroll
-        for (int e = 0; e < F::E; e++) p[g + F::G * e] = v[e];
-    } else {
-        float2* p = dst + ypass_b1(ln, Nx, Ny, Q);
-#pragma unroll
-        for (int e = 0; e < F::E; e++) {
-            const int i = g + F::G * e;
-            if (!pad_half<PY>(e) && i < Ny) p[i] = v[e];
-        }
+    for (int e = 0; e < F::E; e++) {
+        if constexpr (FWD) p[F::G * e] = v[e];
+        else if (!pad_half<PY>(e) && g + F::G * e < Ny) p[F::G * e] = v[e];
     }
 }
 
 template <int PY, bool FWD>
 __global__ __launch_bounds__(kNT) void k_ypass(const float2* __restrict__ src, float2* __restrict__ dst,
-                                               const float2* __restrict__ tw, const EngineState* st, int Nx, int Ny,
-                                               int Q, int nit) {
+                                               const float2* __restrict__ tw, const EngineState* st, FastDiv dx,
+                                               FastDiv dq, int Ny, int nit) {
     using F = RegFFT<PY>;
     constexpr int E = F::E, G = F::G, LPB = kNT / G;
     constexpr bool TWL = PY <= 1024;  // twiddle table in LDS (longer lines keep it in global memory)
@@ -551,23 +645,27 @@ __global__ __launch_bounds__(kNT) void k_ypass(const float2* __restrict__ src, f
     if constexpr (TWL)
         for (int i = threadIdx.x; i < PY; i += kNT) twl[i] = tw[i];
     const int li = threadIdx.x / G, g = threadIdx.x % G;
-    const long nlines = 3L * Nx * Q, stride = (long)gridDim.x * LPB;
-    long line = (long)blockIdx.x * LPB + li;
+    const unsigned nlines = 3 * dx.d * dq.d, stride = gridDim.x * LPB;
+    unsigned line = blockIdx.x * LPB + li;
     constexpr bool PIPE = E <= 16;  // registers for a second line (longer lines load in place)
     float2 nxt[PIPE ? E : 1];
-    if constexpr (PIPE) ypass_load<PY, FWD>(nxt, src, line, line < nlines, Nx, Ny, Q, g);
+    YLine ln = ypass_line(line < nlines ? line : 0, dx, dq, Ny, PY);
+    if constexpr (PIPE) ypass_load<PY, FWD>(nxt, src, ln, line < nlines, Ny, g);
     __syncthreads();  // twiddle table
     for (int it = 0; it < nit; it++, line += stride) {
         float2 v[E];
+        const YLine cur = ln;
+        const unsigned next = line + stride;
+        if (it + 1 < nit) ln = ypass_line(next < nlines ? next : 0, dx, dq, Ny, PY);
         if constexpr (PIPE) {
 #pragma unroll
             for (int e = 0; e < E; e++) v[e] = nxt[e];
-            if (it + 1 < nit) ypass_load<PY, FWD>(nxt, src, line + stride, line + stride < nlines, Nx, Ny, Q, g);
+            if (it + 1 < nit) ypass_load<PY, FWD>(nxt, src, ln, next < nlines, Ny, g);
         } else {
-            ypass_load<PY, FWD>(v, src, line, line < nlines, Nx, Ny, Q, g);
+            ypass_load<PY, FWD>(v, src, cur, line < nlines, Ny, g);
         }
         reg_fft<float, PY, FWD ? -1 : +1>(v, g, lds + li * F::LDS, TWL ? twl : tw);
-        if (line < nlines) ypass_store<PY, FWD>(v, dst, line, Nx, Ny, Q, g);
+        if (line < nlines) ypass_store<PY, FWD>(v, dst, cur, Ny, g);
     }
 }
 
@@ -639,10 +737,10 @@ __device__ __forceinline__ void xmul_kernel(float2 (*v)[RegFFT<PX>::E], const fl
 }
 // column of item t for lane group li: items are (kz, run of lpr ky), with the
 // runs ky and PY - ky adjacent; ky < 0 when the lane group has no column
-__device__ __forceinline__ void xmul_column(long t, long items, int rows, int lpr, int li, int PY, int& kz,
-                                            int& ky) {
+__device__ __forceinline__ void xmul_column(unsigned t, unsigned items, unsigned rows, int lpr, int li, int PY,
+                                            int& kz, int& ky) {
     kz = (int)(t / rows);
-    const int rr = (int)(t % rows);
+    const int rr = (int)(t - kz * rows);
     const int r = (rr & 1) ? rows - 1 - (rr >> 1) : (rr >> 1);
     ky = (t < items && li < lpr && r * lpr + li < PY) ? r * lpr + li : -1;
 }
@@ -721,8 +819,7 @@ __global__ __launch_bounds__(kNT) void k_xmul_v(float2* __restrict__ B2, const f
     const int li = threadIdx.x / G, g = threadIdx.x % G;
     const int lpr = LPB < PY ? LPB : PY;
     const int rows = (PY + lpr - 1) / lpr;
-    const long items = (long)Q * rows;
-    const long t0 = (long)blockIdx.x * nit;
+    const unsigned items = (unsigned)Q * rows, t0 = blockIdx.x * nit;
     float2 nxt[3][E];
     if constexpr (PIPE) {
         int kz, ky;
@@ -731,7 +828,7 @@ __global__ __launch_bounds__(kNT) void k_xmul_v(float2* __restrict__ B2, const f
     }
     __syncthreads();  // twiddle table
     for (int it = 0; it < nit; it++) {
-        const long t = t0 + it;
+        const unsigned t = t0 + it;
         int kz, ky;
         xmul_column(t, items, rows, lpr, li, PY, kz, ky);
         float2 v[3][E];
@@ -770,8 +867,7 @@ __global__ __launch_bounds__(kNT) void k_xmul(float2* __restrict__ B2, const flo
     const int li = threadIdx.x / G, g = threadIdx.x % G;
     const int lpr = LPB < PY ? LPB : PY;  // columns per item
     const int rows = (PY + lpr - 1) / lpr;  // items per kz plane (the last may be partial)
-    const long items = (long)Q * rows;
-    const long t0 = (long)blockIdx.x * nit;
+    const unsigned items = (unsigned)Q * rows, t0 = blockIdx.x * nit;
     float2 nxt[3][E];
     {
         int kz, ky;
@@ -780,7 +876,7 @@ __global__ __launch_bounds__(kNT) void k_xmul(float2* __restrict__ B2, const flo
     }
     __syncthreads();  // twiddle table
     for (int it = 0; it < nit; it++) {
-        const long t = t0 + it;
+        const unsigned t = t0 + it;
         float2 v[3][E];
 #pragma unroll
         for (int c = 0; c < 3; c++)
@@ -1264,137 +1360,114 @@ __global__ __launch_bounds__(kYxyThreads) void k_yxy(float2* __restrict__ B1, co
     yxy_plane<PY, PX>(v, B1, Kc, twY, wx, Nx, Ny, Q, blockIdx.x, lds);
 }
 
-// 2-D: Y forward . kernel . Y inverse of one kz column (3 components) in
-// registers, in place in B1[c][0][kz][y].  Lane group li of a block takes
-// column kz; the 4 stored kernel components (xx, yy, zz, yz) for ky <= PY/2
-// are read with the yz sign restored for ky > PY/2.  Components c0..c0+NC.
-template <int PY, int NC = 3>
-__device__ __forceinline__ void y2r_load(float2 (*v)[RegFFT<PY>::E], const float2* __restrict__ B1, long kz, bool ok,
-                                         int Ny, int Q, int g, int c0 = 0) {
-    using F = RegFFT<PY>;
-    const long cs = (long)Q * Ny;
-    const float2* p = B1 + (ok ? kz : 0) * Ny;
-#pragma unroll
-    for (int c = 0; c < NC; c++)
-#pragma unroll
-        for (int e = 0; e < F::E; e++) {
-            const int i = g + F::G * e;
-            v[c][e] = (!pad_half<PY>(e) && ok && i < Ny) ? p[(c0 + c) * cs + i] : make_float2(0.f, 0.f);
-        }
-}
-template <int PY, int NC = 3>
-__device__ __forceinline__ void y2r_store(float2 (*v)[RegFFT<PY>::E], float2* __restrict__ B1, long kz, int Ny, int Q,
-                                          int g, int c0 = 0) {
-    using F = RegFFT<PY>;
-    const long cs = (long)Q * Ny;
-    float2* p = B1 + kz * Ny;
-#pragma unroll
-    for (int c = 0; c < NC; c++)
-#pragma unroll
-        for (int e = 0; e < F::E; e++) {
-            const int i = g + F::G * e;
-            if (!pad_half<PY>(e) && i < Ny) p[(c0 + c) * cs + i] = v[c][e];
-        }
-}
-// kernel multiply; C0 = 0: all 3 components in v[0..2]; C0 = 1: only x in v[0];
-// C0 = 2: only y, z in v[0..1]
-template <int PY, int C0 = 0>
-__device__ __forceinline__ void y2r_kernel(float2 (*v)[RegFFT<PY>::E], const float* __restrict__ Kc, long kz, int Q,
-                                           int g) {
-    GK_FFT_FP
-    using F = RegFFT<PY>;
-    constexpr int hy = PY / 2 + 1;
-    const long cs = (long)Q * hy;
-#pragma unroll
-    for (int e = 0; e < F::E; e++) {
-        const int ky = g + F::G * e;
-        const bool fy = ky > PY / 2;
-        const long b = kz * hy + (fy ? PY - ky : ky);
-        if constexpr (C0 <= 1) {
-            const float kxx = Kc[b];
-            const float2 a = v[0][e];
-            v[0][e] = make_float2(a.x * kxx, a.y * kxx);
-        }
-        if constexpr (C0 != 1) {
-            constexpr int o = C0 == 0 ? 1 : 0;
-            const float kyy = Kc[cs + b], kzz = Kc[2 * cs + b];
-            const float kyz = fy ? -Kc[3 * cs + b] : Kc[3 * cs + b];
-            const float2 bb = v[o][e], cc = v[o + 1][e];
-            v[o][e] = make_float2(bb.x * kyy + cc.x * kyz, bb.y * kyy + cc.y * kyz);
-            v[o + 1][e] = make_float2(bb.x * kyz + cc.x * kzz, bb.y * kyz + cc.y * kzz);
-        }
-    }
-}
-// transforms of one loaded column (every lane group of the block calls it: the
-// exchanges synchronise the block)
-template <int PY, int NC = 3, int C0 = 0>
-__device__ __forceinline__ void y2r_column(float2 (*v)[RegFFT<PY>::E], const float* __restrict__ Kc, long kz, bool ok,
-                                           int Q, int g, float2* lds, const float2* tw) {
-#pragma unroll
-    for (int c = 0; c < NC; c++) reg_fft<float, PY, -1>(v[c], g, lds, tw);
-    if (ok) y2r_kernel<PY, C0>(v, Kc, kz, Q, g);
-#pragma unroll
-    for (int c = 0; c < NC; c++) reg_fft<float, PY, +1>(v[c], g, lds, tw);
-}
-// long lines (more than 16 elements per lane): x alone, then the y-z pair,
-// to bound the registers of one column
+// 2-D: Y forward . kernel . Y inverse of kz columns, in place in B1[c][0][kz][y].
+// Each component of a column has lanes of its own (block = 3 x W threads, W =
+// max(64, G), thread group c; W / G columns per block), so a column's six
+// transforms run as two after one another; only y and z meet, through LDS, at the
+// kernel multiply (the 4 stored components xx, yy, zz, yz for ky <= PY/2, the yz
+// sign restored beyond).  A lane holds up to 8 (12 for 3 * 2^a) elements, so long
+// lines span several waves, with block barriers in their exchanges.  The kernel
+// values are loaded with the line, before the transforms (of long lines after the
+// forward transform: 80 registers, so that two blocks of 768 threads share a CU).
+//
+// The form this replaces held the 3 components in one lane group with L/64
+// elements per lane: one wave per SIMD, 4 cycles per instruction and nothing to
+// overlap.  Measured per launch (before / now): 1025 columns of 2048 (film 1024 x
+// 1024) 75 / 43 us; 385 of 384 (301 x 180) 15 / 8.2 us; 129 of 64 (128 x 32) 6.0 /
+// 4.4 us.
+constexpr int y2_E(int L) { return L % 3 == 0 ? (L < 12 ? L : 12) : (L < 8 ? L : (L <= 2048 ? 8 : 16)); }
+template <int PY> struct Y2 {
+    static constexpr int E = y2_E(PY), G = PY / E;
+    static constexpr int W = G > 64 ? G : 64;     // threads per component
+    static constexpr int NT = 3 * W, COLS = W / G;  // threads and columns per block
+    static constexpr int LINE = PY + PY / 8;      // exchange buffer of one line
+    static constexpr bool TWL = PY <= 2048;       // twiddle table in LDS
+    static constexpr int LDS = 3 * COLS * LINE + (TWL ? PY : 1);
+};
+// inputs / outputs at index >= PY/2 are padding (compile time, lane-strided i = g + G e)
+template <int PY> __device__ constexpr bool y2_pad(int e) { return Y2<PY>::E % 2 == 0 && e >= Y2<PY>::E / 2; }
+
+// columns kz0 .. kz0 + COLS of the block; every thread of the block calls it
 template <int PY>
-__device__ __forceinline__ void y2r_column_split(float2* __restrict__ B1, const float* __restrict__ Kc, long kz,
-                                                 bool ok, int Ny, int Q, int g, float2* lds, const float2* tw) {
-    constexpr int E = RegFFT<PY>::E;
-    {
-        float2 v[1][E];
-        y2r_load<PY, 1>(v, B1, kz, ok, Ny, Q, g, 0);
-        y2r_column<PY, 1, 1>(v, Kc, kz, ok, Q, g, lds, tw);
-        if (ok) y2r_store<PY, 1>(v, B1, kz, Ny, Q, g, 0);
+__device__ __forceinline__ void y2_columns(float2* __restrict__ B1, const float* __restrict__ Kc,
+                                           const float2* __restrict__ tw, long kz0, int Ny, int Q, float2* lds) {
+    using Y = Y2<PY>;
+    constexpr int E = Y::E, G = Y::G, hy = PY / 2 + 1;
+    constexpr bool WS = G <= 64;
+    const int c = threadIdx.x / Y::W, r = threadIdx.x % Y::W, li = r / G, g = r % G;
+    const long kz = kz0 + li;
+    const bool ok = kz < Q;
+    float2* p = B1 + ((long)c * Q + (ok ? kz : 0)) * Ny;
+    float2* line = lds + (c * Y::COLS + li) * Y::LINE;
+    float2 v[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int i = g + G * e;
+        v[e] = (!y2_pad<PY>(e) && ok && i < Ny) ? p[i] : make_float2(0.f, 0.f);
     }
-    {
-        float2 v[2][E];
-        y2r_load<PY, 2>(v, B1, kz, ok, Ny, Q, g, 1);
-        y2r_column<PY, 2, 2>(v, Kc, kz, ok, Q, g, lds, tw);
-        if (ok) y2r_store<PY, 2>(v, B1, kz, Ny, Q, g, 1);
+    // this component's diagonal value and, for y and z, kyz
+    float kd[E], ko[E];
+    auto load_kernel = [&]() {
+        const float* K = Kc + (ok ? kz : 0) * hy;
+        const long cs = (long)Q * hy;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int ky = g + G * e, kyp = ky > PY / 2 ? PY - ky : ky;
+            kd[e] = K[c * cs + kyp];
+            ko[e] = c ? K[3 * cs + kyp] : 0.f;
+        }
+    };
+    if constexpr (WS) load_kernel();
+    const float2* t = tw;
+    if constexpr (Y::TWL) {
+        float2* twl = lds + 3 * Y::COLS * Y::LINE;
+        for (int i = threadIdx.x; i < PY; i += Y::NT) twl[i] = tw[i];
+        t = twl;
+        __syncthreads();
     }
+    reg_fft<float, PY, -1, 1, E, WS>(v, g, line, t);
+    if (c) {
+#pragma unroll
+        for (int e = 0; e < E; e++) line[g + G * e] = v[e];
+    }
+    if constexpr (!WS) load_kernel();
+    __syncthreads();
+    {
+        GK_FFT_FP
+        const float2* other = lds + ((3 - c) * Y::COLS + li) * Y::LINE;  // the z line for y, the y line for z
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const float k = kd[e], kyz = g + G * e > PY / 2 ? -ko[e] : ko[e];
+            const float2 a = v[e];
+            if (c == 0) {
+                v[e] = make_float2(a.x * k, a.y * k);
+            } else {
+                const float2 o = other[g + G * e];
+                if (c == 1) v[e] = make_float2(a.x * k + o.x * kyz, a.y * k + o.y * kyz);
+                else v[e] = make_float2(o.x * kyz + a.x * k, o.y * kyz + a.y * k);
+            }
+        }
+    }
+    __syncthreads();  // the y and z lines become exchange buffers again
+    reg_fft<float, PY, +1, 1, E, WS>(v, g, line, t);
+    if (ok)
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int i = g + G * e;
+            if (!y2_pad<PY>(e) && i < Ny) p[i] = v[e];
+        }
 }
 
-// single simulation: persistent over kz columns, the next column loaded while
-// the current one is transformed (when its registers fit)
+// single simulation: a block walks nit column sets strided by the grid
 template <int PY>
-__global__ __launch_bounds__(kNT) void k_y2r(float2* __restrict__ B1, const float* __restrict__ Kc,
-                                             const float2* __restrict__ tw, const EngineState* st, int Ny, int Q,
-                                             int nit) {
-    using F = RegFFT<PY>;
-    constexpr int E = F::E, G = F::G, LPB = kNT / G;
-    constexpr bool TWL = PY <= 1024;
-    __shared__ float2 lds[LPB * F::LDS];
-    __shared__ float2 twl[TWL ? PY : 1];
+__global__ __launch_bounds__(Y2<PY>::NT) __attribute__((amdgpu_waves_per_eu(Y2<PY>::G > 128 ? 6 : 1))) void k_y2r(float2* __restrict__ B1, const float* __restrict__ Kc,
+                                                    const float2* __restrict__ tw, const EngineState* st, int Ny,
+                                                    int Q, int nit) {
+    __shared__ float2 lds[Y2<PY>::LDS];
     if (st && !st->trial_active) return;
-    if constexpr (TWL)
-        for (int i = threadIdx.x; i < PY; i += kNT) twl[i] = tw[i];
-    const int li = threadIdx.x / G, g = threadIdx.x % G;
-    const long stride = (long)gridDim.x * LPB;
-    long kz = (long)blockIdx.x * LPB + li;
-    constexpr bool PIPE = E <= 8;
-    float2 nxt[PIPE ? 3 : 1][PIPE ? E : 1];
-    if constexpr (PIPE) y2r_load<PY>(nxt, B1, kz, kz < Q, Ny, Q, g);
-    __syncthreads();  // twiddle table
-    if constexpr (E > 16) {
-        for (int it = 0; it < nit; it++, kz += stride)
-            y2r_column_split<PY>(B1, Kc, kz, kz < Q, Ny, Q, g, lds + li * F::LDS, TWL ? twl : tw);
-    } else {
-        for (int it = 0; it < nit; it++, kz += stride) {
-            float2 v[3][E];
-            if constexpr (PIPE) {
-#pragma unroll
-                for (int c = 0; c < 3; c++)
-#pragma unroll
-                    for (int e = 0; e < E; e++) v[c][e] = nxt[c][e];
-                if (it + 1 < nit) y2r_load<PY>(nxt, B1, kz + stride, kz + stride < Q, Ny, Q, g);
-            } else {
-                y2r_load<PY>(v, B1, kz, kz < Q, Ny, Q, g);
-            }
-            y2r_column<PY>(v, Kc, kz, kz < Q, Q, g, lds + li * F::LDS, TWL ? twl : tw);
-            if (kz < Q) y2r_store<PY>(v, B1, kz, Ny, Q, g);
-        }
+    for (int it = 0; it < nit; it++) {
+        if (it) __syncthreads();
+        y2_columns<PY>(B1, Kc, tw, ((long)it * gridDim.x + blockIdx.x) * Y2<PY>::COLS, Ny, Q, lds);
     }
 }
 
