@@ -33,15 +33,6 @@
 namespace gk {
 
 // ------------------------------------------------------------------ RK pointwise and control
-// FSAL: k_0 <- k_{S-1} for simulations that hold one (rk.go:311-315)
-__global__ __launch_bounds__(256) void kb_fsal_copy(const BSim* sims, const int* idx, const int* start, int n,
-                                                    int last) {
-    const int j = bfind(start, n, blockIdx.x);
-    const BSim& d = sims[idx[j]];
-    if (!d.st->trial_active || !d.st->fsal_init) return;
-    copy_body(d.k[0], d.k[last], 3 * d.N, (int)blockIdx.x - start[j], start[j + 1] - start[j]);
-}
-
 __global__ __launch_bounds__(256) void kb_rk_final(const BSim* sims, const int* idx, const int* start, int n,
                                                    FinalArgs fa) {
     const BBlock bb = bblock(sims, idx, start, n);
@@ -55,10 +46,11 @@ __global__ __launch_bounds__(256) void kb_rk_final(const BSim* sims, const int* 
     rk_final_body(d.m, kp, d.mtmp, d.st, a, (int)d.N, bb.lb, d.nfin);
 }
 
-__global__ __launch_bounds__(256) void kb_commit(const BSim* sims, const int* idx, const int* start, int n) {
+// last: the FSAL tableau's last stage, 0 for the others
+__global__ __launch_bounds__(256) void kb_commit(const BSim* sims, const int* idx, const int* start, int n, int last) {
     const BBlock bb = bblock(sims, idx, start, n);
     const BSim& d = *bb.d;
-    commit_body(d.m, d.mtmp, d.st, d.t.normMap, (int)d.N, bb.lb, d.nfin);
+    commit_body(d.m, d.mtmp, last ? d.k[0] : nullptr, d.k[last], d.st, d.t.normMap, (int)d.N, bb.lb, d.nfin);
 }
 
 // one thread per simulation
@@ -141,7 +133,7 @@ struct mmBatch {
     std::vector<void*> owned;  // device allocations of the tables
     TableImage image;          // set-up only: the tables before upload
     // per pass: one LaunchSet per length class
-    std::vector<LaunchSet> zf, yf, xm, yi, y2, yx, zi, fin, all256;
+    std::vector<LaunchSet> zf, yf, xm, yi, y2, yx, zi, fin;
     int useGraph = 1;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -446,11 +438,6 @@ void enqueue_btrial(mmBatch* b) {
         BStage sg{};
         sg.i = i;
         sg.fsal0 = (i == 0 && t.fsal) ? 1 : 0;
-        if (sg.fsal0)
-            for (auto& ls : b->all256) {
-                kb_fsal_copy<<<ls.blocks, 256, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, t.S - 1);
-                GK_LAUNCH_CHECK();
-            }
         for (int j = 0; j < t.S; j++)
             if (t.a[i][j] != 0.f) {
                 sg.kj[sg.nk] = j;
@@ -504,7 +491,7 @@ void enqueue_btrial(mmBatch* b) {
     GK_LAUNCH_CHECK();
     if (t.adaptive)
         for (auto& ls : b->fin) {
-            kb_commit<<<ls.blocks, 256, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt);
+            kb_commit<<<ls.blocks, 256, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, t.fsal ? t.S - 1 : 0);
             GK_LAUNCH_CHECK();
         }
 }
@@ -567,7 +554,10 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
         d.dx = FastDiv(s->cp.N[0]);
         d.dq = FastDiv(s->cp.Q);
         d.cp = ctrl_params(s);
-        d.cp.n_err = d.nfin;
+        // per-block maxima as this batch's Z inverse writes them: its rows per block are
+        // its own, and so is the number of blocks
+        d.cp.n_k = div_up(d.Ny, epi_rows_host(s->cp.M)) * d.Nx;
+        d.cp.n_err = b->tb.fsal_final() ? d.cp.n_k : d.nfin;
         d.cp.part_e = nullptr;  // the batched epilogue computes no energy
     }
     const size_t sims_off = b->image.put(h.data(), n * sizeof(BSim));
@@ -596,8 +586,6 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
     b->yx = make_sets(b, dt, [](const mmSim* s) { return s->cp.P[1] * 64 + s->cp.P[0]; },
                       [](const mmSim* s) { return s->cp.Q; });
     b->fin = make_sets(b, all, [](const mmSim*) { return 0; }, [](const mmSim* s) { return fin_blocks(s); });
-    b->all256 = make_sets(b, all, [](const mmSim*) { return 0; },
-                          [](const mmSim* s) { return std::max(1, std::min(1024, div_up(3L * s->N, 256 * 4))); });
     // small length classes of each pass: one dispatch launch per pass
     any_kernel_attributes();
     b->zf = merge_small(std::move(b->zf), 0);
@@ -607,7 +595,7 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
     b->yf = merge_small(std::move(b->yf), 4);
     b->yi = merge_small(std::move(b->yi), 4);
     b->xm = merge_small(std::move(b->xm), 5);
-    for (auto* sets : {&b->zf, &b->zi, &b->yf, &b->yi, &b->xm, &b->y2, &b->yx, &b->fin, &b->all256})
+    for (auto* sets : {&b->zf, &b->zi, &b->yf, &b->yi, &b->xm, &b->y2, &b->yx, &b->fin})
         stage_sets(b, *sets);
     // upload the tables: one block, one copy on the batch's stream from pinned memory
     {
@@ -619,7 +607,7 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
         GK_CHECK(hipStreamSynchronize(b->s));
         cached_host_free(host);
         b->dsims = (BSim*)(dev + sims_off);
-        for (auto* sets : {&b->zf, &b->zi, &b->yf, &b->yi, &b->xm, &b->y2, &b->yx, &b->fin, &b->all256})
+        for (auto* sets : {&b->zf, &b->zi, &b->yf, &b->yi, &b->xm, &b->y2, &b->yx, &b->fin})
             for (LaunchSet& ls : *sets) {
                 ls.idx = (int*)(dev + ls.idx_off);
                 ls.start = (int*)(dev + ls.start_off);
@@ -671,7 +659,7 @@ void mm_batch_start(mmBatch* b, const double* seconds, const long long* steps) {
         EngineState h = read_state(s);
         const double stop = seconds ? h.time + seconds[j] / s->unitTime : INFINITY;
         if (seconds) launch_normalize_active(s->m, nullptr, s->normMap, s->N, b->s);
-        launch_set_target(s->st, steps ? steps[j] : -1, stop, b->s);
+        launch_set_target(s->st, steps ? steps[j] : -1, stop, nullptr, b->s);
     }
     GK_CHECK(hipStreamSynchronize(b->s));
 }

@@ -486,6 +486,26 @@ __global__ void k_extract_full(const double2* __restrict__ W, int P0, int P1, in
 }
 
 // =============================================================== plan
+// The row variants of the Z passes that variant 0 stands for on a grid.
+// The passes are bound by instruction issue on small grids: a block's waves share
+// one CU, so rows are spread until every CU has blocks.  Z forward: half the rows
+// (8: 64 B runs of B1) below 4 blocks per CU, a quarter (32 B runs) below one.  Z
+// inverse: half below one block per CU, two rows where that still leaves fewer
+// (its reads of B1 are then 16 B runs, which the small spectra keep in L2).
+// Measured per launch with the length's rows / with these: 301 x 180 film, Z
+// forward of 5 stages 12.8 / 9.7 us, Z inverse 9.6 / 8.5 us; 150 x 91 x 3 slab 8.0 / 7.6
+// and 8.3 / 7.6 us; 70 x 60 x 51 block, Z forward 11.1 / 9.9 us.
+static void grid_rows(const int N[3], int M, int* zr, int* er) {
+    *zr = *er = 0;
+    const int zd = conv_z_rows(M, 0), ed = conv_epi_rows(M, 0);
+    auto zblocks = [&](int rows) { return 3L * N[0] * div_up(N[1], rows); };
+    if (zblocks(zd) < 1024 && conv_zr_valid(M, 1) && zd >= 16) *zr = 1;
+    if (*zr == 1 && zblocks(conv_z_rows(M, 1)) < 256 && conv_zr_valid(M, 3)) *zr = 3;
+    auto eblocks = [&](int rows) { return (long)N[0] * div_up(N[1], rows); };
+    if (eblocks(ed) < 256 && conv_er_valid(M, 1)) *er = 1;
+    if (*er == 1 && eblocks(conv_epi_rows(M, 1)) < 256 && conv_er_valid(M, 2)) *er = 2;
+}
+
 static int pad_len(int n) {
     // smallest register-FFT length 2^a or 3 * 2^a that is >= 2n (any P >= 2n - 1
     // gives the same linear convolution; the reference pads to exactly 2n)
@@ -521,13 +541,14 @@ void conv_plan_init(ConvPlan& cp, const int N[3]) {
     cp.bytes = kc * sizeof(float) + (b1 + b2) * sizeof(float2);
     cp.tp = TuneParams{};
     conv_tune_lookup(N, &cp.tp);
+    grid_rows(N, cp.M, &cp.zr0, &cp.er0);
 }
 
 int conv_epi_blocks_max(const int N[3]) {
     int P2 = pad_len(N[2]);
     if (P2 < 2) P2 = 2;
     const int M = P2 / 2;
-    return div_up(N[1], std::min(conv_epi_rows(M, 0), conv_epi_rows(M, 1))) * N[0];
+    return div_up(N[1], std::min(std::min(conv_epi_rows(M, 0), conv_epi_rows(M, 1)), conv_epi_rows(M, 2))) * N[0];
 }
 
 // ---------------------------------------------------------------- tuning table
@@ -894,9 +915,19 @@ static void launch_zfwd(const ConvPlan& cp, const StageIn& in, hipStream_t s) {
     GK_LAUNCH_CHECK();
 }
 
+int conv_z_rows(int M, int v) {
+    switch (M) {
+#define GK_CASE(n) \
+    case n: return z_rows_v<n>(v);
+        GK_LEN_M(GK_CASE)
+#undef GK_CASE
+    default: abort();
+    }
+}
+
 bool conv_zr_valid(int M, int v) {
     if (v == 0) return true;
-    if (v < 0 || v > 2) return false;
+    if (v < 0 || v > 3) return false;
     switch (M) {
 #define GK_CASE(n) \
     case n: return z_rows_v<n>(v) != z_rows_v<n>(0);
@@ -930,9 +961,11 @@ int conv_epi_rows(int M, int v) {
     }
 }
 
-bool conv_er_valid(int M, int v) { return v == 0 || (v == 1 && conv_epi_rows(M, 1) != conv_epi_rows(M, 0)); }
+bool conv_er_valid(int M, int v) {
+    return v == 0 || ((v == 1 || v == 2) && conv_epi_rows(M, v) != conv_epi_rows(M, 0));
+}
 
-int conv_epi_blocks(const ConvPlan& cp) { return div_up(cp.N[1], conv_epi_rows(cp.M, cp.tp.er)) * cp.N[0]; }
+int conv_epi_blocks(const ConvPlan& cp) { return div_up(cp.N[1], conv_epi_rows(cp.M, cp.er())) * cp.N[0]; }
 
 static void launch_zinv_epi(const ConvPlan& cp, const EpiArgs& ea, const EngineState* st, hipStream_t s) {
     const int M = cp.M;

@@ -16,7 +16,7 @@ template <int M> constexpr int z_rows() {
 }
 
 // rows per Z forward block of shape variant v: 0 the default, 1 half of it, 2
-// double (while the block stays within 1024 threads and 80 KB of LDS).  Short
+// double (while the block stays within 1024 threads and 80 KB of LDS), 3 a quarter.  Short
 // rows (M < 32) have one shape; a variant that does not exist gives the default.
 template <int M> constexpr int z_rows_v(int v) {
     constexpr int d = z_rows<M>();
@@ -27,6 +27,7 @@ template <int M> constexpr int z_rows_v(int v) {
         const int fft = t * RegFFT<M>::LDS, tile = (M + 1) * (t + 1);
         return (t * RegFFT<M>::G <= 1024 && (fft > tile ? fft : tile) * 8 <= 80 * 1024) ? t : d;
     }
+    if (v == 3) return d >= 16 ? d / 4 : d;  // small grids: more blocks
     return d;
 }
 
@@ -43,10 +44,13 @@ template <int M> constexpr int epi_rows() {
     return tr;
 }
 
-// rows per fused Z inverse block of shape variant v: 0 the default, 1 half of it
+// rows per fused Z inverse block of shape variant v: 0 the default, 1 half of it,
+// 2 two rows (where that is less than half; small grids: more blocks)
 template <int M> constexpr int epi_rows_v(int v) {
     constexpr int d = epi_rows<M>();
-    return (v == 1 && M >= 32 && d > 1) ? d / 2 : d;
+    if (M < 32) return d;
+    if (v == 2) return d > 4 ? 2 : d;
+    return (v == 1 && d > 1) ? d / 2 : d;
 }
 
 template <int M>

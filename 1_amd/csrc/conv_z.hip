@@ -46,8 +46,9 @@ static void zinv_epi_launch(const ConvPlan& cp, const EpiArgs& e, const EngineSt
 
 template <int M>
 void zfwd_run(const ConvPlan& cp, const StageIn& si, int NKp, const float2* twM, const float2* twP, hipStream_t s) {
-    if (cp.tp.zr == 1) zfwd_launch<M, z_rows_v<M>(1)>(cp, si, NKp, twM, twP, s);
-    else if (cp.tp.zr == 2) zfwd_launch<M, z_rows_v<M>(2)>(cp, si, NKp, twM, twP, s);
+    if (cp.zr() == 1) zfwd_launch<M, z_rows_v<M>(1)>(cp, si, NKp, twM, twP, s);
+    else if (cp.zr() == 2) zfwd_launch<M, z_rows_v<M>(2)>(cp, si, NKp, twM, twP, s);
+    else if (cp.zr() == 3) zfwd_launch<M, z_rows_v<M>(3)>(cp, si, NKp, twM, twP, s);
     else zfwd_launch<M, z_rows_v<M>(0)>(cp, si, NKp, twM, twP, s);
 }
 
@@ -61,7 +62,8 @@ void zinv_run(const ConvPlan& cp, float* h, const EngineState* st, const float2*
 template <int M>
 void zinv_epi_run(const ConvPlan& cp, const EpiArgs& e, const EngineState* st, const float2* twM, const float2* twP,
                   hipStream_t s) {
-    if (cp.tp.er == 1) zinv_epi_launch<M, epi_rows_v<M>(1)>(cp, e, st, twM, twP, s);
+    if (cp.er() == 1) zinv_epi_launch<M, epi_rows_v<M>(1)>(cp, e, st, twM, twP, s);
+    else if (cp.er() == 2) zinv_epi_launch<M, epi_rows_v<M>(2)>(cp, e, st, twM, twP, s);
     else zinv_epi_launch<M, epi_rows_v<M>(0)>(cp, e, st, twM, twP, s);
 }
 

@@ -45,6 +45,9 @@ struct EngineState {
     int nonfinite;      // max |torque| or the error estimate was NaN or infinite: the run stopped
     float dt_noise;     // dt at the start of the current step: the thermal field's (rk.go:289-292)
     long long noise_step;  // step the thermal field was drawn for (its counter)
+    int begun;          // the pending trial's start (ctrl_begin_body) has run already, with the end of the one before
+    int nk_last;        // per-block maxima the last trial's last stage wrote (alone and in a batch they differ)
+    int commit;         // what the commit after a trial does: 0 nothing, bit 0 the FSAL stage, bit 1 the new m
 };
 
 // |x| for a per-block maximum that must not lose a NaN: fmaxf returns the other
@@ -156,8 +159,8 @@ struct KernelSpec {
 // defaults are hand-picked; the autotuner (mm_sim_tune) times the candidates
 // on the device and a table of tuned values (per data size) feeds new plans.
 struct TuneParams {
-    int zr = 0;   // Z forward rows per block: variant 0 = z_rows<M>(), 1 = half, 2 = double
-    int er = 0;   // fused Z inverse rows per block: variant 0 = epi_rows<M>(), 1 = half
+    int zr = 0;   // Z forward rows per block: variant 0 = by the grid, 1 = half of z_rows<M>(), 2 = double, 3 = a quarter
+    int er = 0;   // fused Z inverse rows per block: variant 0 = by the grid, 1 = half of epi_rows<M>(), 2 = two rows
     int yb = 8;   // blocks per CU of the pipelined 3-D Y passes
     int xb = 4;   // blocks per CU of the pipelined X.K.X pass
     int y2b = 8;  // blocks per CU of the 2-D Y.K.Y pass
@@ -178,6 +181,9 @@ struct ConvPlan {
     int plane3; // 3-D plan the register-resident plane pass fits (used when tp.pp is set)
     size_t bytes;
     TuneParams tp;  // from the tuning table (conv_tune_lookup) when it holds N, else defaults
+    int zr0, er0;   // the row variants that variant 0 stands for on this grid
+    int zr() const { return tp.zr ? tp.zr : zr0; }
+    int er() const { return tp.er ? tp.er : er0; }
 };
 
 // Tuning table: data size N -> launch parameters (process-wide; conv_plan_init
@@ -191,6 +197,7 @@ void conv_tune_clear();
 // rows per block of the fused Z inverse for Z half-length M and variant v, and
 // whether variant v of the Z forward / fused Z inverse rows is a distinct shape
 int conv_epi_rows(int M, int v);
+int conv_z_rows(int M, int v);
 bool conv_zr_valid(int M, int v);
 bool conv_er_valid(int M, int v);
 bool conv_xv_valid(int PX, int v);
@@ -386,7 +393,6 @@ constexpr int kRedBlocks = 1024;
 // fixed step: m = normalize(m_high) in place.
 void launch_rk_final(float* m, const float* const k[7], float* mtmp, EngineState* st, const FinalArgs& a, int N,
                      hipStream_t s);
-void launch_copy_if_active(float* dst, const float* src, long n, const EngineState* st, hipStream_t s);
 
 struct CtrlParams {
     int adaptive;
@@ -406,17 +412,21 @@ struct CtrlParams {
     double cell_volume;     // internal units
     float cmax;             // largest stage node of the tableau (advances field_tmax)
     int thermal;            // T > 0: no dt control after the first torque (rk.go:348)
+    int fsal;               // FSAL tableau: the next trial's first k is this one's last
 };
-void launch_ctrl_begin(EngineState* st, hipStream_t s);
-void launch_ctrl_after_k0(EngineState* st, int fsal_copy, const CtrlParams& p, hipStream_t s);
+// the trial's end (step control), and then the next trial's start
+void launch_ctrl_after_k0(EngineState* st, const CtrlParams& p, hipStream_t s);
 void launch_ctrl_end(EngineState* st, const CtrlParams& p, hipStream_t s);
-void launch_commit(float* m, const float* mtmp, EngineState* st, const float* nmap, int N, hipStream_t s);
+// adaptive tableaux: the new m of an ended step, and the FSAL stage k0 <- klast (null: none)
+void launch_commit(float* m, const float* mtmp, float* k0, const float* klast, EngineState* st, const float* nmap,
+                   int N, hipStream_t s);
 void launch_normalize_active(float* m, const EngineState* st, const float* nmap, int N, hipStream_t s);
 
 void launch_energy(const float* m, const float* h, const float hext[3], int anisType, float kAnis, const float u[3],
                    int N, double* out, hipStream_t s);
-// steps_target = steps + nsteps (nsteps < 0: unlimited), stop time; recomputes `done`
-void launch_set_target(EngineState* st, long long nsteps, double stop, hipStream_t s);
+// steps_target = steps + nsteps (nsteps < 0: unlimited), stop time; recomputes
+// `done`; with p, also starts the first trial (as launch_ctrl_end does for the others)
+void launch_set_target(EngineState* st, long long nsteps, double stop, const CtrlParams* p, hipStream_t s);
 // FP64 reductions for outputs: sums[0..2] = sum of each component; energy
 void launch_sum3(const float* v, int N, double* out_dev, hipStream_t s);
 void launch_sum1(const float* v, int N, double* out_dev, hipStream_t s);

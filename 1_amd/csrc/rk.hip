@@ -61,15 +61,10 @@ __global__ __launch_bounds__(256) void k_rk_final(float* __restrict__ m, KPtrs k
     rk_final_body(m, kp, mtmp, st, a, N, blockIdx.x, gridDim.x);
 }
 
-__global__ void k_copy_if_active(float* __restrict__ dst, const float* __restrict__ src, long n,
-                                 const EngineState* st) {
-    if (!st->trial_active) return;
-    copy_body(dst, src, n, blockIdx.x, gridDim.x);
-}
-
 __global__ __launch_bounds__(256) void k_commit(float* __restrict__ m, const float* __restrict__ mtmp,
+                                                float* __restrict__ k0, const float* __restrict__ klast,
                                                 const EngineState* st, const float* __restrict__ nmap, int N) {
-    commit_body(m, mtmp, st, nmap, N, blockIdx.x, gridDim.x);
+    commit_body(m, mtmp, k0, klast, st, nmap, N, blockIdx.x, gridDim.x);
 }
 
 __global__ void k_normalize_active(float* __restrict__ m, const EngineState* st, const float* __restrict__ nmap,
@@ -85,9 +80,12 @@ __global__ void k_normalize_active(float* __restrict__ m, const EngineState* st,
 }
 
 // ---------------------------------------------------------------- control (one thread / one wave)
-__global__ void k_ctrl_begin(EngineState* st) { ctrl_begin_body(st); }
-__global__ void k_ctrl_after_k0(EngineState* st, int fsal_copy, CtrlParams p) { ctrl_after_k0_body(st, fsal_copy, p); }
-__global__ void k_ctrl_end(EngineState* st, CtrlParams p) { ctrl_end_body(st, p); }
+__global__ __launch_bounds__(64) void k_ctrl_after_k0(EngineState* st, CtrlParams p) { ctrl_after_k0_body(st, 0, p); }
+__global__ __launch_bounds__(64) void k_ctrl_end(EngineState* st, CtrlParams p) {
+    ctrl_end_body(st, p);
+    __syncthreads();
+    ctrl_next_body(st, p);
+}
 
 // ---------------------------------------------------------------- FP64 output reductions
 __global__ __launch_bounds__(256) void k_sum_comp(const float* __restrict__ v, int N, int ncomp,
@@ -134,11 +132,17 @@ __global__ __launch_bounds__(256) void k_energy(const float* __restrict__ m, con
     if (threadIdx.x == 0) atomicAdd(out, wsum[0] + wsum[1] + wsum[2] + wsum[3]);
 }
 
-__global__ void k_set_target(EngineState* st, long long nsteps, double stop) {
-    st->steps_target = nsteps < 0 ? 0x7fffffffffffffffLL : st->steps + nsteps;
-    st->stop = stop;
-    st->done = (st->time >= st->stop || st->steps >= st->steps_target) ? 1 : 0;
-    st->nan_dt = 0;
+__global__ __launch_bounds__(64) void k_set_target(EngineState* st, long long nsteps, double stop, CtrlParams p,
+                                                   int begin) {
+    if (threadIdx.x == 0) {
+        st->steps_target = nsteps < 0 ? 0x7fffffffffffffffLL : st->steps + nsteps;
+        st->stop = stop;
+        st->done = (st->time >= st->stop || st->steps >= st->steps_target) ? 1 : 0;
+        st->nan_dt = 0;
+        st->begun = 0;
+    }
+    __syncthreads();
+    if (begin) ctrl_next_body(st, p);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -160,8 +164,8 @@ void launch_set_active(EngineState* st, hipStream_t s) {
     k_set_active<<<1, 1, 0, s>>>(st);
     GK_LAUNCH_CHECK();
 }
-void launch_set_target(EngineState* st, long long nsteps, double stop, hipStream_t s) {
-    k_set_target<<<1, 1, 0, s>>>(st, nsteps, stop);
+void launch_set_target(EngineState* st, long long nsteps, double stop, const CtrlParams* p, hipStream_t s) {
+    k_set_target<<<1, 64, 0, s>>>(st, nsteps, stop, p ? *p : CtrlParams{}, p != nullptr);
     GK_LAUNCH_CHECK();
 }
 
@@ -186,25 +190,17 @@ void launch_rk_final(float* m, const float* const k[7], float* mtmp, EngineState
     GK_LAUNCH_CHECK();
 }
 
-void launch_copy_if_active(float* dst, const float* src, long n, const EngineState* st, hipStream_t s) {
-    k_copy_if_active<<<gridN(n), 256, 0, s>>>(dst, src, n, st);
-    GK_LAUNCH_CHECK();
-}
-
-void launch_ctrl_begin(EngineState* st, hipStream_t s) {
-    k_ctrl_begin<<<1, 1, 0, s>>>(st);
-    GK_LAUNCH_CHECK();
-}
-void launch_ctrl_after_k0(EngineState* st, int fsal_copy, const CtrlParams& p, hipStream_t s) {
-    k_ctrl_after_k0<<<1, 64, 0, s>>>(st, fsal_copy, p);
+void launch_ctrl_after_k0(EngineState* st, const CtrlParams& p, hipStream_t s) {
+    k_ctrl_after_k0<<<1, 64, 0, s>>>(st, p);
     GK_LAUNCH_CHECK();
 }
 void launch_ctrl_end(EngineState* st, const CtrlParams& p, hipStream_t s) {
     k_ctrl_end<<<1, 64, 0, s>>>(st, p);
     GK_LAUNCH_CHECK();
 }
-void launch_commit(float* m, const float* mtmp, EngineState* st, const float* nmap, int N, hipStream_t s) {
-    k_commit<<<gridN(N), 256, 0, s>>>(m, mtmp, st, nmap, N);
+void launch_commit(float* m, const float* mtmp, float* k0, const float* klast, EngineState* st, const float* nmap,
+                   int N, hipStream_t s) {
+    k_commit<<<gridN(N), 256, 0, s>>>(m, mtmp, k0, klast, st, nmap, N);
     GK_LAUNCH_CHECK();
 }
 void launch_normalize_active(float* m, const EngineState* st, const float* nmap, int N, hipStream_t s) {

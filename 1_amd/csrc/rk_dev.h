@@ -75,18 +75,20 @@ __device__ __forceinline__ void rk_final_body(float* __restrict__ m, const KPtrs
     }
 }
 
-__device__ __forceinline__ void copy_body(float* __restrict__ dst, const float* __restrict__ src, long n, int blk,
-                                          int nblk) {
-    for (long i = blk * (long)blockDim.x + threadIdx.x; i < n; i += (long)nblk * blockDim.x) dst[i] = src[i];
-}
-
 // accepted: m = normalize(m_high); step ended after the last rejected trial:
 // m (restored, i.e. untouched) is normalised (rk.go:426-444); with a norm map
-// each cell to its own norm (sim.go:230-239)
+// each cell to its own norm (sim.go:230-239).  FSAL tableaux: k0 <- klast after
+// every trial, accepted or not, as rk.go:311-315 does at the start of the next
+// (here, where the trial's stages are still in the caches and without a launch
+// of its own).  Bound by memory: 24 B per cell of m and of k.
 __device__ __forceinline__ void commit_body(float* __restrict__ m, const float* __restrict__ mtmp,
+                                            float* __restrict__ k0, const float* __restrict__ klast,
                                             const EngineState* st, const float* __restrict__ nmap, int N, int blk,
                                             int nblk) {
-    if (!st->trial_active || !st->step_end) return;
+    const int what = st->commit;
+    if (k0 && (what & 1))
+        for (long i = blk * (long)blockDim.x + threadIdx.x; i < 3L * N; i += (long)nblk * blockDim.x) k0[i] = klast[i];
+    if (!(what & 2)) return;
     const float* src = st->accept ? mtmp : m;
     for (int i = blk * blockDim.x + threadIdx.x; i < N; i += nblk * blockDim.x) {
         const float x = src[i], y = src[N + i], z = src[2 * N + i];
@@ -99,8 +101,10 @@ __device__ __forceinline__ void commit_body(float* __restrict__ m, const float* 
 
 // ---------------------------------------------------------------- control (single thread)
 __device__ __forceinline__ void ctrl_begin_body(EngineState* st) {
+    if (st->begun) return;
     st->trial_active = !st->done;
     if (!st->trial_active) return;
+    st->begun = 1;
     if (st->new_step) {
         st->time0 = st->time;
         st->trials = 0;
@@ -113,10 +117,17 @@ __device__ __forceinline__ void ctrl_begin_body(EngineState* st) {
     st->dt_used = st->dt;
 }
 
-// one wave reduces n per-block maxima; result valid in every lane
+// one wave reduces n per-block maxima (8 loads in flight per lane: the wave waits
+// for their latency, nothing else); result valid in every lane
 __device__ __forceinline__ float wave_max_partials(const float* part, int n) {
     float v = 0.f;
-    for (int i = threadIdx.x; i < n; i += 64) v = fmaxf(v, part[i]);
+    for (int i0 = threadIdx.x; i0 < n; i0 += 8 * 64) {
+        float w[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) w[u] = i0 + 64 * u < n ? part[i0 + 64 * u] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; u++) v = fmaxf(v, w[u]);
+    }
     for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
     return v;
 }
@@ -124,7 +135,7 @@ __device__ __forceinline__ float wave_max_partials(const float* part, int n) {
 // after k0 is known (rk.go:348-373); run by one wave
 __device__ __forceinline__ void ctrl_after_k0_body(EngineState* st, int fsal_copy, const CtrlParams& p) {
     if (!st->trial_active) return;
-    const float maxTorque = wave_max_partials(fsal_copy ? p.part_k6 : p.part_k0, p.n_k);
+    const float maxTorque = wave_max_partials(fsal_copy ? p.part_k6 : p.part_k0, fsal_copy ? st->nk_last : p.n_k);
     if (threadIdx.x != 0) return;
     if (!isfinite(maxTorque)) st->nonfinite = 1;
     if (p.thermal) return;  // rk.go:348: the dt control after k0 only runs at T = 0
@@ -143,7 +154,10 @@ __device__ __forceinline__ void ctrl_after_k0_body(EngineState* st, int fsal_cop
 
 // after the high/low solutions (rk.go:376-440); run by one wave
 __device__ __forceinline__ void ctrl_end_body(EngineState* st, const CtrlParams& p) {
-    if (!st->trial_active) return;
+    if (!st->trial_active) {
+        if (threadIdx.x == 0) st->commit = 0;
+        return;
+    }
     const float err_red = p.adaptive ? wave_max_partials(p.part_err, p.n_err) : 0.f;
     const float k0_red = p.fold_k0 ? wave_max_partials(p.part_k0, p.n_k) : 0.f;
     double e_red = 0.0;
@@ -185,6 +199,9 @@ __device__ __forceinline__ void ctrl_end_body(EngineState* st, const CtrlParams&
     if (bad) st->rejects_total++;
     st->accept = !bad;
     st->step_end = !bad || st->trials >= kMaxStepTrials || st->nonfinite;
+    st->commit = 1 | (st->step_end ? 2 : 0);
+    st->begun = 0;
+    st->nk_last = p.n_k;
     if (st->log_n < p.log_cap) {
         p.log_dt[st->log_n] = (double)dtu;
         p.log_accept[st->log_n] = !bad;
@@ -200,6 +217,19 @@ __device__ __forceinline__ void ctrl_end_body(EngineState* st, const CtrlParams&
         }
         if (st->time >= st->stop || st->steps >= st->steps_target || st->nan_dt || st->nonfinite) st->done = 1;
     }
+}
+
+// The start of the next trial, by one wave, right after the end of the one before
+// or the run's set-up: with an FSAL k it includes the dt control after k0.
+__device__ __forceinline__ void ctrl_next_body(EngineState* st, const CtrlParams& p) {
+    __shared__ int begun_now;
+    if (threadIdx.x == 0) {
+        begun_now = !st->begun;
+        ctrl_begin_body(st);
+    }
+    __syncthreads();
+    __threadfence_block();
+    if (begun_now && p.fsal && st->fsal_init) ctrl_after_k0_body(st, 1, p);
 }
 
 }  // namespace gk

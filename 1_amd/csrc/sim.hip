@@ -261,6 +261,7 @@ CtrlParams gk::ctrl_params(const mmSim* s) {
     c.log_err = s->log_err;
     c.log_cap = s->log_cap;
     c.thermal = s->p.temperature > 0;
+    c.fsal = s->tb.fsal;
     return c;
 }
 
@@ -288,17 +289,10 @@ static void enqueue_trial(mmSim* s) {
     const Tableau& t = s->tb;
     const CtrlParams cp = ctrl_params(s);
     Prof& pf = s->prof;
-    pf.begin(7, s->s);
-    launch_ctrl_begin(s->st, s->s);
-    pf.end(s->s);
+    // the trial has been started by the one before (launch_ctrl_end) or launch_set_target;
+    // the FSAL stage is in k[0] (launch_commit) and its dt control done
     for (int i = 0; i < t.S; i++) {
-        if (i == 0 && t.fsal && s->fsalHost) {
-            pf.begin(7, s->s);
-            launch_copy_if_active(s->k[0], s->k[t.S - 1], s->N3, s->st, s->s);  // rk.go:311-315
-            launch_ctrl_after_k0(s->st, 1, cp, s->s);
-            pf.end(s->s);
-            continue;
-        }
+        if (i == 0 && t.fsal && s->fsalHost) continue;
         StageIn si{};
         si.m = s->m;
         si.st = s->st;
@@ -349,7 +343,7 @@ static void enqueue_trial(mmSim* s) {
         conv_apply(s->cp, si, nullptr, s->s, &pf, &ea);
         if (i == 0 && needs_after_k0(s)) {
             pf.begin(7, s->s);
-            launch_ctrl_after_k0(s->st, 0, cp, s->s);
+            launch_ctrl_after_k0(s->st, cp, s->s);
             pf.end(s->s);
         }
     }
@@ -371,7 +365,8 @@ static void enqueue_trial(mmSim* s) {
     }
     pf.begin(7, s->s);
     launch_ctrl_end(s->st, cp, s->s);
-    if (t.adaptive) launch_commit(s->m, s->mtmp, s->st, s->normMap, s->N, s->s);
+    if (t.adaptive)
+        launch_commit(s->m, s->mtmp, t.fsal ? s->k[0] : nullptr, s->k[t.S - 1], s->st, s->normMap, s->N, s->s);
     pf.end(s->s);
     if (t.fsal) s->fsalHost = true;
 }
@@ -380,15 +375,29 @@ static long fused_run(mmSim* s, long long nsteps, double stop, bool wait) {
     EngineState h = read_state(s);
     s->fsalHost = h.fsal_init != 0;
     const long long steps0 = h.steps;
-    launch_set_target(s->st, nsteps, stop, s->s);
+    const CtrlParams cp = ctrl_params(s);
+    launch_set_target(s->st, nsteps, stop, &cp, s->s);
     if (!wait) {
         // enqueue exactly nsteps trials (fixed-step tableaux never reject)
         for (long long i = 0; i < nsteps; i++) enqueue_trial(s);
         return nsteps;
     }
+    // Trials enqueued past the end are launches that do nothing: at most as many as
+    // the steps still to take, and for a stop time at most what the time left needs
+    // at the current dt; within that, for adaptive tableaux, doubling batches (dt
+    // grows over the first steps of a run).
     int batch = 4;
     while (true) {
-        for (int i = 0; i < batch; i++) enqueue_trial(s);
+        long long n = batch;
+        if (nsteps >= 0) {
+            const long long left = steps0 + nsteps - h.steps;
+            n = std::min<long long>(left, s->tb.adaptive ? 64 : 1024);
+        } else if (stop < INFINITY && h.dt > 0) {
+            const long long need = (long long)std::min(1e9, std::ceil((stop - h.time) / h.dt));
+            n = std::min<long long>(need, s->tb.adaptive ? batch : 1024);
+        }
+        n = std::max(n, 1LL);
+        for (long long i = 0; i < n; i++) enqueue_trial(s);
         h = read_state(s);
         if (h.nan_dt) {
             fprintf(stderr, "libgpukern: dt = NaN (rk.go:448-452)\n");
@@ -1122,7 +1131,7 @@ void mm_sim_begin_run(mmSim* s, double seconds) {
     EngineState h = read_state(s);
     const double stop = h.time + seconds / s->unitTime;
     launch_normalize_active(s->m, nullptr, s->normMap, s->N, s->s);  // simrun.go:24
-    launch_set_target(s->st, -1, stop, s->s);
+    launch_set_target(s->st, -1, stop, nullptr, s->s);
     GK_CHECK(hipStreamSynchronize(s->s));
 }
 
@@ -1141,7 +1150,7 @@ static double time_pass(mmSim* s, int cls, int n, int nk) {
     }
     EpiArgs ea{};
     ea.m = s->m;
-    ea.out = s->k[0];
+    ea.out = s->mtmp;  // k[0] may hold the next trial's FSAL stage
     ea.t = torque_args(s, s->tb.c[0], s->part);
     launch_set_active(s->st, s->s);
     hipEvent_t e0, e1;
@@ -1203,9 +1212,10 @@ int mm_sim_tune(mmSim* s, int reps, int params[7], double ms_default[8], double 
     };
     for (int i = 0; i < 8; i++) ms_default[i] = ms_tuned[i] = -1;
     std::vector<int> zr{0}, er{0};
-    for (int v = 1; v <= 2; v++)
+    for (int v = 1; v <= 3; v++)
         if (conv_zr_valid(cp.M, v)) zr.push_back(v);
-    if (conv_er_valid(cp.M, 1)) er.push_back(1);
+    for (int v = 1; v <= 2; v++)
+        if (conv_er_valid(cp.M, v)) er.push_back(v);
     const std::vector<int> grid{2, 3, 4, 6, 8, 12, 16};
     tune_one(0, &cp.tp.zr, dflt.zr, zr, 0, -1);
     tune_one(1, &cp.tp.er, dflt.er, er, 4, -1);

@@ -181,7 +181,7 @@ double mm_sim_profile_steps(mmSim* s, int n, double* ms, int* counts);
 /* Fused mode.  n back-to-back launches of one convolution pass class (0..4 as
  * above; the Z inverse with the stage-1 torque epilogue) on the engine's
  * stream between two HIP events; returns the elapsed ms.  The passes work on
- * the engine's scratch spectra and its first stage buffer, so the state m is
+ * the engine's scratch spectra and a scratch field, so the state m is
  * unchanged; the next step recomputes everything they touch. */
 double mm_sim_time_pass(mmSim* s, int cls, int n);
 
@@ -189,8 +189,8 @@ double mm_sim_time_pass(mmSim* s, int cls, int n);
  * every kernel (make1dconf, gpu_conf.cu:68-97, with the size filter of
  * cufftsize.go:14-52); here each pass of a fused-mode simulation has its own
  * tunables, timed on the device: params[6] = {zr: Z forward rows per block
- * (variant 0 default, 1 half, 2 double), er: fused Z inverse rows per block
- * (0 default, 1 half), yb: blocks per CU of the 3-D Y passes, xb: blocks per CU
+ * (variant 0 by the grid, 1 half of the length's default, 2 double, 3 a quarter),
+ * er: fused Z inverse rows per block (0 by the grid, 1 half, 2 two rows), yb: blocks per CU of the 3-D Y passes, xb: blocks per CU
  * of the X.K.X pass, y2b: blocks per CU of the 2-D Y.K.Y pass, pp: for 3-D
  * plans with padded Y 512 and padded X 16 or 32, 1 = Y forward, X.K.X and Y
  * inverse as one register-resident plane pass, 0 = three passes, xv: X.K.X
