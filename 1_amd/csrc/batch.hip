@@ -33,9 +33,9 @@
 namespace gk {
 
 // ------------------------------------------------------------------ RK pointwise and control
-__global__ __launch_bounds__(256) void kb_rk_final(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(256) void kb_rk_final(const BSim* sims, const int2* map,
                                                    FinalArgs fa) {
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (!d.st->trial_active) return;
     KPtrs kp;
@@ -47,8 +47,8 @@ __global__ __launch_bounds__(256) void kb_rk_final(const BSim* sims, const int* 
 }
 
 // last: the FSAL tableau's last stage, 0 for the others
-__global__ __launch_bounds__(256) void kb_commit(const BSim* sims, const int* idx, const int* start, int n, int last) {
-    const BBlock bb = bblock(sims, idx, start, n);
+__global__ __launch_bounds__(256) void kb_commit(const BSim* sims, const int2* map, int last) {
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     commit_body(d.m, d.mtmp, last ? d.k[0] : nullptr, d.k[last], d.st, d.t.normMap, (int)d.N, bb.lb, d.nfin);
 }
@@ -97,10 +97,9 @@ struct LaunchSet {
     int L = 0;       // template length of the class
     int cnt = 0;     // simulations
     int blocks = 0;  // total blocks
-    int* idx = nullptr;
-    int* start = nullptr;
-    size_t idx_off = 0, start_off = 0;  // offsets in the batch's table block (set-up)
-    std::vector<int> hidx, hst;         // host copies of idx and start (set-up)
+    int2* map = nullptr;          // device, per block: simulation, block within it
+    size_t map_off = 0;           // offset in the batch's table block (set-up)
+    std::vector<int> hidx, hst;   // the simulations and their first blocks (set-up)
     int any = 0;                        // 1: small length classes merged, launched by a dispatch kernel
     int nt = 0, lds = 0;                // dispatch launch: threads per block and dynamic LDS bytes
 };
@@ -294,11 +293,13 @@ std::vector<LaunchSet> merge_small(std::vector<LaunchSet> sets, int pass) {
     return out;
 }
 
-// the launch sets' simulation lists and block starts into the table image
+// the launch sets' block tables into the table image
 void stage_sets(mmBatch* b, std::vector<LaunchSet>& sets) {
     for (auto& ls : sets) {
-        ls.idx_off = b->image.put(ls.hidx.data(), ls.cnt * sizeof(int));
-        ls.start_off = b->image.put(ls.hst.data(), (ls.cnt + 1) * sizeof(int));
+        std::vector<int2> map(ls.blocks);
+        for (int i = 0; i < ls.cnt; i++)
+            for (int k = ls.hst[i]; k < ls.hst[i + 1]; k++) map[k] = make_int2(ls.hidx[i], k - ls.hst[i]);
+        ls.map_off = b->image.put(map.data(), map.size() * sizeof(int2));
     }
 }
 
@@ -306,7 +307,7 @@ int fin_blocks(const mmSim* s) { return std::max(1, std::min(kRedBlocks, div_up(
 
 // ---------------------------------------------------------------- launchers (one length class each)
 BLaunch bl(const mmBatch* b, const LaunchSet& ls) {
-    return BLaunch{b->dsims, ls.idx, ls.start, ls.cnt, ls.blocks, ls.nt, ls.lds, b->s};
+    return BLaunch{b->dsims, ls.map, ls.blocks, ls.nt, ls.lds, b->s};
 }
 void bl_zfwd(mmBatch* b, const LaunchSet& ls, const BStage& sg) {
     if (ls.any) {
@@ -335,8 +336,8 @@ void bl_ypass(mmBatch* b, const LaunchSet& ls, const BStage& sg, bool fwd) {
     switch (ls.L) {
 #define GK_CASE(n)                                                                                       \
     case n:                                                                                              \
-        if (fwd) kb_ypass<n, true><<<ls.blocks, kNT, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, sg, tw);  \
-        else kb_ypass<n, false><<<ls.blocks, kNT, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, sg, tw);     \
+        if (fwd) kb_ypass<n, true><<<ls.blocks, kNT, 0, b->s>>>(b->dsims, ls.map, sg, tw);  \
+        else kb_ypass<n, false><<<ls.blocks, kNT, 0, b->s>>>(b->dsims, ls.map, sg, tw);     \
         break;
         GK_LEN_Y(GK_CASE)
 #undef GK_CASE
@@ -353,7 +354,7 @@ void bl_xmul(mmBatch* b, const LaunchSet& ls, const BStage& sg) {
     const float2* tw = twiddle_f32(ls.L);
     switch (ls.L) {
 #define GK_CASE(n)                                                                            \
-    case n: kb_xmul<n><<<ls.blocks, kNT, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, sg, tw); break;
+    case n: kb_xmul<n><<<ls.blocks, kNT, 0, b->s>>>(b->dsims, ls.map, sg, tw); break;
         GK_LEN_X(GK_CASE)
 #undef GK_CASE
     default: abort();
@@ -374,7 +375,7 @@ void bl_yxy(mmBatch* b, const LaunchSet& ls, const BStage& sg) {
 #define GK_YX(n, px)                                                                                              \
     case px:                                                                                                      \
         if constexpr (yxy_fits(px, n))                                                                            \
-            kb_yxy<n, px><<<ls.blocks, kYxyThreads, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, sg, twY, twX); \
+            kb_yxy<n, px><<<ls.blocks, kYxyThreads, 0, b->s>>>(b->dsims, ls.map, sg, twY, twX); \
         else                                                                                                      \
             abort();                                                                                              \
         break;
@@ -401,7 +402,7 @@ void bl_y2d(mmBatch* b, const LaunchSet& ls, const BStage& sg) {
     const float2* tw = twiddle_f32(ls.L);
     switch (ls.L) {
 #define GK_CASE(n)                                                                                           \
-    case n: kb_y2r<n><<<ls.blocks, Y2<n>::NT, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, sg, tw); \
+    case n: kb_y2r<n><<<ls.blocks, Y2<n>::NT, 0, b->s>>>(b->dsims, ls.map, sg, tw); \
         break;
         GK_LEN_Y(GK_CASE)
 #undef GK_CASE
@@ -483,7 +484,7 @@ void enqueue_btrial(mmBatch* b) {
         }
         fa.adaptive = 1;
         for (auto& ls : b->fin) {
-            kb_rk_final<<<ls.blocks, 256, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, fa);
+            kb_rk_final<<<ls.blocks, 256, 0, b->s>>>(b->dsims, ls.map, fa);
             GK_LAUNCH_CHECK();
         }
     }
@@ -491,7 +492,7 @@ void enqueue_btrial(mmBatch* b) {
     GK_LAUNCH_CHECK();
     if (t.adaptive)
         for (auto& ls : b->fin) {
-            kb_commit<<<ls.blocks, 256, 0, b->s>>>(b->dsims, ls.idx, ls.start, ls.cnt, t.fsal ? t.S - 1 : 0);
+            kb_commit<<<ls.blocks, 256, 0, b->s>>>(b->dsims, ls.map, t.fsal ? t.S - 1 : 0);
             GK_LAUNCH_CHECK();
         }
 }
@@ -609,8 +610,7 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
         b->dsims = (BSim*)(dev + sims_off);
         for (auto* sets : {&b->zf, &b->zi, &b->yf, &b->yi, &b->xm, &b->y2, &b->yx, &b->fin})
             for (LaunchSet& ls : *sets) {
-                ls.idx = (int*)(dev + ls.idx_off);
-                ls.start = (int*)(dev + ls.start_off);
+                ls.map = (int2*)(dev + ls.map_off);
             }
         b->image = TableImage{};
     }

@@ -12,15 +12,15 @@ namespace gk {
 template <typename F> static void any_attr(F* f) {
     GK_CHECK(hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, kAnyLds));
 }
-#define GK_ANY_LAUNCH(kern) kern<<<b.blocks, b.nt, b.lds, b.s>>>(b.sims, b.idx, b.start, b.cnt, sg)
+#define GK_ANY_LAUNCH(kern) kern<<<b.blocks, b.nt, b.lds, b.s>>>(b.sims, b.map, sg)
 
 #if GK_PART == 0
 
 template <int NK>
-__global__ __launch_bounds__(1024) void kb_zfwd_any(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(1024) void kb_zfwd_any(const BSim* sims, const int2* map,
                                                     BStage sg) {
     extern __shared__ float2 dyn[];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     switch (d.Q - 1) {
@@ -52,10 +52,10 @@ void any_attr_zfwd() {
 #elif GK_PART <= 2
 
 template <int NU, int FIN>
-__global__ __launch_bounds__(768) void kb_zinv_any(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(768) void kb_zinv_any(const BSim* sims, const int2* map,
                                                    BStage sg) {
     extern __shared__ float2 dyn[];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     switch (d.Q - 1) {
@@ -100,10 +100,10 @@ void any_attr_zinv_fin() {
 
 #else
 
-__global__ __launch_bounds__(kYxyThreads) void kb_yxy_any(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(kYxyThreads) void kb_yxy_any(const BSim* sims, const int2* map,
                                                           BStage sg) {
     extern __shared__ float2 dyn[];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     if (d.PX == 4) {
@@ -121,10 +121,10 @@ __global__ __launch_bounds__(kYxyThreads) void kb_yxy_any(const BSim* sims, cons
     }
 }
 
-__global__ __launch_bounds__(Y2<1024>::NT) void kb_y2r_any(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(Y2<1024>::NT) void kb_y2r_any(const BSim* sims, const int2* map,
                                                   BStage sg) {
     extern __shared__ float2 dyn[];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     switch (d.PY) {
@@ -139,10 +139,10 @@ __global__ __launch_bounds__(Y2<1024>::NT) void kb_y2r_any(const BSim* sims, con
 }
 
 template <bool FWD>
-__global__ __launch_bounds__(kNT) void kb_ypass_any(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(kNT) void kb_ypass_any(const BSim* sims, const int2* map,
                                                     BStage sg) {
     extern __shared__ float2 dyn[];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     switch (d.PY) {
@@ -153,10 +153,10 @@ __global__ __launch_bounds__(kNT) void kb_ypass_any(const BSim* sims, const int*
     }
 }
 
-__global__ __launch_bounds__(kNT) void kb_xmul_any(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(kNT) void kb_xmul_any(const BSim* sims, const int2* map,
                                                    BStage sg) {
     extern __shared__ float2 dyn[];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     switch (d.PX) {

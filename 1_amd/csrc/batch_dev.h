@@ -51,25 +51,18 @@ struct BStage {
     int partslot;  // -1: none, 0: |k0|, 1: |k_last|
 };
 
-// largest j with start[j] <= b (start[0] = 0, increasing)
-__device__ __forceinline__ int bfind(const int* __restrict__ start, int n, int b) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (start[mid] <= b) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-// the simulation of this block and the block's index within it
+// The simulation of this block and the block's index within it, from the launch's
+// table of one int2 per block.  (A binary search over the simulations' first
+// blocks took log2(n) dependent loads at the start of every block, of a few
+// hundred ns each, where the pass itself takes a few us: a 40-member
+// sweep of Dormand-Prince steps 6694 us, 6625 with the table.)
 struct BBlock {
     const BSim* d;
     int lb;
 };
-__device__ __forceinline__ BBlock bblock(const BSim* sims, const int* idx, const int* start, int n) {
-    const int j = bfind(start, n, blockIdx.x);
-    return BBlock{sims + idx[j], (int)blockIdx.x - start[j]};
+__device__ __forceinline__ BBlock bblock(const BSim* sims, const int2* map) {
+    const int2 e = map[blockIdx.x];
+    return BBlock{sims + e.x, e.y};
 }
 __device__ __forceinline__ bool bskip(const BSim& d, const BStage& sg) {
     return !d.st->trial_active || (sg.fsal0 && d.st->fsal_init);
@@ -97,11 +90,10 @@ __device__ __forceinline__ void bz_fwd(const BSim& d, int lb, const BStage& sg, 
 }
 
 template <int M, int TR, int NK>
-__global__ __launch_bounds__(TR * RegFFT<M>::G) void kb_zfwd(const BSim* sims, const int* idx, const int* start,
-                                                               int n, BStage sg, const float2* __restrict__ twM,
+__global__ __launch_bounds__(TR * RegFFT<M>::G) void kb_zfwd(const BSim* sims, const int2* map, BStage sg, const float2* __restrict__ twM,
                                                                const float2* __restrict__ twP) {
     __shared__ float2 lds[zfwd_lds<M, TR>()];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     bz_fwd<M, TR, NK>(d, bb.lb, sg, twM, twP, lds);
@@ -130,10 +122,10 @@ __device__ __forceinline__ void b_ypass(const BSim& d, int lb, const float2* __r
 }
 
 template <int PY, bool FWD>
-__global__ __launch_bounds__(kNT) void kb_ypass(const BSim* sims, const int* idx, const int* start, int n, BStage sg,
+__global__ __launch_bounds__(kNT) void kb_ypass(const BSim* sims, const int2* map, BStage sg,
                                                 const float2* __restrict__ tw) {
     __shared__ float2 lds[ypass_lds<PY>()];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     b_ypass<PY, FWD>(d, bb.lb, tw, lds);
@@ -164,10 +156,10 @@ __device__ __forceinline__ void b_xmul(const BSim& d, int lb, const float2* __re
 }
 
 template <int PX>
-__global__ __launch_bounds__(kNT) void kb_xmul(const BSim* sims, const int* idx, const int* start, int n, BStage sg,
+__global__ __launch_bounds__(kNT) void kb_xmul(const BSim* sims, const int2* map, BStage sg,
                                                const float2* __restrict__ tw) {
     __shared__ float2 lds[xmul_lds<PX>()];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     b_xmul<PX>(d, bb.lb, tw, lds);
@@ -186,11 +178,11 @@ __device__ __forceinline__ void b_yxy(const BSim& d, int lb, const float2* __res
 }
 
 template <int PY, int PX>
-__global__ __launch_bounds__(kYxyThreads) void kb_yxy(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(kYxyThreads) void kb_yxy(const BSim* sims, const int2* map,
                                                        BStage sg, const float2* __restrict__ twY,
                                                        const float2* __restrict__ twX) {
     __shared__ float2 lds[yxy_lds<PY, PX>()];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     b_yxy<PY, PX>(d, bb.lb, twY, twX, lds);
@@ -203,10 +195,10 @@ __device__ __forceinline__ void b_y2r(const BSim& d, int lb, const float2* __res
 }
 
 template <int PY>
-__global__ __launch_bounds__(Y2<PY>::NT) void kb_y2r(const BSim* sims, const int* idx, const int* start, int n,
+__global__ __launch_bounds__(Y2<PY>::NT) void kb_y2r(const BSim* sims, const int2* map,
                                                      BStage sg, const float2* __restrict__ tw) {
     __shared__ float2 lds[Y2<PY>::LDS];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     b_y2r<PY>(d, bb.lb, tw, lds);
@@ -241,14 +233,13 @@ __device__ __forceinline__ void bz_inv(const BSim& d, int lb, const BStage& sg, 
 }
 
 template <int M, int TR, int NU, int FIN>
-__global__ __launch_bounds__(3 * TR * RegFFT<M>::G) void kb_zinv_epi(const BSim* sims, const int* idx,
-                                                                       const int* start, int n, BStage sg,
+__global__ __launch_bounds__(3 * TR * RegFFT<M>::G) void kb_zinv_epi(const BSim* sims, const int2* map, BStage sg,
                                                                        const float2* __restrict__ twM,
                                                                        const float2* __restrict__ twP) {
     __shared__ float2 lds[zinv_epi_lds<M, TR>()];
     __shared__ float hext_s[3];
     __shared__ float red[3 * TR * RegFFT<M>::G];
-    const BBlock bb = bblock(sims, idx, start, n);
+    const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     bz_inv<M, TR, NU, FIN>(d, bb.lb, sg, twM, twP, lds, hext_s, red);
@@ -311,12 +302,11 @@ template <int M> constexpr int zinv_any_bytes() {
     return zinv_epi_lds<M, TR>() * 8 + 16 + 3 * NR * 4;
 }
 
-// the batch's table, the simulations of a launch and its geometry
+// the batch's table, the blocks of a launch and its geometry
 struct BLaunch {
     const BSim* sims;
-    const int* idx;
-    const int* start;
-    int cnt, blocks;
+    const int2* map;  // per block: simulation, block within it
+    int blocks;
     int nt, lds;  // dispatch launch: threads per block and dynamic LDS bytes
     hipStream_t s;
 };

@@ -13,18 +13,18 @@ namespace gk {
 template <int M> void bz_fwd_run(const BLaunch& b, const BStage& sg, const float2* twM, const float2* twP) {
     constexpr int TR = z_rows_c<M>(), nt = TR * RegFFT<M>::G;
     switch (zfwd_nk(sg.nk)) {
-    case 0: kb_zfwd<M, TR, 0><<<b.blocks, nt, 0, b.s>>>(b.sims, b.idx, b.start, b.cnt, sg, twM, twP); break;
-    case 1: kb_zfwd<M, TR, 1><<<b.blocks, nt, 0, b.s>>>(b.sims, b.idx, b.start, b.cnt, sg, twM, twP); break;
-    case 2: kb_zfwd<M, TR, 2><<<b.blocks, nt, 0, b.s>>>(b.sims, b.idx, b.start, b.cnt, sg, twM, twP); break;
-    case 3: kb_zfwd<M, TR, 3><<<b.blocks, nt, 0, b.s>>>(b.sims, b.idx, b.start, b.cnt, sg, twM, twP); break;
-    default: kb_zfwd<M, TR, 5><<<b.blocks, nt, 0, b.s>>>(b.sims, b.idx, b.start, b.cnt, sg, twM, twP); break;
+    case 0: kb_zfwd<M, TR, 0><<<b.blocks, nt, 0, b.s>>>(b.sims, b.map, sg, twM, twP); break;
+    case 1: kb_zfwd<M, TR, 1><<<b.blocks, nt, 0, b.s>>>(b.sims, b.map, sg, twM, twP); break;
+    case 2: kb_zfwd<M, TR, 2><<<b.blocks, nt, 0, b.s>>>(b.sims, b.map, sg, twM, twP); break;
+    case 3: kb_zfwd<M, TR, 3><<<b.blocks, nt, 0, b.s>>>(b.sims, b.map, sg, twM, twP); break;
+    default: kb_zfwd<M, TR, 5><<<b.blocks, nt, 0, b.s>>>(b.sims, b.map, sg, twM, twP); break;
     }
 }
 
 template <int M, int NU, int FIN>
 static void epi_launch(const BLaunch& b, const BStage& sg, const float2* twM, const float2* twP) {
     constexpr int TR = epi_rows_c<M>(), nt = 3 * TR * RegFFT<M>::G;
-    kb_zinv_epi<M, TR, NU, FIN><<<b.blocks, nt, 0, b.s>>>(b.sims, b.idx, b.start, b.cnt, sg, twM, twP);
+    kb_zinv_epi<M, TR, NU, FIN><<<b.blocks, nt, 0, b.s>>>(b.sims, b.map, sg, twM, twP);
 }
 template <int M> void bz_epi_run(const BLaunch& b, const BStage& sg, const float2* twM, const float2* twP) {
     if (sg.fin == 1) {
