@@ -422,13 +422,16 @@ void launch_commit(float* m, const float* mtmp, float* k0, const float* klast, E
                    int N, hipStream_t s);
 void launch_normalize_active(float* m, const EngineState* st, const float* nmap, int N, hipStream_t s);
 
+// energy of m in field h as per-block FP64 sums in out[0..sum_blocks(N)), host memory
+// the device can write; the caller adds them up after the stream has finished
+constexpr int kSumBlocks = 256;
+int sum_blocks(int N);
 void launch_energy(const float* m, const float* h, const float hext[3], int anisType, float kAnis, const float u[3],
                    int N, double* out, hipStream_t s);
 // steps_target = steps + nsteps (nsteps < 0: unlimited), stop time; recomputes
 // `done`; with p, also starts the first trial (as launch_ctrl_end does for the others)
 void launch_set_target(EngineState* st, long long nsteps, double stop, const CtrlParams* p, hipStream_t s);
-// FP64 reductions for outputs: sums[0..2] = sum of each component; energy
-void launch_sum3(const float* v, int N, double* out_dev, hipStream_t s);
-void launch_sum1(const float* v, int N, double* out_dev, hipStream_t s);
+// per-block FP64 sums of each component for outputs: out[c * sum_blocks(N) + block]
+void launch_sum3(const float* v, int N, double* out, hipStream_t s);
 
 }  // namespace gk

@@ -15,6 +15,7 @@
 
 #include "../../include/gpukern.h"
 #include "gk_common.h"
+#include "gk_enqueue.h"
 
 namespace gk {
 
@@ -253,6 +254,14 @@ __global__ void k_add_constant(float* __restrict__ a, float c, int n) {
 }
 __global__ void k_lincomb(float* __restrict__ a, const float* __restrict__ b, float wa, float wb, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) a[i] = wa * a[i] + wb * b[i];
+}
+
+__global__ void k_combine(float* dst, const float* src, CombineTerms t, int n) {  // dst may be src
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        float a = src[i];
+        for (int j = 0; j < t.n; j++) a += t.c[j] * t.k[j][i];
+        dst[i] = a;
+    }
 }
 
 struct LinCombMany {
@@ -619,6 +628,61 @@ static dim3 g1(long n) {
     return dim3((unsigned)g);
 }
 
+static LocalParams local_params(const float* Hext, int anisType, const float* anisK, const float* anisAxes);
+
+namespace gk {
+void enq_copy(const float* src, float* dst, int n) {
+    GK_ASSERT(n > 0, "memcpy_on_gpu: n=%d", n);
+    GK_CHECK(hipMemcpyAsync(dst, src, (size_t)n * sizeof(float), hipMemcpyDeviceToDevice, stream()));
+}
+void enq_combine(float* dst, const float* src, const CombineTerms& t, int n) {
+    k_combine<<<g1(n), kBlock, 0, stream()>>>(dst, src, t, n);
+    GK_LAUNCH_CHECK();
+}
+void enq_linear_combination(float* a, float* b, float wa, float wb, int N) {
+    k_lincomb<<<g1(N), kBlock, 0, stream()>>>(a, b, wa, wb, N);
+    GK_LAUNCH_CHECK();
+}
+void enq_normalize(float* m, float* map, int N) {
+    k_normalize<<<g1(N), kBlock, 0, stream()>>>(m, map, N);
+    GK_LAUNCH_CHECK();
+}
+void enq_deltaM(float* m, float* h, float alpha_mul, float* alpha_map, float dt_gilb, int N) {
+    k_deltaM<<<g1(N), kBlock, 0, stream()>>>(m, h, alpha_mul, alpha_map, dt_gilb, N);
+    GK_LAUNCH_CHECK();
+}
+void enq_spintorque_deltaM(float* m, float* h, float alpha, float beta, float eps, const float* u, float* jmap,
+                           float dt_gilb, int N0, int N1, int N2) {
+    k_spintorque<<<g1((long)N0 * N1 * N2), kBlock, 0, stream()>>>(m, h, alpha, beta, eps, u[0], u[1], u[2], jmap,
+                                                                  dt_gilb, N0, N1, N2);
+    GK_LAUNCH_CHECK();
+}
+void enq_add_local_fields(float* m, float* h, int N, const float* Hext, float* hmap, int anisType, const float* anisK,
+                          const float* anisAxes) {
+    LocalParams p = local_params(Hext, anisType, anisK, anisAxes);
+    k_local_fields<false><<<g1(N), kBlock, 0, stream()>>>(m, h, nullptr, hmap, p, N);
+    GK_LAUNCH_CHECK();
+}
+void enq_anal_fw_step(float dt, float alpha, int N, float* m_in, float* m_out, float* h) {
+    k_anal_fw<<<g1(N), kBlock, 0, stream()>>>(m_in, m_out, h, dt, alpha, N);
+    GK_LAUNCH_CHECK();
+}
+void enq_kernelmul6(float* mx, float* my, float* mz, float* kxx, float* kyy, float* kzz, float* kyz, float* kxz,
+                    float* kxy, int nReal) {
+    GK_ASSERT(nReal > 0 && nReal % 2 == 0, "gpu_kernelmul6: nRealNumbers=%d", nReal);
+    int n = nReal / 2;
+    k_kernelmul6<<<g1(n), kBlock, 0, stream()>>>((float2*)mx, (float2*)my, (float2*)mz, kxx, kyy, kzz, kyz, kxz, kxy,
+                                                 n);
+    GK_LAUNCH_CHECK();
+}
+void enq_kernelmul4(float* mx, float* my, float* mz, float* kxx, float* kyy, float* kzz, float* kyz, int nReal) {
+    GK_ASSERT(nReal > 0 && nReal % 2 == 0, "gpu_kernelmul4: nRealNumbers=%d", nReal);
+    int n = nReal / 2;
+    k_kernelmul4<<<g1(n), kBlock, 0, stream()>>>((float2*)mx, (float2*)my, (float2*)mz, kxx, kyy, kzz, kyz, n);
+    GK_LAUNCH_CHECK();
+}
+}  // namespace gk
+
 extern "C" {
 
 // ---------------------------------------------------------------- init (gpu_init.cu, gpu_conf.cu)
@@ -726,8 +790,7 @@ void memcpy_from_gpu(float* source, float* dest, int n) {
     sync();
 }
 void memcpy_on_gpu(float* source, float* dest, int n) {
-    GK_ASSERT(n > 0, "memcpy_on_gpu: n=%d", n);
-    GK_CHECK(hipMemcpyAsync(dest, source, (size_t)n * sizeof(float), hipMemcpyDeviceToDevice, stream()));
+    enq_copy(source, dest, n);
     sync();
 }
 void memcpy_gpu_dir(float* source, float* dest, int n, int direction) {
@@ -770,7 +833,7 @@ void gpu_add_constant(float* a, float c, int N) {
     sync();
 }
 void gpu_linear_combination(float* a, float* b, float wa, float wb, int N) {
-    k_lincomb<<<g1(N), kBlock, 0, stream()>>>(a, b, wa, wb, N);
+    enq_linear_combination(a, b, wa, wb, N);
     sync();
 }
 void gpu_linear_combination_many(float* result, float** vectors, float* weights, int nv, int N) {
@@ -833,15 +896,15 @@ float gpu_reduce(int op, float* input, float* devbuf, float* hostbuf, int blocks
 
 // ---------------------------------------------------------------- normalize / torque
 void gpu_normalize_uniform(float* m, int N) {
-    k_normalize<<<g1(N), kBlock, 0, stream()>>>(m, nullptr, N);
+    enq_normalize(m, nullptr, N);
     sync();
 }
 void gpu_normalize_map(float* m, float* map, int N) {
-    k_normalize<<<g1(N), kBlock, 0, stream()>>>(m, map, N);
+    enq_normalize(m, map, N);
     sync();
 }
 void gpu_deltaM(float* m, float* h, float alpha_mul, float* alpha_map, float dt_gilb, int N) {
-    k_deltaM<<<g1(N), kBlock, 0, stream()>>>(m, h, alpha_mul, alpha_map, dt_gilb, N);
+    enq_deltaM(m, h, alpha_mul, alpha_map, dt_gilb, N);
     sync();
 }
 
@@ -863,8 +926,7 @@ static LocalParams local_params(const float* Hext, int anisType, const float* an
 }
 void gpu_add_local_fields(float* m, float* h, int N, float* Hext, float* hmap, int anisType, float* anisK,
                           float* anisAxes) {
-    LocalParams p = local_params(Hext, anisType, anisK, anisAxes);
-    k_local_fields<false><<<g1(N), kBlock, 0, stream()>>>(m, h, nullptr, hmap, p, N);
+    enq_add_local_fields(m, h, N, Hext, hmap, anisType, anisK, anisAxes);
     sync();
 }
 void gpu_add_local_fields_H_and_phi(float* m, float* h, float* phi, int N, float* Hext, float* hmap, int anisType,
@@ -908,16 +970,11 @@ void gpu_add_exch(float* m, float* h, int* size, int* periodic, int* exchInConv,
 // ---------------------------------------------------------------- kernel multiply (gpu_kernmul.cu:25-141)
 void gpu_kernelmul6(float* mx, float* my, float* mz, float* kxx, float* kyy, float* kzz, float* kyz, float* kxz,
                     float* kxy, int nReal) {
-    GK_ASSERT(nReal > 0 && nReal % 2 == 0, "gpu_kernelmul6: nRealNumbers=%d", nReal);
-    int n = nReal / 2;
-    k_kernelmul6<<<g1(n), kBlock, 0, stream()>>>((float2*)mx, (float2*)my, (float2*)mz, kxx, kyy, kzz, kyz, kxz, kxy,
-                                                 n);
+    enq_kernelmul6(mx, my, mz, kxx, kyy, kzz, kyz, kxz, kxy, nReal);
     sync();
 }
 void gpu_kernelmul4(float* mx, float* my, float* mz, float* kxx, float* kyy, float* kzz, float* kyz, int nReal) {
-    GK_ASSERT(nReal > 0 && nReal % 2 == 0, "gpu_kernelmul4: nRealNumbers=%d", nReal);
-    int n = nReal / 2;
-    k_kernelmul4<<<g1(n), kBlock, 0, stream()>>>((float2*)mx, (float2*)my, (float2*)mz, kxx, kyy, kzz, kyz, n);
+    enq_kernelmul4(mx, my, mz, kxx, kyy, kzz, kyz, nReal);
     sync();
 }
 
@@ -938,14 +995,12 @@ void gpu_copy_unpad(float* src, float* dst, int S0, int S1, int S2, int D0, int 
 // ---------------------------------------------------------------- STT / semi-analytical (gpu_spintorque.cu:188-211, gpu_anal.cu:87-98)
 void gpu_spintorque_deltaM(float* m, float* h, float alpha, float beta, float epsillon, float* u, float* jmap,
                            float dt_gilb, int N0, int N1, int N2) {
-    long N = (long)N0 * N1 * N2;
-    k_spintorque<<<g1(N), kBlock, 0, stream()>>>(m, h, alpha, beta, epsillon, u[0], u[1], u[2], jmap, dt_gilb, N0, N1,
-                                                 N2);
+    enq_spintorque_deltaM(m, h, alpha, beta, epsillon, u, jmap, dt_gilb, N0, N1, N2);
     sync();
 }
 
 void gpu_anal_fw_step(float dt, float alpha, int N, float* m_in, float* m_out, float* h) {
-    k_anal_fw<<<g1(N), kBlock, 0, stream()>>>(m_in, m_out, h, dt, alpha, N);
+    enq_anal_fw_step(dt, alpha, N, m_in, m_out, h);
     sync();
 }
 

@@ -23,6 +23,8 @@ struct LineArgs {
     unsigned nlines, n_inner;   // line l starts at (l / n_inner) outer + (l % n_inner) inner
     long inner, outer, estride;  // elements at stride estride
     int nvalid, nkeep;           // inputs read (the rest are zeros), outputs stored
+    int ncomp;                   // transforms of the same shape, one per blockIdx.y ...
+    long cstride;                // ... at this distance
     __device__ __forceinline__ long start(unsigned l) const { return (long)(l / n_inner) * outer + (long)(l % n_inner) * inner; }
 };
 // Rows of n_real floats (row r at (r / n_inner)*real_outer + (r % n_inner)*real_inner)
@@ -32,6 +34,8 @@ struct RowArgs {
     unsigned nrows, n_inner;
     long real_inner, real_outer, cplx_inner, cplx_outer;
     int n_real, vec;
+    int ncomp;                // transforms of the same shape, one per blockIdx.y
+    long real_comp, cplx_comp;
     __device__ __forceinline__ long real_at(unsigned r) const {
         return (long)(r / n_inner) * real_outer + (long)(r % n_inner) * real_inner;
     }
@@ -49,12 +53,14 @@ void fft_rows_c2r_reg(const float2* in, float* out, int P, const RowArgs& a, hip
 // a runtime radix list, others through Bluestein's chirp-z convolution.
 template <typename T, int DIR>
 void fft_lines_any(C2<T>* data, int L, long nlines, long n_inner, long inner, long outer, long estride, int nvalid,
-                   int nkeep, hipStream_t s);
+                   int nkeep, hipStream_t s, int ncomp = 1, long cstride = 0);
 // rows: n_real floats -> P/2+1 complex, and the unnormalised inverse
 void fft_rows_r2c_any(const float* in, float2* out, int P, long nrows, long n_inner, long in_inner, long in_outer,
-                      long out_inner, long out_outer, int n_real, hipStream_t s);
+                      long out_inner, long out_outer, int n_real, hipStream_t s, int ncomp = 1, long in_comp = 0,
+                      long out_comp = 0);
 void fft_rows_c2r_any(const float2* in, float* out, int P, long nrows, long n_inner, long in_inner, long in_outer,
-                      long out_inner, long out_outer, int n_real, hipStream_t s);
+                      long out_inner, long out_outer, int n_real, hipStream_t s, int ncomp = 1, long in_comp = 0,
+                      long out_comp = 0);
 // Build (once, cached) every twiddle / chirp table the FP32 transforms of this
 // length and direction read, so that a later call finds them all.
 void fft_lines_any_tables(int L, int dir);

@@ -16,6 +16,7 @@
 
 #include "../../include/gpukern.h"
 #include "fft_device.h"
+#include "gk_enqueue.h"
 #include "gk_fft.h"
 
 namespace gk {
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(1024) void k_lines_reg(float2* __restrict__ data, c
     const int i = threadIdx.x & ((1 << sh) - 1), g = threadIdx.x >> sh;
     const unsigned l = (blockIdx.x << sh) + i;
     const bool ok = l < a.nlines;
-    float2* p = data + a.start(ok ? l : 0);
+    float2* p = data + blockIdx.y * a.cstride + a.start(ok ? l : 0);
     float2 v[E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(1024) void k_rows_r2c_reg(const float* __restrict__
     float2* buf = dyn_lines + M + row * line_buf(M);
     const unsigned r = blockIdx.x * nr + row;
     const bool ok = r < a.nrows;
-    const float* src = in + a.real_at(ok ? r : 0);
+    const float* src = in + blockIdx.y * a.real_comp + a.real_at(ok ? r : 0);
     float2 v[E], wp[E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(1024) void k_rows_r2c_reg(const float* __restrict__
     for (int e = 0; e < E; e++) buf[g + G * e] = v[e];
     __syncthreads();
     if (!ok) return;
-    float2* dst = out + a.cplx_at(r);
+    float2* dst = out + blockIdx.y * a.cplx_comp + a.cplx_at(r);
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const int k = g + G * e;
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(1024) void k_rows_c2r_reg(const float2* __restrict_
     float2* buf = dyn_lines + M + row * line_buf(M);
     const unsigned r = blockIdx.x * nr + row;
     const bool ok = r < a.nrows;
-    const float2* src = in + a.cplx_at(ok ? r : 0);
+    const float2* src = in + blockIdx.y * a.cplx_comp + a.cplx_at(ok ? r : 0);
     float2 v[E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(1024) void k_rows_c2r_reg(const float2* __restrict_
     __syncthreads();
     reg_fft<float, M, +1, 1, E, false>(v, g, buf, twl);
     if (!ok) return;
-    float* dst = out + a.real_at(r);
+    float* dst = out + blockIdx.y * a.real_comp + a.real_at(r);
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const int n = g + G * e;
@@ -285,8 +286,8 @@ template <int DIR> void fft_lines_reg(float2* data, int L, const LineArgs& a, hi
     switch (L) {
 #define GK_CASE(n)                                                                                              \
     case n: {                                                                                                   \
-        const int sh = lines_shift(n, line_G(n), a.nlines);                                                     \
-        k_lines_reg<n, DIR><<<div_up(a.nlines, 1L << sh), line_G(n) << sh, ((line_buf(n) << sh) + n) * 8, s>>>( \
+        const int sh = lines_shift(n, line_G(n), a.nlines * a.ncomp);                                                     \
+        k_lines_reg<n, DIR><<<dim3(div_up(a.nlines, 1L << sh), a.ncomp), line_G(n) << sh, ((line_buf(n) << sh) + n) * 8, s>>>( \
             data, tw, a, sh);                                                                                   \
         break;                                                                                                  \
     }
@@ -306,8 +307,8 @@ void fft_rows_r2c_reg(const float* in, float2* out, int P, const RowArgs& a, hip
     switch (M) {
 #define GK_CASE(n)                                                                                       \
     case n: {                                                                                            \
-        const int nr = rows_per_launch_block(n, line_G(n), a.nrows);                                     \
-        k_rows_r2c_reg<n><<<div_up(a.nrows, nr), line_G(n) * nr, (line_buf(n) * nr + n) * 8, s>>>(       \
+        const int nr = rows_per_launch_block(n, line_G(n), a.nrows * a.ncomp);                                     \
+        k_rows_r2c_reg<n><<<dim3(div_up(a.nrows, nr), a.ncomp), line_G(n) * nr, (line_buf(n) * nr + n) * 8, s>>>(       \
             in, out, twM, twP, a, nr);                                                                   \
         break;                                                                                           \
     }
@@ -325,8 +326,8 @@ void fft_rows_c2r_reg(const float2* in, float* out, int P, const RowArgs& a, hip
     switch (M) {
 #define GK_CASE(n)                                                                                       \
     case n: {                                                                                            \
-        const int nr = rows_per_launch_block(n, line_G(n), a.nrows);                                     \
-        k_rows_c2r_reg<n><<<div_up(a.nrows, nr), line_G(n) * nr, (line_buf(n) * nr + n) * 8, s>>>(       \
+        const int nr = rows_per_launch_block(n, line_G(n), a.nrows * a.ncomp);                                     \
+        k_rows_c2r_reg<n><<<dim3(div_up(a.nrows, nr), a.ncomp), line_G(n) * nr, (line_buf(n) * nr + n) * 8, s>>>(       \
             in, out, twM, twP, a, nr);                                                                   \
         break;                                                                                           \
     }
@@ -366,6 +367,36 @@ struct gpuFFT3dPlan {
     int padded[3];
     int pzc;
 };
+
+namespace gk {
+// rows, then columns; twiddle and chirp tables come from the plan's construction
+void enq_fft_forward(gpuFFT3dPlan* p, const float* real, long real_stride, float* cplx, long cplx_stride, int nc) {
+    const int N0 = p->size[0], N1 = p->size[1], N2 = p->size[2];
+    const int P0 = p->padded[0], P1 = p->padded[1], P2 = p->padded[2], Q = p->pzc;
+    float2* out = (float2*)cplx;
+    const long cs = cplx_stride / 2;
+    hipStream_t s = stream();
+    // Z: real rows (x<N0, y<N1) -> out[x][y][0..Q)
+    fft_rows_r2c_any(real, out, P2, (long)N0 * N1, N1, N2, (long)N1 * N2, Q, (long)P1 * Q, N2, s, nc, real_stride, cs);
+    // Y: columns (x<N0, kz) over y; rows y>=N1 are zero padding and not read
+    if (P1 > 1) fft_lines_any<float, -1>(out, P1, (long)N0 * Q, Q, 1, (long)P1 * Q, Q, N1, P1, s, nc, cs);
+    // X: every (ky,kz) column; planes x>=N0 are zero padding and not read
+    if (P0 > 1) fft_lines_any<float, -1>(out, P0, (long)P1 * Q, (long)P1 * Q, 1, 0, (long)P1 * Q, N0, P0, s, nc, cs);
+}
+void enq_fft_inverse(gpuFFT3dPlan* p, float* cplx, long cplx_stride, float* real, long real_stride, int nc) {
+    const int N0 = p->size[0], N1 = p->size[1], N2 = p->size[2];
+    const int P0 = p->padded[0], P1 = p->padded[1], P2 = p->padded[2], Q = p->pzc;
+    float2* in = (float2*)cplx;
+    const long cs = cplx_stride / 2;
+    hipStream_t s = stream();
+    // X: all columns, only planes x<N0 are kept
+    if (P0 > 1) fft_lines_any<float, +1>(in, P0, (long)P1 * Q, (long)P1 * Q, 1, 0, (long)P1 * Q, P0, N0, s, nc, cs);
+    // Y: columns of the kept planes, only rows y<N1 are kept
+    if (P1 > 1) fft_lines_any<float, +1>(in, P1, (long)N0 * Q, Q, 1, (long)P1 * Q, Q, P1, N1, s, nc, cs);
+    // Z: complex rows (x<N0, y<N1) -> first N2 reals
+    fft_rows_c2r_any(in, real, P2, (long)N0 * N1, N1, Q, (long)P1 * Q, N2, (long)N1 * N2, N2, s, nc, cs, real_stride);
+}
+}  // namespace gk
 
 extern "C" {
 
@@ -413,21 +444,8 @@ static size_t forward_scratch_elems(const gpuFFT3dPlan* p) {
     return need;
 }
 
-// the forward transform on stream s: rows, then columns; twiddle and chirp tables
-// come from the plan's construction
-static void plan_forward(gpuFFT3dPlan* p, const float* input, float2* out, hipStream_t s) {
-    const int N0 = p->size[0], N1 = p->size[1], N2 = p->size[2];
-    const int P0 = p->padded[0], P1 = p->padded[1], P2 = p->padded[2], Q = p->pzc;
-    // Z: real rows (x<N0, y<N1) -> out[x][y][0..Q)
-    fft_rows_r2c_any(input, out, P2, (long)N0 * N1, N1, N2, (long)N1 * N2, Q, (long)P1 * Q, N2, s);
-    // Y: columns (x<N0, kz) over y; rows y>=N1 are zero padding and not read
-    if (P1 > 1) fft_lines_any<float, -1>(out, P1, (long)N0 * Q, Q, 1, (long)P1 * Q, Q, N1, P1, s);
-    // X: every (ky,kz) column; planes x>=N0 are zero padding and not read
-    if (P0 > 1) fft_lines_any<float, -1>(out, P0, (long)P1 * Q, (long)P1 * Q, 1, 0, (long)P1 * Q, N0, P0, s);
-}
-
 void gpuFFT3dPlan_forward(gpuFFT3dPlan* p, float* input, float* output) {
-    plan_forward(p, input, (float2*)output, stream());
+    enq_fft_forward(p, input, 0, output, 0, 1);
     sync();
 }
 
@@ -438,22 +456,13 @@ void gpuFFT3dPlan_forward_noalloc(gpuFFT3dPlan* p, float* input, float* output) 
               "the maximum is %zu (use gpuFFT3dPlan_forward)",
               p->padded[0], p->padded[1], p->padded[2], need, kFFTScratchElems);
     tables_frozen(true);
-    plan_forward(p, input, (float2*)output, stream());
+    enq_fft_forward(p, input, 0, output, 0, 1);
     tables_frozen(false);
     sync();
 }
 
 void gpuFFT3dPlan_inverse(gpuFFT3dPlan* p, float* input, float* output) {
-    const int N0 = p->size[0], N1 = p->size[1], N2 = p->size[2];
-    const int P0 = p->padded[0], P1 = p->padded[1], P2 = p->padded[2], Q = p->pzc;
-    float2* in = (float2*)input;
-    hipStream_t s = stream();
-    // X: all columns, only planes x<N0 are kept
-    if (P0 > 1) fft_lines_any<float, +1>(in, P0, (long)P1 * Q, (long)P1 * Q, 1, 0, (long)P1 * Q, P0, N0, s);
-    // Y: columns of the kept planes, only rows y<N1 are kept
-    if (P1 > 1) fft_lines_any<float, +1>(in, P1, (long)N0 * Q, Q, 1, (long)P1 * Q, Q, P1, N1, s);
-    // Z: complex rows (x<N0, y<N1) -> first N2 reals
-    fft_rows_c2r_any(in, output, P2, (long)N0 * N1, N1, Q, (long)P1 * Q, N2, (long)N1 * N2, N2, s);
+    enq_fft_inverse(p, input, 0, output, 0, 1);
     sync();
 }
 

@@ -102,6 +102,7 @@ __global__ __launch_bounds__(256) void k_fft_lines_rt(C2<T>* __restrict__ data, 
     C2<T>* b = a + ((long)L << sh);
     const unsigned l0 = blockIdx.x << sh, mask = (1u << sh) - 1, nl = min(la.nlines - l0, 1u << sh);
     const bool col = la.estride != 1;
+    data += blockIdx.y * la.cstride;
     for (unsigned t = threadIdx.x; t < ((unsigned)L << sh); t += blockDim.x) {
         const unsigned q = col ? t & mask : t / L, n = col ? t >> sh : t - q * L;
         const bool in = q < nl && (int)n < la.nvalid;
@@ -124,6 +125,8 @@ __global__ __launch_bounds__(256) void k_rows_r2c_rt(const float* __restrict__ i
     float2* a = reinterpret_cast<float2*>(smem_rt);
     float2* b = a + ((long)H << sh);
     const unsigned r0 = blockIdx.x << sh, nr = min(ra.nrows - r0, 1u << sh);
+    in += blockIdx.y * ra.real_comp;
+    out += blockIdx.y * ra.cplx_comp;
     for (unsigned t = threadIdx.x; t < ((unsigned)H << sh); t += blockDim.x) {
         const unsigned q = t / H, n = t - q * H;
         float2 v = make_float2(0.f, 0.f);
@@ -161,6 +164,8 @@ __global__ __launch_bounds__(256) void k_rows_c2r_rt(const float2* __restrict__ 
     float2* a = reinterpret_cast<float2*>(smem_rt);
     float2* b = a + ((long)H << sh);
     const unsigned r0 = blockIdx.x << sh, nr = min(ra.nrows - r0, 1u << sh);
+    in += blockIdx.y * ra.cplx_comp;
+    out += blockIdx.y * ra.real_comp;
     for (unsigned t = threadIdx.x; t < ((unsigned)H << sh); t += blockDim.x) {
         const unsigned q = t / H, k = t - q * H;
         float2 v = make_float2(0.f, 0.f);
@@ -296,7 +301,7 @@ __global__ __launch_bounds__(1024) void k_lines_blue(float2* __restrict__ data, 
     const int i = threadIdx.x & ((1 << sh) - 1), g = threadIdx.x >> sh;
     const unsigned l = (blockIdx.x << sh) + i;
     const bool ok = l < a.nlines;
-    float2* p = data + a.start(ok ? l : 0);
+    float2* p = data + blockIdx.y * a.cstride + a.start(ok ? l : 0);
     float2 v[8];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -334,7 +339,7 @@ __global__ __launch_bounds__(1024) void k_rows_blue(const float* __restrict__ ri
         float2 x = make_float2(0.f, 0.f);
         if (ok && n < H) {
             if constexpr (MODE == BLUE_R2C) {
-                const float* src = rin + a.real_at(r);
+                const float* src = rin + blockIdx.y * a.real_comp + a.real_at(r);
                 if (even) {
                     if (2 * n < a.n_real) x.x = src[2 * n];
                     if (2 * n + 1 < a.n_real) x.y = src[2 * n + 1];
@@ -342,7 +347,7 @@ __global__ __launch_bounds__(1024) void k_rows_blue(const float* __restrict__ ri
                     x.x = src[n];
                 }
             } else {
-                const float2* X = cin + a.cplx_at(r);
+                const float2* X = cin + blockIdx.y * a.cplx_comp + a.cplx_at(r);
                 if (even) x = c2r_merge<float>(X[n], X[H - n], twP[n]);
                 else x = n <= H / 2 ? X[n] : cconj<float>(X[H - n]);
             }
@@ -361,7 +366,7 @@ __global__ __launch_bounds__(1024) void k_rows_blue(const float* __restrict__ ri
             __syncthreads();
         }
         if (!ok) return;
-        float2* dst = cout + a.cplx_at(r);
+        float2* dst = cout + blockIdx.y * a.cplx_comp + a.cplx_at(r);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int k = g + G * e;
@@ -374,7 +379,7 @@ __global__ __launch_bounds__(1024) void k_rows_blue(const float* __restrict__ ri
         }
     } else {
         if (!ok) return;
-        float* dst = rout + a.real_at(r);
+        float* dst = rout + blockIdx.y * a.real_comp + a.real_at(r);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int n = g + G * e;
@@ -418,11 +423,11 @@ static int blue_rows(int Lp, unsigned nrows) {
 template <int DIR> static void lines_blue(float2* data, int L, const LineArgs& a, hipStream_t s) {
     const BlueTables& bt = blue_tables(L, DIR);
     const float2* tw = twiddle_f32(bt.Lp);
-    const int sh = blue_shift(bt.Lp, a.nlines);
+    const int sh = blue_shift(bt.Lp, a.nlines * a.ncomp);
     switch (bt.Lp) {
 #define GK_CASE(n)                                                                                               \
     case n:                                                                                                      \
-        k_lines_blue<n, DIR><<<div_up(a.nlines, 1L << sh), blue_G(n) << sh, ((blue_buf(n) << sh) + n) * 8, s>>>( \
+        k_lines_blue<n, DIR><<<dim3(div_up(a.nlines, 1L << sh), a.ncomp), blue_G(n) << sh, ((blue_buf(n) << sh) + n) * 8, s>>>( \
             data, bt.w, bt.B, tw, L, a, sh);                                                                     \
         break;
         GK_FOR_EACH_BLUE(GK_CASE)
@@ -438,11 +443,11 @@ static void rows_blue(const float* rin, float* rout, const float2* cin, float2* 
     const BlueTables& bt = blue_tables(H, MODE == BLUE_R2C ? -1 : +1);
     const float2* tw = twiddle_f32(bt.Lp);
     const float2* twP = even ? twiddle_f32(P) : nullptr;
-    const int nr = blue_rows(bt.Lp, a.nrows);
+    const int nr = blue_rows(bt.Lp, a.nrows * a.ncomp);
     switch (bt.Lp) {
 #define GK_CASE(n)                                                                                                \
     case n:                                                                                                       \
-        k_rows_blue<n, MODE><<<div_up(a.nrows, nr), blue_G(n) * nr, (blue_buf(n) * nr + n) * 8, s>>>(             \
+        k_rows_blue<n, MODE><<<dim3(div_up(a.nrows, nr), a.ncomp), blue_G(n) * nr, (blue_buf(n) * nr + n) * 8, s>>>(             \
             rin, rout, cin, cout, bt.w, bt.B, tw, twP, H, even, a, nr);                                           \
         break;
         GK_FOR_EACH_BLUE(GK_CASE)
@@ -465,16 +470,17 @@ void fft_lines_any_tables(int L, int dir) {
 
 template <typename T, int DIR>
 void fft_lines_any(C2<T>* data, int L, long nlines, long n_inner, long inner, long outer, long estride, int nvalid,
-                   int nkeep, hipStream_t s) {
+                   int nkeep, hipStream_t s, int ncomp, long cstride) {
     if (nlines <= 0) return;
     if constexpr (sizeof(T) == 8) {
+        GK_ASSERT(ncomp == 1, "one FP64 transform per call");
         if (fft_length_supported(L)) {
             fft_lines<T, DIR>(data, L, nlines, n_inner, inner, outer, estride, nvalid, nkeep, s);
             return;
         }
     }
     GK_ASSERT(nlines < (1L << 31) && n_inner < (1L << 31), "FFT of %ld lines", nlines);
-    const LineArgs a{(unsigned)nlines, (unsigned)n_inner, inner, outer, estride, nvalid, nkeep};
+    const LineArgs a{(unsigned)nlines, (unsigned)n_inner, inner, outer, estride, nvalid, nkeep, ncomp, cstride};
     if constexpr (sizeof(T) == 4) {
         if (fft_reg_length(L)) {
             fft_lines_reg<DIR>(data, L, a, s);
@@ -487,8 +493,8 @@ void fft_lines_any(C2<T>* data, int L, long nlines, long n_inner, long inner, lo
         const C2<T>* tw;
         if constexpr (sizeof(T) == 4) tw = twiddle_f32(L);
         else tw = twiddle_f64(L);
-        const int sh = rt_shift<T>(L, a.nlines);
-        k_fft_lines_rt<T, DIR><<<div_up(nlines, 1L << sh), 256, (2 * L * sizeof(C2<T>)) << sh, s>>>(data, tw, L, rl, a, sh);
+        const int sh = rt_shift<T>(L, a.nlines * ncomp);
+        k_fft_lines_rt<T, DIR><<<dim3(div_up(nlines, 1L << sh), ncomp), 256, (2 * L * sizeof(C2<T>)) << sh, s>>>(data, tw, L, rl, a, sh);
         GK_LAUNCH_CHECK();
         return;
     }
@@ -496,10 +502,14 @@ void fft_lines_any(C2<T>* data, int L, long nlines, long n_inner, long inner, lo
     else GK_ASSERT(false, "FP64 FFT length %d is not supported", L);
 }
 
-template void fft_lines_any<float, -1>(float2*, int, long, long, long, long, long, int, int, hipStream_t);
-template void fft_lines_any<float, +1>(float2*, int, long, long, long, long, long, int, int, hipStream_t);
-template void fft_lines_any<double, -1>(double2*, int, long, long, long, long, long, int, int, hipStream_t);
-template void fft_lines_any<double, +1>(double2*, int, long, long, long, long, long, int, int, hipStream_t);
+template void fft_lines_any<float, -1>(float2*, int, long, long, long, long, long, int, int, hipStream_t, int,
+                                        long);
+template void fft_lines_any<float, +1>(float2*, int, long, long, long, long, long, int, int, hipStream_t, int,
+                                        long);
+template void fft_lines_any<double, -1>(double2*, int, long, long, long, long, long, int, int, hipStream_t, int,
+                                        long);
+template void fft_lines_any<double, +1>(double2*, int, long, long, long, long, long, int, int, hipStream_t, int,
+                                        long);
 
 void fft_rows_any_tables(int P, int dir) {
     const int H = P % 2 == 0 ? P / 2 : P;
@@ -508,25 +518,29 @@ void fft_rows_any_tables(int P, int dir) {
 }
 
 static RowArgs row_args(const void* real, long nrows, long n_inner, long real_inner, long real_outer, long cplx_inner,
-                        long cplx_outer, int n_real) {
+                        long cplx_outer, int n_real, int ncomp, long real_comp, long cplx_comp) {
     GK_ASSERT(nrows < (1L << 31) && n_inner < (1L << 31), "FFT of %ld rows", nrows);
-    const int vec = n_real % 2 == 0 && real_inner % 2 == 0 && real_outer % 2 == 0 && (uintptr_t)real % 8 == 0;
-    return RowArgs{(unsigned)nrows, (unsigned)n_inner, real_inner, real_outer, cplx_inner, cplx_outer, n_real, vec};
+    const int vec = n_real % 2 == 0 && real_inner % 2 == 0 && real_outer % 2 == 0 && real_comp % 2 == 0 &&
+                    (uintptr_t)real % 8 == 0;
+    return RowArgs{(unsigned)nrows, (unsigned)n_inner, real_inner, real_outer, cplx_inner, cplx_outer, n_real, vec, ncomp,
+                   real_comp, cplx_comp};
 }
 
 void fft_rows_r2c_any(const float* in, float2* out, int P, long nrows, long n_inner, long in_inner, long in_outer,
-                      long out_inner, long out_outer, int n_real, hipStream_t s) {
+                      long out_inner, long out_outer, int n_real, hipStream_t s, int ncomp, long in_comp,
+                      long out_comp) {
     if (nrows <= 0) return;
     GK_ASSERT(n_real <= P, "real FFT length %d (data %d)", P, n_real);
-    const RowArgs a = row_args(in, nrows, n_inner, in_inner, in_outer, out_inner, out_outer, n_real);
+    const RowArgs a = row_args(in, nrows, n_inner, in_inner, in_outer, out_inner, out_outer, n_real, ncomp, in_comp,
+                               out_comp);
     const int even = P % 2 == 0, H = even ? P / 2 : P;
     RadixList rl;
     if (even && fft_reg_length(H)) {
         fft_rows_r2c_reg(in, out, P, a, s);
     } else if (factor_radices(H, rl)) {
         GK_ASSERT(2L * H * 8 <= 65536, "FFT length %d is too long for one block", H);
-        const int sh = rt_shift<float>(H, a.nrows);
-        k_rows_r2c_rt<<<div_up(nrows, 1L << sh), 256, (2 * H * 8) << sh, s>>>(
+        const int sh = rt_shift<float>(H, a.nrows * ncomp);
+        k_rows_r2c_rt<<<dim3(div_up(nrows, 1L << sh), ncomp), 256, (2 * H * 8) << sh, s>>>(
             in, out, twiddle_f32(H), even ? twiddle_f32(P) : nullptr, H, even, rl, a, sh);
         GK_LAUNCH_CHECK();
     } else {
@@ -535,18 +549,20 @@ void fft_rows_r2c_any(const float* in, float2* out, int P, long nrows, long n_in
 }
 
 void fft_rows_c2r_any(const float2* in, float* out, int P, long nrows, long n_inner, long in_inner, long in_outer,
-                      long out_inner, long out_outer, int n_real, hipStream_t s) {
+                      long out_inner, long out_outer, int n_real, hipStream_t s, int ncomp, long in_comp,
+                      long out_comp) {
     if (nrows <= 0) return;
     GK_ASSERT(n_real <= P, "real FFT length %d (data %d)", P, n_real);
-    const RowArgs a = row_args(out, nrows, n_inner, out_inner, out_outer, in_inner, in_outer, n_real);
+    const RowArgs a = row_args(out, nrows, n_inner, out_inner, out_outer, in_inner, in_outer, n_real, ncomp, out_comp,
+                               in_comp);
     const int even = P % 2 == 0, H = even ? P / 2 : P;
     RadixList rl;
     if (even && fft_reg_length(H)) {
         fft_rows_c2r_reg(in, out, P, a, s);
     } else if (factor_radices(H, rl)) {
         GK_ASSERT(2L * H * 8 <= 65536, "FFT length %d is too long for one block", H);
-        const int sh = rt_shift<float>(H, a.nrows);
-        k_rows_c2r_rt<<<div_up(nrows, 1L << sh), 256, (2 * H * 8) << sh, s>>>(
+        const int sh = rt_shift<float>(H, a.nrows * ncomp);
+        k_rows_c2r_rt<<<dim3(div_up(nrows, 1L << sh), ncomp), 256, (2 * H * 8) << sh, s>>>(
             in, out, twiddle_f32(H), even ? twiddle_f32(P) : nullptr, H, even, rl, a, sh);
         GK_LAUNCH_CHECK();
     } else {

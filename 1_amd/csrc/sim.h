@@ -64,7 +64,7 @@ struct mmSim {
     int* log_acc = nullptr;
     float* log_err = nullptr;  // per trial: the error estimate (adaptive) or 0
     int log_cap = 1 << 16;
-    double* dsum = nullptr;
+    double* hsum = nullptr;  // pinned: per-block sums of the output reductions
     float* part = nullptr;  // 3 x npart: |k0|, |k_last|, error
     int npart = 0;          // max(kRedBlocks, blocks of the fused Z inverse + torque pass)
     int nk_part = 0;        // partial maxima written per torque evaluation
@@ -97,6 +97,7 @@ struct mmSim {
     gpuFFT3dPlan* plan = nullptr;
     int Pabi[3] = {};
     float* abuf[3] = {};
+    long abufStride = 0;  // floats between abuf[c] when they are one array, 0 if separate
     float* akern[6] = {};
     float* am1 = nullptr;
     float* abackup = nullptr;

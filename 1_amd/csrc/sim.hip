@@ -19,6 +19,7 @@
 #include "../../include/gpukern.h"
 #include "../../include/mumax_engine.h"
 #include "engine.h"
+#include "gk_enqueue.h"
 #include "sim.h"
 
 using namespace gk;
@@ -414,18 +415,28 @@ static long fused_run(mmSim* s, long long nsteps, double stop, bool wait) {
 }
 
 // ---------------------------------------------------------------- ABI mode (reference call sequence)
+// The drop-in operations in the reference's order, on the library stream without
+// a wait between them (gk_enqueue.h): the host reads nothing before the step's
+// reductions, and ~10 us of synchronisation per call were two thirds of a small
+// film's step.  A field's three components share their transforms' launches and a
+// stage's input is one combination.  256 x 64 film with spin torque, 4 RK4 steps:
+// 2987 us with a wait per call, 693 us.
 static void abi_calc_heff(mmSim* s, float* m, float* h) {
     // conv.go:57-100
     const int N = s->N;
-    for (int c = 0; c < 3; c++) gpuFFT3dPlan_forward(s->plan, m + c * N, s->abuf[c]);
+    if (s->abufStride) enq_fft_forward(s->plan, m, N, s->abuf[0], s->abufStride, 3);
+    else
+        for (int c = 0; c < 3; c++) enq_fft_forward(s->plan, m + (long)c * N, 0, s->abuf[c], 0, 1);
     const int nReal = s->Pabi[0] * s->Pabi[1] * (s->Pabi[2] + 2);
     if (s->Pabi[0] > 1)
-        gpu_kernelmul6(s->abuf[0], s->abuf[1], s->abuf[2], s->akern[0], s->akern[1], s->akern[2], s->akern[3],
+        enq_kernelmul6(s->abuf[0], s->abuf[1], s->abuf[2], s->akern[0], s->akern[1], s->akern[2], s->akern[3],
                        s->akern[4], s->akern[5], nReal);
     else
-        gpu_kernelmul4(s->abuf[0], s->abuf[1], s->abuf[2], s->akern[0], s->akern[1], s->akern[2], s->akern[3],
+        enq_kernelmul4(s->abuf[0], s->abuf[1], s->abuf[2], s->akern[0], s->akern[1], s->akern[2], s->akern[3],
                        nReal);
-    for (int c = 0; c < 3; c++) gpuFFT3dPlan_inverse(s->plan, s->abuf[c], h + c * N);
+    if (s->abufStride) enq_fft_inverse(s->plan, s->abuf[0], s->abufStride, h, N, 3);
+    else
+        for (int c = 0; c < 3; c++) enq_fft_inverse(s->plan, s->abuf[c], 0, h + (long)c * N, 0, 1);
     // addLocalFields (field.go:36-61)
     float b[3];
     s->fieldTmaxHost = std::max(s->fieldTmaxHost, s->htime);
@@ -434,7 +445,7 @@ static void abi_calc_heff(mmSim* s, float* m, float* h) {
     for (int c = 0; c < 3; c++) hext[c] = b[c] / (float)s->unitField;
     float kk = s->kAnis;
     float ax[3] = {s->u[0], s->u[1], s->u[2]};
-    gpu_add_local_fields(m, h, N, hext, nullptr, s->p.anisType, &kk, ax);
+    enq_add_local_fields(m, h, N, hext, nullptr, s->p.anisType, &kk, ax);
 }
 
 static bool has_current(const mmParams& p) { return p.current[0] != 0 || p.current[1] != 0 || p.current[2] != 0; }
@@ -472,7 +483,7 @@ static void abi_spintorque(mmSim* s, float* m, float* h) {
     float j[3], u[3];
     current_at(s, j);
     for (int i = 0; i < 3; i++) u[i] = 0.5f * (j[i] / (Ms / L)) / (float)s->cell[i];
-    gpu_spintorque_deltaM(m, h, alpha, beta, eps, u, s->jMask, dtGilb, s->p.size[0], s->p.size[1], s->p.size[2]);
+    enq_spintorque_deltaM(m, h, alpha, beta, eps, u, s->jMask, dtGilb, s->p.size[0], s->p.size[1], s->p.size[2]);
 }
 
 static void abi_torque(mmSim* s, float* m, float* h) {
@@ -482,15 +493,12 @@ static void abi_torque(mmSim* s, float* m, float* h) {
         return;
     }
     const float alpha = (float)s->p.alpha;
-    gpu_deltaM(m, h, alpha, s->alphaMap, 1.f / (1.f + alpha * alpha), s->N);
+    enq_deltaM(m, h, alpha, s->alphaMap, 1.f / (1.f + alpha * alpha), s->N);
 }
 
 // Sim.Normalize (sim.go:230-239): to the norm map when there is one
 static void normalize_abi(mmSim* s, float* m) {
-    if (s->normMap)
-        gpu_normalize_map(m, s->normMap, s->N);
-    else
-        gpu_normalize_uniform(m, s->N);
+    enq_normalize(m, s->normMap, s->N);
 }
 
 static bool semianal(const mmSim* s) { return s->p.solver == MM_SEMIANAL1 || s->p.solver == MM_SEMIANAL2; }
@@ -503,25 +511,25 @@ static void abi_semianal_step(mmSim* s) {
     float *m1 = s->m, *m2 = s->am1, *m3 = s->k[1], *h = s->k[0];
     if (s->hsteps == 0) {
         abi_calc_heff(s, m1, h);
-        gpu_anal_fw_step(dt / 2.f, alpha, N, m1, m2, h);
+        enq_anal_fw_step(dt / 2.f, alpha, N, m1, m2, h);
         abi_calc_heff(s, m2, h);
-        gpu_anal_fw_step(dt, alpha, N, m1, m1, h);
+        enq_anal_fw_step(dt, alpha, N, m1, m1, h);
     } else if (s->p.solver == MM_SEMIANAL1) {
         abi_calc_heff(s, m1, h);
-        gpu_anal_fw_step(dt, alpha, N, m2, m2, h);
+        enq_anal_fw_step(dt, alpha, N, m2, m2, h);
         abi_calc_heff(s, m2, h);
-        gpu_anal_fw_step(dt, alpha, N, m1, m1, h);
+        enq_anal_fw_step(dt, alpha, N, m1, m1, h);
     } else {
         abi_calc_heff(s, m1, h);
-        gpu_anal_fw_step(dt, alpha, N, m2, m3, h);
-        gpu_linear_combination(m3, m2, 0.5f, 0.5f, n3);
+        enq_anal_fw_step(dt, alpha, N, m2, m3, h);
+        enq_linear_combination(m3, m2, 0.5f, 0.5f, n3);
         abi_calc_heff(s, m3, h);
-        gpu_anal_fw_step(dt, alpha, N, m2, m2, h);
+        enq_anal_fw_step(dt, alpha, N, m2, m2, h);
         abi_calc_heff(s, m2, h);
-        gpu_anal_fw_step(dt, alpha, N, m1, m3, h);
-        gpu_linear_combination(m3, m1, 0.5f, 0.5f, n3);
+        enq_anal_fw_step(dt, alpha, N, m1, m3, h);
+        enq_linear_combination(m3, m1, 0.5f, 0.5f, n3);
         abi_calc_heff(s, m3, h);
-        gpu_anal_fw_step(dt, alpha, N, m1, m1, h);
+        enq_anal_fw_step(dt, alpha, N, m1, m1, h);
     }
     if (s->hsteps % 100 == 0) {
         normalize_abi(s, m1);
@@ -542,7 +550,17 @@ static void abi_step(mmSim* s) {
     float* m = s->m;
     float* m1 = s->am1;
     const double time0 = s->htime;
-    memcpy_on_gpu(m, s->abackup, n3);
+    enq_copy(m, s->abackup, n3);
+    // dt times the nonzero coefficients of a tableau row, with their stages
+    auto terms = [&](const float* a) {
+        CombineTerms c{};
+        for (int j = 0; j < order; j++)
+            if (a[j] != 0.f) {
+                c.k[c.n] = s->k[j];
+                c.c[c.n++] = s->hdt * a[j];
+            }
+        return c;
+    };
     bool good = false;
     int trials = 0;
     while (!good && trials < kMaxStepTrials) {
@@ -550,12 +568,10 @@ static void abi_step(mmSim* s) {
         s->htrials++;
         for (int i = 0; i < order; i++) {
             if (t.fsal && i == 0 && s->hfsal) {
-                memcpy_on_gpu(s->k[order - 1], s->k[0], n3);
+                enq_copy(s->k[order - 1], s->k[0], n3);
             } else {
                 s->htime = time0 + (double)(t.c[i] * s->hdt);
-                memcpy_on_gpu(m, m1, n3);
-                for (int j = 0; j < order; j++)
-                    if (t.a[i][j] != 0.f) gpu_madd(m1, s->hdt * t.a[i][j], s->k[j], n3);
+                enq_combine(m1, m, terms(t.a[i]), n3);
                 abi_calc_heff(s, m1, s->k[i]);
                 abi_torque(s, m1, s->k[i]);
                 s->hfsal = true;
@@ -576,15 +592,14 @@ static void abi_step(mmSim* s) {
         const float dtu = s->hdt;
         s->htime = time0 + (double)s->hdt;
         if (t.adaptive) {
-            memcpy_on_gpu(m, m1, n3);
-            for (int i = 0; i < order; i++)
-                if (t.b2[i] != 0.f) gpu_madd(m1, t.b2[i] * s->hdt, s->k[i], n3);
+            enq_combine(m1, m, terms(t.b2), n3);
         }
-        for (int i = 0; i < order; i++)
-            if (t.b[i] != 0.f) gpu_madd(m, t.b[i] * s->hdt, s->k[i], n3);
+        enq_combine(m, m, terms(t.b), n3);
         bool bad = false;
         if (t.adaptive) {
-            gpu_madd(m1, -1.f, m, n3);
+            CombineTerms diff{};
+            diff.k[0] = m, diff.c[0] = -1.f, diff.n = 1;
+            enq_combine(m1, m1, diff, n3);
             float err = gpu_reduce(REDUCE_MAXABS, m1, s->redDev, s->redHost.data(), s->redBlocks, s->redThreads, n3);
             s->herr = err;
             float factor = (float)pow((double)((float)s->p.maxError / err), 1.0 / (double)t.order);
@@ -593,7 +608,7 @@ static void abi_step(mmSim* s) {
             s->hdt = s->hdt * factor;
             GK_ASSERT(!std::isnan(s->hdt), "dt = NaN");
             if (err > 2.f * (float)s->p.maxError) {
-                memcpy_on_gpu(s->abackup, m, n3);
+                enq_copy(s->abackup, m, n3);
                 bad = true;
                 s->hrejects++;
             } else {
@@ -630,7 +645,14 @@ static void abi_init(mmSim* s, const double cellInt[3]) {
     for (int i = 0; i < 3; i++) s->Pabi[i] = size[i] > 1 && !s->p.periodic[i] ? 2 * size[i] : size[i];
     s->plan = new_gpuFFT3dPlan_padded(size, s->Pabi);
     const long phys = (long)s->Pabi[0] * s->Pabi[1] * (s->Pabi[2] + 2);
-    for (int c = 0; c < 3; c++) s->abuf[c] = new_gpu_array((int)phys);
+    // the three spectra as one array, so that their transforms share launches
+    if (3 * phys <= INT_MAX) {
+        s->abuf[0] = new_gpu_array((int)(3 * phys));
+        s->abufStride = phys;
+        for (int c = 1; c < 3; c++) s->abuf[c] = s->abuf[0] + c * phys;
+    } else {
+        for (int c = 0; c < 3; c++) s->abuf[c] = new_gpu_array((int)phys);
+    }
     // real-space kernel in FP64 on the device (FaceKernel6 + Exch6), rounded to float32;
     // the spectrum of the real-space kernel is taken with the drop-in plan, as loadKernel6 does
     const int nK = s->Pabi[0] == 1 ? 4 : 6;
@@ -751,7 +773,6 @@ mmSim* mm_sim_new(const mmParams* p, const float* m0, int mode) {
     s->log_dt = (double*)dmalloc(s, s->log_cap * sizeof(double));
     s->log_acc = (int*)dmalloc(s, s->log_cap * sizeof(int));
     s->log_err = (float*)dmalloc(s, s->log_cap * sizeof(float));
-    s->dsum = (double*)dmalloc(s, 4 * sizeof(double));
     EngineState h{};
     h.dt = (float)(p->dt / s->unitTime);  // init.go:280-284
     if (h.dt == 0.f) h.dt = 1e-4f;
@@ -809,13 +830,14 @@ void mm_sim_free(mmSim* s) {
     for (int i = 0; i < 7; i++)
         cached_free(s->k[i]);
     for (float* p : {s->m, s->mi, s->mtmp, s->fB, s->alphaMap, s->normMap, s->jMask}) cached_free(p);
-    for (void* p : {(void*)s->st, (void*)s->log_dt, (void*)s->log_acc, (void*)s->log_err, (void*)s->dsum, (void*)s->fT,
+    for (void* p : {(void*)s->st, (void*)s->log_dt, (void*)s->log_acc, (void*)s->log_err, (void*)s->fT,
                     (void*)s->part, (void*)s->epart})
         cached_free(p);
+    cached_host_free(s->hsum);
     conv_plan_free(s->cp);
     if (s->plan) delete_gpuFFT3dPlan(s->plan);
     for (int c = 0; c < 3; c++)
-        if (s->abuf[c]) free_gpu_array(s->abuf[c]);
+        if (s->abuf[c] && (c == 0 || !s->abufStride)) free_gpu_array(s->abuf[c]);
     for (int k = 0; k < 6; k++)
         if (s->akern[k]) free_gpu_array(s->akern[k]);
     for (float* p : {s->am1, s->abackup, s->redDev})
@@ -833,6 +855,7 @@ long mm_sim_run(mmSim* s, double seconds) {
             abi_step(s);
             n++;
         }
+        sync();
         return n;
     }
     EngineState h = read_state(s);
@@ -849,6 +872,7 @@ long mm_sim_run_until(mmSim* s, double stop) {
             abi_step(s);
             n++;
         }
+        sync();
         return n;
     }
     return fused_run(s, -1, stop, true);
@@ -857,6 +881,7 @@ long mm_sim_run_until(mmSim* s, double stop) {
 void mm_sim_steps(mmSim* s, int n) {
     if (s->mode == MM_MODE_ABI) {
         for (int i = 0; i < n; i++) abi_step(s);
+        sync();
         return;
     }
     fused_run(s, n, INFINITY, true);
@@ -949,6 +974,7 @@ static void eval_heff(mmSim* s, const float* m_host, float* h_dev) {
     if (s->mode == MM_MODE_ABI) {
         GK_CHECK(hipStreamSynchronize(s->s));
         abi_calc_heff(s, s->mi, h_dev);
+        sync();
         return;
     }
     StageIn si{};
@@ -975,6 +1001,7 @@ void mm_sim_torque(mmSim* s, const float* m, float* k) {
     eval_heff(s, m, s->mtmp);
     if (has_current(s)) {
         abi_spintorque(s, s->mi, s->mtmp);  // torque.go:40-49
+        sync();
     } else {
         const float alpha = (float)s->p.alpha;
         gpu_deltaM(s->mi, s->mtmp, alpha, s->alphaMap, (float)(1.0 / (1.0 + s->p.alpha * s->p.alpha)), s->N);
@@ -982,15 +1009,21 @@ void mm_sim_torque(mmSim* s, const float* m, float* k) {
     GK_CHECK(hipMemcpy(k, s->mtmp, s->N3 * sizeof(float), hipMemcpyDeviceToHost));
 }
 
+// pinned buffer of the output reductions' block sums, from the first of them on
+static double* sum_buffer(mmSim* s) {
+    if (!s->hsum) s->hsum = (double*)cached_host_malloc(3 * kSumBlocks * sizeof(double));
+    return s->hsum;
+}
+
 double mm_sim_energy(mmSim* s) {
     StageIn si{};
     si.m = s->m;
     conv_apply(s->cp, si, s->mtmp, s->s);
-    double t, ts;
+    double t = 0, ts = 0;
     if (s->mode == MM_MODE_ABI) {
         t = s->htime;
         ts = std::max(s->fieldTmaxHost, t);
-    } else {
+    } else if (s->field.fn || s->p.nField >= 2) {  // a static field needs no time, and no wait for it
         const EngineState h = read_state(s);
         t = h.time;
         ts = std::max(h.field_tmax, t);
@@ -998,20 +1031,22 @@ double mm_sim_energy(mmSim* s) {
     float b[3], hext[3];
     applied_field_host(s, t, ts, b);
     for (int c = 0; c < 3; c++) hext[c] = b[c] / (float)s->unitField;
-    GK_CHECK(hipMemsetAsync(s->dsum, 0, sizeof(double), s->s));
-    launch_energy(s->m, s->mtmp, hext, s->p.anisType, s->kAnis, s->u, s->N, s->dsum, s->s);
-    double e = 0;
-    GK_CHECK(hipMemcpyAsync(&e, s->dsum, sizeof(double), hipMemcpyDeviceToHost, s->s));
+    launch_energy(s->m, s->mtmp, hext, s->p.anisType, s->kAnis, s->u, s->N, sum_buffer(s), s->s);
     GK_CHECK(hipStreamSynchronize(s->s));
+    double e = 0;
+    for (int i = 0; i < sum_blocks(s->N); i++) e += s->hsum[i];
     return e * s->cell[0] * s->cell[1] * s->cell[2];
 }
 
 void mm_sim_average_m(mmSim* s, double* avg) {
-    GK_CHECK(hipMemsetAsync(s->dsum, 0, 3 * sizeof(double), s->s));
-    launch_sum3(s->m, s->N, s->dsum, s->s);
-    GK_CHECK(hipMemcpyAsync(avg, s->dsum, 3 * sizeof(double), hipMemcpyDeviceToHost, s->s));
+    launch_sum3(s->m, s->N, sum_buffer(s), s->s);
     GK_CHECK(hipStreamSynchronize(s->s));
-    for (int c = 0; c < 3; c++) avg[c] /= (double)s->N;
+    const int nb = sum_blocks(s->N);
+    for (int c = 0; c < 3; c++) {
+        double a = 0;
+        for (int i = 0; i < nb; i++) a += s->hsum[c * nb + i];
+        avg[c] = a / (double)s->N;
+    }
 }
 
 long mm_sim_kernel_spectrum(mmSim* s, float* out) {
@@ -1078,7 +1113,7 @@ unsigned long long mm_sim_footprint(const mmParams* p) {
     size_t b = conv_plan_footprint(p->size, &epi);
     const int npart = std::max(kRedBlocks, epi);
     b += N3 * sizeof(float) * (size_t)(1 + t.S + 2);  // m, k_0..k_{S-1}, m_i, m_tmp
-    b += sizeof(EngineState) + (size_t)(1 << 16) * (sizeof(double) + sizeof(int) + sizeof(float)) + 4 * sizeof(double);
+    b += sizeof(EngineState) + (size_t)(1 << 16) * (sizeof(double) + sizeof(int) + sizeof(float));
     b += 3 * (size_t)npart * sizeof(float) + (size_t)npart * sizeof(double);  // part, epart
     if (p->nField >= 2) b += (size_t)p->nField * (sizeof(double) + 3 * sizeof(float));
     if (p->alphaMap) b += (size_t)(N3 / 3) * sizeof(float);
