@@ -16,7 +16,7 @@ LIB = os.path.join(HERE, "libgpukern.so")
 
 SOURCES = ["gk_basic.hip", "gk_fft.hip", "gk_fft_any.hip", "conv.hip", "rk.hip", "sim.hip", "batch.hip", "io.cpp"]
 # kernels with many length instantiations, compiled in parts (-DGK_PART=i): they set the build's time
-PARTS = {"conv_z.hip": 5, "batch_z.hip": 5, "batch_any.hip": 4}
+PARTS = {"conv_z.hip": 7, "batch_z.hip": 7, "batch_any.hip": 4}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -44,7 +44,10 @@ def _compile(job):
 
 def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
+    # the longest first: the conv_z parts, the dispatch kernels of the Z inverse, batch and conv
     jobs = [(src, i) for src, n in PARTS.items() for i in range(n)] + [(src, None) for src in SOURCES]
+    slow = {"conv_z.hip": 0, "batch.hip": 1, "conv.hip": 1, "batch_any.hip": 2, "batch_z.hip": 3}
+    jobs.sort(key=lambda j: slow.get(j[0], 4))
     with ThreadPoolExecutor(max_workers=min(len(jobs), os.cpu_count() or 4)) as ex:
         objs = list(ex.map(_compile, jobs))
     tmp = LIB + ".tmp"

@@ -210,6 +210,7 @@ __device__ __forceinline__ void bz_inv(const BSim& d, int lb, const BStage& sg, 
     const int nyb = (d.Ny + TR - 1) / TR;
     const int yb = lb % nyb, x = lb / nyb;
     EpiArgs ea{};
+    ea.nx = -1;
     ea.m = sg.use_mi ? d.mi : d.m;
     ea.out = FIN == 1 ? d.m : d.k[sg.i];
     for (int j = 0; j < 6; j++) {

@@ -972,6 +972,8 @@ static void launch_zinv_epi(const ConvPlan& cp, const EpiArgs& ea, const EngineS
     GK_ASSERT(st != nullptr && ea.nu >= 0 && ea.nu <= 6 && (ea.fin != 1 || ea.nu <= 3) &&
                   (ea.fin != 2 || (ea.mhigh && ea.part_err)),
               "fused Z inverse: bad epilogue");
+    GK_ASSERT(ea.nx < 0 || (ea.nx <= 4 && ea.fin != 2 && (ea.fin == 1 || (ea.nu <= 1 && ea.xm)) && z_fwd_fused(M)),
+              "fused Z inverse: bad next stage");
     // pad the list of earlier stages to the kernel's bound with (m, 0, 0): fmaf(0, m, z) == z
     const int nu = ea.nu;
     EpiArgs e = ea;
@@ -980,6 +982,10 @@ static void launch_zinv_epi(const ConvPlan& cp, const EpiArgs& ea, const EngineS
         e.a[j] = 0.f;
         e.b[j] = 0.f;
         e.ce[j] = 0.0;
+    }
+    for (int j = std::max(ea.nx, 0); j < 4; j++) {
+        e.xk[j] = ea.xm;
+        e.xa[j] = 0.f;
     }
     const float2* twM = twiddle_f32(M);
     const float2* twP = twiddle_f32(cp.P[2]);
@@ -1192,40 +1198,55 @@ void conv_run_pass(const ConvPlan& cp, int cls, const StageIn& in, float* h, con
     }
 }
 
-void conv_apply(const ConvPlan& cp, const StageIn& in, float* h, hipStream_t s, Prof* prof, const EpiArgs* epi) {
+// Up to 4 waves of the Z inverse per SIMD (1024 of them): there the launches'
+// latencies count and one kernel less gains (20 RK4 steps of a 128 x 32 film 1453 ->
+// 1164 us, 150 x 91 x 3 slab 1240 -> 1173, 1024 x 1024 film, 3072 waves, 1809 -> 1784).
+// Larger grids keep the passes apart, whose own shapes and overlap are worth more
+// (256 x 256 x 16, 6144 waves: 10 RK4 steps 3711 us apart, 3818 fused).
+bool conv_fwd_fused(const ConvPlan& cp) {
+    if (!z_fwd_fused(cp.M)) return false;
+    const int tr = conv_epi_rows(cp.M, cp.er());
+    const long blocks = (long)div_up(cp.N[1], tr) * cp.N[0];
+    return blocks * div_up(3 * tr * reg_fft_G(cp.M), 64) <= 4096;
+}
+
+void conv_apply(const ConvPlan& cp, const StageIn* in, const EngineState* st, float* h, hipStream_t s, Prof* prof,
+                const EpiArgs* epi) {
     Prof dummy;
     Prof& p = prof ? *prof : dummy;
-    p.begin(0, s);
-    launch_zfwd(cp, in, s);
-    p.end(s);
+    if (in) {
+        p.begin(0, s);
+        launch_zfwd(cp, *in, s);
+        p.end(s);
+    }
     if (cp.P[0] == 1) {
         p.begin(2, s);
-        launch_y2d(cp, in.st, s);
+        launch_y2d(cp, st, s);
         p.end(s);
     } else if (cp.yxy) {
         p.begin(2, s);
-        launch_yxy(cp, in.st, s);
+        launch_yxy(cp, st, s);
         p.end(s);
     } else if (cp.plane3 && cp.tp.pp) {
         p.begin(2, s);
-        launch_plane3(cp, in.st, s);
+        launch_plane3(cp, st, s);
         p.end(s);
     } else {
         p.begin(1, s);
-        launch_y3d(cp, in.st, true, s);
+        launch_y3d(cp, st, true, s);
         p.end(s);
         p.begin(2, s);
-        launch_xmul(cp, in.st, s);
+        launch_xmul(cp, st, s);
         p.end(s);
         p.begin(3, s);
-        launch_y3d(cp, in.st, false, s);
+        launch_y3d(cp, st, false, s);
         p.end(s);
     }
     p.begin(4, s);
     if (epi)
-        launch_zinv_epi(cp, *epi, in.st, s);
+        launch_zinv_epi(cp, *epi, st, s);
     else
-        launch_zinv(cp, h, in.st, s);
+        launch_zinv(cp, h, st, s);
     p.end(s);
 }
 

@@ -53,6 +53,10 @@ template <int M> constexpr int epi_rows_v(int v) {
     return (v == 1 && d > 1) ? d / 2 : d;
 }
 
+// lengths whose fused Z inverse can end with the next stage's Z forward (a block of
+// longer rows has two of them, whose 16 B runs of B1 would make the stores partial lines)
+constexpr bool z_fwd_fused(int M) { return M >= 2 && M <= 1024; }
+
 template <int M>
 void zfwd_run(const ConvPlan& cp, const StageIn& si, int NKp, const float2* twM, const float2* twP, hipStream_t s);
 template <int M>

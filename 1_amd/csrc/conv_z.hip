@@ -30,6 +30,23 @@ static void zinv_epi_launch(const ConvPlan& cp, const EpiArgs& e, const EngineSt
                             const float2* twP, hipStream_t s) {
     const int Nx = cp.N[0], Ny = cp.N[1], Nz = cp.N[2], nu = e.nu;
     const dim3 g(div_up(Ny, TR), Nx), b(3 * TR * RegFFT<M>::G);
+    if constexpr (z_fwd_fused(M))
+        if (e.nx >= 0) {
+#define GK_ZX(NU, FIN, NX) k_zinv_epi<M, TR, NU, FIN, NX><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz)
+            if (e.fin == 1) {
+                if (nu <= 1) GK_ZX(1, 1, 0);
+                else GK_ZX(3, 1, 0);
+            } else if (nu == 0) {
+                if (e.nx == 0) GK_ZX(0, 0, 0);
+                else GK_ZX(0, 0, 4);
+            } else {
+                if (e.nx == 0) GK_ZX(1, 0, 0);
+                else if (e.nx == 1) GK_ZX(1, 0, 1);
+                else GK_ZX(1, 0, 4);
+            }
+#undef GK_ZX
+            return;
+        }
     if (e.fin == 1) {
         if (nu <= 1) k_zinv_epi<M, TR, 1, 1><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);
         else k_zinv_epi<M, TR, 3, 1><<<g, b, 0, s>>>(cp.B1, e, twM, twP, st, Nx, Ny, Nz);

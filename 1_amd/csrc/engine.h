@@ -243,8 +243,12 @@ struct EpiArgs;
 // h = K * m (planar 3N each); in = stage build description, out = 3N floats.
 // With epi != null the Z inverse pass ends in the torque / final-combination
 // epilogue described by *epi instead of writing h.
-void conv_apply(const ConvPlan& cp, const StageIn& in, float* h, hipStream_t s, Prof* prof = nullptr,
-                const EpiArgs* epi = nullptr);
+// in == null (with epi): B1 already holds the input's Z forward, from the epilogue
+// of the stage before (epi->nx >= 0 there); st is in->st then.
+void conv_apply(const ConvPlan& cp, const StageIn* in, const EngineState* st, float* h, hipStream_t s,
+                Prof* prof = nullptr, const EpiArgs* epi = nullptr);
+// whether the plan's Z inverse ends with the next stage's Z forward
+bool conv_fwd_fused(const ConvPlan& cp);
 // number of blocks (= per-block partial maxima) of the fused Z inverse + torque pass
 int conv_epi_blocks(const ConvPlan& cp);  // blocks of the fused Z inverse at cp.tp.er
 int conv_epi_blocks_max(const int N[3]);   // ... the most over every row variant
@@ -376,6 +380,14 @@ struct EpiArgs {
     double ce_self;
     float* mhigh;
     float* part_err;
+    // the next stage's Z forward in the same kernel (zinv_epi_tile's NX >= 0): its
+    // input is xm + dt (sum_j xa_j xk_j + xself k_i), or the new m where fin == 1,
+    // stored to xmi if that is not null
+    int nx;
+    const float* xm;
+    const float* xk[4];
+    float xa[4], xself;
+    float* xmi;
 };
 
 struct FinalArgs {

@@ -286,12 +286,17 @@ TorqueArgs gk::torque_args(const mmSim* s, float c, float* part) {
 }
 
 // ---------------------------------------------------------------- fused mode
-static void enqueue_trial(mmSim* s) {
+// fwd: B1 holds the Z forward of m, from the trial before; next: the last stage of a
+// fixed-step tableau leaves the Z forward of the new m there for the next trial.
+// Returns whether it did.
+static bool enqueue_trial(mmSim* s, bool fwd, bool next) {
     const Tableau& t = s->tb;
     const CtrlParams cp = ctrl_params(s);
     Prof& pf = s->prof;
     // the trial has been started by the one before (launch_ctrl_end) or launch_set_target;
     // the FSAL stage is in k[0] (launch_commit) and its dt control done
+    const bool fusable = conv_fwd_fused(s->cp);
+    const float* mi_ready = nullptr;  // the stage input, where the stage before has stored it
     for (int i = 0; i < t.S; i++) {
         if (i == 0 && t.fsal && s->fsalHost) continue;
         StageIn si{};
@@ -323,9 +328,31 @@ static void enqueue_trial(mmSim* s) {
         if (!fin && !efin && ea.nu >= 2) {
             // the Z forward pass stores m_i, which the epilogue reads instead of
             // rebuilding it from m and nu earlier stages (same fmaf chain, same bits)
+            GK_ASSERT(!fwd || mi_ready, "stage input of a fused forward pass");
             si.mout = s->mi;
             ea.m = s->mi;
             ea.nu = 0;
+        }
+        // the next stage's Z forward at the end of this one's epilogue, unless the dt
+        // control after k0 comes between them
+        ea.nx = -1;
+        mi_ready = nullptr;
+        if (fin && next && fusable) {
+            ea.nx = 0;
+        } else if (fusable && i + 1 < t.S && !(i == 0 && needs_after_k0(s)) && t.a[i + 1][i] != 0.f && ea.nu <= 1) {
+            int used = 0;
+            ea.xm = s->m;
+            ea.nx = 0;
+            for (int j = 0; j < i; j++)
+                if (t.a[i + 1][j] != 0.f) {
+                    ea.xk[ea.nx] = s->k[j];
+                    ea.xa[ea.nx++] = t.a[i + 1][j];
+                    used++;
+                }
+            ea.xself = t.a[i + 1][i];
+            // the next stage reads a stored input if it has two or more earlier stages (as above)
+            const bool nfin = !t.adaptive && i + 1 == t.S - 1, nefin = t.fsal_final() && i + 1 == t.S - 1;
+            if (!nfin && !nefin && used + 1 >= 2) mi_ready = ea.xmi = s->mi;
         }
         if (efin) {
             ea.ce_self = (double)t.b2[i] - (double)t.b[i];
@@ -341,7 +368,8 @@ static void enqueue_trial(mmSim* s) {
         // wantEnergy: the energy of the new state (FSAL, last stage) or of the step's start
         // (rk.go:324-333)
         if (s->wantEnergy && i == (t.fsal ? t.S - 1 : 0)) ea.epart = s->epart;
-        conv_apply(s->cp, si, nullptr, s->s, &pf, &ea);
+        conv_apply(s->cp, fwd ? nullptr : &si, s->st, nullptr, s->s, &pf, &ea);
+        fwd = ea.nx >= 0;
         if (i == 0 && needs_after_k0(s)) {
             pf.begin(7, s->s);
             launch_ctrl_after_k0(s->st, cp, s->s);
@@ -370,6 +398,7 @@ static void enqueue_trial(mmSim* s) {
         launch_commit(s->m, s->mtmp, t.fsal ? s->k[0] : nullptr, s->k[t.S - 1], s->st, s->normMap, s->N, s->s);
     pf.end(s->s);
     if (t.fsal) s->fsalHost = true;
+    return !t.adaptive && fwd;
 }
 
 static long fused_run(mmSim* s, long long nsteps, double stop, bool wait) {
@@ -380,7 +409,8 @@ static long fused_run(mmSim* s, long long nsteps, double stop, bool wait) {
     launch_set_target(s->st, nsteps, stop, &cp, s->s);
     if (!wait) {
         // enqueue exactly nsteps trials (fixed-step tableaux never reject)
-        for (long long i = 0; i < nsteps; i++) enqueue_trial(s);
+        bool fwd = false;
+        for (long long i = 0; i < nsteps; i++) fwd = enqueue_trial(s, fwd, i + 1 < nsteps);
         return nsteps;
     }
     // Trials enqueued past the end are launches that do nothing: at most as many as
@@ -398,7 +428,8 @@ static long fused_run(mmSim* s, long long nsteps, double stop, bool wait) {
             n = std::min<long long>(need, s->tb.adaptive ? batch : 1024);
         }
         n = std::max(n, 1LL);
-        for (long long i = 0; i < n; i++) enqueue_trial(s);
+        bool fwd = false;
+        for (long long i = 0; i < n; i++) fwd = enqueue_trial(s, fwd, i + 1 < n);
         h = read_state(s);
         if (h.nan_dt) {
             fprintf(stderr, "libgpukern: dt = NaN (rk.go:448-452)\n");
@@ -979,7 +1010,7 @@ static void eval_heff(mmSim* s, const float* m_host, float* h_dev) {
     }
     StageIn si{};
     si.m = s->mi;
-    conv_apply(s->cp, si, h_dev, s->s);
+    conv_apply(s->cp, &si, nullptr, h_dev, s->s);
     EngineState h = read_state(s);
     float b[3], hext[3];
     applied_field_host(s, h.time, std::max(h.field_tmax, h.time), b);
@@ -1018,7 +1049,7 @@ static double* sum_buffer(mmSim* s) {
 double mm_sim_energy(mmSim* s) {
     StageIn si{};
     si.m = s->m;
-    conv_apply(s->cp, si, s->mtmp, s->s);
+    conv_apply(s->cp, &si, nullptr, s->mtmp, s->s);
     double t = 0, ts = 0;
     if (s->mode == MM_MODE_ABI) {
         t = s->htime;
@@ -1185,6 +1216,7 @@ static double time_pass(mmSim* s, int cls, int n, int nk) {
     }
     EpiArgs ea{};
     ea.m = s->m;
+    ea.nx = -1;
     ea.out = s->mtmp;  // k[0] may hold the next trial's FSAL stage
     ea.t = torque_args(s, s->tb.c[0], s->part);
     launch_set_active(s->st, s->s);

@@ -36,6 +36,31 @@ def test_film_column_lengths_vs_oracle(mm, orc, ny):
     assert np.abs(h - ref).max() < 5e-6 * np.abs(ref).max()
 
 
+# every tableau's stages with their forward passes in the epilogues: even and odd rows, the shortest, partly
+# filled tiles, and the dt control after the first stage (which keeps the passes apart)
+@pytest.mark.parametrize("solver", ["rk2", "rk12", "rk3", "rk23", "rk4", "rkck", "rkdp"])
+@pytest.mark.parametrize("size,kw", [((1, 21, 30), {}), ((3, 9, 51), {}), ((2, 12, 3), {}), ((2, 5, 2), {}),
+                                     ((4, 10, 16), {"max_dt": 1.5e-14})])
+def test_fused_stages_vs_oracle(mm, orc, solver, size, kw):
+    m0 = random_m(size, 9)
+    cfg = cfg_of(size, m0, solver=solver, dt=1e-14, maxerror=1e-4, field=("static", (1e-2, 2e-2, -3e-2)), **kw)
+    s = mm.workloads.make_sim(cfg)
+    s.steps(6)
+    dts, acc = s.trial_log()
+    o = orc.sim(m0, **mm.workloads.oracle_kwargs(cfg))
+    i = 0
+    while i < len(dts):
+        j = i
+        while not acc[j]:
+            j += 1
+        o.step_replay(dts[i:j + 1], acc[i:j + 1])
+        i = j + 1
+    assert s.state()["steps"] == 6
+    dm = np.abs(s.m.reshape(-1) - np.asarray(o.m).reshape(-1)).max()
+    s.free()
+    assert dm < 1e-5
+
+
 # row lengths of every part of the Z kernels, odd and even, with partly filled row tiles
 @pytest.mark.parametrize("size", [(2, 9, 40), (3, 21, 51), (1, 17, 130), (1, 35, 301), (2, 5, 640), (1, 3, 1601)])
 def test_row_variants_give_the_same_steps(mm, lib, tmp_path, size):
