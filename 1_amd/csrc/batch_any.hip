@@ -51,8 +51,10 @@ void any_attr_zfwd() {
 
 #elif GK_PART <= 2
 
+// (96 registers, 5 waves per SIMD; the last stage of an adaptive tableau, with six
+// earlier stages and their FP64 errors, would spill: 91 us, 136 with the bound)
 template <int NU, int FIN>
-__global__ __launch_bounds__(768) void kb_zinv_any(const BSim* sims, const int2* map,
+__global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(FIN == 2 ? 1 : 5))) void kb_zinv_any(const BSim* sims, const int2* map,
                                                    BStage sg) {
     extern __shared__ float2 dyn[];
     const BBlock bb = bblock(sims, map);

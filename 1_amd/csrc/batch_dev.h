@@ -261,6 +261,10 @@ template <int M> constexpr int epi_rows_c() {
     int p = 1;
     while (p * 2 <= tr) p *= 2;
     tr = p;
+    // three blocks per CU by their LDS: a dispatch launch gives every block the LDS of
+    // its largest length, so at 80 KB all of them ran two to a CU (40-member sweep,
+    // the launch of the short lengths 44.4 us, now 38.4)
+    while (tr > 4 && zinv_epi_lds_elems(M, tr) * 8 > 48 * 1024) tr /= 2;
     while (tr > 1 && zinv_epi_lds_elems(M, tr) * 8 > 80 * 1024) tr /= 2;
     return tr;
 }

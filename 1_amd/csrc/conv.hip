@@ -1043,9 +1043,9 @@ static void launch_y3d(const ConvPlan& cp, const EngineState* st, bool fwd, hipS
     GK_LAUNCH_CHECK();
 }
 
-// X . K . X launch variants (TuneParams::xv) for padded X 16, 32, 64: 1 = no
-// prefetch of the next item, 2 = half the elements per lane over twice the
-// lanes, 3 = both; 0 and other lengths: k_xmul
+// X . K . X launch variants (TuneParams::xv) for padded X 16, 32, 64: 2 = half the
+// elements per lane over twice the lanes with the next item prefetched, 3 =
+// without the prefetch; 0, 1 and other lengths: k_xmul
 template <int PX, int EE, bool PIPE>
 static void xmul_v_launch(const ConvPlan& cp, const EngineState* st, const float2* tw, hipStream_t s) {
     constexpr int LPB = kNT / (PX / EE);
@@ -1060,10 +1060,9 @@ bool conv_xv_valid(int PX, int v) { return v == 0 || ((PX == 16 || PX == 32 || P
 static void launch_xmul(const ConvPlan& cp, const EngineState* st, hipStream_t s) {
     const int PX = cp.P[0], PY = cp.P[1], Nx = cp.N[0], Q = cp.Q;
     const float2* tw = twiddle_f32(PX);
-    if (cp.tp.xv && conv_xv_valid(PX, cp.tp.xv)) {
+    if (cp.tp.xv >= 2 && conv_xv_valid(PX, cp.tp.xv)) {
         switch (PX * 4 + cp.tp.xv) {
 #define GK_XV(n)                                                                            \
-    case n * 4 + 1: xmul_v_launch<n, RegFFT<n>::E, false>(cp, st, tw, s); break;            \
     case n * 4 + 2: xmul_v_launch<n, RegFFT<n>::E / 2, true>(cp, st, tw, s); break;        \
     case n * 4 + 3: xmul_v_launch<n, RegFFT<n>::E / 2, false>(cp, st, tw, s); break;
             GK_XV(16) GK_XV(32) GK_XV(64)

@@ -165,7 +165,7 @@ struct TuneParams {
     int xb = 4;   // blocks per CU of the pipelined X.K.X pass
     int y2b = 8;  // blocks per CU of the 2-D Y.K.Y pass
     int pp = 0;   // 3-D plans that fit it: 1 = Y.X K X.Y in one plane pass (k_plane3), 0 = separate passes
-    int xv = 0;   // X.K.X variant (padded X 16-64): 0 default, 1 no prefetch, 2 half the elements per lane, 3 both
+    int xv = 0;   // X.K.X variant (padded X 16-64): 0, 1 default, 2 half the elements per lane and a prefetch, 3 without it
 };
 
 struct ConvPlan {

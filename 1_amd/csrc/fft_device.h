@@ -178,6 +178,38 @@ template <typename T, int R, int DIR> __device__ __forceinline__ void dft(C2<T>*
     else dft7<T, DIR>(v);
 }
 
+// DFT of N = R1 R2 values in registers (Cooley-Tukey: R2 transforms of R1, twiddles
+// wx[n2 k1] = exp(-2 pi i n2 k1 / N), R1 transforms of R2), natural order in and out
+template <int N> constexpr int small_r1() { return N == 6 ? 2 : 4; }  // 6 = 2 x 3, 12 = 4 x 3, 16 = 4 x 4
+template <typename T, int N, int DIR> __device__ __forceinline__ void dft_small(C2<T>* v, const C2<T>* wx) {
+    GK_FFT_FP
+    constexpr int R1 = small_r1<N>(), R2 = N / R1;
+    static_assert(R1 * R2 == N, "6, 12 or 16");
+    C2<T> o[N];
+#pragma unroll
+    for (int n2 = 0; n2 < R2; n2++) {
+        C2<T> b[R1];
+#pragma unroll
+        for (int n1 = 0; n1 < R1; n1++) b[n1] = v[R2 * n1 + n2];
+        dft<T, R1, DIR>(b);
+#pragma unroll
+        for (int k1 = 0; k1 < R1; k1++) {
+            if (n2 * k1) {
+                C2<T> w = wx[n2 * k1];
+                if (DIR > 0) w.y = -w.y;
+                b[k1] = cmul<T>(b[k1], w);
+            }
+            o[R2 * k1 + n2] = b[k1];
+        }
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < R1; k1++) {
+        dft<T, R2, DIR>(o + R2 * k1);
+#pragma unroll
+        for (int k2 = 0; k2 < R2; k2++) v[k1 + R1 * k2] = o[R2 * k1 + k2];
+    }
+}
+
 // radix chosen for the remaining length `rem` (product of the radices still to do)
 constexpr int next_radix(int rem) {
     return rem % 8 == 0 ? 8 : rem % 4 == 0 ? 4 : rem % 2 == 0 ? 2 : rem % 3 == 0 ? 3 : rem % 5 == 0 ? 5 : 7;

@@ -766,13 +766,12 @@ __global__ __launch_bounds__(kNT) void k_ypass(const float2* __restrict__ src, f
     }
 }
 
-// 3-D X forward . kernel . X inverse, software-pipelined.  One (kz, ky) column
+// 3-D X forward . kernel . X inverse.  One (kz, ky) column
 // per group of G lanes, all 3 components in registers (lane-strided x = g + G e):
 // the loads and stores touch G rows of consecutive ky per instruction, the
 // 6-component symmetric multiply is lane-local, and each transform needs one
 // LDS exchange per radix pass.  A block item is one kz and a run of lpr
-// consecutive ky; a block walks `nit` consecutive items, loading the columns of
-// the next item before transforming the current one.  Items are ordered so that
+// consecutive ky; a block walks `nit` consecutive items.  Items are ordered so that
 // the runs ky and Py - ky (which read the same kernel rows) follow each other.
 // the 3 components of column (kz, ky) into lane g's registers (ky < 0: zeros)
 template <int PX>
@@ -842,9 +841,9 @@ __device__ __forceinline__ void xmul_column(unsigned t, unsigned items, unsigned
     ky = (t < items && li < lpr && r * lpr + li < PY) ? r * lpr + li : -1;
 }
 
-// Launch variants of the X . K . X pass (TuneParams::xv): EE elements per lane
-// (the default RegFFT<PX>::E, or half of it over twice the lanes: fewer live
-// registers, one more LDS exchange per transform) and PIPE, the next item's
+// Launch variants of the X . K . X pass (TuneParams::xv 2 and 3): EE elements per
+// lane, half of the default RegFFT<PX>::E over twice the lanes (fewer live
+// registers, one more LDS exchange per transform), and PIPE, the next item's
 // columns loaded before the current one is transformed (twice the data
 // registers) or after.  Lane g of a line holds x = g + (PX / EE) e.
 template <int PX, int EE>
@@ -951,6 +950,9 @@ __global__ __launch_bounds__(kNT) void k_xmul_v(float2* __restrict__ B2, const f
     }
 }
 
+// every other length, and the default: RegFFT<PX>::E elements per lane, no prefetch
+// (it doubles the data registers, and the waves it costs hide more latency than
+// it does: padded X 128, 70 x 60 x 51, 23.3 us a launch with it, 19.3 without)
 template <int PX>
 __global__ __launch_bounds__(kNT) void k_xmul(float2* __restrict__ B2, const float* __restrict__ Kc,
                                               const float2* __restrict__ tw, const EngineState* st, int Nx, int PY,
@@ -965,27 +967,12 @@ __global__ __launch_bounds__(kNT) void k_xmul(float2* __restrict__ B2, const flo
     const int lpr = LPB < PY ? LPB : PY;  // columns per item
     const int rows = (PY + lpr - 1) / lpr;  // items per kz plane (the last may be partial)
     const unsigned items = (unsigned)Q * rows, t0 = blockIdx.x * nit;
-    float2 nxt[3][E];
-    {
-        int kz, ky;
-        xmul_column(t0, items, rows, lpr, li, PY, kz, ky);
-        xmul_load<PX>(nxt, B2, kz, ky, Nx, PY, Q, g);
-    }
     __syncthreads();  // twiddle table
     for (int it = 0; it < nit; it++) {
-        const unsigned t = t0 + it;
-        float2 v[3][E];
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-#pragma unroll
-            for (int e = 0; e < E; e++) v[c][e] = nxt[c][e];
-        if (it + 1 < nit) {
-            int kz1, ky1;
-            xmul_column(t + 1, items, rows, lpr, li, PY, kz1, ky1);
-            xmul_load<PX>(nxt, B2, kz1, ky1, Nx, PY, Q, g);
-        }
         int kz, ky;
-        xmul_column(t, items, rows, lpr, li, PY, kz, ky);
+        xmul_column(t0 + it, items, rows, lpr, li, PY, kz, ky);
+        float2 v[3][E];
+        xmul_load<PX>(v, B2, kz, ky, Nx, PY, Q, g);
 #pragma unroll
         for (int c = 0; c < 3; c++) reg_fft<float, PX, -1>(v[c], g, lds + li * F::LDS, twl);
         if (ky >= 0) xmul_kernel<PX>(v, Kc, kz, ky, PY, g);
@@ -1266,7 +1253,7 @@ __global__ __launch_bounds__(kPlaneThreads) void k_plane3(float2* __restrict__ B
 // so per field evaluation the pass reads and writes B1 once, where the three
 // separate passes move B1 twice and the Y-padded B2 four times.  The X
 // transforms of length PX (Nx <= PX/2 nonzero inputs, Nx outputs kept) are
-// direct sums with the table exp(-2 pi i j / PX).
+// register butterflies with the table exp(-2 pi i j / PX).
 constexpr int kYxyThreads = 256;
 constexpr int kYxyLdsBytes = 80 * 1024;
 // Which plans take the plane pass: a plane of 3 (PX/2) lines plus separate
@@ -1347,33 +1334,25 @@ __device__ __forceinline__ void yxy_plane(float2 (*v)[RegFFT<PY>::E], float2* __
     // X . K . X for every ky of the plane
     for (int ky = threadIdx.x; ky < PY; ky += NT) {
         GK_FFT_FP
-        constexpr bool BF = PX == 4 || PX == 8;  // radix-4 / radix-8 butterflies, else direct sums
+        // radix-4 / radix-8 butterflies, or two factors for 6, 12 and 16 (the direct sums
+        // these replace took 3 x PX^2 / 2 complex products a transform, more than
+        // everything else in the pass: 150 x 91 x 3, PX 6, 7.9 us a launch, now 7.5;
+        // 128 x 128 x 8, PX 16, 21.8 us, now 14.0)
+        constexpr bool R48 = PX == 4 || PX == 8;
         float2 a[3][PX];
 #pragma unroll
         for (int c = 0; c < 3; c++)
 #pragma unroll
             for (int kx = 0; kx < PX; kx++) a[c][kx] = make_float2(0.f, 0.f);
-        if constexpr (BF) {
 #pragma unroll
-            for (int x = 0; x < PX / 2; x++)
-                if (x < Nx)
+        for (int x = 0; x < PX / 2; x++)
+            if (x < Nx)
 #pragma unroll
-                    for (int c = 0; c < 3; c++) a[c][x] = plane[(long)(c * Nx + x) * PY + ky];
+                for (int c = 0; c < 3; c++) a[c][x] = plane[(long)(c * Nx + x) * PY + ky];
 #pragma unroll
-            for (int c = 0; c < 3; c++) dft<float, PX, -1>(a[c]);
-        } else {
-#pragma unroll
-            for (int x = 0; x < PX / 2; x++) {
-                if (x < Nx) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++) {
-                        const float2 u = plane[(long)(c * Nx + x) * PY + ky];
-#pragma unroll
-                        for (int kx = 0; kx < PX; kx++)
-                            a[c][kx] = cadd<float>(a[c][kx], cmul<float>(u, wx[(kx * x) % PX]));
-                    }
-                }
-            }
+        for (int c = 0; c < 3; c++) {
+            if constexpr (R48) dft<float, PX, -1>(a[c]);
+            else dft_small<float, PX, -1>(a[c], wx);
         }
         // kernel layout of plane-pass plans: [kz][component][kx <= PX/2][ky <= PY/2], so that
         // consecutive ky (threads) read consecutive floats
@@ -1393,29 +1372,16 @@ __device__ __forceinline__ void yxy_plane(float2 (*v)[RegFFT<PY>::E], float2* __
             a[1][kx] = make_float2(p.x * kxy + q.x * kyy + w.x * kyz, p.y * kxy + q.y * kyy + w.y * kyz);
             a[2][kx] = make_float2(p.x * kxz + q.x * kyz + w.x * kzz, p.y * kxz + q.y * kyz + w.y * kzz);
         }
-        if constexpr (BF) {
 #pragma unroll
-            for (int c = 0; c < 3; c++) dft<float, PX, +1>(a[c]);
-#pragma unroll
-            for (int x = 0; x < PX / 2; x++)
-                if (x < Nx)
-#pragma unroll
-                    for (int c = 0; c < 3; c++) plane[(long)(c * Nx + x) * PY + ky] = a[c][x];
-        } else {
-#pragma unroll
-            for (int x = 0; x < PX / 2; x++) {
-                if (x < Nx) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++) {
-                        float2 t = make_float2(0.f, 0.f);
-#pragma unroll
-                        for (int kx = 0; kx < PX; kx++)
-                            t = cadd<float>(t, cmul<float>(a[c][kx], cconj<float>(wx[(kx * x) % PX])));
-                        plane[(long)(c * Nx + x) * PY + ky] = t;
-                    }
-                }
-            }
+        for (int c = 0; c < 3; c++) {
+            if constexpr (R48) dft<float, PX, +1>(a[c]);
+            else dft_small<float, PX, +1>(a[c], wx);
         }
+#pragma unroll
+        for (int x = 0; x < PX / 2; x++)
+            if (x < Nx)
+#pragma unroll
+                for (int c = 0; c < 3; c++) plane[(long)(c * Nx + x) * PY + ky] = a[c][x];
     }
     __syncthreads();
     // Y inverse, first Ny kept; the last round first, whose rows the exchange

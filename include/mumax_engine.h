@@ -194,8 +194,8 @@ double mm_sim_time_pass(mmSim* s, int cls, int n);
  * of the X.K.X pass, y2b: blocks per CU of the 2-D Y.K.Y pass, pp: for 3-D
  * plans with padded Y 512 and padded X 16 or 32, 1 = Y forward, X.K.X and Y
  * inverse as one register-resident plane pass, 0 = three passes, xv: X.K.X
- * variant for padded X 16-64, 0 default, 1 without the next item's prefetch,
- * 2 half the elements per lane over twice the lanes, 3 both}.  Each tunable's
+ * variant for padded X 16-64, 0 and 1 default, 2 half the elements per lane over
+ * twice the lanes with the next item prefetched, 3 without the prefetch}.  Each tunable's
  * candidates run `reps` back-to-back launches (least of 3 runs); the fastest is
  * kept in s and stored in the process's tuning table under s's data size.
  * ms_default / ms_tuned [0..6]: ms per launch of the affected pass(es) at the
