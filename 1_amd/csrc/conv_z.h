@@ -40,7 +40,10 @@ template <int M> constexpr int epi_rows() {
     int p = 1;
     while (p * 2 <= tr) p *= 2;
     tr = p;
-    while (tr > 1 && zinv_epi_lds_elems(M, tr) * 8 > 80 * 1024) tr /= 2;
+    // two blocks per CU (80 KB of LDS), except for long rows that this would leave
+    // with two rows per block and 16 B runs of B1
+    const int cap = M >= 1024 ? 150 * 1024 : 80 * 1024;
+    while (tr > 1 && zinv_epi_lds_elems(M, tr) * 8 > cap) tr /= 2;
     return tr;
 }
 

@@ -83,10 +83,13 @@ __global__ __launch_bounds__(NT) void k_fft_lines(C2<T>* __restrict__ data, cons
 // index fastest.  All of a lane's loads and the block's copy of the twiddle
 // table are issued together, one memory latency for the whole kernel (the LDS
 // Stockham kernels these replace read the table from global memory in every
-// pass).  Blocks hold as many lines as leave about two blocks per CU: small
-// transforms are latency-bound and need the CUs, not the occupancy.
-// Measured per launch (before / now): 2064 lines of 256 12.9 / 9.0 us, 33024 of 32
-// 8.0 / 5.7 us, 2048 rows of 256 reals 8.9 / 4.2 us; 64 rows of 512 12.4 / 4.0 us.
+// pass).  Strided lines go 16 to a block, whole 128 B cache lines: with 4, for more
+// blocks, neighbours on other XCDs wrote parts of the same line.  Rows go as many
+// to a block as leave about two blocks per CU: small transforms are latency-bound
+// and need the CUs, not the occupancy.
+// Measured per launch (before / now): 2064 lines of 256 12.9 / 6.9 us (4 lines a
+// block 9.0), 33024 of 32 8.0 / 5.5 us, 2048 rows of 256 reals 8.9 / 4.3 us; 64 rows
+// of 512 12.4 / 4.0 us.
 constexpr int line_E(int L) { return L % 3 == 0 ? (L < 12 ? L : 12) : (L < 8 ? L : 8); }
 constexpr int line_G(int L) { return L / line_E(L); }
 constexpr int line_buf(int L) { return L + L / 8 + 1; }
@@ -262,14 +265,14 @@ bool fft_reg_length(int L) {
     }
 }
 
-// log2 of the lines per block: up to 256 threads (64 B or longer runs: at least
-// 8 lines) and 60 KB of LDS, then fewer while the launch has under two blocks per
-// CU (512) and a block a whole wave and 4 lines (32 B runs)
+// log2 of the lines per block: up to 256 threads, at least 16 lines (128 B runs, a
+// cache line) and 60 KB of LDS, then fewer, down to 4 lines (32 B runs), while the
+// launch has under 64 blocks
 static int lines_shift(int L, int G, unsigned nlines) {
-    int sh = 3;
+    int sh = 4;
     while ((G << (sh + 1)) <= 256) sh++;
     while (sh > 0 && ((G << sh) > 1024 || (((line_buf(L) << sh) + L) * 8) > 60 * 1024)) sh--;
-    while (sh > 2 && (G << (sh - 1)) >= 64 && (nlines >> sh) < 512) sh--;
+    while (sh > 2 && (G << (sh - 1)) >= 64 && (nlines >> sh) < 64) sh--;
     return sh;
 }
 // rows per block: 256 threads, fewer while the launch has under 512 blocks and a block a whole wave
