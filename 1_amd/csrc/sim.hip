@@ -295,7 +295,7 @@ static bool enqueue_trial(mmSim* s, bool fwd, bool next) {
     Prof& pf = s->prof;
     // the trial has been started by the one before (launch_ctrl_end) or launch_set_target;
     // the FSAL stage is in k[0] (launch_commit) and its dt control done
-    const bool fusable = conv_fwd_fused(s->cp);
+    const bool fusable = conv_fwd_fused(s->cp) && !pf.on;  // a profile times each pass by itself
     const float* mi_ready = nullptr;  // the stage input, where the stage before has stored it
     for (int i = 0; i < t.S; i++) {
         if (i == 0 && t.fsal && s->fsalHost) continue;

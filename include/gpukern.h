@@ -118,13 +118,12 @@ void gpuFFT3dPlan_inverse(gpuFFT3dPlan* plan, float* input, float* output); /* g
 int gpuFFT3dPlan_normalization(gpuFFT3dPlan* plan);                        /* gpu_fft0.cu:112 */
 /* No counterpart in the reference.  gpuFFT3dPlan_forward for callers that
  * cannot allocate device memory (HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc): the same transform and the same bits, but
- * the temporaries of non-power-of-two lengths (packed rows, Bluestein buffers)
- * live in a fixed 32 MiB device array per GPU instead of per-call allocations,
- * and the plan's tables come from new_gpuFFT3dPlan_padded.  Plans whose
- * temporaries exceed 4 Mi complex elements are rejected (abort with a message).
- * Every call on one GPU shares that array: calls that overlap on one GPU (other
- * host threads) race. */
+ * harnesses that forbid hipMalloc): the same transform and the same bits.
+ * Neither call allocates (every length runs in registers and LDS on the
+ * caller's buffers; the plan's tables come from new_gpuFFT3dPlan_padded), but
+ * this one keeps a limit on the plan: lengths that are not powers of two whose
+ * packed rows and chirp buffers would exceed 4 Mi complex elements are rejected
+ * (abort with a message). */
 void gpuFFT3dPlan_forward_noalloc(gpuFFT3dPlan* plan, float* input, float* output);
 
 /* ---- thermal noise (gpu_temperature.h:25) ---- */

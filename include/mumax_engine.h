@@ -175,7 +175,8 @@ unsigned long long mm_memory_trim(void);
  * engine's stream; returns the elapsed ms.  The _profile variant also brackets
  * every kernel class (0 Z fwd, 1 Y fwd, 2 X.K.X or Y.K.Y, 3 Y inv, 4 Z inv,
  * 5 torque, 6 RK final, 7 control) and returns per-class total ms and launch
- * counts in ms[8], counts[8]. */
+ * counts in ms[8], counts[8]; every pass has a launch of its own there (small
+ * grids otherwise run a stage's Z inverse and the next one's Z forward in one). */
 double mm_sim_time_steps(mmSim* s, int n);
 double mm_sim_profile_steps(mmSim* s, int n, double* ms, int* counts);
 /* Fused mode.  n back-to-back launches of one convolution pass class (0..4 as
