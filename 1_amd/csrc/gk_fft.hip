@@ -447,9 +447,25 @@ static size_t forward_scratch_elems(const gpuFFT3dPlan* p) {
     return need;
 }
 
+// The row pass reads rows of one length and stores rows of another, block by
+// block in any order, so real data that share memory with the spectrum go
+// through an array of their own (from the engine's cache of device memory).
+static float* aside_if_shared(const gpuFFT3dPlan* p, const float* real, const float* cplx) {
+    const long n = (long)p->size[0] * p->size[1] * p->size[2], nc = (long)p->padded[0] * p->padded[1] * p->pzc * 2;
+    return real < cplx + nc && cplx < real + n ? (float*)cached_malloc(n * sizeof(float)) : nullptr;
+}
+static size_t real_bytes(const gpuFFT3dPlan* p) { return (size_t)p->size[0] * p->size[1] * p->size[2] * sizeof(float); }
+static float* enq_forward_any(gpuFFT3dPlan* p, const float* input, float* output) {
+    float* aside = aside_if_shared(p, input, output);
+    if (aside) GK_CHECK(hipMemcpyAsync(aside, input, real_bytes(p), hipMemcpyDeviceToDevice, stream()));
+    enq_fft_forward(p, aside ? aside : input, 0, output, 0, 1);
+    return aside;
+}
+
 void gpuFFT3dPlan_forward(gpuFFT3dPlan* p, float* input, float* output) {
-    enq_fft_forward(p, input, 0, output, 0, 1);
+    float* aside = enq_forward_any(p, input, output);
     sync();
+    cached_free(aside);
 }
 
 void gpuFFT3dPlan_forward_noalloc(gpuFFT3dPlan* p, float* input, float* output) {
@@ -459,14 +475,18 @@ void gpuFFT3dPlan_forward_noalloc(gpuFFT3dPlan* p, float* input, float* output) 
               "the maximum is %zu (use gpuFFT3dPlan_forward)",
               p->padded[0], p->padded[1], p->padded[2], need, kFFTScratchElems);
     tables_frozen(true);
-    enq_fft_forward(p, input, 0, output, 0, 1);
+    float* aside = enq_forward_any(p, input, output);
     tables_frozen(false);
     sync();
+    cached_free(aside);
 }
 
 void gpuFFT3dPlan_inverse(gpuFFT3dPlan* p, float* input, float* output) {
-    enq_fft_inverse(p, input, 0, output, 0, 1);
+    float* aside = aside_if_shared(p, output, input);
+    enq_fft_inverse(p, input, 0, aside ? aside : output, 0, 1);
+    if (aside) GK_CHECK(hipMemcpyAsync(output, aside, real_bytes(p), hipMemcpyDeviceToDevice, stream()));
     sync();
+    cached_free(aside);
 }
 
 }  // extern "C"

@@ -108,7 +108,8 @@ void gpu_copy_unpad(float* source, float* dest, int S0, int S1, int S2, int D0, 
 /* ---- padded real FFT (gpu_fft0.h:30-75) ---- */
 /* Layout of the transform: real [size] in, half-complex [paddedSize0][paddedSize1][paddedSize2+2]
  * floats out (interleaved complex, Z halved), as cufftPlan3d/2d R2C in the reference.
- * Rows and planes that are known zeros because of the padding are never transformed. */
+ * Rows and planes that are known zeros because of the padding are never transformed.
+ * Input and output may share memory: the real data then go through an array of their own. */
 typedef struct gpuFFT3dPlan gpuFFT3dPlan; /* gpu_fft0.h:30-38 (opaque here) */
 gpuFFT3dPlan* new_gpuFFT3dPlan_padded(int* size, int* paddedSize);        /* gpu_fft0.h:51 */
 void delete_gpuFFT3dPlan(gpuFFT3dPlan* plan);                             /* gpu_fft0.h:56 */
@@ -120,7 +121,8 @@ int gpuFFT3dPlan_normalization(gpuFFT3dPlan* plan);                        /* gp
  * cannot allocate device memory (HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): the same transform and the same bits.
  * Neither call allocates (every length runs in registers and LDS on the
- * caller's buffers; the plan's tables come from new_gpuFFT3dPlan_padded), but
+ * caller's buffers, which must not overlap for that; the plan's tables come
+ * from new_gpuFFT3dPlan_padded), but
  * this one keeps a limit on the plan: lengths that are not powers of two whose
  * packed rows and chirp buffers would exceed 4 Mi complex elements are rejected
  * (abort with a message). */

@@ -150,3 +150,32 @@ def test_dropin_transform_lengths(lib, size, P):
     for p in (d, back):
         lib.free_gpu_array(p)
     lib.delete_gpuFFT3dPlan(plan)
+
+
+# the real data at the start of the spectrum's memory and further in: register rows, LDS rows, Bluestein rows, odd length
+@pytest.mark.parametrize("size,P", [((4, 16, 32), (8, 32, 64)), ((2, 9, 15), (4, 18, 30)), ((2, 11, 13), (4, 22, 26)),
+                                    ((3, 6, 45), (6, 12, 45)), ((1, 1, 2), (1, 1, 4))])
+@pytest.mark.parametrize("call", ["gpuFFT3dPlan_forward", "gpuFFT3dPlan_forward_noalloc"])
+def test_dropin_transform_of_shared_memory(lib, size, P, call):
+    """Input and output that overlap give the bits that separate arrays give, both ways."""
+    from test_zz_no_alloc import download, i3, upload
+
+    n, n_out = int(np.prod(size)), P[0] * P[1] * 2 * (P[2] // 2 + 1)
+    x = np.random.default_rng(8).standard_normal(size).astype(np.float32)
+    plan = lib.new_gpuFFT3dPlan_padded(i3(*size), i3(*P))
+    a, b, c = upload(lib, x), lib.new_gpu_array(n_out), lib.new_gpu_array(n)
+    getattr(lib, call)(plan, a, b)
+    spec = download(lib, b, n_out)
+    lib.gpuFFT3dPlan_inverse(plan, b, c)
+    back = download(lib, c, n)
+    for at in (0, (n_out - n) // 4 * 2):
+        d = lib.new_gpu_array(n_out)
+        lib.memcpy_to_gpu(x.ctypes.data, d + 4 * at, n)
+        getattr(lib, call)(plan, d + 4 * at, d)
+        assert np.array_equal(download(lib, d, n_out).view(np.uint32), spec.view(np.uint32)), at
+        lib.gpuFFT3dPlan_inverse(plan, d, d + 4 * at)
+        assert np.array_equal(download(lib, d + 4 * at, n).view(np.uint32), back.view(np.uint32)), at
+        lib.free_gpu_array(d)
+    for p in (a, b, c):
+        lib.free_gpu_array(p)
+    lib.delete_gpuFFT3dPlan(plan)
