@@ -489,10 +489,17 @@ void fft_lines_any(C2<T>* data, int L, long nlines, long n_inner, long inner, lo
     }
     RadixList rl;
     if (factor_radices(L, rl)) {
-        GK_ASSERT(2L * L * (long)sizeof(C2<T>) <= 65536, "FFT length %d is too long for one block", L);
+        // FP64: up to 3072 (96 KB, one block per CU), which the engine pads 1025..1536 cells to
+        constexpr int max_lds = sizeof(T) == 8 ? 96 * 1024 : 64 * 1024;
+        GK_ASSERT(2L * L * (long)sizeof(C2<T>) <= max_lds, "FFT length %d is too long for one block", L);
         const C2<T>* tw;
-        if constexpr (sizeof(T) == 4) tw = twiddle_f32(L);
-        else tw = twiddle_f64(L);
+        if constexpr (sizeof(T) == 4) {
+            tw = twiddle_f32(L);
+        } else {
+            tw = twiddle_f64(L);
+            GK_CHECK(hipFuncSetAttribute((const void*)k_fft_lines_rt<T, DIR>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         max_lds));
+        }
         const int sh = rt_shift<T>(L, a.nlines * ncomp);
         k_fft_lines_rt<T, DIR><<<dim3(div_up(nlines, 1L << sh), ncomp), 256, (2 * L * sizeof(C2<T>)) << sh, s>>>(data, tw, L, rl, a, sh);
         GK_LAUNCH_CHECK();

@@ -23,7 +23,6 @@ def random_m(size, seed):
 
 
 # padded Y 4, 6, 8, 12, 64, 96, 128, 1024, 1536, 2048, 4096: one lane group per wave up to one block per line
-# (the FP64 set-up transforms take no 3072)
 @pytest.mark.parametrize("ny", [2, 3, 4, 5, 31, 47, 64, 400, 700, 1000, 1600])
 def test_film_column_lengths_vs_oracle(mm, orc, ny):
     size = (1, ny, 5)
@@ -34,6 +33,35 @@ def test_film_column_lengths_vs_oracle(mm, orc, ny):
     ref = o.heff(m0).reshape(h.shape)
     s.free()
     assert np.abs(h - ref).max() < 5e-6 * np.abs(ref).max()
+
+
+# 1025..1536 cells are padded to 3072, the longest 3 * 2^a: columns, rows, and the Y passes of a 3-D grid
+@pytest.mark.parametrize("size", [(1, 1100, 5), (1, 3, 1536), (2, 1025, 3), (2, 2, 1201)])
+def test_axes_padded_to_3072(mm, orc, size):
+    m0 = random_m(size, 4)
+    cfg = cfg_of(size, m0, solver="rkdp", maxerror=1e-4, dt=1e-14, max_dt=1e-14)
+    s = mm.workloads.make_sim(cfg)
+    o = orc.sim(m0, **mm.workloads.oracle_kwargs(cfg))
+    h = s.heff(m0)
+    ref = o.heff(m0).reshape(h.shape)
+    assert np.abs(h - ref).max() < 5e-6 * np.abs(ref).max()
+    t = mm.workloads.make_sim(cfg)
+    b = mm.Batch([t])
+    b.start(steps=2)
+    while b.trials(2):
+        pass
+    b.free()
+    s.steps(2)
+    assert s.state()["steps"] == t.state()["steps"] == 2
+    assert np.array_equal(s.m, t.m)
+    dts, acc = s.trial_log()
+    assert all(acc) and len(dts) == 2
+    o.step_replay(dts[:1], acc[:1])
+    o.step_replay(dts[1:], acc[1:])
+    dm = np.abs(s.m.reshape(-1) - np.asarray(o.m).reshape(-1)).max()
+    for x in (s, t):
+        x.free()
+    assert dm < 1e-5
 
 
 # every tableau's stages with their forward passes in the epilogues: even and odd rows, the shortest, partly
