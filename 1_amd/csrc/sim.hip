@@ -401,7 +401,8 @@ static bool enqueue_trial(mmSim* s, bool fwd, bool next) {
     return !t.adaptive && fwd;
 }
 
-static long fused_run(mmSim* s, long long nsteps, double stop, bool wait) {
+// relax: the run may end at any step, however many are left (relax.go:14-25)
+static long fused_run(mmSim* s, long long nsteps, double stop, bool wait, bool relax = false) {
     EngineState h = read_state(s);
     s->fsalHost = h.fsal_init != 0;
     const long long steps0 = h.steps;
@@ -415,17 +416,22 @@ static long fused_run(mmSim* s, long long nsteps, double stop, bool wait) {
     }
     // Trials enqueued past the end are launches that do nothing: at most as many as
     // the steps still to take, and for a stop time at most what the time left needs
-    // at the current dt; within that, for adaptive tableaux, doubling batches (dt
-    // grows over the first steps of a run).
+    // at the current dt.  Within that, doubling batches where the end cannot be
+    // told: dt changes from step to step (it grows over the first steps of a run),
+    // or a relaxation ends once the energy rises.  (A 128 x 32 film relaxed again
+    // with 20000 steps allowed, which ends after a few: 1024 RK4 trials at once took
+    // 25 ms, these 0.3 ms.)
+    const bool fixed_dt = !s->tb.adaptive && !needs_after_k0(s);
+    const int most = s->tb.adaptive || relax ? 64 : 1024;
     int batch = 4;
     while (true) {
         long long n = batch;
         if (nsteps >= 0) {
             const long long left = steps0 + nsteps - h.steps;
-            n = std::min<long long>(left, s->tb.adaptive ? 64 : 1024);
+            n = std::min<long long>(left, relax ? batch : most);
         } else if (stop < INFINITY && h.dt > 0) {
             const long long need = (long long)std::min(1e9, std::ceil((stop - h.time) / h.dt));
-            n = std::min<long long>(need, s->tb.adaptive ? batch : 1024);
+            n = std::min<long long>(need, fixed_dt ? most : batch);
         }
         n = std::max(n, 1LL);
         bool fwd = false;
@@ -440,7 +446,7 @@ static long fused_run(mmSim* s, long long nsteps, double stop, bool wait) {
             abort();
         }
         if (h.done) break;
-        if (batch < 64) batch *= 2;
+        if (batch < most) batch *= 2;
     }
     return (long)(h.steps - steps0);
 }
@@ -1186,7 +1192,7 @@ long mm_sim_relax(mmSim* s, long max_steps) {
     GK_ASSERT(s->mode == MM_MODE_FUSED, "mm_sim_relax needs the fused mode");
     s->wantEnergy = true;  // relax.go:16
     launch_set_relax(s->st, 1, s->s);
-    const long n = fused_run(s, max_steps > 0 ? max_steps : -1, INFINITY, true);
+    const long n = fused_run(s, max_steps > 0 ? max_steps : -1, INFINITY, true, true);
     launch_set_relax(s->st, 0, s->s);
     GK_CHECK(hipStreamSynchronize(s->s));
     return n;

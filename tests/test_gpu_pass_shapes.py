@@ -158,6 +158,29 @@ def test_run_to_a_stop_time_in_pieces(mm):
     b.free()
 
 
+def test_a_relaxation_enqueues_no_further_than_its_end(mm):
+    """A relaxed state ends its next relaxation within a few steps, also where many
+    more are allowed: nearly all of 1024 trials enqueued at once would do nothing
+    (each a dozen launches, some 25 us: 25 ms). The allowance of 5 ms is a fifth of that."""
+    import time
+
+    size = (1, 24, 40)
+    m0 = np.zeros((3,) + size, np.float32)
+    m0[2] = 1
+    s = mm.workloads.make_sim(cfg_of(size, m0, alpha=1.0, dt=1e-13))
+    s.relax(4000)
+    took = {}
+    for most in (0, 20000):
+        took[most] = []
+        for _ in range(4):
+            s.sync()
+            t = time.perf_counter()
+            s.relax(most)
+            took[most].append(time.perf_counter() - t)
+    s.free()
+    assert min(took[20000]) < min(took[0]) + 5e-3
+
+
 # columns and rows of the drop-in plan: register lengths, LDS lengths, Bluestein lengths, their largest
 @pytest.mark.parametrize("size,P", [((1, 11, 13), (1, 22, 26)), ((1, 2039, 3), (1, 2039, 6)), ((2, 1500, 3), (4, 3072, 6)),
                                     ((1, 4096, 4), (1, 4096, 8)), ((3, 7, 1536), (6, 14, 3072)), ((2, 9, 4078), (3, 9, 4078)),
