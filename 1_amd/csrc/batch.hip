@@ -5,8 +5,8 @@
 // Each simulation keeps its own device state exactly as in the single-simulation
 // engine (sim.hip): m, k_i, spectra B1/B2, kernel spectrum, EngineState, trial
 // log.  A batched kernel covers every simulation whose padded length matches its
-// template: blocks are numbered per simulation and prefix tables map a block to
-// (simulation, local block), after which the kernel runs the same device body
+// template: a table per launch maps each of its blocks to (simulation, local
+// block), after which the kernel runs the same device body
 // as the single-simulation kernel (passes.h, rk_dev.h).  So a simulation gets
 // bit-identical arithmetic alone and in a batch; only its scheduling differs.
 //
@@ -85,6 +85,18 @@ __global__ void kb_done(const BSim* sims, int n, int* done, float* rem) {
     }
 }
 
+// one simulation of a launch: the table entries of its blocks
+struct BlockRun {
+    int first, sim, n;
+};
+// The launches' block tables (batch_dev.h, BBlock), one wave per run.  Filled on the
+// device: filling them on the host and copying 8 bytes per block, a batch of 400
+// simulations of a sweep took 315 us to build, from the runs 155 us (64: 61 and 45 us).
+__global__ __launch_bounds__(64) void kb_block_tables(const BlockRun* runs, int2* __restrict__ table) {
+    const BlockRun r = runs[blockIdx.x];
+    for (int i = threadIdx.x; i < r.n; i += 64) table[r.first + i] = make_int2(r.sim, i);
+}
+
 }  // namespace gk
 
 using namespace gk;
@@ -98,7 +110,7 @@ struct LaunchSet {
     int cnt = 0;     // simulations
     int blocks = 0;  // total blocks
     int2* map = nullptr;          // device, per block: simulation, block within it
-    size_t map_off = 0;           // offset in the batch's table block (set-up)
+    int map_first = 0;            // its first entry in the batch's block tables (set-up)
     std::vector<int> hidx, hst;   // the simulations and their first blocks (set-up)
     int any = 0;                        // 1: small length classes merged, launched by a dispatch kernel
     int nt = 0, lds = 0;                // dispatch launch: threads per block and dynamic LDS bytes
@@ -132,7 +144,7 @@ struct mmBatch {
     std::vector<void*> owned;  // device allocations of the tables
     TableImage image;          // set-up only: the tables before upload
     // per pass: one LaunchSet per length class
-    std::vector<LaunchSet> zf, yf, xm, yi, y2, yx, zi, fin;
+    std::vector<LaunchSet> zf, y3, xm, y2, yx, zi, fin;
     int useGraph = 1;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -293,13 +305,13 @@ std::vector<LaunchSet> merge_small(std::vector<LaunchSet> sets, int pass) {
     return out;
 }
 
-// the launch sets' block tables into the table image
-void stage_sets(mmBatch* b, std::vector<LaunchSet>& sets) {
+// the runs of the launch sets' block tables, which follow each other from entry `entries` on
+void stage_sets(std::vector<LaunchSet>& sets, std::vector<BlockRun>& runs, int& entries) {
     for (auto& ls : sets) {
-        std::vector<int2> map(ls.blocks);
+        ls.map_first = entries;
         for (int i = 0; i < ls.cnt; i++)
-            for (int k = ls.hst[i]; k < ls.hst[i + 1]; k++) map[k] = make_int2(ls.hidx[i], k - ls.hst[i]);
-        ls.map_off = b->image.put(map.data(), map.size() * sizeof(int2));
+            runs.push_back({entries + ls.hst[i], ls.hidx[i], ls.hst[i + 1] - ls.hst[i]});
+        entries += ls.blocks;
     }
 }
 
@@ -464,9 +476,9 @@ void enqueue_btrial(mmBatch* b) {
         sg.cmax = t.cmax(i);
         sg.partslot = i == 0 ? 0 : (t.fsal && i == t.S - 1) ? 1 : -1;
         for (auto& ls : b->zf) bl_zfwd(b, ls, sg);
-        for (auto& ls : b->yf) bl_ypass(b, ls, sg, true);
+        for (auto& ls : b->y3) bl_ypass(b, ls, sg, true);
         for (auto& ls : b->xm) bl_xmul(b, ls, sg);
-        for (auto& ls : b->yi) bl_ypass(b, ls, sg, false);
+        for (auto& ls : b->y3) bl_ypass(b, ls, sg, false);
         for (auto& ls : b->y2) bl_y2d(b, ls, sg);
         for (auto& ls : b->yx) bl_yxy(b, ls, sg);
         for (auto& ls : b->zi) bl_zinv_epi(b, ls, sg);
@@ -576,8 +588,7 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
     b->zf = make_sets(b, all, M, [](const mmSim* s) { return div_up(s->cp.N[1], z_rows_host(s->cp.M)) * s->cp.N[0] * 3; });
     b->zi = make_sets(b, all, M, [](const mmSim* s) { return div_up(s->cp.N[1], epi_rows_host(s->cp.M)) * s->cp.N[0]; });
     auto ylines = [](const mmSim* s) { return div_up(3L * s->cp.N[0] * s->cp.Q, 256 / lanes_host(s->cp.P[1])); };
-    b->yf = make_sets(b, d3, PY, ylines);
-    b->yi = make_sets(b, d3, PY, ylines);
+    b->y3 = make_sets(b, d3, PY, ylines);
     b->xm = make_sets(b, d3, PX, [](const mmSim* s) {
         const int lpb = 256 / lanes_host(s->cp.P[0]);
         const int lpr = std::min(lpb, s->cp.P[1]);
@@ -593,11 +604,13 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
     b->zi = merge_small(std::move(b->zi), 1);
     b->yx = merge_small(std::move(b->yx), 2);
     b->y2 = merge_small(std::move(b->y2), 3);
-    b->yf = merge_small(std::move(b->yf), 4);
-    b->yi = merge_small(std::move(b->yi), 4);
+    b->y3 = merge_small(std::move(b->y3), 4);
     b->xm = merge_small(std::move(b->xm), 5);
-    for (auto* sets : {&b->zf, &b->zi, &b->yf, &b->yi, &b->xm, &b->y2, &b->yx, &b->fin})
-        stage_sets(b, *sets);
+    std::vector<BlockRun> runs;
+    int entries = 0;
+    for (auto* sets : {&b->zf, &b->zi, &b->y3, &b->xm, &b->y2, &b->yx, &b->fin})
+        stage_sets(*sets, runs, entries);
+    const size_t runs_off = b->image.put(runs.data(), runs.size() * sizeof(BlockRun));
     // upload the tables: one block, one copy on the batch's stream from pinned memory
     {
         const size_t nb = b->image.bytes.size();
@@ -605,13 +618,14 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
         char* host = (char*)cached_host_malloc(nb);
         memcpy(host, b->image.bytes.data(), nb);
         GK_CHECK(hipMemcpyAsync(dev, host, nb, hipMemcpyHostToDevice, b->s));
+        int2* tables = (int2*)balloc(b, (size_t)entries * sizeof(int2));
+        kb_block_tables<<<(unsigned)runs.size(), 64, 0, b->s>>>((const BlockRun*)(dev + runs_off), tables);
+        GK_LAUNCH_CHECK();
         GK_CHECK(hipStreamSynchronize(b->s));
         cached_host_free(host);
         b->dsims = (BSim*)(dev + sims_off);
-        for (auto* sets : {&b->zf, &b->zi, &b->yf, &b->yi, &b->xm, &b->y2, &b->yx, &b->fin})
-            for (LaunchSet& ls : *sets) {
-                ls.map = (int2*)(dev + ls.map_off);
-            }
+        for (auto* sets : {&b->zf, &b->zi, &b->y3, &b->xm, &b->y2, &b->yx, &b->fin})
+            for (LaunchSet& ls : *sets) ls.map = tables + ls.map_first;
         b->image = TableImage{};
     }
     // twiddle tables are created on first use: make them now, outside any graph capture

@@ -219,3 +219,32 @@ def test_batch_keeps_its_field_table_when_the_simulation_replaces_it(mm):
     assert np.array_equal(s.trial_log()[0], dt2) and np.array_equal(s.m, m2)
     assert not np.array_equal(m1, m2)
     s.free()
+
+
+def test_building_a_batch_does_not_depend_on_its_blocks(mm):
+    """A batch is built from a few rows per simulation; its blocks' tables are filled on the
+    device. 64 simulations of 4 x 256 x 256 have some 100 000 blocks more than 64 of 4 x 16 x 16:
+    filled one by one on the host and copied, 800 KB, they take well over 100 us more (the least
+    of ten builds of each; the allowance is 60 us)."""
+    import time
+
+    least = []
+    for size in ((4, 16, 16), (4, 256, 256)):
+        m0 = np.zeros((3,) + size, np.float32)
+        m0[2] = 1
+        cfg = dict(size=size, cellsize=(4e-9, 4e-9, 4e-9), msat=8e5, aexch=1.3e-11, alpha=0.1, solver="rkdp",
+                   maxerror=1e-4, dt=1e-14, m0=m0)
+        sims = [mm.workloads.make_sim(cfg) for _ in range(64)]
+        for s in sims:
+            s.state()
+        took = []
+        for _ in range(10):
+            t = time.perf_counter()
+            b = mm.Batch(sims)
+            took.append(time.perf_counter() - t)
+            b.free()
+        least.append(min(took))
+        for s in sims:
+            s.free()
+    print("batch of 64 built: %.1f us, %.1f us" % tuple(1e6 * t for t in least), flush=True)
+    assert least[1] < least[0] + 60e-6, least
