@@ -927,7 +927,8 @@ int conv_z_rows(int M, int v) {
 
 bool conv_zr_valid(int M, int v) {
     if (v == 0) return true;
-    if (v < 0 || v > 3) return false;
+    if (v < 0 || v > 4) return false;
+    if (v == 4) v = 1;  // the length's own rows: a shape to ask for where there are others
     switch (M) {
 #define GK_CASE(n) \
     case n: return z_rows_v<n>(v) != z_rows_v<n>(0);
@@ -962,6 +963,7 @@ int conv_epi_rows(int M, int v) {
 }
 
 bool conv_er_valid(int M, int v) {
+    if (v == 3) v = 1;  // the length's own rows, as in conv_zr_valid
     return v == 0 || ((v == 1 || v == 2) && conv_epi_rows(M, v) != conv_epi_rows(M, 0));
 }
 

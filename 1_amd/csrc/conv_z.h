@@ -15,9 +15,11 @@ template <int M> constexpr int z_rows() {
     return tr;
 }
 
-// rows per Z forward block of shape variant v: 0 the default, 1 half of it, 2
-// double (while the block stays within 1024 threads and 80 KB of LDS), 3 a quarter.  Short
-// rows (M < 32) have one shape; a variant that does not exist gives the default.
+// rows per Z forward block of shape variant v: 0 and 4 the length's own, 1 half of
+// them, 2 double (while the block stays within 1024 threads and 80 KB of LDS), 3 a
+// quarter.  Short rows (M < 32) have one shape; a variant that does not exist gives
+// the length's own.  (A plan's variant 0 is the one grid_rows chose, conv.hip; 4 and
+// the Z inverse's 3 ask for the length's own rows on any grid.)
 template <int M> constexpr int z_rows_v(int v) {
     constexpr int d = z_rows<M>();
     if (M < 32) return d;
@@ -47,8 +49,8 @@ template <int M> constexpr int epi_rows() {
     return tr;
 }
 
-// rows per fused Z inverse block of shape variant v: 0 the default, 1 half of it,
-// 2 two rows (where that is less than half; small grids: more blocks)
+// rows per fused Z inverse block of shape variant v: 0 and 3 the length's own, 1
+// half of them, 2 two rows (where that is less than half; small grids: more blocks)
 template <int M> constexpr int epi_rows_v(int v) {
     constexpr int d = epi_rows<M>();
     if (M < 32) return d;

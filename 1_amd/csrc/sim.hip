@@ -1284,11 +1284,12 @@ int mm_sim_tune(mmSim* s, int reps, int params[7], double ms_default[8], double 
         ms_tuned[slot] = t_best;
     };
     for (int i = 0; i < 8; i++) ms_default[i] = ms_tuned[i] = -1;
+    // every row count once: 0 is the one of the grid's rule
     std::vector<int> zr{0}, er{0};
+    for (int v = 1; v <= 4; v++)
+        if (conv_zr_valid(cp.M, v) && conv_z_rows(cp.M, v) != conv_z_rows(cp.M, cp.zr0)) zr.push_back(v);
     for (int v = 1; v <= 3; v++)
-        if (conv_zr_valid(cp.M, v)) zr.push_back(v);
-    for (int v = 1; v <= 2; v++)
-        if (conv_er_valid(cp.M, v)) er.push_back(v);
+        if (conv_er_valid(cp.M, v) && conv_epi_rows(cp.M, v) != conv_epi_rows(cp.M, cp.er0)) er.push_back(v);
     const std::vector<int> grid{2, 3, 4, 6, 8, 12, 16};
     tune_one(0, &cp.tp.zr, dflt.zr, zr, 0, -1);
     tune_one(1, &cp.tp.er, dflt.er, er, 4, -1);

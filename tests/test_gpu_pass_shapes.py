@@ -95,7 +95,7 @@ def test_row_variants_give_the_same_steps(mm, lib, tmp_path, size):
     m0 = random_m(size, 3)
     out = []
     try:
-        for zr, er in [(0, 0), (1, 1), (2, 2), (3, 1)]:
+        for zr, er in [(0, 0), (1, 1), (2, 2), (3, 1), (4, 3)]:
             table = tmp_path / "t.txt"
             table.write_text("%d %d %d %d %d 8 4 8 0 0\n" % (size + (zr, er)))
             lib.mm_tune_clear()

@@ -40,6 +40,20 @@ def test_table_round_trip_and_validation(tmp_path):
     assert lib.mm_tune_load(str(tmp_path / "missing.txt").encode()) == -1
 
 
+def test_the_lengths_own_rows_are_a_choice(tmp_path):
+    """Variants 4 (Z forward) and 3 (Z inverse): the row counts of the length, whatever the
+    grid's rule takes; short rows have one count and no such variant."""
+    lib = _lib()
+    src, out = tmp_path / "in.txt", tmp_path / "out.txt"
+    src.write_text("1 32 128 4 3 8 4 8 0 0\n1 32 8 4 3 8 4 8 0 0\n1 32 64 5 4 8 4 8 0 0\n")
+    lib.mm_tune_clear()
+    assert lib.mm_tune_load(str(src).encode()) == 3
+    assert lib.mm_tune_save(str(out).encode()) == 3
+    lib.mm_tune_clear()
+    rows = sorted(l.split() for l in out.read_text().splitlines() if not l.startswith("#"))
+    assert [r[2:5] for r in rows] == [["128", "4", "3"], ["64", "0", "0"], ["8", "0", "0"]]
+
+
 def test_committed_table_parses():
     table = os.path.join(ROOT, "1_amd", "tune_gfx950.txt")
     if not os.path.exists(table):
