@@ -1208,8 +1208,10 @@ void mm_sim_begin_run(mmSim* s, double seconds) {
 }
 
 // n back-to-back launches of pass class cls; the Z forward's stage build reads
-// nk earlier stages (the first stage of a step reads none, most others one)
-static double time_pass(mmSim* s, int cls, int n, int nk) {
+// nk earlier stages (the first stage of a step reads none, most others one); the Z
+// inverse ends with the next stage's Z forward where `fwd` (of m: nothing of the
+// scratch field enters, so that repeated launches stay at the same numbers)
+static double time_pass(mmSim* s, int cls, int n, int nk, bool fwd = false) {
     GK_ASSERT(s->mode == MM_MODE_FUSED && n > 0 && cls >= 0 && cls <= 4, "time_pass: fused mode, class 0..4");
     GK_ASSERT(nk >= 0 && nk < s->tb.S, "time_pass: %d earlier stages", nk);
     StageIn si{};
@@ -1222,7 +1224,8 @@ static double time_pass(mmSim* s, int cls, int n, int nk) {
     }
     EpiArgs ea{};
     ea.m = s->m;
-    ea.nx = -1;
+    ea.nx = fwd ? 0 : -1;
+    ea.xm = s->m;
     ea.out = s->mtmp;  // k[0] may hold the next trial's FSAL stage
     ea.t = torque_args(s, s->tb.c[0], s->part);
     launch_set_active(s->st, s->s);
@@ -1252,26 +1255,30 @@ int mm_sim_tune(mmSim* s, int reps, int params[7], double ms_default[8], double 
     // back-to-back launches, after 2 untimed launches
     // (the Z forward with one earlier stage in its stage build, as in most stages)
     const int nk0 = s->tb.S >= 2 ? 1 : 0;
-    auto timed = [&](int cls_a, int cls_b) {
-        double t = 0;
-        for (int cls : {cls_a, cls_b}) {
-            if (cls < 0) continue;
-            const int nk = cls == 0 ? nk0 : 0;
-            time_pass(s, cls, 2, nk);
-            double best = INFINITY;
-            for (int r = 0; r < 3; r++) best = std::min(best, time_pass(s, cls, reps, nk) / reps);
-            t += best;
-        }
-        return t;
+    auto least = [&](int cls, bool fwd) {
+        const int nk = cls == 0 ? nk0 : 0;
+        time_pass(s, cls, 2, nk, fwd);
+        double best = INFINITY;
+        for (int r = 0; r < 3; r++) best = std::min(best, time_pass(s, cls, reps, nk, fwd) / reps);
+        return best;
+    };
+    auto timed = [&](int cls_a, int cls_b) { return least(cls_a, false) + (cls_b < 0 ? 0.0 : least(cls_b, false)); };
+    // The Z inverse and, if it is one kernel with the next stage's Z forward for some
+    // row count of this grid (which a row count also decides), that pass too: as the
+    // one kernel where the plan runs that, else as the two.
+    bool z_pair = false;
+    auto timed_zinv = [&](int, int) {
+        if (!z_pair) return least(4, false);
+        return conv_fwd_fused(cp) ? least(4, true) : least(4, false) + least(0, false);
     };
     // one tunable: try its candidates, keep the fastest (ties keep the earlier)
-    auto tune_one = [&](int slot, int* field, int dval, const std::vector<int>& cands, int cls_a, int cls_b) {
+    auto tune_by = [&](auto cost, int slot, int* field, int dval, const std::vector<int>& cands, int cls_a, int cls_b) {
         double t_d = -1, t_best = INFINITY;
         int v_best = dval;
         for (int v : cands) {
             *field = v;
             if (field == &cp.tp.er) s->nk_part = conv_epi_blocks(cp);
-            const double t = timed(cls_a, cls_b);
+            const double t = cost(cls_a, cls_b);
             if (v == dval) t_d = t;
             if (t < t_best) {
                 t_best = t;
@@ -1283,6 +1290,9 @@ int mm_sim_tune(mmSim* s, int reps, int params[7], double ms_default[8], double 
         ms_default[slot] = t_d;
         ms_tuned[slot] = t_best;
     };
+    auto tune_one = [&](int slot, int* field, int dval, const std::vector<int>& cands, int cls_a, int cls_b) {
+        tune_by(timed, slot, field, dval, cands, cls_a, cls_b);
+    };
     for (int i = 0; i < 8; i++) ms_default[i] = ms_tuned[i] = -1;
     // every row count once: 0 is the one of the grid's rule
     std::vector<int> zr{0}, er{0};
@@ -1292,7 +1302,11 @@ int mm_sim_tune(mmSim* s, int reps, int params[7], double ms_default[8], double 
         if (conv_er_valid(cp.M, v) && conv_epi_rows(cp.M, v) != conv_epi_rows(cp.M, cp.er0)) er.push_back(v);
     const std::vector<int> grid{2, 3, 4, 6, 8, 12, 16};
     tune_one(0, &cp.tp.zr, dflt.zr, zr, 0, -1);
-    tune_one(1, &cp.tp.er, dflt.er, er, 4, -1);
+    for (int v : er) {
+        cp.tp.er = v;
+        z_pair = z_pair || conv_fwd_fused(cp);
+    }
+    tune_by(timed_zinv, 1, &cp.tp.er, dflt.er, er, 4, -1);
     if (sep) {
         // separate Y and X.K.X passes first (the plane pass off), then the choice between them
         const int pp0 = cp.tp.pp;

@@ -201,7 +201,8 @@ double mm_sim_time_pass(mmSim* s, int cls, int n);
  * candidates run `reps` back-to-back launches (least of 3 runs); the fastest is
  * kept in s and stored in the process's tuning table under s's data size.
  * ms_default / ms_tuned [0..6]: ms per launch of the affected pass(es) at the
- * default and the chosen value (-1 where the plan has no such pass); [7]: the
+ * default and the chosen value (-1 where the plan has no such pass; er: of the Z
+ * inverse and the next stage's Z forward on grids that run them as one); [7]: the
  * three separate passes and the plane pass (-1 where it does not fit).  m is
  * unchanged.
  * Row counts, blocks per CU and the prefetch change no result bit, except that

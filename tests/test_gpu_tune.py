@@ -95,3 +95,22 @@ def test_every_launch_shape_gives_the_same_steps(mm, lib, tmp_path, size, cell):
         table = os.path.join(os.path.dirname(mm.gpukern.__file__), "tune_gfx950.txt")
         if os.path.exists(table):
             lib.mm_tune_load(table.encode())
+
+
+def test_the_tuner_times_the_kernel_the_steps_run(mm, lib):
+    """A small film's Z inverse ends with the next stage's Z forward, so its row count is
+    chosen on that kernel, not on the Z inverse alone (8.8 against 6.0 us for 128 x 32)."""
+    size, cell = CASES[3]
+    try:
+        lib.mm_tune_clear()
+        s = make(mm, size, cell)
+        s.steps(1)
+        alone = min(lib.mm_sim_time_pass(s._ptr, 4, 50) / 50 for _ in range(5))
+        m = s.m
+        _, default, _ = s.tune(reps=50)["er"]
+        assert default > 1.15 * alone, (default, alone)
+        assert np.array_equal(s.m, m)
+        s.free()
+    finally:
+        lib.mm_tune_clear()
+        lib.mm_tune_load(mm.gpukern.TUNE_TABLE.encode())
