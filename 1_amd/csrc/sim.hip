@@ -1314,7 +1314,7 @@ int mm_sim_tune(mmSim* s, int reps, int params[7], double ms_default[8], double 
         tune_one(2, &cp.tp.yb, dflt.yb, grid, 1, 3);
         tune_one(3, &cp.tp.xb, dflt.xb, grid, 2, -1);
         std::vector<int> xv{0};
-        for (int v = 1; v <= 3; v++)
+        for (int v = 2; v <= 3; v++)  // 1 is 0
             if (conv_xv_valid(cp.P[0], v)) xv.push_back(v);
         if (xv.size() > 1) tune_one(6, &cp.tp.xv, dflt.xv, xv, 2, -1);
         cp.tp.pp = pp0;

@@ -25,15 +25,17 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 DESCR = {
-    "zr": "Z forward rows per block (0 default, 1 half, 2 double)",
-    "er": "fused Z inverse rows per block (0 default, 1 half)",
+    "zr": "Z forward rows per block (0 by the grid, 1 half of the length's own, 2 double, 3 a quarter, 4 the length's "
+          "own)",
+    "er": "fused Z inverse rows per block (0 by the grid, 1 half of the length's own, 2 two rows, 3 the length's own); "
+          "on grids where it ends with the next stage's Z forward the ms are of both",
     "yb": "3-D Y passes, blocks per CU (both passes)",
     "xb": "X.K.X pass, blocks per CU",
     "y2b": "2-D Y.K.Y pass, blocks per CU",
     "pp": "3-D plans with padded Y 512, padded X 16/32: 1 = one register-resident plane pass for Y, X.K.X, Y "
           "inverse; 0 = three passes (ms: the passes it replaces)",
-    "xv": "X.K.X variant, padded X 16-64: 0 default, 1 no prefetch of the next item, 2 half the elements per lane "
-          "over twice the lanes, 3 both",
+    "xv": "X.K.X variant, padded X 16-64: 0 default (1 is the same), 2 half the elements per lane over twice the "
+          "lanes with the next item prefetched, 3 without the prefetch",
 }
 
 
@@ -81,10 +83,11 @@ def main():
     text = "\n".join(lines + (extra if len(extra) > 5 else []))
     print(text)
     print("\n%d entries written to %s" % (n, args.out))
-    print("\n" + "\n".join("- `%s`: %s" % kv for kv in DESCR.items()))
+    notes = "\n".join("- `%s`: %s" % kv for kv in DESCR.items())
+    print("\n" + notes)
     if args.report:
         with open(args.report, "w") as f:
-            f.write(text + "\n")
+            f.write(text + "\n\n" + notes + "\n")
 
 
 if __name__ == "__main__":

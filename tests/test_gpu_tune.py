@@ -73,7 +73,7 @@ def test_every_launch_shape_gives_the_same_steps(mm, lib, tmp_path, size, cell):
         lib.mm_tune_clear()
         s = make(mm, size, cell)
         res = s.tune(reps=3)
-        assert "zr" in res and "er" in res
+        assert "zr" in res and "er" in res and res.get("xv", (0,))[0] != 1  # 1 is 0: no candidate
         for k, val in res.items():
             if k == "plane_vs_three":
                 assert min(val) > 0
