@@ -58,9 +58,10 @@ def test_python_binding_tables_match_headers():
 
 
 def test_noalloc_forward_rejects_plans_beyond_its_scratch():
-    """gpuFFT3dPlan_forward_noalloc checks its fixed scratch (4 Mi complex
-    elements) before any device call: Z rows of half-length 3001 (prime) over
-    2000 rows need 2000 x 3001 packed elements plus a Bluestein buffer, so it
+    """gpuFFT3dPlan_forward_noalloc checks its limit on the plan (4 Mi complex
+    elements of packed rows and chirp buffers, as they are counted, though the
+    transform holds neither) before any device call: Z rows of half-length 3001
+    (prime) over 2000 rows count 2000 x 3001 packed elements plus a chirp buffer, so it
     aborts with a message (the library's error behaviour).  Runs in a child
     process on the CPU; input and output are never touched."""
     import subprocess

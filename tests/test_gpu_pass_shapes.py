@@ -190,7 +190,7 @@ def test_dropin_transform_lengths(lib, size, P):
     from test_zz_no_alloc import download, forward_both, i3, upload
 
     ref, got, npref = forward_both(lib, size, P, 5)
-    assert np.array_equal(ref.view(np.uint32), got.view(np.uint32))
+    assert np.array_equal(ref.view(np.uint32), got.view(np.uint32))  # the two calls run the same kernels
     assert np.abs(ref.view(np.complex64).reshape(npref.shape) - npref).max() < 2e-6 * np.abs(npref).max()
     plan = lib.new_gpuFFT3dPlan_padded(i3(*size), i3(*P))
     d, back = upload(lib, ref), lib.new_gpu_array(int(np.prod(size)))

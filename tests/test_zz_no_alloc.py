@@ -1,12 +1,13 @@
-"""gpuFFT3dPlan_forward_noalloc (include/gpukern.h) against gpuFFT3dPlan_forward.
+"""gpuFFT3dPlan_forward_noalloc (include/gpukern.h): numpy's transform, on device
+memory that stays as it is during the call.
 
-The no-allocation variant runs the same kernels with their temporaries in the
-library's fixed device scratch array, so its output must equal the allocating
-forward transform's bit for bit.  Two calls in a row, the second on a smaller
-plan, check that what the first left in the shared array does not leak into
-the second.  The sizes make every scratch user run: Z rows of half-length 13
-(packed rows plus a Bluestein buffer), Y lines of length 22 (Bluestein), Z
-rows of half-length 7 (packed rows, radix-7 Stockham).
+Both forward calls run a plan's kernels in registers and LDS on the caller's
+buffers, so their outputs are the same bits; what the no-allocation call adds is
+that it refuses large plans (tests/test_abi_exports.py) and a missing table.  The
+sizes take Z rows of half-length 13 (Bluestein), Y lines of length 22 (Bluestein), Z
+rows of half-length 7 (radix-7 Stockham) and powers of two (registers).
+
+Tolerance: 2e-6 of the largest value (FP32 transforms, a few 1e-7 x log2 P).
 """
 import ctypes as C
 
@@ -36,6 +37,13 @@ def download(lib, p, n):
     return out
 
 
+def device_memory():
+    """free bytes of the device, as the HIP runtime that the library is linked to gives them"""
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
 def forward_both(lib, size, P, seed):
     rng = np.random.default_rng(seed)
     x = rng.standard_normal(size).astype(F32)
@@ -44,8 +52,10 @@ def forward_both(lib, size, P, seed):
     din = upload(lib, x)
     d_ref = lib.new_gpu_array(n_out)
     d_na = lib.new_gpu_array(n_out)
-    lib.gpuFFT3dPlan_forward(plan, din, d_ref)
+    lib.gpuFFT3dPlan_forward(plan, din, d_ref)  # (also loads the kernels' code)
+    before = device_memory(), lib.mm_memory_cached()
     lib.gpuFFT3dPlan_forward_noalloc(plan, din, d_na)
+    assert (device_memory(), lib.mm_memory_cached()) == before, "the call took device memory"
     ref = download(lib, d_ref, n_out)
     got = download(lib, d_na, n_out)
     for p in (din, d_ref, d_na):
