@@ -1022,6 +1022,24 @@ static int pipeline_split(long items, long blocks, int* grid) {
     return (int)nit;
 }
 
+// FastDiv at the ends of its quotients' ranges, for every d up to 1024 and about the powers of two
+constexpr bool fast_div_exact(unsigned d) {
+    const FastDiv f(d);
+    const unsigned last = 0x7fffffffu, k = last / d;
+    for (unsigned n : {0u, d - 1, d, (k / 2 + 1) * d - 1, (k / 2 + 1) * d, k * d - 1, k * d, last})
+        if (n <= last && f.div(n) != n / d) return false;
+    return true;
+}
+constexpr bool fast_div_exact() {
+    for (unsigned d = 1; d <= 1024; d++)
+        if (!fast_div_exact(d)) return false;
+    for (unsigned p = 1024; p <= 1u << 30; p *= 2)
+        for (unsigned d : {p - 1, p, p + 1, p + p / 3})
+            if (!fast_div_exact(d)) return false;
+    return fast_div_exact(0x7fffffffu);
+}
+static_assert(fast_div_exact(), "FastDiv");
+
 static void launch_y3d(const ConvPlan& cp, const EngineState* st, bool fwd, hipStream_t s) {
     const int PY = cp.P[1], Nx = cp.N[0], Ny = cp.N[1], Q = cp.Q;
     const float2* tw = twiddle_f32(PY);

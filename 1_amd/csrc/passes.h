@@ -44,14 +44,6 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
     return (b % kXcd) * (nb / kXcd) + b / kXcd;
 }
 
-template <int L> constexpr int rows_per_block() {
-    int n = 71680 / ((L + 1) * 8);
-    n = n < 1 ? 1 : (n > 16 ? 16 : n);
-    int p = 1;
-    while (p * 2 <= n) p *= 2;
-    return p;
-}
-
 // shuffle of a complex value within groups of W lanes
 template <int W> __device__ __forceinline__ float2 shfl2(float2 v, int src) {
     return make_float2(__shfl(v.x, src, W), __shfl(v.y, src, W));
@@ -677,6 +669,23 @@ __global__ __launch_bounds__(3 * TR * RegFFT<M>::G) void k_zinv_epi(float2* B1, 
                                   blockIdx.y * gridDim.x + blockIdx.x, lds, hext_s, red);
 }
 
+// Division of n < 2^31 by a runtime constant d >= 1 as a product: a pass's lines
+// cost two of these instead of four 64-bit divisions (about 100 instructions each,
+// twice the line's transform).  With 2^(shift - 31) >= d, mul = ceil(2^shift / d) is
+// over 2^shift / d by less than 1, the quotient by less than n / 2^shift < 1 / d: the
+// floor is exact.  mul is below 2^32 (2^31 for d = 1 and powers of two, more for others:
+// it needs all 32 bits), the product below 2^63.
+struct FastDiv {
+    unsigned d, mul, shift;
+    FastDiv() = default;
+    constexpr explicit FastDiv(unsigned dv) : d(dv), mul(0), shift(31) {
+        while ((1ull << (shift - 31)) < dv) shift++;
+        mul = (unsigned)(((1ull << shift) + dv - 1) / dv);
+    }
+    __host__ __device__ __forceinline__ constexpr unsigned div(unsigned n) const {
+        return (unsigned)(((unsigned long long)n * mul) >> shift);
+    }
+};
 // 3-D Y passes, software-pipelined.  One line per lane group and iteration:
 //   forward  B1[c][x][kz][0..Ny) -> B2[c][kz][x][0..Py)   (zero padded)
 //   inverse  B2[c][kz][x][0..Py) -> B1[c][x][kz][0..Ny)   (rows >= Ny dropped)
@@ -685,18 +694,6 @@ __global__ __launch_bounds__(3 * TR * RegFFT<M>::G) void k_zinv_epi(float2* B1, 
 // before transforming line i, so the memory of one line overlaps the FFT of
 // the previous one; twiddles come from LDS, so no global load sits between a
 // prefetch and its use.
-// Division of n < 2^31 by a runtime constant d >= 1 as a product: a pass's lines
-// cost two of these instead of four 64-bit divisions (about 100 instructions each,
-// twice the line's transform).
-struct FastDiv {
-    unsigned d, mul, shift;
-    FastDiv() = default;
-    explicit FastDiv(unsigned dv) : d(dv), mul(0), shift(31) {
-        while ((1ull << (shift - 31)) < dv) shift++;               // 2^(shift-31) >= d
-        mul = (unsigned)(((1ull << shift) + dv - 1) / dv);         // ceil(2^shift / d) <= 2^31 + 1
-    }
-    __device__ __forceinline__ unsigned div(unsigned n) const { return (unsigned)(((unsigned long long)n * mul) >> shift); }
-};
 // offsets of B1 line (c, x, kz) and B2 line (c, kz, x) of a Y-pass line number (x fastest)
 struct YLine {
     long b1, b2;
@@ -1523,9 +1520,9 @@ __device__ __forceinline__ void y2_columns(float2* __restrict__ B1, const float*
 
 // single simulation: a block walks nit column sets strided by the grid
 template <int PY>
-__global__ __launch_bounds__(Y2<PY>::NT) __attribute__((amdgpu_waves_per_eu(Y2<PY>::G > 128 ? 6 : 1))) void k_y2r(float2* __restrict__ B1, const float* __restrict__ Kc,
-                                                    const float2* __restrict__ tw, const EngineState* st, int Ny,
-                                                    int Q, int nit) {
+__global__ __launch_bounds__(Y2<PY>::NT) __attribute__((amdgpu_waves_per_eu(Y2<PY>::G > 128 ? 6 : 1))) void k_y2r(
+    float2* __restrict__ B1, const float* __restrict__ Kc, const float2* __restrict__ tw, const EngineState* st, int Ny,
+    int Q, int nit) {
     __shared__ float2 lds[Y2<PY>::LDS];
     if (st && !st->trial_active) return;
     for (int it = 0; it < nit; it++) {
