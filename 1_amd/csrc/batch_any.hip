@@ -24,9 +24,14 @@ __global__ __launch_bounds__(1024) void kb_zfwd_any(const BSim* sims, const int2
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     switch (d.Q - 1) {
-#define GK_CASE(m)                                                              \
-    case m: {                                                                   \
-        constexpr int TR = z_rows_c<m>();                                           if (threadIdx.x >= TR * RegFFT<m>::G) return;                               bz_fwd<m, TR, NK>(d, bb.lb, sg, d.twM, d.twP, dyn);                         break;                                                                  }
+#define GK_CASE(m)                                    \
+    case m: {                                         \
+        constexpr int TR = z_rows_c<m>();             \
+        if (threadIdx.x >= TR * RegFFT<m>::G) return; \
+        bz_fwd<m, TR, NK>(d, bb.lb, sg, d.twM, d.twP, \
+                          dyn);                       \
+        break;                                        \
+    }
         GK_ANY_M(GK_CASE)
 #undef GK_CASE
     }
@@ -54,16 +59,21 @@ void any_attr_zfwd() {
 // (96 registers, 5 waves per SIMD; the last stage of an adaptive tableau, with six
 // earlier stages and their FP64 errors, would spill: 91 us, 136 with the bound)
 template <int NU, int FIN>
-__global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(FIN == 2 ? 1 : 5))) void kb_zinv_any(const BSim* sims, const int2* map,
-                                                   BStage sg) {
+__global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(FIN == 2 ? 1 : 5))) void kb_zinv_any(
+    const BSim* sims, const int2* map, BStage sg) {
     extern __shared__ float2 dyn[];
     const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;
     if (bskip(d, sg)) return;
     switch (d.Q - 1) {
-#define GK_CASE(m)                                                                              \
-    case m: {                                                                   \
-        constexpr int TR = epi_rows_c<m>(), NT = 3 * TR * RegFFT<m>::G;                             if (threadIdx.x >= NT) return;                                                              float* hext_s = reinterpret_cast<float*>(dyn + zinv_epi_lds<m, TR>());                      bz_inv<m, TR, NU, FIN>(d, bb.lb, sg, d.twM, d.twP, dyn, hext_s, hext_s + 4);                break;                                                                                  }
+#define GK_CASE(m)                                                                   \
+    case m: {                                                                        \
+        constexpr int TR = epi_rows_c<m>(), NT = 3 * TR * RegFFT<m>::G;              \
+        if (threadIdx.x >= NT) return;                                               \
+        float* hext_s = reinterpret_cast<float*>(dyn + zinv_epi_lds<m, TR>());       \
+        bz_inv<m, TR, NU, FIN>(d, bb.lb, sg, d.twM, d.twP, dyn, hext_s, hext_s + 4); \
+        break;                                                                       \
+    }
         GK_ANY_M(GK_CASE)
 #undef GK_CASE
     }

@@ -90,8 +90,9 @@ __device__ __forceinline__ void bz_fwd(const BSim& d, int lb, const BStage& sg, 
 }
 
 template <int M, int TR, int NK>
-__global__ __launch_bounds__(TR * RegFFT<M>::G) void kb_zfwd(const BSim* sims, const int2* map, BStage sg, const float2* __restrict__ twM,
-                                                               const float2* __restrict__ twP) {
+__global__ __launch_bounds__(TR * RegFFT<M>::G) void kb_zfwd(const BSim* sims, const int2* map, BStage sg,
+                                                             const float2* __restrict__ twM,
+                                                             const float2* __restrict__ twP) {
     __shared__ float2 lds[zfwd_lds<M, TR>()];
     const BBlock bb = bblock(sims, map);
     const BSim& d = *bb.d;

@@ -159,10 +159,10 @@ struct KernelSpec {
 // defaults are hand-picked; the autotuner (mm_sim_tune) times the candidates
 // on the device and a table of tuned values (per data size) feeds new plans.
 struct TuneParams {
-    int zr = 0;   // Z forward rows per block: variant 0 = by the grid, 1 = half of z_rows<M>(), 2 = double, 3 = a quarter, 4 = z_rows<M>()
-    int er = 0;   // fused Z inverse rows per block: variant 0 = by the grid, 1 = half of epi_rows<M>(), 2 = two rows, 3 = epi_rows<M>()
+    int zr = 0;   // Z forward rows per block: 0 by the grid, 1 half of z_rows<M>(), 2 double, 3 a quarter, 4 z_rows<M>()
+    int er = 0;   // fused Z inverse rows per block: 0 by the grid, 1 half of epi_rows<M>(), 2 two rows, 3 epi_rows<M>()
     int yb = 8;   // blocks per CU of the pipelined 3-D Y passes
-    int xb = 4;   // blocks per CU of the pipelined X.K.X pass
+    int xb = 4;   // blocks per CU of the X.K.X pass
     int y2b = 8;  // blocks per CU of the 2-D Y.K.Y pass
     int pp = 0;   // 3-D plans that fit it: 1 = Y.X K X.Y in one plane pass (k_plane3), 0 = separate passes
     int xv = 0;   // X.K.X variant (padded X 16-64): 0, 1 default, 2 half the elements per lane and a prefetch, 3 without it

@@ -83,10 +83,12 @@ __global__ __launch_bounds__(NT) void k_fft_lines(C2<T>* __restrict__ data, cons
 // index fastest.  All of a lane's loads and the block's copy of the twiddle
 // table are issued together, one memory latency for the whole kernel (the LDS
 // Stockham kernels these replace read the table from global memory in every
-// pass).  Strided lines go 16 to a block, whole 128 B cache lines: with 4, for more
-// blocks, neighbours on other XCDs wrote parts of the same line.  Rows go as many
-// to a block as leave about two blocks per CU: small transforms are latency-bound
-// and need the CUs, not the occupancy.
+// pass).  Strided lines go 16 (short lengths more) to a block, whole 128 B cache
+// lines: with 4, for more blocks, neighbours on other XCDs wrote parts of the same
+// line.  Threads and LDS allow that up to length 384: 8 lines at 512, 4 at 768 and
+// 1024, 2 at 1536 and 2048, one at 3072 and 4096 share parts of cache lines.  Rows go
+// as many to a block as leave about two blocks per CU: small transforms are
+// latency-bound and need the CUs, not the occupancy.
 // Measured per launch (before / now): 2064 lines of 256 12.9 / 6.9 us (4 lines a
 // block 9.0), 33024 of 32 8.0 / 5.5 us, 2048 rows of 256 reals 8.9 / 4.3 us; 64 rows
 // of 512 12.4 / 4.0 us.
@@ -265,9 +267,10 @@ bool fft_reg_length(int L) {
     }
 }
 
-// log2 of the lines per block: up to 256 threads, at least 16 lines (128 B runs, a
-// cache line) and 60 KB of LDS, then fewer, down to 4 lines (32 B runs), while the
-// launch has under 64 blocks
+// log2 of the lines per block: 16 (128 B runs, a cache line) or as many more as 256
+// threads take, fewer where they pass 1024 threads or 60 KB of LDS (8 at length 512
+// down to one at 3072 and at 4096, whose line takes 70 KB), and down to 4 (32 B runs)
+// while the launch has under 64 blocks of more than a wave
 static int lines_shift(int L, int G, unsigned nlines) {
     int sh = 4;
     while ((G << (sh + 1)) <= 256) sh++;

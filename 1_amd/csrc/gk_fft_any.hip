@@ -2,13 +2,14 @@
 // every size cuFFT does; the Go driver pads each axis to 2N, kernel.go:80-90,
 // so lengths such as 2^a 3^b 5^c 7^d and 2p for a prime p all occur).
 //
-// Lengths whose factors are 2, 3, 5 and 7 run as Stockham passes in LDS with
-// a runtime list of radices (8, 4, 2, 3, 5, 7), one line per block.  Any other
-// length uses Bluestein's chirp-z identity nk = (n^2 + k^2 - (k-n)^2)/2:
+// Lengths whose factors are 2, 3, 5 and 7 (beyond the register lengths of
+// gk_fft.hip) run as Stockham passes in LDS with a runtime list of radices (8, 4,
+// 2, 3, 5, 7), up to 8 neighbouring lines per block.  Any other length uses
+// Bluestein's chirp-z identity nk = (n^2 + k^2 - (k-n)^2)/2:
 //   X[k] = w[k] sum_n (x[n] w[n]) conj(w)[k-n],   w[n] = exp(DIR pi i n^2 / L),
-// i.e. a circular convolution of length Lp >= 2L-1 (a power of two) done with
-// the power-of-two line transforms; the chirp and the transformed filter are
-// computed on the host in long double.  Real rows of even length P use the
+// i.e. a circular convolution of length Lp >= 2L-1 (a power of two), both of whose
+// transforms run in registers in one kernel; the chirp and the transformed filter
+// are computed on the host in long double.  Real rows of even length P use the
 // half-length complex transform (same split / merge as the power-of-two path);
 // odd P (a periodic axis) uses the full complex transform of length P.
 #include <hip/hip_runtime.h>
