@@ -1065,7 +1065,8 @@ static void launch_y3d(const ConvPlan& cp, const EngineState* st, bool fwd, hipS
 
 // X . K . X launch variants (TuneParams::xv) for padded X 16, 32, 64: 2 = half the
 // elements per lane over twice the lanes with the next item prefetched, 3 =
-// without the prefetch; 0, 1 and other lengths: k_xmul
+// without the prefetch; 0, 1 and other lengths: k_xmul, or k_xmul_v with the prefetch
+// where xmul_walks says so
 template <int PX, int EE, bool PIPE>
 static void xmul_v_launch(const ConvPlan& cp, const EngineState* st, const float2* tw, hipStream_t s) {
     constexpr int LPB = kNT / (PX / EE);
@@ -1076,6 +1077,10 @@ static void xmul_v_launch(const ConvPlan& cp, const EngineState* st, const float
     k_xmul_v<PX, EE, PIPE><<<g, kNT, 0, s>>>(cp.B2, cp.Kc, tw, st, cp.N[0], PY, cp.Q, nit);
 }
 bool conv_xv_valid(int PX, int v) { return v == 0 || ((PX == 16 || PX == 32 || PX == 64) && v >= 1 && v <= 3); }
+
+bool conv_xmul_walks(const ConvPlan& cp) {
+    return (cp.tp.xv >= 2 && conv_xv_valid(cp.P[0], cp.tp.xv)) || xmul_walks(cp.P[0]);
+}
 
 static void launch_xmul(const ConvPlan& cp, const EngineState* st, hipStream_t s) {
     const int PX = cp.P[0], PY = cp.P[1], Nx = cp.N[0], Q = cp.Q;
@@ -1094,14 +1099,15 @@ static void launch_xmul(const ConvPlan& cp, const EngineState* st, hipStream_t s
     }
     switch (PX) {
 #define GK_CASE(n)                                                                              \
-    case n: {                                                                                   \
-        constexpr int LPB = kNT / RegFFT<n>::G;                                                 \
-        const int lpr = LPB < PY ? LPB : PY;                                                    \
-        int g = 0;                                                                              \
-        const int nit = pipeline_split((long)Q * div_up(PY, lpr), (long)cp.tp.xb * cu_count(), &g); \
-        k_xmul<n><<<g, kNT, 0, s>>>(cp.B2, cp.Kc, tw, st, Nx, PY, Q, nit);                      \
-        break;                                                                                  \
-    }
+    case n:                                                                                     \
+        if constexpr (xmul_walks(n)) {                                                          \
+            xmul_v_launch<n, RegFFT<n>::E, true>(cp, st, tw, s);                                \
+        } else {                                                                                \
+            constexpr int LPB = kNT / RegFFT<n>::G;                                             \
+            const int g = Q * div_up(PY, LPB < PY ? LPB : PY);                                  \
+            k_xmul<n><<<g, kNT, 0, s>>>(cp.B2, cp.Kc, tw, st, Nx, PY, Q);                       \
+        }                                                                                       \
+        break;
         GK_LEN_X(GK_CASE)
 #undef GK_CASE
     default: abort();

@@ -162,7 +162,7 @@ struct TuneParams {
     int zr = 0;   // Z forward rows per block: 0 by the grid, 1 half of z_rows<M>(), 2 double, 3 a quarter, 4 z_rows<M>()
     int er = 0;   // fused Z inverse rows per block: 0 by the grid, 1 half of epi_rows<M>(), 2 two rows, 3 epi_rows<M>()
     int yb = 8;   // blocks per CU of the pipelined 3-D Y passes
-    int xb = 4;   // blocks per CU of the X.K.X pass
+    int xb = 4;   // blocks per CU of the X.K.X pass where its blocks walk items (conv_xmul_walks)
     int y2b = 8;  // blocks per CU of the 2-D Y.K.Y pass
     int pp = 0;   // 3-D plans that fit it: 1 = Y.X K X.Y in one plane pass (k_plane3), 0 = separate passes
     int xv = 0;   // X.K.X variant (padded X 16-64): 0, 1 default, 2 half the elements per lane and a prefetch, 3 without it
@@ -201,6 +201,8 @@ int conv_z_rows(int M, int v);
 bool conv_zr_valid(int M, int v);
 bool conv_er_valid(int M, int v);
 bool conv_xv_valid(int PX, int v);
+// whether the X.K.X pass runs a kernel whose blocks walk items, xb per CU, and not one item per block
+bool conv_xmul_walks(const ConvPlan& cp);
 
 // Choose padded sizes, allocate buffers.  Kc is set by conv_acquire_kernel.
 void conv_plan_init(ConvPlan& cp, const int N[3]);

@@ -768,8 +768,8 @@ __global__ __launch_bounds__(kNT) void k_ypass(const float2* __restrict__ src, f
 // the loads and stores touch G rows of consecutive ky per instruction, the
 // 6-component symmetric multiply is lane-local, and each transform needs one
 // LDS exchange per radix pass.  A block item is one kz and a run of lpr
-// consecutive ky; a block walks `nit` consecutive items.  Items are ordered so that
-// the runs ky and Py - ky (which read the same kernel rows) follow each other.
+// consecutive ky.  Items are ordered so that the runs ky and Py - ky (which read the
+// same kernel rows) follow each other.
 // the 3 components of column (kz, ky) into lane g's registers (ky < 0: zeros)
 template <int PX>
 __device__ __forceinline__ void xmul_load(float2 (*v)[RegFFT<PX>::E], const float2* __restrict__ B2, int kz, int ky,
@@ -838,11 +838,17 @@ __device__ __forceinline__ void xmul_column(unsigned t, unsigned items, unsigned
     ky = (t < items && li < lpr && r * lpr + li < PY) ? r * lpr + li : -1;
 }
 
-// Launch variants of the X . K . X pass (TuneParams::xv 2 and 3): EE elements per
-// lane, half of the default RegFFT<PX>::E over twice the lanes (fewer live
+// Variants of the X . K . X pass whose blocks walk `nit` consecutive items: EE
+// elements per lane, RegFFT<PX>::E or half of it over twice the lanes (fewer live
 // registers, one more LDS exchange per transform), and PIPE, the next item's
 // columns loaded before the current one is transformed (twice the data
-// registers) or after.  Lane g of a line holds x = g + (PX / EE) e.
+// registers) or after.  Lane g of a line holds x = g + (PX / EE) e.  Halves are
+// TuneParams::xv 2 (PIPE) and 3; padded X 192 and 384 take the whole with PIPE: their
+// 180 and 194 registers allow two waves per SIMD with the prefetch or without
+// (233 and 256), so there it costs no waves.  90 x 90 x 90 (padded X 192) 51 us a launch
+// with it, 59 without walking as many items, 50 an item per block; 75 x 270 x 74 136,
+// 163 and 158 us; 133 x 11 x 323 (384) 59, 64 and 52 us.
+constexpr bool xmul_walks(int PX) { return PX == 192 || PX == 384; }
 template <int PX, int EE>
 __device__ __forceinline__ void xmul_load_e(float2 (*v)[EE], const float2* __restrict__ B2, int kz, int ky, int Nx,
                                             int PY, int Q, int g) {
@@ -947,13 +953,16 @@ __global__ __launch_bounds__(kNT) void k_xmul_v(float2* __restrict__ B2, const f
     }
 }
 
-// every other length, and the default: RegFFT<PX>::E elements per lane, no prefetch
-// (it doubles the data registers, and the waves it costs hide more latency than
-// it does: padded X 128, 70 x 60 x 51, 23.3 us a launch with it, 19.3 without)
+// every other length, and the default: RegFFT<PX>::E elements per lane, an item per
+// block.  A prefetch of the next item doubles the data registers, and the waves it
+// costs hide more latency than it does; and without one, a block that walks items
+// only makes later ones wait: 70 x 60 x 51 (padded X 128) 21.2 us a launch with the
+// prefetch and 4 blocks per CU, 18.4 walking items without it, 18.0 an item per block;
+// 256 x 256 x 16 36.8, 33.8 and 31.0 us; 300 x 300 x 24 148, 135 and 113 us.
 template <int PX>
 __global__ __launch_bounds__(kNT) void k_xmul(float2* __restrict__ B2, const float* __restrict__ Kc,
                                               const float2* __restrict__ tw, const EngineState* st, int Nx, int PY,
-                                              int Q, int nit) {
+                                              int Q) {
     using F = RegFFT<PX>;
     constexpr int E = F::E, G = F::G, LPB = kNT / G;
     __shared__ float2 lds[LPB * F::LDS];
@@ -963,20 +972,17 @@ __global__ __launch_bounds__(kNT) void k_xmul(float2* __restrict__ B2, const flo
     const int li = threadIdx.x / G, g = threadIdx.x % G;
     const int lpr = LPB < PY ? LPB : PY;  // columns per item
     const int rows = (PY + lpr - 1) / lpr;  // items per kz plane (the last may be partial)
-    const unsigned items = (unsigned)Q * rows, t0 = blockIdx.x * nit;
+    int kz, ky;
+    xmul_column(blockIdx.x, (unsigned)Q * rows, rows, lpr, li, PY, kz, ky);
+    float2 v[3][E];
+    xmul_load<PX>(v, B2, kz, ky, Nx, PY, Q, g);
     __syncthreads();  // twiddle table
-    for (int it = 0; it < nit; it++) {
-        int kz, ky;
-        xmul_column(t0 + it, items, rows, lpr, li, PY, kz, ky);
-        float2 v[3][E];
-        xmul_load<PX>(v, B2, kz, ky, Nx, PY, Q, g);
 #pragma unroll
-        for (int c = 0; c < 3; c++) reg_fft<float, PX, -1>(v[c], g, lds + li * F::LDS, twl);
-        if (ky >= 0) xmul_kernel<PX>(v, Kc, kz, ky, PY, g);
+    for (int c = 0; c < 3; c++) reg_fft<float, PX, -1>(v[c], g, lds + li * F::LDS, twl);
+    if (ky >= 0) xmul_kernel<PX>(v, Kc, kz, ky, PY, g);
 #pragma unroll
-        for (int c = 0; c < 3; c++) reg_fft<float, PX, +1>(v[c], g, lds + li * F::LDS, twl);
-        if (ky >= 0) xmul_store<PX>(v, B2, kz, ky, Nx, PY, Q, g);
-    }
+    for (int c = 0; c < 3; c++) reg_fft<float, PX, +1>(v[c], g, lds + li * F::LDS, twl);
+    if (ky >= 0) xmul_store<PX>(v, B2, kz, ky, Nx, PY, Q, g);
 }
 
 // 3-D Y forward . X.K.X . Y inverse of one kz plane in one pass, for padded

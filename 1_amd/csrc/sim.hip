@@ -1312,11 +1312,11 @@ int mm_sim_tune(mmSim* s, int reps, int params[7], double ms_default[8], double 
         const int pp0 = cp.tp.pp;
         cp.tp.pp = 0;
         tune_one(2, &cp.tp.yb, dflt.yb, grid, 1, 3);
-        tune_one(3, &cp.tp.xb, dflt.xb, grid, 2, -1);
         std::vector<int> xv{0};
         for (int v = 2; v <= 3; v++)  // 1 is 0
             if (conv_xv_valid(cp.P[0], v)) xv.push_back(v);
         if (xv.size() > 1) tune_one(6, &cp.tp.xv, dflt.xv, xv, 2, -1);
+        if (conv_xmul_walks(cp)) tune_one(3, &cp.tp.xb, dflt.xb, grid, 2, -1);
         cp.tp.pp = pp0;
         if (cp.plane3) {
             double t[2];

@@ -158,6 +158,27 @@ def test_run_to_a_stop_time_in_pieces(mm):
     b.free()
 
 
+# padded X of every X.K.X kernel: an item per block (24 to 128, 256, 512) and walked with a prefetch (192, 384)
+@pytest.mark.parametrize("size", [(9, 34, 4), (13, 9, 4), (40, 3, 6), (50, 4, 5), (66, 5, 6), (96, 34, 2), (100, 3, 4),
+                                  (130, 6, 5), (192, 9, 3), (200, 4, 4)])
+def test_x_axis_lengths_vs_oracle(mm, orc, size):
+    m0 = random_m(size, 6)
+    cfg = cfg_of(size, m0, solver="rkdp", maxerror=1e-4, dt=1e-14, max_dt=1e-14)
+    s, t = mm.workloads.make_sim(cfg), mm.workloads.make_sim(cfg)
+    o = orc.sim(m0, **mm.workloads.oracle_kwargs(cfg))
+    h = s.heff(m0)
+    ref = o.heff(m0).reshape(h.shape)
+    assert np.abs(h - ref).max() < 5e-6 * np.abs(ref).max()
+    s.steps(2)
+    b = mm.Batch([t])
+    b.start(steps=2)
+    b.trials(2)
+    b.free()
+    assert np.array_equal(s.m, t.m)
+    for x in (s, t):
+        x.free()
+
+
 def test_a_relaxation_enqueues_no_further_than_its_end(mm):
     """A relaxed state ends its next relaxation within a few steps, also where many
     more are allowed: nearly all of 1024 trials enqueued at once would do nothing
