@@ -491,10 +491,20 @@ __global__ void k_extract_full(const double2* __restrict__ W, int P0, int P1, in
 // one CU, so rows are spread until every CU has blocks.  Z forward: half the rows
 // (8: 64 B runs of B1) below 4 blocks per CU, a quarter (32 B runs) below one.  Z
 // inverse: half below one block per CU, two rows where that still leaves fewer
-// (its reads of B1 are then 16 B runs, which the small spectra keep in L2).
+// (its reads of B1 are then 16 B runs, which the small spectra keep in L2); and half
+// below 480 blocks for rows of 96 to 512 pairs where it goes on with the next stage's
+// Z forward: 256 to 480 blocks that are a whole stage leave the CUs with one waiting
+// for those with two (longer rows would have 16 B runs or shorter).
 // Measured per launch with the length's rows / with these: 301 x 180 film, Z
 // forward of 5 stages 12.8 / 9.7 us, Z inverse 9.6 / 8.5 us; 150 x 91 x 3 slab 8.0 / 7.6
-// and 8.3 / 7.6 us; 70 x 60 x 51 block, Z forward 11.1 / 9.9 us.
+// and 8.3 / 7.6 us; 70 x 60 x 51 block, Z forward 11.1 / 9.9 us.  RK4 step with the
+// length's rows / with half in the combined kernel: 184 x 45 x 78 455 / 400 us, 323 x 11 x
+// 133 535 / 510, 500 x 300 x 4 355 / 322, 90 x 100 x 48 305 / 296; rows of 64 pairs 168 / 167
+// (64 x 64 x 64) and 222 / 234 (60 x 120 x 60).
+constexpr long kFusedWaves = 4096;  // conv_fwd_fused
+static long zinv_waves(const int N[3], int M, int rows) {
+    return (long)div_up(N[1], rows) * N[0] * div_up(3 * rows * reg_fft_G(M), 64);
+}
 static void grid_rows(const int N[3], int M, int* zr, int* er) {
     *zr = *er = 0;
     const int zd = conv_z_rows(M, 0), ed = conv_epi_rows(M, 0);
@@ -502,7 +512,8 @@ static void grid_rows(const int N[3], int M, int* zr, int* er) {
     if (zblocks(zd) < 1024 && conv_zr_valid(M, 1) && zd >= 16) *zr = 1;
     if (*zr == 1 && zblocks(conv_z_rows(M, 1)) < 256 && conv_zr_valid(M, 3)) *zr = 3;
     auto eblocks = [&](int rows) { return (long)N[0] * div_up(N[1], rows); };
-    if (eblocks(ed) < 256 && conv_er_valid(M, 1)) *er = 1;
+    const bool combined = z_fwd_fused(M) && zinv_waves(N, M, ed) <= kFusedWaves;
+    if (eblocks(ed) < (combined && M >= 96 && M <= 512 ? 480 : 256) && conv_er_valid(M, 1)) *er = 1;
     if (*er == 1 && eblocks(conv_epi_rows(M, 1)) < 256 && conv_er_valid(M, 2)) *er = 2;
 }
 
@@ -1229,10 +1240,7 @@ void conv_run_pass(const ConvPlan& cp, int cls, const StageIn& in, float* h, con
 // Larger grids keep the passes apart, whose own shapes and overlap are worth more
 // (256 x 256 x 16, 6144 waves: 10 RK4 steps 3711 us apart, 3818 fused).
 bool conv_fwd_fused(const ConvPlan& cp) {
-    if (!z_fwd_fused(cp.M)) return false;
-    const int tr = conv_epi_rows(cp.M, cp.er());
-    const long blocks = (long)div_up(cp.N[1], tr) * cp.N[0];
-    return blocks * div_up(3 * tr * reg_fft_G(cp.M), 64) <= 4096;
+    return z_fwd_fused(cp.M) && zinv_waves(cp.N, cp.M, conv_epi_rows(cp.M, cp.er())) <= kFusedWaves;
 }
 
 void conv_apply(const ConvPlan& cp, const StageIn* in, const EngineState* st, float* h, hipStream_t s, Prof* prof,
