@@ -20,6 +20,7 @@
 #include <mutex>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <vector>
 
@@ -129,7 +130,7 @@ struct TableImage {
     }
 };
 
-int epi_rows_host(int M);
+int epi_rows_host(int M, bool any);
 int z_rows_host(int M);
 
 }  // namespace
@@ -165,10 +166,10 @@ int z_rows_host(int M) {
     }
     abort();
 }
-int epi_rows_host(int M) {
+int epi_rows_host(int M, bool any) {
     switch (M) {
 #define GK_CASE(n) \
-    case n: return epi_rows_c<n>();
+    case n: return any ? epi_rows_any<n>() : epi_rows_c<n>();
         GK_LEN_M(GK_CASE)
 #undef GK_CASE
     }
@@ -192,7 +193,7 @@ AnyShape any_shape(int pass, int L) {
         break;
     case 1:  // Z inverse + epilogue, L = M
         switch (L) {
-#define GK_CASE(n) case n: return {3 * epi_rows_c<n>() * RegFFT<n>::G, zinv_any_bytes<n>()};
+#define GK_CASE(n) case n: return {3 * epi_rows_any<n>() * RegFFT<n>::G, zinv_any_bytes<n>()};
             GK_ANY_M(GK_CASE)
 #undef GK_CASE
         }
@@ -271,7 +272,9 @@ std::vector<LaunchSet> make_sets(mmBatch* b, const std::vector<int>& members, Ke
 // fewer blocks than this are merged into one dispatch launch when two or more
 // of them are small and have a body in the dispatch kernel.
 std::atomic<int> g_merge_blocks{1024};
-std::vector<LaunchSet> merge_small(std::vector<LaunchSet> sets, int pass) {
+// any_blocks(j), if given: simulation j's blocks in the dispatch launch (else the same).
+std::vector<LaunchSet> merge_small(std::vector<LaunchSet> sets, int pass,
+                                   const std::function<int(int)>& any_blocks = nullptr) {
     std::vector<LaunchSet> out, small;
     const int limit = g_merge_blocks.load();
     for (auto& ls : sets) {
@@ -295,7 +298,7 @@ std::vector<LaunchSet> merge_small(std::vector<LaunchSet> sets, int pass) {
         m.lds = std::max(m.lds, a.lds);
         for (int i = 0; i < ls.cnt; i++) {
             m.hidx.push_back(ls.hidx[i]);
-            m.hst.push_back(m.hst.back() + ls.hst[i + 1] - ls.hst[i]);
+            m.hst.push_back(m.hst.back() + (any_blocks ? any_blocks(ls.hidx[i]) : ls.hst[i + 1] - ls.hst[i]));
         }
         m.cnt += ls.cnt;
     }
@@ -567,13 +570,8 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
         d.dx = FastDiv(s->cp.N[0]);
         d.dq = FastDiv(s->cp.Q);
         d.cp = ctrl_params(s);
-        // per-block maxima as this batch's Z inverse writes them: its rows per block are
-        // its own, and so is the number of blocks
-        d.cp.n_k = div_up(d.Ny, epi_rows_host(s->cp.M)) * d.Nx;
-        d.cp.n_err = b->tb.fsal_final() ? d.cp.n_k : d.nfin;
         d.cp.part_e = nullptr;  // the batched epilogue computes no energy
     }
-    const size_t sims_off = b->image.put(h.data(), n * sizeof(BSim));
     b->ddone = (int*)balloc(b, n * sizeof(int));
     b->drem = (float*)balloc(b, n * sizeof(float));
     // launch sets per pass and length class
@@ -586,7 +584,8 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
     auto PY = [](const mmSim* s) { return s->cp.P[1]; };
     auto PX = [](const mmSim* s) { return s->cp.P[0]; };
     b->zf = make_sets(b, all, M, [](const mmSim* s) { return div_up(s->cp.N[1], z_rows_host(s->cp.M)) * s->cp.N[0] * 3; });
-    b->zi = make_sets(b, all, M, [](const mmSim* s) { return div_up(s->cp.N[1], epi_rows_host(s->cp.M)) * s->cp.N[0]; });
+    auto zinv_blocks = [](const mmSim* s, bool any) { return div_up(s->cp.N[1], epi_rows_host(s->cp.M, any)) * s->cp.N[0]; };
+    b->zi = make_sets(b, all, M, [&](const mmSim* s) { return zinv_blocks(s, false); });
     auto ylines = [](const mmSim* s) { return div_up(3L * s->cp.N[0] * s->cp.Q, 256 / lanes_host(s->cp.P[1])); };
     b->y3 = make_sets(b, d3, PY, ylines);
     b->xm = make_sets(b, d3, PX, [](const mmSim* s) {
@@ -601,11 +600,19 @@ mmBatch* mm_batch_new(mmSim* const* sims, int n) {
     // small length classes of each pass: one dispatch launch per pass
     any_kernel_attributes();
     b->zf = merge_small(std::move(b->zf), 0);
-    b->zi = merge_small(std::move(b->zi), 1);
+    b->zi = merge_small(std::move(b->zi), 1, [&](int j) { return zinv_blocks(sims[j], true); });
     b->yx = merge_small(std::move(b->yx), 2);
     b->y2 = merge_small(std::move(b->y2), 3);
     b->y3 = merge_small(std::move(b->y3), 4);
     b->xm = merge_small(std::move(b->xm), 5);
+    // per-block maxima as this batch's Z inverse writes them: one per block of its launch
+    for (const LaunchSet& ls : b->zi)
+        for (int i = 0; i < ls.cnt; i++) {
+            BSim& d = h[ls.hidx[i]];
+            d.cp.n_k = ls.hst[i + 1] - ls.hst[i];
+            d.cp.n_err = b->tb.fsal_final() ? d.cp.n_k : d.nfin;
+        }
+    const size_t sims_off = b->image.put(h.data(), n * sizeof(BSim));
     std::vector<BlockRun> runs;
     int entries = 0;
     for (auto* sets : {&b->zf, &b->zi, &b->y3, &b->xm, &b->y2, &b->yx, &b->fin})

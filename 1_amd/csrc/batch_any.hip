@@ -68,7 +68,7 @@ __global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(FIN == 2 ? 
     switch (d.Q - 1) {
 #define GK_CASE(m)                                                                   \
     case m: {                                                                        \
-        constexpr int TR = epi_rows_c<m>(), NT = 3 * TR * RegFFT<m>::G;              \
+        constexpr int TR = epi_rows_any<m>(), NT = 3 * TR * RegFFT<m>::G;            \
         if (threadIdx.x >= NT) return;                                               \
         float* hext_s = reinterpret_cast<float*>(dyn + zinv_epi_lds<m, TR>());       \
         bz_inv<m, TR, NU, FIN>(d, bb.lb, sg, d.twM, d.twP, dyn, hext_s, hext_s + 4); \

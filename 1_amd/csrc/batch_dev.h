@@ -262,11 +262,16 @@ template <int M> constexpr int epi_rows_c() {
     int p = 1;
     while (p * 2 <= tr) p *= 2;
     tr = p;
-    // three blocks per CU by their LDS: a dispatch launch gives every block the LDS of
-    // its largest length, so at 80 KB all of them ran two to a CU (40-member sweep,
-    // the launch of the short lengths 44.4 us, now 38.4)
-    while (tr > 4 && zinv_epi_lds_elems(M, tr) * 8 > 48 * 1024) tr /= 2;
     while (tr > 1 && zinv_epi_lds_elems(M, tr) * 8 > 80 * 1024) tr /= 2;
+    return tr;
+}
+// rows of a dispatch launch's block: it has the LDS of the launch's largest length,
+// so at 80 KB all of them ran two to a CU; three by their LDS (40-member sweep, the
+// launch of the short lengths 44.4 us, now 38.1).  A launch of one length keeps its
+// rows: half of them made 24 members of 256 x 256 3.8 % slower, of 256 x 256 x 4 3.1 %.
+template <int M> constexpr int epi_rows_any() {
+    int tr = epi_rows_c<M>();
+    while (tr > 4 && zinv_epi_lds_elems(M, tr) * 8 > 48 * 1024) tr /= 2;
     return tr;
 }
 
@@ -304,7 +309,7 @@ inline bool any_yx(int PY, int PX) { return any_y(PY) && (PX == 4 || PX == 8) &&
 inline bool any_x(int PX) { return PX == 4 || PX == 8 || PX == 16 || PX == 32; }
 
 template <int M> constexpr int zinv_any_bytes() {
-    constexpr int TR = epi_rows_c<M>(), NR = TR * RegFFT<M>::G;
+    constexpr int TR = epi_rows_any<M>(), NR = TR * RegFFT<M>::G;
     return zinv_epi_lds<M, TR>() * 8 + 16 + 3 * NR * 4;
 }
 
