@@ -189,11 +189,13 @@ __global__ __launch_bounds__(256) void k_rows_c2r_rt(const float2* __restrict__ 
 }
 
 // log2 of the lines per block: 8 (64 B runs of float2), fewer where both buffers
-// pass 48 KB or, down to 4, where the launch has under 512 blocks
+// pass 48 KB or, down to 4, where the launch has under 512 blocks, and one where it
+// has under 16 (9 lines of 210: the transform padded to 210 x 1 x 16 23.2 us with 4, 20.7 with one)
 template <typename T> static int rt_shift(int L, unsigned nlines) {
     int sh = 3;
     while (sh > 0 && (2L * L * (long)sizeof(C2<T>) << sh) > 48 * 1024) sh--;
     while (sh > 2 && (nlines >> sh) < 512) sh--;
+    while (sh > 0 && (nlines >> sh) < 16) sh--;
     return sh;
 }
 
