@@ -1116,7 +1116,7 @@ static void launch_xmul(const ConvPlan& cp, const EngineState* st, hipStream_t s
         } else {                                                                                \
             constexpr int LPB = kNT / RegFFT<n>::G;                                             \
             const int g = Q * div_up(PY, LPB < PY ? LPB : PY);                                  \
-            k_xmul<n><<<g, kNT, 0, s>>>(cp.B2, cp.Kc, tw, st, Nx, PY, Q);                       \
+            k_xmul<n><<<g, kNT, 0, s>>>(cp.B2, cp.Kc, tw, st, Nx, PY, Q, 1);                    \
         }                                                                                       \
         break;
         GK_LEN_X(GK_CASE)

@@ -957,12 +957,14 @@ __global__ __launch_bounds__(kNT) void k_xmul_v(float2* __restrict__ B2, const f
 // block.  A prefetch of the next item doubles the data registers, and the waves it
 // costs hide more latency than it does; and without one, a block that walks items
 // only makes later ones wait: 70 x 60 x 51 (padded X 128) 21.2 us a launch with the
-// prefetch and 4 blocks per CU, 18.4 walking items without it, 18.0 an item per block;
-// 256 x 256 x 16 36.8, 33.8 and 31.0 us; 300 x 300 x 24 148, 135 and 113 us.
+// prefetch and 4 blocks per CU, 18.0 an item per block; 256 x 256 x 16 36.8, walking items
+// without it 33.8, an item per block 31.0 us; 300 x 300 x 24 148, 135 and 113 us.
+// (The launch gives nit = 1; written without the loop, the compiler's schedule was up
+// to 12 % faster in the pass on its own, but 64 x 64 x 64 steps went 164 -> 167 us.)
 template <int PX>
 __global__ __launch_bounds__(kNT) void k_xmul(float2* __restrict__ B2, const float* __restrict__ Kc,
                                               const float2* __restrict__ tw, const EngineState* st, int Nx, int PY,
-                                              int Q) {
+                                              int Q, int nit) {
     using F = RegFFT<PX>;
     constexpr int E = F::E, G = F::G, LPB = kNT / G;
     __shared__ float2 lds[LPB * F::LDS];
@@ -972,17 +974,20 @@ __global__ __launch_bounds__(kNT) void k_xmul(float2* __restrict__ B2, const flo
     const int li = threadIdx.x / G, g = threadIdx.x % G;
     const int lpr = LPB < PY ? LPB : PY;  // columns per item
     const int rows = (PY + lpr - 1) / lpr;  // items per kz plane (the last may be partial)
-    int kz, ky;
-    xmul_column(blockIdx.x, (unsigned)Q * rows, rows, lpr, li, PY, kz, ky);
-    float2 v[3][E];
-    xmul_load<PX>(v, B2, kz, ky, Nx, PY, Q, g);
+    const unsigned items = (unsigned)Q * rows, t0 = blockIdx.x * nit;
     __syncthreads();  // twiddle table
+    for (int it = 0; it < nit; it++) {
+        int kz, ky;
+        xmul_column(t0 + it, items, rows, lpr, li, PY, kz, ky);
+        float2 v[3][E];
+        xmul_load<PX>(v, B2, kz, ky, Nx, PY, Q, g);
 #pragma unroll
-    for (int c = 0; c < 3; c++) reg_fft<float, PX, -1>(v[c], g, lds + li * F::LDS, twl);
-    if (ky >= 0) xmul_kernel<PX>(v, Kc, kz, ky, PY, g);
+        for (int c = 0; c < 3; c++) reg_fft<float, PX, -1>(v[c], g, lds + li * F::LDS, twl);
+        if (ky >= 0) xmul_kernel<PX>(v, Kc, kz, ky, PY, g);
 #pragma unroll
-    for (int c = 0; c < 3; c++) reg_fft<float, PX, +1>(v[c], g, lds + li * F::LDS, twl);
-    if (ky >= 0) xmul_store<PX>(v, B2, kz, ky, Nx, PY, Q, g);
+        for (int c = 0; c < 3; c++) reg_fft<float, PX, +1>(v[c], g, lds + li * F::LDS, twl);
+        if (ky >= 0) xmul_store<PX>(v, B2, kz, ky, Nx, PY, Q, g);
+    }
 }
 
 // 3-D Y forward . X.K.X . Y inverse of one kz plane in one pass, for padded
