@@ -843,12 +843,13 @@ __device__ __forceinline__ void xmul_column(unsigned t, unsigned items, unsigned
 // registers, one more LDS exchange per transform), and PIPE, the next item's
 // columns loaded before the current one is transformed (twice the data
 // registers) or after.  Lane g of a line holds x = g + (PX / EE) e.  Halves are
-// TuneParams::xv 2 (PIPE) and 3; padded X 192 and 384 take the whole with PIPE: their
-// 180 and 194 registers allow two waves per SIMD with the prefetch or without
-// (233 and 256), so there it costs no waves.  90 x 90 x 90 (padded X 192) 51 us a launch
-// with it, 59 without walking as many items, 50 an item per block; 75 x 270 x 74 136,
-// 163 and 158 us; 133 x 11 x 323 (384) 59, 64 and 52 us.
-constexpr bool xmul_walks(int PX) { return PX == 192 || PX == 384; }
+// TuneParams::xv 2 (PIPE) and 3; padded X 192 takes the whole with PIPE: its 180
+// registers allow two waves per SIMD, the prefetch's 233 as many, so there it costs
+// none.  With it / walking items without it / an item per block: 75 x 270 x 74 136 / 163 /
+// 158 us a launch, 100 x 45 x 78 32 / 36 / 36, 90 x 90 x 90 51 / 59 / 50.  (At 384, where it
+// costs none either, 323 x 11 x 133 59 / 64 / 52 and 90 x 90 x 180 117 / 125 / 111: an item per
+// block.)
+constexpr bool xmul_walks(int PX) { return PX == 192; }
 template <int PX, int EE>
 __device__ __forceinline__ void xmul_load_e(float2 (*v)[EE], const float2* __restrict__ B2, int kz, int ky, int Nx,
                                             int PY, int Q, int g) {

@@ -30,7 +30,7 @@ DESCR = {
     "er": "fused Z inverse rows per block (0 by the grid, 1 half of the length's own, 2 two rows, 3 the length's own); "
           "on grids where it ends with the next stage's Z forward the ms are of both",
     "yb": "3-D Y passes, blocks per CU (both passes)",
-    "xb": "X.K.X pass, blocks per CU where they walk items (padded X 192 and 384, xv 2 and 3)",
+    "xb": "X.K.X pass, blocks per CU where they walk items (padded X 192, xv 2 and 3)",
     "y2b": "2-D Y.K.Y pass, blocks per CU",
     "pp": "3-D plans with padded Y 512, padded X 16/32: 1 = one register-resident plane pass for Y, X.K.X, Y "
           "inverse; 0 = three passes (ms: the passes it replaces)",

@@ -193,8 +193,8 @@ double mm_sim_time_pass(mmSim* s, int cls, int n);
  * (variant 0 by the grid, 1 half of the length's own, 2 double, 3 a quarter, 4
  * the length's own), er: fused Z inverse rows per block (0 by the grid, 1 half, 2
  * two rows, 3 the length's own), yb: blocks per CU of the 3-D Y passes, xb: blocks
- * per CU of the X.K.X pass where they walk items (padded X 192 and 384, xv 2 and
- * 3; the others run an item per block), y2b: blocks per CU of the 2-D Y.K.Y pass, pp: for 3-D
+ * per CU of the X.K.X pass where they walk items (padded X 192, xv 2 and 3; the
+ * others run an item per block), y2b: blocks per CU of the 2-D Y.K.Y pass, pp: for 3-D
  * plans with padded Y 512 and padded X 16 or 32, 1 = Y forward, X.K.X and Y
  * inverse as one register-resident plane pass, 0 = three passes, xv: X.K.X
  * variant for padded X 16-64, 0 and 1 default, 2 half the elements per lane over

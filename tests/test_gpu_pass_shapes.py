@@ -158,7 +158,7 @@ def test_run_to_a_stop_time_in_pieces(mm):
     b.free()
 
 
-# padded X of every X.K.X kernel: an item per block (24 to 128, 256, 512) and walked with a prefetch (192, 384)
+# padded X of every X.K.X kernel: an item per block (24 to 128, 256 to 512) and walked with a prefetch (192)
 @pytest.mark.parametrize("size", [(9, 34, 4), (13, 9, 4), (40, 3, 6), (50, 4, 5), (66, 5, 6), (96, 34, 2), (100, 3, 4),
                                   (130, 6, 5), (192, 9, 3), (200, 4, 4)])
 def test_x_axis_lengths_vs_oracle(mm, orc, size):
